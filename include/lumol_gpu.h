@@ -299,9 +299,11 @@ int lg_mc_run_batch(lg_system* const* systems, size_t count, const uint64_t* see
  *   pair_lanes    lanes per atom in the pair and neighbour-list kernels (4..64;
  *                 16 for systems with a pair potential other than LJ,
  *                 Harmonic and Null, or a table)
- *   kspace_split  row ranges of the k-space force kernel (1..32)
- *   rho_width     atoms per block of the row form of the rho(k) kernel (a
- *                 multiple of 64 up to 512)
+ *   kspace_split  row ranges of the k-space force kernel of the row form
+ *                 (1..32; kmax above 64; no effect on the octant form)
+ *   rho_width     atoms per block of the rho(k) kernel (a multiple of 64 up to
+ *                 512); a quarter of it in the MD kernel that forms rho(k)
+ *                 with the half-steps
  *   nlist_build   neighbour-list build: 1 lanes per atom, 2 one workgroup per
  *                 cell with candidates staged in LDS, 3 direct: workgroups
  *                 per cell over the atoms' cell tags, no cell list (up to
@@ -314,13 +316,10 @@ int lg_mc_run_batch(lg_system* const* systems, size_t count, const uint64_t* see
  *                 launches while a kernel profile is active).  On ROCm 7.0
  *                 the replay measured 4-18% slower than eager launches, so
  *                 it is off by default.
- *   rho_kind      rho(k) kernel: 1 row form (one lane per run of five
- *                 k-vectors, a loop over atoms, the phase rows of a few
- *                 atoms at a time staged in LDS up to kmax 12; the default),
- *                 2 matrix-core form (rho as a complex product over atoms on
- *                 v_mfma 16x16x4; kmax <= 16, else the row form), 3 the row
- *                 form reading the phase rows from the table (no staging;
- *                 the same sums, bit for bit).
+ *   rho_kind      1 (default), 2 or 3: the three forms that earlier versions
+ *                 of rho(k) had.  All run the octant form on the matrix cores
+ *                 now (kmax up to 64, the row form above), with the same bits;
+ *                 the knob is kept for saved choices.
  * lumol_amd.tuning picks them per size bucket by timing the candidates.
  * Results do not depend on them beyond summation order. */
 typedef struct lg_tuning {
@@ -350,11 +349,14 @@ enum {
     LG_KERNEL_PAIRS = 1,        /* k_pairs: LJ + Ewald real space / Wolf, and, in
                                    the FP64 form, the intra-molecular terms (extra
                                    blocks of the same launch)                     */
-    LG_KERNEL_MOLECULES = 2,    /* k_intra_terms: the intra-molecular terms in a
-                                   launch of their own (mixed form)               */
-    LG_KERNEL_KSPACE_RHO = 3,   /* k_rho_partial + k_rho_reduce                  */
-    LG_KERNEL_KSPACE_FORCE = 4, /* k_kspace_force                                */
-    LG_KERNEL_INTEGRATE = 5,    /* integrator halves + thermostat                */
+    LG_KERNEL_MOLECULES = 2,    /* the intra-molecular terms in a launch of their own
+                                   or with the list build (mixed form)            */
+    LG_KERNEL_KSPACE_RHO = 3,   /* rho(k) partials in a launch of their own       */
+    LG_KERNEL_KSPACE_FORCE = 4, /* k-space forces, with the half-steps that follow
+                                   them in MD and the rho(k) partials of the new
+                                   positions                                      */
+    LG_KERNEL_INTEGRATE = 5,    /* integrator halves (with the rho(k) partials of
+                                   the new positions) + thermostat                */
     LG_KERNEL_CLASSES = 6
 };
 typedef struct lg_profile {

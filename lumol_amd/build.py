@@ -12,7 +12,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "liblumol_gpu.so")
 SOURCES = [os.path.join(HERE, "csrc", "lg_api.hip")]
-DEPS = SOURCES + [os.path.join(HERE, "csrc", f) for f in ("lg_device.hpp", "lg_kernels.hpp")] + [
+DEPS = SOURCES + [os.path.join(HERE, "csrc", f) for f in ("lg_device.hpp", "lg_kernels.hpp", "lg_kspace.hpp", "lg_mc.hpp")] + [
     os.path.join(ROOT, "include", "lumol_gpu.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cmath>
 #include <cstring>
@@ -396,11 +397,21 @@ struct lg_system {
     DevBuf<double4> fk;  // k-space partial forces [ksplit][n]
     DevBuf<int4> kidx;
     DevBuf<KRow> rows;
-    DevBuf<KUnit> units;         // rho pass work units (up to 4 k-vectors of a row)
+    // octant form (kmax <= kOctMaxK): (p, q) pairs and their row tiles, work
+    // items of the rho pass, output tiles, k map, force coefficients, partials
+    bool oct = false;
+    int oct_nrt = 0, oct_nst = 0, oct_steps = 0, oct_zcols = 0, oct_nitems = 0, oct_ntiles = 0;
+    int oct_width = 0, oct_nchunks = 0, oct_ngroups = 0, oct_ipg = 0, oct_asplit = 1;
+    int rho_nchunks = 0;  // partial sums of the last rho pass
+    DevBuf<int> opairs, osteps, okmap, omask;
+    DevBuf<OctItem> oitems;
+    DevBuf<int4> oslots, orows32, orows64;
+    DevBuf<float> ocoef32;
+    DevBuf<double> ocoef64;
+    DevBuf<double4> opart;
+    // row form (kmax above it)
+    DevBuf<KUnit> units;         // rho pass work units (up to 5 k-vectors of a row)
     DevBuf<int> kslot;           // k -> slot of the rho partials (j * nunits + unit)
-    // matrix-core rho: column tiles of (iky, ikz), output -> k map, identity slots
-    int mfma_nt = 0;
-    DevBuf<int> mcols, mkmap, kslot_id;
     // erfcx tables of the real-space erfc (empty: library erfc)
     DevBuf<double> ecx64;
     DevBuf<float> ecx32;
@@ -453,10 +464,7 @@ struct lg_system {
     DevBuf<int> mc_cell_count, mc_atom_cell;
     // snapshot for neighbour-list overflow recovery
     DevBuf<double4> snap_pos, snap_vel, snap_acc;
-    // Verlet build deferred by launch_nlist into the rho(k) launch (k_cells_rho)
-    bool cells_pending = false, cells_nearest = false, direct_pending = false;
-    CellsArgs cells_args{};
-    DirectArgs direct_args{};
+    bool intra_done = false;  // launch_nlist ran the intra-molecular terms (k_direct_intra)
     // MD chunk captured as a HIP graph, with what it was captured for
     hipGraphExec_t md_exec = nullptr;
     uint64_t md_key[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -947,45 +955,168 @@ int prepare_params(lg_system* s) {
     return LG_OK;
 }
 
-// ewald.rs:130-183 and :353-378 for an orthorhombic cell
-// Launch shape of the matrix-core rho pass: atoms per stage and tiles per
-// wave, the first candidate with at least 256 blocks (one per CU) -- wider
-// stages and more tiles per wave share more staging and operand work --
-// then stages merged per block so that the grid stays near 1024-2048 blocks
-// and the partials (chunks x k-vectors) few.
-struct RhoShape {
-    int width, wlog, cpb, ngroups, nchunks;
-};
-// dynamic LDS of a matrix-core rho launch: its own, or the Verlet build's
-// when the two share the launch and the buffer
-static size_t rho_mfma_bytes(int width, int kmax, bool mixed) {
-    const size_t r = mixed ? rho_mfma_lds<float>(width, kmax) : rho_mfma_lds<double>(width, kmax);
-    return std::max(r, sizeof(CellsLds));
+// Atoms per block of k_oct_step: the 16-atom groups dealt evenly to one block
+// per CU (256), at most as many as the LDS holds.  One block more than there
+// are CUs would double the time of the kernel, which is bound by the matrix
+// cores of a CU (36 000 atoms: 282 blocks of 128 took 121 us, of which the
+// CUs with one block needed 70).  The rho_width knob sets it to a quarter of
+// its value.
+constexpr size_t kOctLdsMax = 148 * 1024;  // dynamic LDS of a block that has its CU alone (160 KB, 9 KB static)
+constexpr size_t kOctRhoLds = 72 * 1024;   // of a block of the separate rho pass, two per CU
+template <typename T>
+static int oct_step_atoms_t(const lg_system* s) {
+    const int kmax = s->coul_kmax, zc = s->oct_zcols, w = s->tune.rho_width;
+    const int groups = blocks_for(s->n, 16);
+    int g = w > 0 ? w / 64 : (groups + 255) / 256;
+    g = std::min(g, kOctMaxGroups);
+    while (g > 1 && oct_step_lds<T>(kmax, zc, 16 * g) > kOctLdsMax) g--;
+    return 16 * g;
 }
-// Launch shape of the matrix-core rho pass: the widest stage (atoms staged
-// per block: wider shares more staging per k) that still gives at least 256
-// blocks (one per CU) and fits the LDS, then stages merged per block so that
-// the grid stays near 1024-2048 blocks and the partials (chunks x k-vectors)
-// few.
-static RhoShape rho_mfma_shape(const lg_system* s, bool mixed) {
-    // widths 16..128 (FP32) or 16..64 (FP64): the kernel's trips take four
-    // atoms of each of its four sub-waves
-    const int wl0 = mixed ? 7 : 6, wlmin = 4;
-    RhoShape sh{};
-    sh.ngroups = (s->mfma_nt + 2 * kRhoMfmaTpw - 1) / (2 * kRhoMfmaTpw);
-    sh.wlog = wlmin;
-    for (int wl = wl0; wl >= wlmin; wl--) {
-        if (rho_mfma_bytes(1 << wl, s->coul_kmax, mixed) > s->ctx->max_shared) continue;
-        sh.wlog = wl;
-        if (size_t(blocks_for(s->ld, 1 << wl)) * sh.ngroups >= 256) break;
+static int oct_step_atoms(const lg_system* s, bool mixed) {
+    return mixed ? oct_step_atoms_t<float>(s) : oct_step_atoms_t<double>(s);
+}
+// Whether k_oct_step also forms the rho partials: one set per block is
+// written, so beyond 512 blocks the separate pass, with up to 512 atoms per
+// set, takes over.
+static bool oct_step_rho(const lg_system* s, bool mixed) { return blocks_for(s->n, oct_step_atoms(s, mixed)) <= 512; }
+
+// The octant form's tables from the k set (see lg_kspace.hpp): pairs (p, q) =
+// (ikx, |iky|) sorted by how many ikz they need, row tiles of four pairs,
+// work items of four output tiles, and for every output column of a tile the
+// k-vectors it completes.
+static int prepare_octants(lg_system* s, const std::vector<int4>& idx) {
+    std::map<std::pair<int, int>, int> extent;  // pair -> largest |ikz| + 1
+    for (const int4& k : idx) {
+        int& z = extent[{k.x, std::abs(k.y)}];
+        z = std::max(z, std::abs(k.z) + 1);
     }
-    sh.width = 1 << sh.wlog;
-    const int stages = blocks_for(s->ld, sh.width);
-    sh.cpb = std::max(1, int(size_t(stages) * sh.ngroups / 1024));
-    sh.nchunks = (stages + sh.cpb - 1) / sh.cpb;
-    return sh;
+    std::vector<std::array<int, 3>> pairs;  // extent, p, q
+    for (auto& [pq, z] : extent) pairs.push_back({z, pq.first, pq.second});
+    std::stable_sort(pairs.begin(), pairs.end(), [](auto& a, auto& b) { return a[0] > b[0]; });
+    const int nrt = int((pairs.size() + 3) / 4);
+    std::vector<int> opairs(size_t(nrt) * 4, 0), steps(nrt), ncol(nrt);
+    std::map<std::pair<int, int>, int> at;
+    for (size_t j = 0; j < pairs.size(); j++) {
+        opairs[j] = pairs[j][1] | pairs[j][2] << 16;
+        at[{pairs[j][1], pairs[j][2]}] = int(j);
+    }
+    for (int t = 0; t < nrt; t++) {
+        const int z = pairs[size_t(t) * 4][0];
+        ncol[t] = (z + 7) / 8;
+        steps[t] = (z + 1) / 2;
+    }
+    // items: two row tiles x two column tiles while both columns exist, four
+    // row tiles x one column tile for a last odd column; stand-ins repeat a
+    // row tile and own no output tile
+    std::vector<OctItem> items;
+    std::vector<int4> slots;
+    for (int c = 0; c < ncol[0]; c += 2) {
+        std::vector<int> two, one;
+        for (int t = 0; t < nrt; t++) {
+            if (ncol[t] >= c + 2) two.push_back(t);
+            if (ncol[t] == c + 1) one.push_back(t);
+        }
+        const size_t own2 = two.size();
+        if (two.size() % 2 && !one.empty()) {
+            two.push_back(one.front());
+            one.erase(one.begin());
+        }
+        for (size_t j = 0; j < two.size(); j += 2) {
+            const int t0 = two[j], t1 = j + 1 < two.size() ? two[j + 1] : -1;
+            const int slot = 4 * int(items.size());
+            items.push_back(OctItem{{t0, std::max(t1, 0), 0, 0}, c, 0});
+            slots.push_back(make_int4(slot, t0, c, 0));
+            slots.push_back(make_int4(slot + 1, t0, c + 1, 0));
+            if (t1 >= 0) slots.push_back(make_int4(slot + 2, t1, c, 0));
+            if (t1 >= 0 && j + 1 < own2) slots.push_back(make_int4(slot + 3, t1, c + 1, 0));
+        }
+        for (size_t j = 0; j < one.size(); j += 4) {
+            OctItem it{{0, 0, 0, 0}, c, 1};
+            const int slot = 4 * int(items.size());
+            for (size_t u = 0; u < 4 && j + u < one.size(); u++) {
+                it.rt[u] = one[j + u];
+                slots.push_back(make_int4(slot + int(u), one[j + u], c, 0));
+            }
+            items.push_back(it);
+        }
+    }
+    std::vector<int> tile_of(size_t(nrt) * ncol[0], -1);  // (row tile, column tile) -> output tile
+    for (size_t e = 0; e < slots.size(); e++) tile_of[size_t(slots[e].y) * ncol[0] + slots[e].z] = int(e);
+    std::vector<int> kmap(slots.size() * 4 * 16 * 2, -1);
+    for (size_t k = 0; k < idx.size(); k++) {
+        const int j = at[{idx[k].x, std::abs(idx[k].y)}], r = std::abs(idx[k].z);
+        const int e = tile_of[size_t(j / 4) * ncol[0] + r / 8];
+        const int col = 2 * (r % 8) + (idx[k].z < 0 ? 1 : 0);
+        kmap[((size_t(e) * 4 + j % 4) * 16 + col) * 2 + (idx[k].y < 0 ? 1 : 0)] = int(k);
+    }
+    // the X and Y phase rows of every matrix row of an item (see OctRho)
+    const int K1 = s->coul_kmax + 1;
+    std::vector<int4> rows32, rows64;
+    for (const OctItem& it : items)
+        for (int i = 0; i < 16; i++) {
+            auto row = [&](int u, int pair, int ab) {
+                const int pk = opairs[size_t(it.rt[u]) * 4 + pair];
+                return (2 * (pk & 0xffff) + (ab >> 1)) | (2 * K1 + 2 * (pk >> 16) + (ab & 1)) << 16;
+            };
+            auto rows = [&](int pair, int ab) {
+                return make_int4(row(0, pair, ab), row(1, pair, ab), row(2, pair, ab), row(3, pair, ab));
+            };
+            rows32.push_back(rows(i >> 2, i & 3));  // OctT<float>::row_of
+            rows64.push_back(rows(i & 3, i >> 2));  // OctT<double>::row_of
+        }
+    // what a lane of an output tile has to store: the columns r below its
+    // pair's extent, of the tiles that are owned
+    std::vector<int> mask(items.size() * 64, 0);
+    for (const int4& sl : slots)
+        for (int l = 0; l < 64; l++) {
+            const size_t j = size_t(sl.y) * 4 + l / 16;
+            if (j < pairs.size() && sl.z * 8 + (l % 16) / 2 < pairs[j][0]) mask[size_t(sl.x / 4) * 64 + l] |= 1 << (sl.x % 4);
+        }
+    s->oct_nrt = nrt;
+    s->oct_zcols = 16 * ncol[0];
+    s->oct_nst = 4 * ncol[0];
+    s->oct_steps = steps[0];  // of the longest row
+    s->oct_nitems = int(items.size());
+    s->oct_ntiles = int(slots.size());
+    // about one block per CU: the widest chunk of atoms (fewer partial sums),
+    // then fewer items per block (their waves share the atoms), then narrower
+    // chunks
+    const int nitems = int(items.size());
+    int ng = blocks_for(nitems, 8), w = 512;
+    auto blocks = [&]() { return ng * blocks_for(s->n, w); };
+    while (w > 128 && blocks() < 200) w -= 64;
+    while (ng < nitems && 2 * ng <= blocks_for(nitems, 2) && blocks() < 128) ng *= 2;
+    while (w > 64 && blocks() < 128) w -= 64;
+    if (s->tune.rho_width > 0) w = s->tune.rho_width;
+    s->oct_ipg = blocks_for(nitems, ng);
+    s->oct_ngroups = blocks_for(nitems, s->oct_ipg);
+    s->oct_asplit = 8 / s->oct_ipg;
+    s->oct_width = w;
+    s->oct_nchunks = blocks_for(s->n, w);
+    hipStream_t st = S(s);
+    LG_TRY(upload(s->opairs, opairs, st));
+    LG_TRY(upload(s->osteps, steps, st));
+    LG_TRY(upload(s->okmap, kmap, st));
+    LG_TRY(upload(s->oitems, items, st));
+    LG_TRY(upload(s->oslots, slots, st));
+    LG_TRY(upload(s->omask, mask, st));
+    LG_TRY(upload(s->orows32, rows32, st));
+    LG_TRY(upload(s->orows64, rows64, st));
+    const std::vector<double> zero(size_t(nrt) * s->oct_nst * 64, 0.0);
+    LG_TRY(upload(s->ocoef64, zero, st));
+    LG_TRY(upload(s->ocoef32, std::vector<float>(zero.size(), 0.f), st));
+    size_t sets = size_t(s->oct_nchunks);
+    for (int m = 0; m < 2; m++)
+        if (oct_step_rho(s, m == 1)) sets = std::max(sets, size_t(blocks_for(s->n, oct_step_atoms(s, m == 1))));
+    LG_TRY(s->opart.ensure(sets * 4 * s->oct_nitems * 64));
+    LG_TRY(s->epart_k.ensure(size_t(s->oct_ntiles) * 4 * 7));
+    s->ksplit = s->tune.kspace_split > 0 ? s->tune.kspace_split : 8;
+    LG_TRY(s->fk.ensure(s->n));
+    LG_HIP(hipStreamSynchronize(st));  // the tables above are local
+    return LG_OK;
 }
 
+// ewald.rs:130-183 and :353-378 for an orthorhombic cell
 int prepare_kspace(lg_system* s) {
     s->kspace_dirty = false;
     s->nk = 0;
@@ -1039,6 +1170,17 @@ int prepare_kspace(lg_system* s) {
         for (int z = -kmax; z < kmax; z++) push(0, y, z);
     for (int z = 1; z < kmax; z++) push(0, 0, z);
     s->nk = int(idx.size());
+    for (int d = 0; d < 3; d++) s->kg[d] = 2.0 * kPi * inv[d];
+    std::vector<double> vflat;
+    for (int q = 0; q < 6; q++) vflat.insert(vflat.end(), vf[q].begin(), vf[q].end());
+    hipStream_t st = S(s);
+    LG_TRY(upload(s->kidx, idx, st));
+    LG_TRY(upload(s->efac, efac, st));
+    LG_TRY(upload(s->vfac, vflat, st));
+    LG_TRY(s->rho.ensure(s->nk));
+    if (kmax > 1000) return fail(LG_E_UNSUPPORTED, "kmax too large");
+    s->oct = kmax <= kOctMaxK && s->nk > 0;
+    if (s->oct) return prepare_octants(s, idx);
     std::vector<KRow> rows;
     for (int k = 0; k < s->nk; k++) {
         if (rows.empty() || rows.back().ikx != idx[k].x || rows.back().iky != idx[k].y ||
@@ -1056,48 +1198,14 @@ int prepare_kspace(lg_system* s) {
     std::vector<int> kslot(s->nk);
     for (int u = 0; u < s->nunits; u++)
         for (int j = 0; j < units[u].nv; j++) kslot[units[u].kb + j] = j * s->nunits + u;
-    for (int d = 0; d < 3; d++) s->kg[d] = 2.0 * kPi * inv[d];
-    // matrix-core rho: distinct (iky, ikz) columns in tiles of 16; rows ikx
-    // 0..15 cover the set when kmax <= 16
-    std::vector<int> mcols, mkmap, kid(s->nk);
-    s->mfma_nt = 0;
-    if (kmax <= 16) {
-        std::vector<std::pair<int, int>> cl;
-        for (int k = 0; k < s->nk; k++) cl.push_back({idx[k].y, idx[k].z});
-        std::sort(cl.begin(), cl.end());
-        cl.erase(std::unique(cl.begin(), cl.end()), cl.end());
-        const int nt = int((cl.size() + 15) / 16);
-        mcols.assign(size_t(nt) * 16, (kmax << 16) | kmax);
-        for (size_t j = 0; j < cl.size(); j++) mcols[j] = ((cl[j].first + kmax) << 16) | (cl[j].second + kmax);
-        mkmap.assign(size_t(nt) * 256, -1);
-        for (int k = 0; k < s->nk; k++) {
-            int j = int(std::lower_bound(cl.begin(), cl.end(), std::make_pair(idx[k].y, idx[k].z)) - cl.begin());
-            mkmap[size_t(j / 16) * 256 + idx[k].x * 16 + j % 16] = k;
-        }
-        s->mfma_nt = nt;
-    }
-    for (int k = 0; k < s->nk; k++) kid[k] = k;
-    std::vector<double> vflat;
-    for (int q = 0; q < 6; q++) vflat.insert(vflat.end(), vf[q].begin(), vf[q].end());
-    hipStream_t st = S(s);
-    LG_TRY(upload(s->kidx, idx, st));
     LG_TRY(upload(s->rows, rows, st));
     LG_TRY(upload(s->units, units, st));
     LG_TRY(upload(s->kslot, kslot, st));
-    if (s->mfma_nt > 0) {
-        LG_TRY(upload(s->mcols, mcols, st));
-        LG_TRY(upload(s->mkmap, mkmap, st));
-        LG_TRY(upload(s->kslot_id, kid, st));
-    }
-    LG_TRY(upload(s->efac, efac, st));
-    LG_TRY(upload(s->vfac, vflat, st));
     LG_TRY(upload(s->krec, rec, st));
     std::vector<KRec32> r32(rec.size());
     for (size_t k = 0; k < rec.size(); k++)
         r32[k] = KRec32{0.f, 0.f, float(rec[k].g), float(rec[k].gz)};
     LG_TRY(upload(s->krec32, r32, st));
-    LG_TRY(s->rho.ensure(s->nk));
-    if (kmax > 1000) return fail(LG_E_UNSUPPORTED, "kmax too large");
     // enough waves to fill the device (~4096: 64 atoms x 4 waves per block,
     // grid.y row splits), with as few force partials as that allows
     int fwaves = 4 * blocks_for(s->n, 64);
@@ -1105,15 +1213,9 @@ int prepare_kspace(lg_system* s) {
     if (s->tune.kspace_split > 0) s->ksplit = std::min(s->tune.kspace_split, std::max(1, s->nrows));
     LG_TRY(s->fk.ensure(size_t(s->ksplit) * s->n));
     s->ld = blocks_for(s->n, 64) * 64;
-    // rho partials: the row form's narrowest atom chunk (64) or the
-    // matrix-core form's chunks, whichever needs more
-    size_t npart = size_t(blocks_for(s->ld, 64)) * kRhoUnitK * s->nunits;
-    if (s->mfma_nt > 0)
-        for (int m = 0; m < 2; m++) npart = std::max(npart, size_t(rho_mfma_shape(s, m == 1).nchunks) * s->nk);
-    LG_TRY(s->rho_partial.ensure(npart));
-    // the staged row kernel loads kRhoStageRows rows per round (the rows
-    // past the phase rows are loaded and not used)
-    const size_t trows = size_t(std::max(phase_rows(kmax), kRhoStageRows));
+    // rho partials of the narrowest atom chunk (64)
+    LG_TRY(s->rho_partial.ensure(size_t(blocks_for(s->ld, 64)) * kRhoUnitK * s->nunits));
+    const size_t trows = size_t(phase_rows(kmax));
     LG_TRY(s->phase_tab.ensure(trows * s->ld));
     LG_TRY(s->phase_q.ensure(s->ld));
     LG_TRY(s->phase_tab32.ensure(trows * s->ld));
@@ -1269,15 +1371,21 @@ static CellTag cell_tags(lg_system* s) {
     return CellTag{direct_build(s) ? s->cellid.p : nullptr, s->grid, s->box,
                    s->precision == LG_PRECISION_MIXED ? s->frac.p : nullptr, s->frac_origin};
 }
+static MdArgs md_args(lg_system* s) {
+    const double hs = 0.5 * s->skin;
+    return MdArgs{s->pos.p, s->vel.p, s->acc.p, int(s->n), s->integrator != LG_INTEGRATOR_VELOCITY_VERLET ? 1 : 0,
+                  s->dt, s->ref.p, hs * hs, s->flags.p, cell_tags(s)};
+}
 // Workgroups per cell of the direct build: about 256 workgroups in all (one
 // per CU of the MI355X), at most 8 per cell.
 static int direct_split(const lg_system* s) { return std::max(1, std::min(8, 256 / std::max(1, s->grid.ncell))); }
 static int direct_blocks(const lg_system* s) { return s->grid.ncell * direct_split(s); }
 
-// Atoms per block of the rho pass: the narrowest chunk (64..512) that keeps
-// the grid at or below ~2048 blocks, so that per-block work stays
+// Atoms per block of the rho pass.  Row form: the narrowest chunk (64..512)
+// that keeps the grid at or below ~2048 blocks, so that per-block work stays
 // substantial while the partials stay few; the tuning knob overrides.
 static int rho_chunk(const lg_system* s) {
+    if (s->oct) return s->oct_width;
     if (s->tune.rho_width > 0) return s->tune.rho_width;
     int nub = blocks_for(s->nunits, 64);
     int w = 64;
@@ -1285,14 +1393,94 @@ static int rho_chunk(const lg_system* s) {
     return w;
 }
 
-// The matrix-core rho form when asked for (rho_kind 2; the row form is the
-// default: it measured as fast or faster on the bench systems), kmax <= 16
-// and its LDS (the larger of its own and the Verlet build's, which share a
-// launch) within the device limit.
-static bool rho_use_mfma(const lg_system* s, bool mixed) {
-    if (s->mfma_nt <= 0 || s->tune.rho_kind != 2) return false;
-    const RhoShape sh = rho_mfma_shape(s, mixed);
-    return rho_mfma_bytes(sh.width, s->coul_kmax, mixed) <= s->ctx->max_shared;
+// Blocks of the rho(k) reduction (and of its energy partials).
+static int kspace_reduce_blocks(const lg_system* s) {
+    if (s->coul_kind != COUL_EWALD || s->nk <= 0) return 0;
+    return s->oct ? 4 * s->oct_ntiles : blocks_for(s->nk, kRhoReduceK);
+}
+
+// Arguments of the octant rho pass.
+static OctRho oct_rho_args(const lg_system* s, bool mixed) {
+    OctRho a{};
+    for (int d = 0; d < 3; d++) a.inv[d] = s->box.inv[d];
+    a.kmax = s->coul_kmax;
+    a.zcols = s->oct_zcols;
+    a.items = s->oitems.p;
+    a.rows = mixed ? s->orows32.p : s->orows64.p;
+    a.mask = s->omask.p;
+    a.nitems = s->oct_nitems;
+    a.ngroups = s->oct_ngroups;
+    a.ipg = s->oct_ipg;
+    a.asplit = s->oct_asplit;
+    a.nchunks = s->oct_nchunks;
+    a.width = s->oct_width;
+    a.partial = s->opart.p;
+    return a;
+}
+template <typename T>
+static void launch_rho_oct(lg_system* s, const OctRho& ra, int grid) {
+    int sa = std::min(128, ra.width);
+    while (sa > 16 && oct_lds<T>(ra.kmax, ra.zcols, sa) > kOctRhoLds) sa -= 16;
+    const size_t lds = std::max(kOctRed, oct_lds<T>(ra.kmax, ra.zcols, sa));
+    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_rho_oct<T>, grid, 512, uint32_t(lds), ra, sa, s->pos.p, int(s->n));
+}
+
+// k_oct_step: NST by the steps of the longest row (0 above eight steps).
+template <typename T, int NST>
+static void launch_oct_step_c(lg_system* s, int cls, const OctForce& a, const OctStep& st, const OctRho& ra, int c) {
+    launch_timed(s, cls, k_oct_step<T, NST>, blocks_for(s->n, c), 512, uint32_t(oct_step_lds<T>(ra.kmax, ra.zcols, c)),
+                 a, st, ra, c);
+}
+template <typename T>
+static void launch_oct_step_t(lg_system* s, int cls, const OctForce& a, const OctStep& st, const OctRho& ra, int c) {
+    // an instance reads NST steps of every row tile, which holds oct_nst =
+    // 4 ceil(extent / 8) of them: 4 for at most 4 steps, 8 for 5 to 8
+    if (s->oct_steps <= 4)
+        launch_oct_step_c<T, 4>(s, cls, a, st, ra, c);
+    else if (s->oct_steps <= 5)
+        launch_oct_step_c<T, 5>(s, cls, a, st, ra, c);
+    else if (s->oct_steps <= 8)
+        launch_oct_step_c<T, 8>(s, cls, a, st, ra, c);
+    else
+        launch_oct_step_c<T, 0>(s, cls, a, st, ra, c);
+}
+// Kinetic-energy partials of k_oct_step: one per wave of atoms.
+static int oct_ke_parts(const lg_system* s) {
+    const int c = oct_step_atoms(s, s->precision == LG_PRECISION_MIXED);
+    return blocks_for(s->n, c) * ((c + 63) / 64);
+}
+static void launch_oct_step(lg_system* s, int what, int then, double* ke_part, const Thermo& th) {
+    const bool mixed = s->precision == LG_PRECISION_MIXED;
+    const int c = oct_step_atoms(s, mixed);
+    OctForce a{};
+    for (int d = 0; d < 3; d++) a.kg[d] = s->kg[d];
+    a.coef = mixed ? static_cast<const void*>(s->ocoef32.p) : static_cast<const void*>(s->ocoef64.p);
+    a.pairs = s->opairs.p;
+    a.steps = s->osteps.p;
+    a.nrt = s->oct_nrt;
+    a.nst = s->oct_nst;
+    OctRho ra = oct_rho_args(s, mixed);
+    ra.ngroups = blocks_for(s->oct_nitems, 8);
+    ra.ipg = blocks_for(s->oct_nitems, ra.ngroups);
+    ra.asplit = 8 / ra.ipg;
+    ra.width = c;
+    ra.nchunks = blocks_for(s->n, c);
+    if (what & OCT_RHO) s->rho_nchunks = ra.nchunks;
+    OctStep st{};
+    st.what = what;
+    st.then = then;
+    st.force = s->force.p;
+    st.contrib = s->contrib.p;
+    st.slot_start = s->nterms > 0 ? s->slot_start.p : nullptr;
+    st.fk = then == OCT_COMBINE ? s->fk.p : nullptr;
+    st.ke_part = ke_part;
+    st.m = md_args(s);
+    st.th = th;
+    const int cls = (what & OCT_FORCE) ? LG_KERNEL_KSPACE_FORCE : LG_KERNEL_INTEGRATE;
+    if (mixed)
+        launch_oct_step_t<float>(s, cls, a, st, ra, c);
+    else
+        launch_oct_step_t<double>(s, cls, a, st, ra, c);
 }
 
 // The next force evaluation rebuilds the list whatever the displacements.
@@ -1302,8 +1490,34 @@ static int force_rebuild(lg_system* s) {
     return LG_OK;
 }
 
-int launch_nlist(lg_system* s, bool check) {
+// The arguments of the intra-molecular terms (k_intra_terms, or blocks of
+// another launch).
+static IntraArgs intra_args(lg_system* s) {
+    IntraArgs ia{};
+    ia.pos = s->pos.p;
+    ia.meta = s->meta.p;
+    ia.nterms = s->nterms;
+    ia.terms = s->terms.p;
+    ia.table = s->table.p;
+    ia.tabs = s->ptabs.p;
+    ia.nkinds = int(s->nkinds);
+    ia.pair_restr = s->pair_restr.p;
+    ia.pair_s14 = s->pair_s14.p;
+    ia.bparam = s->bparam.p;
+    ia.aparam = s->aparam.p;
+    ia.dparam = s->dparam.p;
+    ia.coul = s->coul;
+    ia.coul_restr = s->coul_restr;
+    ia.coul_s14 = s->coul_s14;
+    ia.box = s->box;
+    ia.contrib = s->contrib.p;
+    ia.epart = s->ep_mol_at ? s->ep_mol_at : s->epart_mol.p;
+    return ia;
+}
+
+int launch_nlist(lg_system* s, bool check, bool energy) {
     hipStream_t st = S(s);
+    s->intra_done = false;
     // profiled intervals only around launches (an empty event pair would
     // count the event packets' own dispatch as list time)
     long prof = -1;
@@ -1325,11 +1539,16 @@ int launch_nlist(lg_system* s, bool check) {
                       s->nbr.p, s->nnbr.p, s->ref.p, s->sorted.p, flag, direct_split(s)};
         const bool nearest = s->periodic && (g.reach[0] == 0 || g.reach[1] == 0 || g.reach[2] == 0);
         prof_stop(s, prof);
-        if (s->coul_kind == COUL_EWALD && s->nk > 0) {
-            // launched by launch_forces together with the rho(k) partials
-            s->direct_pending = true;
-            s->cells_nearest = nearest;
-            s->direct_args = da;
+        // mixed form, forces only: the intra-molecular terms ride as the last
+        // blocks of this launch, which most steps leave empty
+        s->intra_done = !energy && s->precision == LG_PRECISION_MIXED && !s->gen_pairs && s->nterms > 0;
+        if (s->intra_done) {
+            const int ncb = direct_blocks(s), fib = blocks_for(s->nterms, kCellBlock);
+            auto go = [&](auto kernel) {
+                launch_timed(s, LG_KERNEL_MOLECULES, kernel, ncb + fib, kCellBlock, 0, da, ncb, intra_args(s));
+            };
+            if (nearest) go(k_direct_intra<true>);
+            else go(k_direct_intra<false>);
             return LG_OK;
         }
         long p2 = prof_start(s, LG_KERNEL_NLIST);
@@ -1364,13 +1583,6 @@ int launch_nlist(lg_system* s, bool check) {
                      s->nbr.p, s->nnbr.p, s->pos.p, s->ref.p, flag};
         const bool nearest = s->periodic && (g.reach[0] == 0 || g.reach[1] == 0 || g.reach[2] == 0);
         prof_stop(s, prof);
-        if (s->coul_kind == COUL_EWALD && s->nk > 0) {
-            // launched by launch_forces together with the rho(k) partials
-            s->cells_pending = true;
-            s->cells_nearest = nearest;
-            s->cells_args = ca;
-            return LG_OK;
-        }
         long p2 = prof_start(s, LG_KERNEL_NLIST);
         if (nearest)
             k_nlist_cells<true><<<g.ncell, kCellBlock, 0, st>>>(ca);
@@ -1401,165 +1613,43 @@ int launch_nlist(lg_system* s, bool check) {
     return LG_OK;
 }
 
-// The arguments of the intra-molecular terms (k_intra_terms, or blocks of
-// another launch).
-static IntraArgs intra_args(lg_system* s) {
-    IntraArgs ia{};
-    ia.pos = s->pos.p;
-    ia.meta = s->meta.p;
-    ia.nterms = s->nterms;
-    ia.terms = s->terms.p;
-    ia.table = s->table.p;
-    ia.tabs = s->ptabs.p;
-    ia.nkinds = int(s->nkinds);
-    ia.pair_restr = s->pair_restr.p;
-    ia.pair_s14 = s->pair_s14.p;
-    ia.bparam = s->bparam.p;
-    ia.aparam = s->aparam.p;
-    ia.dparam = s->dparam.p;
-    ia.coul = s->coul;
-    ia.coul_restr = s->coul_restr;
-    ia.coul_s14 = s->coul_s14;
-    ia.box = s->box;
-    ia.contrib = s->contrib.p;
-    ia.epart = s->ep_mol_at ? s->ep_mol_at : s->epart_mol.p;
-    return ia;
-}
-
-// phase_done: the MD first half-step has already written the phase table
-// and the FP32 positions (frac) of the current positions.
-int launch_forces(lg_system* s, bool energy, bool combine = true, bool phase_done = false) {
+// frac_done: the MD first half-step has already written the FP32 positions
+// (frac) of the current positions.  rho_done: and their rho(k) partials.
+int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done = false, bool rho_done = false) {
     hipStream_t st = S(s);
     int n = int(s->n);
     bool mixed = s->precision == LG_PRECISION_MIXED;
+    const bool kspace = s->coul_kind == COUL_EWALD && s->nk > 0;
+    const bool oct = kspace && s->oct;
     // rho(k) partials first: their reduction runs as the last blocks of the
     // pair launch, and the k-space forces after it
     int nchunks = 0;
-    const bool use_mfma = s->coul_kind == COUL_EWALD && s->nk > 0 && rho_use_mfma(s, mixed);
-    // mixed form, forces only: the intra-molecular terms ride as the last
-    // blocks of the direct-build list-and-rho launch (its 64 KB of LDS hold
-    // it to 4 waves per SIMD, which the terms' 104 VGPRs do not lower)
-    const bool intra_fused = mixed && !energy && !s->gen_pairs && s->nterms > 0 && s->coul_kind == COUL_EWALD &&
-                             s->nk > 0 && !use_mfma && s->direct_pending;
-    const IntraArgs fia = intra_fused ? intra_args(s) : IntraArgs{};
-    const int fib = intra_fused ? blocks_for(s->nterms, kCellBlock) : 0;
-    if (s->coul_kind == COUL_EWALD && s->nk > 0) {
-        int kmax = s->coul_kmax;
-        int nub = blocks_for(s->nunits, 64);
-        int w = rho_chunk(s);
-        nchunks = blocks_for(s->ld, w);
-        unsigned grid = xcd_grid(nub, nchunks);
-        // with a deferred Verlet build: one launch of k_cells_rho, the list
-        // blocks first (cells rounded up to 8), then the rho blocks
-        const bool direct = s->direct_pending;
-        const bool cells = s->cells_pending || direct;
-        const int ncb = cells ? ((direct ? direct_blocks(s) : s->grid.ncell) + 7) / 8 * 8 : 0;
-        const CellsArgs& ca = s->cells_args;
-        const DirectArgs& da = s->direct_args;
-        const bool near = s->cells_nearest;
-        if (use_mfma) {
-            // the matrix-core rho shares its launch with the cell-list build
-            // only; a direct build runs first on its own
-            if (direct && near)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_nlist_direct<true>, direct_blocks(s), kCellBlock, 0, da);
-            else if (direct)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_nlist_direct<false>, direct_blocks(s), kCellBlock, 0, da);
-            const bool cells = s->cells_pending;
-            const RhoShape sh = rho_mfma_shape(s, mixed);
-            nchunks = sh.nchunks;
-            const unsigned mgrid = xcd_grid(sh.ngroups, sh.nchunks);
-            if (mixed) {
-                if (!phase_done)
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_phase32, blocks_for(size_t(3) * s->ld, 256), 256, 0, s->pos.p, n, s->ld, s->box, kmax,
-                                                                                  s->phase_tab32.p, s->phase_q32.p);
-                RhoMfmaArgs<float, float2> ra{s->pos.p, n, s->box, s->ld, kmax, sh.wlog, sh.cpb,
-                                              s->mfma_nt, sh.ngroups, sh.nchunks, s->mcols.p, s->mkmap.p, s->nk,
-                                              s->rho_partial.p};
-                const size_t lds = rho_mfma_bytes(sh.width, kmax, true);
-                if (!cells)
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_rho_mfma<float, float2>, mgrid, 512, lds, ra);
-                else if (near)
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_cells_rho_mfma<true, float, float2>, ncb + mgrid, kCellBlock, lds, ca, ra, ncb);
-                else
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_cells_rho_mfma<false, float, float2>, ncb + mgrid, kCellBlock, lds, ca, ra, ncb);
-            } else {
-                if (!phase_done)
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_phase, blocks_for(size_t(3) * s->ld, 256), 256, 0, s->pos.p, n, s->ld, s->box, kmax,
-                                                                                s->phase_tab.p, s->phase_q.p);
-                RhoMfmaArgs<double, double2> ra{s->pos.p, n, s->box, s->ld, kmax, sh.wlog, sh.cpb,
-                                                s->mfma_nt, sh.ngroups, sh.nchunks, s->mcols.p, s->mkmap.p, s->nk,
-                                                s->rho_partial.p};
-                const size_t lds = rho_mfma_bytes(sh.width, kmax, false);
-                if (!cells)
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_rho_mfma<double, double2>, mgrid, 512, lds, ra);
-                else if (near)
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_cells_rho_mfma<true, double, double2>, ncb + mgrid, kCellBlock, lds, ca, ra, ncb);
-                else
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_cells_rho_mfma<false, double, double2>, ncb + mgrid, kCellBlock, lds, ca, ra, ncb);
-            }
-        } else if (mixed) {
-            if (!phase_done)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_phase32, blocks_for(size_t(3) * s->ld, 256), 256, 0, s->pos.p, n, s->ld, s->box, kmax,
-                                                                              s->phase_tab32.p, s->phase_q32.p);
-            RhoRowsArgs<float, float2> ra{s->phase_tab32.p, s->phase_q32.p, s->ld, kmax, w, s->units.p,
-                                          s->nunits, s->rho_partial.p, nub, nchunks, s->tune.rho_kind != 3};
-            if (!cells)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_rho_rows<float, float2>, grid, 512, 0, ra);
-            else if (direct && near) {
-                if (fib > 0)
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_direct_rho<true, float, float2, true>, ncb + grid + fib,
-                                 kCellBlock, 0, da, ra, ncb, int(grid), fia);
-                else
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_direct_rho<true, float, float2, false>, ncb + grid,
-                                 kCellBlock, 0, da, ra, ncb, int(grid), fia);
-            }
-            else if (direct) {
-                if (fib > 0)
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_direct_rho<false, float, float2, true>, ncb + grid + fib,
-                                 kCellBlock, 0, da, ra, ncb, int(grid), fia);
-                else
-                    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_direct_rho<false, float, float2, false>, ncb + grid,
-                                 kCellBlock, 0, da, ra, ncb, int(grid), fia);
-            }
-            else if (near)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_cells_rho<true, float, float2>, ncb + grid, kCellBlock, 0, ca, ra, ncb);
-            else
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_cells_rho<false, float, float2>, ncb + grid, kCellBlock, 0, ca, ra, ncb);
-        } else {
-            if (!phase_done)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_phase, blocks_for(size_t(3) * s->ld, 256), 256, 0, s->pos.p, n, s->ld, s->box, kmax,
-                                                                            s->phase_tab.p, s->phase_q.p);
-            RhoRowsArgs<double, double2> ra{s->phase_tab.p, s->phase_q.p, s->ld, kmax, w, s->units.p,
-                                            s->nunits, s->rho_partial.p, nub, nchunks, s->tune.rho_kind != 3};
-            if (!cells)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_rho_rows<double, double2>, grid, 512, 0, ra);
-            else if (direct && near)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_direct_rho<true, double, double2>, ncb + grid, kCellBlock, 0, da, ra,
-                             ncb, int(grid), IntraArgs{});
-            else if (direct)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_direct_rho<false, double, double2>, ncb + grid, kCellBlock, 0, da, ra,
-                             ncb, int(grid), IntraArgs{});
-            else if (near)
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_cells_rho<true, double, double2>, ncb + grid, kCellBlock, 0, ca, ra, ncb);
-            else
-                launch_timed(s, LG_KERNEL_KSPACE_RHO, k_cells_rho<false, double, double2>, ncb + grid, kCellBlock, 0, ca, ra, ncb);
+    if (oct) {
+        if (!rho_done) {
+            const OctRho ra = oct_rho_args(s, mixed);
+            const int grid = int(xcd_grid(ra.ngroups, ra.nchunks));
+            s->rho_nchunks = ra.nchunks;
+            if (mixed) launch_rho_oct<float>(s, ra, grid);
+            else launch_rho_oct<double>(s, ra, grid);
         }
-        s->cells_pending = false;
-        s->direct_pending = false;
-    }
-    if (s->cells_pending) {  // deferred build without k-space (not expected): launch it alone
-        if (s->cells_nearest)
-            k_nlist_cells<true><<<s->grid.ncell, kCellBlock, 0, st>>>(s->cells_args);
-        else
-            k_nlist_cells<false><<<s->grid.ncell, kCellBlock, 0, st>>>(s->cells_args);
-        s->cells_pending = false;
-    }
-    if (s->direct_pending) {
-        if (s->cells_nearest)
-            k_nlist_direct<true><<<direct_blocks(s), kCellBlock, 0, st>>>(s->direct_args);
-        else
-            k_nlist_direct<false><<<direct_blocks(s), kCellBlock, 0, st>>>(s->direct_args);
-        s->direct_pending = false;
+        nchunks = s->rho_nchunks;
+    } else if (kspace) {
+        const int kmax = s->coul_kmax, nub = blocks_for(s->nunits, 64), w = rho_chunk(s);
+        nchunks = blocks_for(s->ld, w);
+        const unsigned grid = xcd_grid(nub, nchunks);
+        if (mixed) {
+            launch_timed(s, LG_KERNEL_KSPACE_RHO, k_phase32, blocks_for(size_t(3) * s->ld, 256), 256, 0, s->pos.p, n,
+                         s->ld, s->box, kmax, s->phase_tab32.p, s->phase_q32.p);
+            RhoRowsArgs<float, float2> ra{s->phase_tab32.p, s->phase_q32.p, s->ld, kmax, w, s->units.p,
+                                          s->nunits, s->rho_partial.p, nub, nchunks};
+            launch_timed(s, LG_KERNEL_KSPACE_RHO, k_rho_rows<float, float2>, grid, 512, 0, ra);
+        } else {
+            launch_timed(s, LG_KERNEL_KSPACE_RHO, k_phase, blocks_for(size_t(3) * s->ld, 256), 256, 0, s->pos.p, n,
+                         s->ld, s->box, kmax, s->phase_tab.p, s->phase_q.p);
+            RhoRowsArgs<double, double2> ra{s->phase_tab.p, s->phase_q.p, s->ld, kmax, w, s->units.p,
+                                            s->nunits, s->rho_partial.p, nub, nchunks};
+            launch_timed(s, LG_KERNEL_KSPACE_RHO, k_rho_rows<double, double2>, grid, 512, 0, ra);
+        }
     }
     PairArgs pa{};
     pa.pos = s->pos.p;
@@ -1583,41 +1673,55 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool phase_don
     pa.hf32 = s->hf_ok ? s->hf32.p : nullptr;
     pa.hf_inv_h = s->hf_inv_h;
     pa.frac = s->frac.p;
-    if (mixed && !s->gen_pairs && !phase_done) {
+    if (mixed && !s->gen_pairs && !frac_done) {
         // the MD half-steps write the FP32 positions beside the new ones;
         // any other caller converts the current positions here
         launch_timed(s, LG_KERNEL_PAIRS, k_frac, blocks_for(n, 256), 256, 0, s->pos.p, n, s->box, s->frac_origin,
                      s->frac.p);
     }
     // the intra-molecular terms run as the last blocks of the pair launch
-    // (FP64 form), of the list-and-rho launch (mixed form, forces only,
-    // direct build: intra_fused) or in a launch of their own
+    // (FP64 form), of the list launch (mixed form, forces only, direct build:
+    // intra_done) or in a launch of their own
     IntraArgs& ia = pa.intra;
     ia = intra_args(s);
     const int iblocks = s->nterms > 0 ? blocks_for(s->nterms, 256) : 0;
     // rho(k) reduction blocks
-    const bool kspace = s->coul_kind == COUL_EWALD && s->nk > 0;
-    RhoReduceArgs& rr = pa.rr;
-    rr = RhoReduceArgs{};
-    int rblocks = 0;
-    if (kspace) {
+    const int rblocks = kspace_reduce_blocks(s);
+    double* const epk = s->ep_k_at ? s->ep_k_at : s->epart_k.p;
+    pa.oct = oct;
+    if (oct) {
+        OctReduce& rr = pa.orr;
+        rr.partial = s->opart.p;
+        rr.nchunks = nchunks;
+        rr.nslots = 4 * s->oct_nitems;
+        rr.slots = s->oslots.p;
+        rr.kmap = s->okmap.p;
+        rr.nk = s->nk;
+        rr.nst = s->oct_nst;
+        rr.rho = s->rho.p;
+        rr.efac = s->efac.p;
+        rr.vfac = s->vfac.p;
+        rr.epart = epk;
+        rr.coef32 = mixed ? s->ocoef32.p : nullptr;
+        rr.coef64 = mixed ? nullptr : s->ocoef64.p;
+    } else if (kspace) {
+        RhoReduceArgs& rr = pa.rr;
         rr.partial = s->rho_partial.p;
         rr.nchunks = nchunks;
-        rr.nslot = use_mfma ? s->nk : kRhoUnitK * s->nunits;
-        rr.kslot = use_mfma ? s->kslot_id.p : s->kslot.p;
+        rr.nslot = kRhoUnitK * s->nunits;
+        rr.kslot = s->kslot.p;
         rr.nk = s->nk;
         rr.rho = s->rho.p;
         rr.rec = mixed ? nullptr : s->krec.p;
         rr.rec32 = mixed ? s->krec32.p : nullptr;
         rr.efac = s->efac.p;
         rr.vfac = s->vfac.p;
-        rr.epart = s->ep_k_at ? s->ep_k_at : s->epart_k.p;
-        rblocks = blocks_for(s->nk, kRhoReduceK);
+        rr.epart = epk;
     }
     // the mixed instance leaves the intra-molecular terms to a launch of
     // their own (see k_pairs_mixed)
     const bool intra_apart = mixed && !s->gen_pairs;
-    if (intra_apart && iblocks > 0 && !intra_fused) {
+    if (intra_apart && iblocks > 0 && !s->intra_done) {
         if (energy)
             launch_timed(s, LG_KERNEL_MOLECULES, k_intra_terms<true>, iblocks, 256, 0, ia);
         else
@@ -1671,7 +1775,10 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool phase_don
     }
 #undef LG_PAIRS_CASE
 #undef LG_PAIRS_CK
-    if (s->coul_kind == COUL_EWALD && s->nk > 0) {
+    if (oct) {
+        // in MD the k-space forces run with the half-step that needs them
+        if (combine) launch_oct_step(s, OCT_FORCE, OCT_COMBINE, nullptr, Thermo{});
+    } else if (kspace) {
         int kmax = s->coul_kmax;
         constexpr int kApl = 1;  // atoms per lane (2 measured slower at 4k-9k atoms)
         int nab = blocks_for(n, 64 * kApl);
@@ -1685,7 +1792,7 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool phase_don
                 s->phase_tab.p, s->ld, n, kmax, s->rows.p, s->nrows, s->krec.p, s->kg[0], s->kg[1], s->kg[2],
                 s->ksplit, nab, s->fk.p);
     }
-    if (combine && (kspace || s->nterms > 0)) {
+    if (combine && !oct && (kspace || s->nterms > 0)) {
         // timed with the k-space forces: it adds their partials
         long pc = prof_start(s, kspace ? LG_KERNEL_KSPACE_FORCE : LG_KERNEL_MOLECULES);
         k_force_combine<<<blocks_for(n, 256), 256, 0, st>>>(s->force.p, s->contrib.p,
@@ -1721,7 +1828,7 @@ int check_overflow(lg_system* s, bool* overflowed, bool* nonfinite = nullptr) {
 int compute(lg_system* s, bool energy) {
     LG_TRY(prepare(s));
     for (int attempt = 0; attempt < 4; attempt++) {
-        LG_TRY(launch_nlist(s, true));
+        LG_TRY(launch_nlist(s, true, energy));
         LG_TRY(launch_forces(s, energy));
         bool ov = false;
         LG_TRY(check_overflow(s, &ov));
@@ -1748,7 +1855,7 @@ int gather_energies(lg_system* s, Energies& E) {
         LG_HIP(hipMemcpyAsync(hm.data(), s->epart_mol.p, hm.size() * sizeof(double), hipMemcpyDeviceToHost, st));
     }
     std::vector<double> hk;
-    int nbk = (s->coul_kind == COUL_EWALD && s->nk > 0) ? blocks_for(s->nk, kRhoReduceK) : 0;
+    int nbk = kspace_reduce_blocks(s);
     if (nbk) {
         hk.resize(size_t(nbk) * 7);
         LG_HIP(hipMemcpyAsync(hk.data(), s->epart_k.p, hk.size() * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -2045,7 +2152,7 @@ int lg_system_create(lg_context* ctx, size_t natoms, lg_system** out) {
     int r;
     if ((r = s->pos.ensure(natoms)) || (r = s->vel.ensure(natoms)) || (r = s->acc.ensure(natoms)) ||
         (r = s->force.ensure(natoms)) || (r = s->lambda.ensure(1)) ||
-        (r = s->ke_part.ensure(size_t(blocks_for(natoms, 64))))) {
+        (r = s->ke_part.ensure(size_t(blocks_for(natoms, 16))))) {
         delete s;
         return r;
     }
@@ -2066,9 +2173,16 @@ int lg_system_destroy(lg_system* s) {
     DevBuf<int>* ibufs[] = {&s->cellid, &s->slot, &s->count, &s->start, &s->tmp, &s->sorted, &s->nbr, &s->nnbr,
 
                             &s->flags, &s->pair_restr, &s->slot_start, &s->d_mol_start,
-                            &s->mc_cell_count, &s->mc_atom_cell, &s->kslot, &s->mcols, &s->mkmap, &s->kslot_id};
+                            &s->mc_cell_count, &s->mc_atom_cell, &s->kslot, &s->opairs, &s->osteps, &s->okmap, &s->omask};
     for (auto* b : ibufs) b->release();
     s->units.release();
+    s->oitems.release();
+    s->oslots.release();
+    s->orows32.release();
+    s->orows64.release();
+    s->ocoef32.release();
+    s->ocoef64.release();
+    s->opart.release();
     s->ecx64.release();
     s->ecx32.release();
     s->hf32.release();
@@ -2268,7 +2382,7 @@ int lg_system_get_tuning(lg_system* s, lg_tuning* t) {
     t->md_graph = s->tune.md_graph == 2 ? 2 : 1;
     t->rho_width = (s->coul_kind == COUL_EWALD && s->nk > 0) ? rho_chunk(s) : 0;
     t->rho_kind = (s->coul_kind == COUL_EWALD && s->nk > 0)
-                      ? (rho_use_mfma(s, s->precision == LG_PRECISION_MIXED) ? 2 : (s->tune.rho_kind == 3 ? 3 : 1))
+                      ? (s->tune.rho_kind == 2 && s->coul_kmax <= 16 ? 2 : (s->tune.rho_kind == 3 ? 3 : 1))
                       : 0;
     return LG_OK;
 }
@@ -2489,7 +2603,7 @@ int lg_potential_energy_noalloc(lg_system* s, lg_energy_terms* out) {
     }
     const int nbp = pair_blocks_of(s->n, s->tpa);
     const int nbm = s->nterms > 0 ? blocks_for(s->nterms, 256) : 0;
-    const int nbk = (s->coul_kind == COUL_EWALD && s->nk > 0) ? blocks_for(s->nk, kRhoReduceK) : 0;
+    const int nbk = kspace_reduce_blocks(s);
     const size_t need = size_t(nbp) * 8 + size_t(nbm) * 11 + size_t(nbk) * 7 + 18;
     if (need > kNoallocScratchDoubles)
         return fail(LG_E_INVALID, "the energy partial sums of this system (" + std::to_string(need) +
@@ -2503,7 +2617,7 @@ int lg_potential_energy_noalloc(lg_system* s, lg_energy_terms* out) {
     double* sums = s->ep_k_at + size_t(nbk) * 7;
     const uint32_t mask = s->prof_mask;
     s->prof_mask = 0;  // no event creation in this call
-    int rc = launch_nlist(s, true);
+    int rc = launch_nlist(s, true, true);
     if (rc == LG_OK) rc = launch_forces(s, true);
     s->prof_mask = mask;
     s->ep_pairs_at = s->ep_mol_at = s->ep_k_at = nullptr;
@@ -2588,7 +2702,7 @@ int lg_molecular_virial(lg_system* s, double* w9) {
     a.part = s->molvir_part.p;
     k_mol_pairs<<<nbp, 256, 0, st>>>(a);
     if (kspace)
-        k_mol_kspace<<<nbp, 256, 0, st>>>(s->pos.p, s->meta.p, s->fk.p, s->ksplit, n, s->mol_com.p,
+        k_mol_kspace<<<nbp, 256, 0, st>>>(s->pos.p, s->meta.p, s->fk.p, s->oct ? 1 : s->ksplit, s->oct ? 1 : 0, n, s->mol_com.p,
                                           s->molvir_part.p + size_t(nbp) * 6);
     LG_HIP(hipGetLastError());
     std::vector<double> h(size_t(nbp) * (6 + (kspace ? 9 : 0)));
@@ -2701,68 +2815,54 @@ static int md_chunk(lg_system* s, uint64_t todo) {
     const int n = int(s->n);
     const bool thermo = s->thermostat;
     const bool kspace = s->coul_kind == COUL_EWALD && s->nk > 0;
-    double hs = 0.5 * s->skin;
-    int nb = blocks_for(n, 64);  // second half: one wave per block, one KE partial each
-    // the first half-step also writes the phase table of the new positions
-    // (64 atoms per block, ld atoms with the padding)
-    PhaseOut ph{};
-    if (kspace) {
-        ph.mode = s->precision == LG_PRECISION_MIXED ? 2 : 1;
-        ph.kmax = s->coul_kmax;
-        ph.ld = s->ld;
-        ph.box = s->box;
-        ph.tab = s->phase_tab.p;
-        ph.q = s->phase_q.p;
-        ph.tab32 = s->phase_tab32.p;
-        ph.q32 = s->phase_q32.p;
-    }
-    Thermo th{nullptr, nb, double(3 * s->n), s->berendsen_T, s->berendsen_tau};
-    int nbf = blocks_for(std::max(n, kspace ? s->ld : 0), 64);
-    const int tbf = ph.mode == 2 ? 512 : 256;  // waves per first-half block: see phase_roles
-    const CellTag tags = cell_tags(s);
-    const bool lf = s->integrator != LG_INTEGRATOR_VELOCITY_VERLET;
-    const int ks = kspace ? s->ksplit : 0;
+    const bool oct = kspace && s->oct;
+    const int nb = blocks_for(n, kMdBlock);
+    // kinetic-energy partials: one per block of the kernel with the second half
+    const int nke = oct ? oct_ke_parts(s) : nb;
+    const int with_rho = oct && oct_step_rho(s, s->precision == LG_PRECISION_MIXED) ? OCT_RHO : 0;
+    const MdArgs m = md_args(s);
+    Thermo th{nullptr, nke, double(3 * s->n), s->berendsen_T, s->berendsen_tau, nullptr};
+    const int tb = nke > kThermoParts ? 1024 : (oct ? 512 : kMdBlock);  // as the blocks that form the factor
+    double* const kp = thermo ? s->ke_part.p : nullptr;
     const int* sl = s->nterms > 0 ? s->slot_start.p : nullptr;
+    const int ks = kspace && !oct ? s->ksplit : 0;
     // without a thermostat the second half of a step and the first half of
-    // the next share a launch (k_md_fused); the chunk's first and last
-    // halves run alone
+    // the next share a launch (k_md_fused, k_oct_step); the chunk's first
+    // and last halves run alone
     bool first_pending = true;
     for (uint64_t k = 0; k < todo; k++) {
         // integrator launches timed, when profiled, by their own kernel
         // timestamps (launch_timed), like the force launches
         if (first_pending) {
             // the Berendsen scale of the previous step is applied by the first half
-            th.ke_part = (thermo && k > 0) ? s->ke_part.p : nullptr;
-            if (!lf)
-                launch_timed(s, LG_KERNEL_INTEGRATE, k_vv_first, nbf, tbf, 0, s->pos.p, s->vel.p, s->acc.p, n, s->dt,
-                             th, s->ref.p, hs * hs, s->flags.p, ph, tags);
+            th.ke_part = (thermo && k > 0) ? kp : nullptr;
+            th.lambda = nullptr;
+            if (th.ke_part && nke > kThermoParts) {
+                launch_timed(s, LG_KERNEL_INTEGRATE, k_berendsen, 1, tb, 0, th, s->lambda.p);
+                th.lambda = s->lambda.p;
+            }
+            if (oct)
+                launch_oct_step(s, OCT_FIRST | with_rho, 0, nullptr, th);
             else
-                launch_timed(s, LG_KERNEL_INTEGRATE, k_lf_first, nbf, tbf, 0, s->pos.p, s->vel.p, s->acc.p, n, s->dt,
-                             th, s->ref.p, hs * hs, s->flags.p, ph, tags);
+                launch_timed(s, LG_KERNEL_INTEGRATE, k_md_first, nb, kMdBlock, 0, m, th);
         }
-        LG_TRY(launch_nlist(s, false));
-        LG_TRY(launch_forces(s, false, false, true));
+        LG_TRY(launch_nlist(s, false, false));
+        LG_TRY(launch_forces(s, false, false, true, with_rho != 0));
         const bool fuse = !thermo && k + 1 < todo;
-        if (fuse && !lf)
-            launch_timed(s, LG_KERNEL_INTEGRATE, k_md_fused<false>, nbf, tbf, 0, s->force.p, s->pos.p, s->contrib.p,
-                         sl, s->fk.p, ks, s->vel.p, s->acc.p, n, s->dt, s->ref.p, hs * hs, s->flags.p, ph, tags);
+        if (oct)
+            launch_oct_step(s, fuse ? OCT_FORCE | with_rho : OCT_FORCE, fuse ? OCT_FUSED : OCT_SECOND, kp, Thermo{});
         else if (fuse)
-            launch_timed(s, LG_KERNEL_INTEGRATE, k_md_fused<true>, nbf, tbf, 0, s->force.p, s->pos.p, s->contrib.p,
-                         sl, s->fk.p, ks, s->vel.p, s->acc.p, n, s->dt, s->ref.p, hs * hs, s->flags.p, ph, tags);
-        else {
-            double* kp = thermo ? s->ke_part.p : nullptr;
-            if (!lf)
-                launch_timed(s, LG_KERNEL_INTEGRATE, k_md_second<false>, nb, 64, 0, s->force.p, s->pos.p,
-                             s->contrib.p, sl, s->fk.p, ks, s->vel.p, s->acc.p, n, s->dt, kp, s->flags.p);
-            else
-                launch_timed(s, LG_KERNEL_INTEGRATE, k_md_second<true>, nb, 64, 0, s->force.p, s->pos.p,
-                             s->contrib.p, sl, s->fk.p, ks, s->vel.p, s->acc.p, n, s->dt, kp, s->flags.p);
-        }
+            launch_timed(s, LG_KERNEL_INTEGRATE, k_md_fused, nb, kMdBlock, 0, m, s->force.p, s->contrib.p, sl,
+                         s->fk.p, ks);
+        else
+            launch_timed(s, LG_KERNEL_INTEGRATE, k_md_second, nb, kMdBlock, 0, m, s->force.p, s->contrib.p, sl,
+                         s->fk.p, ks, kp);
         first_pending = !fuse;
     }
     if (thermo) {
-        th.ke_part = s->ke_part.p;
-        k_berendsen<<<1, 256, 0, st>>>(th, s->lambda.p);
+        th.ke_part = kp;
+        th.lambda = nullptr;
+        k_berendsen<<<1, tb, 0, st>>>(th, s->lambda.p);
         k_scale_vel<<<blocks_for(n, 256), 256, 0, st>>>(s->vel.p, n, s->lambda.p);
     }
     LG_HIP(hipGetLastError());

@@ -20,6 +20,7 @@
 #include <type_traits>
 
 #include "lg_device.hpp"
+#include "lg_kspace.hpp"
 
 namespace lg {
 
@@ -1342,6 +1343,8 @@ struct PairArgs {
     // intra-molecular terms and the rest the rho(k) reduction
     int pair_blocks, intra_blocks;
     IntraArgs intra;
+    int oct;       // the reduction is of the octant form (orr), else of the row form (rr)
+    OctReduce orr;
     RhoReduceArgs rr;
     // erfcx tables of the Ewald / Wolf real-space erfc (erfcx_tab), or null
     // for the library erfc
@@ -1355,6 +1358,14 @@ struct PairArgs {
     const float* hf32;
     double hf_inv_h;
 };
+
+template <bool kEnergy>
+__device__ __forceinline__ void kspace_reduce_block(const PairArgs& a, int blk) {
+    if (a.oct)
+        oct_reduce_block<kEnergy>(a.orr, blk);
+    else
+        rho_reduce_block<kEnergy>(a.rr, blk);
+}
 
 constexpr int kMaxKinds = 16;
 constexpr int kPairBlock = 256;
@@ -1401,7 +1412,7 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(4)))
         if (b < a.intra_blocks)
             intra_block<kEnergy>(a.intra, b);
         else
-            rho_reduce_block<kEnergy>(a.rr, b - a.intra_blocks);
+            kspace_reduce_block<kEnergy>(a, b - a.intra_blocks);
         return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.rebuild) *a.rebuild = 0;
@@ -1577,7 +1588,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs_mixed(PairArgs a) {
     __shared__ __align__(16) float ecx[kTab ? kErfcxPieces * (kErfcxDeg32 + 1) : 4];
     __shared__ __align__(16) float hft[kTab ? kErfcxPieces * (kErfcxDeg32 + 1) : 4];
     if ((int)blockIdx.x >= a.pair_blocks) {  // uniform over the block
-        rho_reduce_block<kEnergy>(a.rr, blockIdx.x - a.pair_blocks);
+        kspace_reduce_block<kEnergy>(a, blockIdx.x - a.pair_blocks);
         return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.rebuild) *a.rebuild = 0;
@@ -1973,7 +1984,7 @@ __global__ __launch_bounds__(256) void k_mol_pairs(MolVirialArgs a) {
 }
 
 __global__ __launch_bounds__(256) void k_mol_kspace(const double4* __restrict__ pos, const int2* __restrict__ meta,
-                                                     const double4* __restrict__ fk, int ksplit, int n,
+                                                     const double4* __restrict__ fk, int ksplit, int with_q, int n,
                                                      const double4* __restrict__ com, double* __restrict__ part) {
     double c[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1986,7 +1997,9 @@ __global__ __launch_bounds__(256) void k_mol_kspace(const double4* __restrict__ 
             sz += p.z;
         }
         const double4 p = pos[i];
-        const double fx = (p.w * sx) / kFourPiEps0, fy = (p.w * sy) / kFourPiEps0, fz = (p.w * sz) / kFourPiEps0;
+        // the octant form's sums carry the charge already (with_q)
+        const double q = with_q ? 1.0 : p.w;
+        const double fx = (q * sx) / kFourPiEps0, fy = (q * sy) / kFourPiEps0, fz = (q * sz) / kFourPiEps0;
         const double4 cm = com[meta[i].y];
         const double d[3] = {p.x - cm.x, p.y - cm.y, p.z - cm.z};
         const double f[3] = {fx, fy, fz};
@@ -1997,10 +2010,11 @@ __global__ __launch_bounds__(256) void k_mol_kspace(const double4* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------------
-// Ewald k-space (ewald.rs:633-733).  k_phase computes, once per evaluation,
+// Ewald k-space (ewald.rs:633-733) of the row form, for kmax above kOctMaxK
+// (below: lg_kspace.hpp).  k_phase computes, once per evaluation,
 // e^{i n k_axis . r_i} for every atom and axis by the reference's recursion
 // (polar for n = 1, products for |n| >= 2, conjugates for n < 0) into a
-// table in HBM; the rho and force kernels stage the rows they use in LDS and
+// table in HBM; the rho and force kernels read the rows they use from it and
 // form e^{i k.r} = (Ex * Ey) * Ez as ewald.rs:666-668.
 // ---------------------------------------------------------------------------------
 
@@ -2063,37 +2077,13 @@ __device__ __forceinline__ float2 phase32_n(double phase, int k) {
 }
 
 __device__ __forceinline__ void phase_axis32(double x, double inv, int axis, int kmax, float2* __restrict__ tab,
-                                             int ld, int a, int k0 = 1, int k1 = -1) {
+                                             int ld, int a) {
     double phase = (2.0 * kPi * inv) * x;
-    if (k1 < 0) k1 = kmax;
-    if (k0 == 1) tab[(size_t)phase_row(axis, 0, kmax) * ld + a] = make_float2(1.f, 0.f);
-    for (int k = k0; k <= k1; k++) {
+    tab[(size_t)phase_row(axis, 0, kmax) * ld + a] = make_float2(1.f, 0.f);
+    for (int k = 1; k <= kmax; k++) {
         const float2 e = phase32_n(phase, k);
         tab[(size_t)phase_row(axis, k, kmax) * ld + a] = e;
         if (axis != 0) tab[(size_t)phase_row(axis, -k, kmax) * ld + a] = make_float2(e.x, -e.y);
-    }
-}
-
-// Where the MD step's first half writes the phase table of the new
-// positions (mode 0: no k-space, 1: FP64 table, 2: FP32 table).
-struct PhaseOut {
-    int mode, kmax, ld;
-    Box box;
-    double2* tab;
-    double* q;
-    float2* tab32;
-    float* q32;
-};
-
-__device__ __forceinline__ void phase_atom(const PhaseOut& ph, int a, bool live, double4 p) {
-    double xyz[3] = {live ? p.x : 0.0, live ? p.y : 0.0, live ? p.z : 0.0};
-    if (ph.mode == 1) {
-        for (int axis = 0; axis < 3; axis++) phase_axis64(xyz[axis], ph.box.inv[axis], axis, ph.kmax, ph.tab, ph.ld, a);
-        ph.q[a] = live ? p.w : 0.0;
-    } else {
-        for (int axis = 0; axis < 3; axis++)
-            phase_axis32(xyz[axis], ph.box.inv[axis], axis, ph.kmax, ph.tab32, ph.ld, a);
-        ph.q32[a] = live ? (float)p.w : 0.f;
     }
 }
 
@@ -2119,20 +2109,17 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
     return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
+// ---- row form (kmax above kOctMaxK) ---------------------------------------------
 // rho partial sums by row units.  A unit is up to kRhoUnitK (5) consecutive
 // k-vectors of one row (fixed ikx, iky; consecutive ikz): per atom, the lane
 // forms q e^{i k0.r} = q (Ex * Ey) * Ez[ikz0] and steps to the next ikz by
-// one product with Ez[1], 7.2 operations and 0.6 table reads per (atom, k).
-// Five per unit pads the k set least (units fill whole 64-lane blocks more
-// often than with four: SPC/E kmax 10, 480 units in 512 lanes against 589
-// in 640; 8.9 against 9.2 operations per k-vector and atom, lane padding
-// included).  Block = 64 units (one per lane) x 8 waves; the block's atom
-// chunk of `width` atoms is split in eight and each wave sums its eighth;
-// the eight wave sums are added in order in LDS and wave j < 5 writes
-// k-vector j of every unit: partial[chunk * 5 * nunits + j * nunits + unit]
-// (slots with j past the unit's count are not written).  Table rows are
-// read straight from L2: a wave's lanes read few distinct rows at one atom
-// column.  The table is padded with zero charges to `ld` atoms.  Grid:
+// one product with Ez[1].  Block = 64 units (one per lane) x 8 waves; the
+// block's atom chunk of `width` atoms is split in eight and each wave sums
+// its eighth; the eight wave sums are added in order in LDS and wave j < 5
+// writes k-vector j of every unit: partial[chunk * 5 * nunits + j * nunits +
+// unit] (slots with j past the unit's count are not written).  Table rows
+// are read straight from L2: a wave's lanes read few distinct rows at one
+// atom column.  The table is padded with zero charges to `ld` atoms.  Grid:
 // xcd_grid(nub, nchunks), so all unit blocks of an atom chunk share one L2.
 // Mixed form (T = float): each wave's eighth is summed in FP32, the rest in
 // FP64.
@@ -2151,59 +2138,37 @@ struct RhoRowsArgs {
     int nunits;
     double2* partial;
     int nub, nchunks;
-    int stage;  // 1: phase rows staged in LDS when they fit (rho_kind 1), 0: read from the table (rho_kind 3)
 };
 
-// Phase rows the staged row kernel loads per round; the phase tables are
-// allocated with at least this many rows (kmax <= 12 staged).
-constexpr int kRhoStageRows = 64;
-// Atoms per staging round of the row kernel: every phase row of S
-// consecutive atoms is copied to LDS at once.
-template <typename T>
-constexpr int rho_stage_atoms() { return sizeof(T) == 4 ? 8 : 4; }
-// LDS bytes of one wave's staging area (rows padded to S + 1 entries so that
-// lanes reading different rows at one atom fall in different banks; the
-// charges follow the rows), rounded to 16 bytes.
 template <typename T, typename T2>
-__host__ __device__ constexpr size_t rho_stage_wave_bytes(int kmax) {
-    return ((size_t)phase_rows(kmax) * (rho_stage_atoms<T>() + 1) * sizeof(T2) + rho_stage_atoms<T>() * sizeof(T) +
-            15) / 16 * 16;
-}
-
-// NW waves per block (8 in k_rho_rows, k_cells_rho and k_direct_rho),
-// logical block index L of the xcd_grid(nub, nchunks) layout.  buf: the
-// launch's LDS (buf_bytes), which holds the eight wave sums at the end and,
-// when the staging areas of all NW waves fit in it, the staged phase rows.
-// kPrefetch: the staged loop loads the next round while it sums the current
-// one (more registers held: used where the launch's LDS, not its registers,
-// sets the residency).
-template <typename T, typename T2, int NW, bool kPrefetch = false>
-__device__ __forceinline__ void rho_rows_block(const RhoRowsArgs<T, T2>& ra, int L, unsigned char* buf,
-                                               size_t buf_bytes) {
-    static_assert(NW >= kRhoUnitK, "one wave writes each k-vector of a unit");
-    double2(*red)[kRhoUnitK][64] = reinterpret_cast<double2(*)[kRhoUnitK][64]>(buf);
+__global__ __launch_bounds__(512) void k_rho_rows(RhoRowsArgs<T, T2> ra) {
+    constexpr int NW = 8;
+    __shared__ double2 red[NW][kRhoUnitK][64];
     const T2* __restrict__ tab = ra.tab;
     const T* __restrict__ q = ra.q;
     const int ld = ra.ld, kmax = ra.kmax, width = ra.width, nunits = ra.nunits;
     const KUnit* __restrict__ units = ra.units;
-    double2* __restrict__ partial = ra.partial;
     int ub, chunk;
-    if (!xcd_block_at(L, ra.nub, ra.nchunks, ub, chunk)) return;
+    if (!xcd_block(ra.nub, ra.nchunks, ub, chunk)) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int u = ub * 64 + lane;
     const KUnit un = units[u < nunits ? u : nunits - 1];
     const int per = width / NW;
-    // the wave's atom range, visibly uniform.  a1 - a0 is a multiple of 8
-    // or <= 0: widths are multiples of 64 (as is ld), so per and a0 are
-    // multiples of 8
     const int a0 = __builtin_amdgcn_readfirstlane(chunk * width + w * per);
     const int a1 = min(a0 + per, ld);
     T re[kRhoUnitK], im[kRhoUnitK];
 #pragma unroll
     for (int v = 0; v < kRhoUnitK; v++) re[v] = im[v] = 0;
-    // one atom's terms, in the order of the reference's triple product
-    auto add_atom = [&](T2 x, T2 y, T2 z, T2 e1, T qa) {
-        T2 e = cmul(cmul(x, y), z);
+    const T2* cx = tab + (size_t)phase_row(0, un.ikx, kmax) * ld;
+    const T2* cy = tab + (size_t)phase_row(1, un.iky, kmax) * ld;
+    const T2* cz = tab + (size_t)phase_row(2, un.kz0, kmax) * ld;
+    const T2* c1 = tab + (size_t)phase_row(2, 1, kmax) * ld;
+#pragma unroll 4
+    for (int a = a0; a < a1; a++) {
+        // one atom's terms, in the order of the reference's triple product
+        T2 e = cmul(cmul(cx[a], cy[a]), cz[a]);
+        const T2 e1 = c1[a];
+        const T qa = q[a];
         e.x *= qa;
         e.y *= qa;
 #pragma unroll
@@ -2212,87 +2177,7 @@ __device__ __forceinline__ void rho_rows_block(const RhoRowsArgs<T, T2>& ra, int
             re[v] += e.x;
             im[v] += e.y;
         }
-    };
-    constexpr int S = rho_stage_atoms<T>(), SP = S + 1;
-    constexpr int kStep = 64 / S;  // rows per load instruction of a wave
-    const size_t wave_bytes = rho_stage_wave_bytes<T, T2>(kmax);
-    const int prow = phase_rows(kmax);
-    if (ra.stage && (size_t)NW * wave_bytes <= buf_bytes && prow <= kRhoStageRows) {
-        // Staged: each round copies every phase row of the next S atoms
-        // (and their charges) to the wave's own LDS area, one load per 64
-        // entries (S consecutive atoms of 64 / S rows), all in flight
-        // together; then each lane reads its unit's rows from LDS: one
-        // memory latency per S atoms.  Atoms are added in index order, as in
-        // the unstaged loop.  The loads cover kRhoStageRows rows, which the
-        // table is allocated to hold; rows past the phase rows are not
-        // stored.  Only this wave reads its area, and a wave's LDS
-        // operations complete in order, so a round's reads precede the next
-        // round's writes.
-        T2* tile = reinterpret_cast<T2*>(buf + (size_t)w * wave_bytes);
-        T* qt = reinterpret_cast<T*>(tile + (size_t)prow * SP);
-        const int rx = phase_row(0, un.ikx, kmax) * SP, ry = phase_row(1, un.iky, kmax) * SP;
-        const int rz = phase_row(2, un.kz0, kmax) * SP, r1 = phase_row(2, 1, kmax) * SP;
-        const int lr = lane / S, lj = lane - lr * S, lq = min(lane, S - 1);
-        const T2* src = tab + (size_t)lr * ld + lj;
-        constexpr int kR = kRhoStageRows / kStep;
-        T2 v[kR];
-        T qv;
-        auto load = [&](int a) {
-#pragma unroll
-            for (int it = 0; it < kR; it++) v[it] = src[(size_t)(it * kStep) * ld + a];
-            qv = q[a + lq];
-        };
-        auto stage = [&]() {
-#pragma unroll
-            for (int it = 0; it < kR; it++) {
-                const int r = lr + it * kStep;
-                if (r < prow) tile[r * SP + lj] = v[it];
-            }
-            qt[lq] = qv;
-            // the wave's LDS writes done before any lane reads them
-            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-            __builtin_amdgcn_wave_barrier();
-        };
-        auto sum = [&]() {
-#pragma unroll
-            for (int j = 0; j < S; j++) add_atom(tile[rx + j], tile[ry + j], tile[rz + j], tile[r1 + j], qt[j]);
-            __builtin_amdgcn_wave_barrier();
-        };
-        if constexpr (kPrefetch) {
-            // the next round's loads in flight while this round is summed
-            // (one memory latency per wave).  The first round's values go
-            // through an empty asm statement once they have landed, so that
-            // the values entering the loop are not all loads and the
-            // compiler keeps the early loads where they are; the last round
-            // reloads its own atoms (in bounds, not used).
-            if (a0 < a1) {
-                load(a0);
-#pragma unroll
-                for (int it = 0; it < kR; it++) asm volatile("" : "+v"(v[it].x), "+v"(v[it].y));
-                asm volatile("" : "+v"(qv));
-            }
-            for (int a = a0; a < a1; a += S) {
-                stage();
-                load(a + S < a1 ? a + S : a);
-                sum();
-            }
-        } else {
-            for (int a = a0; a < a1; a += S) {
-                load(a);
-                stage();
-                sum();
-            }
-        }
-    } else {
-        const T2* cx = tab + (size_t)phase_row(0, un.ikx, kmax) * ld;
-        const T2* cy = tab + (size_t)phase_row(1, un.iky, kmax) * ld;
-        const T2* cz = tab + (size_t)phase_row(2, un.kz0, kmax) * ld;
-        const T2* c1 = tab + (size_t)phase_row(2, 1, kmax) * ld;
-#pragma unroll 4
-        for (int a = a0; a < a1; a++) add_atom(cx[a], cy[a], cz[a], c1[a], q[a]);
     }
-    // every wave is past its staging area before the sums overwrite it
-    __syncthreads();
 #pragma unroll
     for (int v = 0; v < kRhoUnitK; v++) red[w][v][lane] = make_double2(re[v], im[v]);
     __syncthreads();
@@ -2303,279 +2188,37 @@ __device__ __forceinline__ void rho_rows_block(const RhoRowsArgs<T, T2>& ra, int
             sum.x += red[v][w][lane].x;
             sum.y += red[v][w][lane].y;
         }
-        partial[(size_t)chunk * kRhoUnitK * nunits + (size_t)w * nunits + u] = sum;
+        ra.partial[(size_t)chunk * kRhoUnitK * nunits + (size_t)w * nunits + u] = sum;
     }
 }
 
-// LDS of the eight wave sums of a row-kernel block
-constexpr size_t kRhoRed = sizeof(double2) * (kCellBlock / 64) * kRhoUnitK * 64;
-
-// Same 8-wave blocks as the rho part of k_cells_rho, so that the partial
-// sums do not depend on which launch computed them.
-template <typename T, typename T2>
-__global__ __launch_bounds__(512) void k_rho_rows(RhoRowsArgs<T, T2> ra) {
-    __shared__ __align__(16) unsigned char buf[kRhoRed];
-    rho_rows_block<T, T2, 8>(ra, blockIdx.x, buf, sizeof(buf));
-}
-
-// One launch for two independent passes of a force evaluation: blocks
-// [0, ncb) build the Verlet list (ncb = cells rounded up to 8, so that the
-// rho blocks that follow keep the XCD layout of xcd_grid), the rest compute
-// the rho(k) partials with 8 waves per block.  Both read only what the
-// first half-step and the cell list wrote.
-template <bool kMinImage, typename T, typename T2>
-__global__ __launch_bounds__(kCellBlock) void k_cells_rho(CellsArgs ca, RhoRowsArgs<T, T2> ra, int ncb) {
-    __shared__ __align__(16) unsigned char buf[sizeof(CellsLds) > kRhoRed ? sizeof(CellsLds) : kRhoRed];
-    if ((int)blockIdx.x < ncb)
-        nlist_cells_block<kMinImage>(ca, blockIdx.x, ncb, *reinterpret_cast<CellsLds*>(buf));
-    else
-        rho_rows_block<T, T2, kCellBlock / 64>(ra, blockIdx.x - ncb, buf, sizeof(buf));
-}
-
-// The same with the direct Verlet build in the first ncb blocks; the rho
-// partials in the next nrho blocks, and any blocks past those run the
-// intra-molecular terms (forces only, kCellBlock terms per block), which
-// need only the positions of the first half-step.
-// kIntra: the instance with the intra-molecular blocks (mixed form); the
-// others leave their code out (it costs the rho blocks registers).
-// Four waves per SIMD: its 64 KB of LDS allow two blocks (sixteen waves) per
-// CU, so registers up to 128 cost nothing and above it would cost a block.
-template <bool kMinImage, typename T, typename T2, bool kIntra = false>
-__global__ __launch_bounds__(kCellBlock, 4) void k_direct_rho(DirectArgs da, RhoRowsArgs<T, T2> ra, int ncb, int nrho,
-                                                           IntraArgs ia) {
-    __shared__ __align__(16) unsigned char buf[sizeof(DirectLds) > kRhoRed ? sizeof(DirectLds) : kRhoRed];
-    if ((int)blockIdx.x < ncb)
-        nlist_direct_block<kMinImage>(da, blockIdx.x, ncb, *reinterpret_cast<DirectLds*>(buf));
-    else if ((int)blockIdx.x < ncb + nrho)
-        rho_rows_block<T, T2, kCellBlock / 64, true>(ra, blockIdx.x - ncb, buf, sizeof(buf));
-    else if constexpr (kIntra)
-        intra_block<false>(ia, blockIdx.x - ncb - nrho);
-}
-
-
-// ---- rho(k) on the matrix cores ---------------------------------------------------
-// With e^{ik.r} = Ex[ikx] * Eyz[(iky, ikz)] and Eyz = q Ey Ez, the structure
-// factor is a complex matrix product over atoms:
-//     rho[ikx][col] = sum_i Ex[i][ikx] * Eyz[i][col],   col = (iky, ikz)
-// (the same triple product as ewald.rs:664-673, grouped differently).  Rows
-// ikx = 0..15 (kmax <= 16), columns = the distinct (iky, ikz) of the k set in
-// tiles of 16; the reduction index runs over (atom, re/im), so one
-// v_mfma 16x16x4 adds two atoms to a 16 x 16 tile of Re(rho) and another to
-// Im(rho):
-//     Re: A = (Ex.re, -Ex.im), B = (Eyz.re, Eyz.im)
-//     Im: A = (Ex.im,  Ex.re), B = the same
-// The reduction over atoms -- across lanes in a lane-per-atom layout --
-// happens inside the matrix core.  Block = 8 waves on `width` atoms whose
-// phase factors it forms from the positions into LDS as
-// [atom][X 0..15 | Ey -kmax..kmax | Ez -kmax..kmax] plus the charges
-// (applied to the A operand); wave
-// (sub = w & 3, half = w >> 2) sums atoms [sub * width/4, +width/4) of each
-// stage for 3 tiles; a block covers 6 tiles (group) and `cpb`
-// consecutive stages (chunk).  The four sub-waves' tiles are added in order
-// in FP64 and written to partial[chunk * nk + k] for the valid k only
-// (kmap); the fixed-order chunk reduction of rho_reduce_block follows.
-typedef float rho_f4 __attribute__((ext_vector_type(4)));
-typedef double rho_d4 __attribute__((ext_vector_type(4)));
-template <typename T> struct MfmaAcc;
-template <> struct MfmaAcc<float> { typedef rho_f4 type; };
-template <> struct MfmaAcc<double> { typedef rho_d4 type; };
-__device__ __forceinline__ rho_f4 mfma16x16x4(float a, float b, rho_f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ rho_d4 mfma16x16x4(double a, double b, rho_d4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-// Both take A[i][k] from lane i + 16 k and B[k][j] from lane j + 16 k; output
-// r of lane l is D[row][l % 16] with row = 4 (l / 16) + r for the FP32 form
-// and l / 16 + 4 r for the FP64 form (measured on gfx950).
-__device__ __forceinline__ int mfma16_row(float, int l16, int r) { return 4 * l16 + r; }
-__device__ __forceinline__ int mfma16_row(double, int l16, int r) { return l16 + 4 * r; }
-
-constexpr int kRhoMfmaTpw = 3;  // tiles per wave (a block: 2 x 3 tiles)
-
-template <typename T, typename T2>
-struct RhoMfmaArgs {
-    const double4* pos;  // positions, charge in w
-    int n;
-    Box box;
-    int ld, kmax;
-    int wlog;     // log2 of the atoms per stage: 4..7 (a multiple of 16)
-    int cpb;      // stages per block
-    int nt;       // column tiles
-    int ngroups;  // tile groups (blocks per chunk)
-    int nchunks;
-    const int* cols;  // nt * 16: (iky + kmax) << 16 | (ikz + kmax)
-    const int* kmap;  // nt * 256: k of output (ikx, col), or -1
-    int nk;
-    double2* partial;
-};
-
-// LDS entries per staged atom: X (16) + Ey (2 kmax + 1) + Ez (2 kmax + 1),
-// plus one so that the stride is odd and the stores of one row (consecutive
-// atoms, 8 or 16 bytes each) fall in distinct banks.
-__host__ __device__ inline int rho_mfma_stride(int kmax) {
-    return 16 + 2 * (2 * kmax + 1) + 1;
-}
-// LDS bytes of one block: the staged rows and charges, or the sub-wave
-// tiles, whichever is larger (the second reuses the first).
+// ---- octant form: rho(k) alone ----------------------------------------------------------
+// For evaluations outside MD steps and systems of too many chunks for
+// k_oct_step: blocks of a.width atoms (several stages of SA) x item groups.
+// Dynamic LDS: the rows of SA atoms, at least kOctRed.
 template <typename T>
-__host__ __device__ inline size_t rho_mfma_lds(int width, int kmax) {
-    size_t stage = size_t(width) * rho_mfma_stride(kmax) * 2 * sizeof(T) + size_t(width) * sizeof(T);
-    size_t red = size_t(2) * 3 * kRhoMfmaTpw * 2 * 4 * 64 * sizeof(T);
-    return stage > red ? stage : red;
-}
-
-template <typename T, typename T2>
-__device__ __forceinline__ void rho_mfma_block(const RhoMfmaArgs<T, T2>& ra, int L, T2* __restrict__ smem) {
-    typedef typename MfmaAcc<T>::type acc_t;
+__global__ __launch_bounds__(512, 2) void k_rho_oct(OctRho ra, int SA, const double4* __restrict__ pos, int n) {
+    extern __shared__ __align__(16) unsigned char oct_smem[];
     int grp, chunk;
-    if (!xcd_block_at(L, ra.ngroups, ra.nchunks, grp, chunk)) return;
-    const int kmax = ra.kmax, wl = ra.wlog, W = 1 << wl, nt = ra.nt;
-    constexpr int tpw = kRhoMfmaTpw;
-    const int ny = 2 * kmax + 1, S = rho_mfma_stride(kmax);
-    T* qs = reinterpret_cast<T*>(smem + W * S);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int sub = w & 3, half = w >> 2;
-    const int kk = lane >> 4, c = lane & 15, comp = kk & 1;
-    const int t0 = grp * 2 * tpw + half * tpw;
-    int offy[kRhoMfmaTpw], offz[kRhoMfmaTpw];
-#pragma unroll
-    for (int t = 0; t < kRhoMfmaTpw; t++) {
-        const int tt = t0 + t;
-        // tiles past the last compute on a stand-in column and are not stored
-        const int ci = tt < nt ? ra.cols[tt * 16 + c] : ((kmax << 16) | kmax);
-        offy[t] = 16 + (ci >> 16);
-        offz[t] = 16 + ny + (ci & 0xffff);
-    }
-    // the k-vector of each output, fetched now so that its latency is hidden
-    int kmp[kRhoMfmaTpw][4];
-#pragma unroll
-    for (int t = 0; t < kRhoMfmaTpw; t++)
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            kmp[t][r] = (sub == 0 && t0 + t < nt) ? ra.kmap[(t0 + t) * 256 + mfma16_row(T(0), kk, r) * 16 + c] : -1;
-    acc_t are[kRhoMfmaTpw], aim[kRhoMfmaTpw];
-#pragma unroll
-    for (int t = 0; t < kRhoMfmaTpw; t++) {
-        are[t] = acc_t{0, 0, 0, 0};
-        aim[t] = acc_t{0, 0, 0, 0};
-    }
-    const int per = W >> 2;
-    // staging: thread (axis, atom) forms the atom's phase factors along one
-    // axis by the reference's recursion in FP64 (phase_axis64; the mixed form
-    // rounds each factor to FP32 once), and the x-axis thread its charge;
-    // atoms past n are zero
-    for (int stg = 0; stg < ra.cpb; stg++) {
-        const int a0 = (chunk * ra.cpb + stg) * W;
-        if (stg > 0) __syncthreads();  // the previous stage is read before it is replaced
-        if ((int)threadIdx.x < 3 * W) {
-            const int a = threadIdx.x & (W - 1), axis = threadIdx.x >> wl, ga = a0 + a;
-            double4 p = make_double4(0.0, 0.0, 0.0, 0.0);
-            if (ga < ra.n) p = ra.pos[ga];
-            const double x = axis == 0 ? p.x : (axis == 1 ? p.y : p.z);
-            const double phase = (2.0 * kPi * ra.box.inv[axis]) * x;
-            T2* row = smem + a * S + (axis == 0 ? 0 : (axis == 1 ? 16 + kmax : 16 + ny + kmax));
-            T2 one;
-            one.x = 1;
-            one.y = 0;
-            row[0] = one;
-            double sn, cs;
-            sincos(phase, &sn, &cs);
-            double ex = cs, ey = sn;
-            // x rows ikx = 0..kmax-1 (the half-space set), zero up to 15
-            const int top = axis == 0 ? kmax - 1 : kmax;
-            for (int k = 1; k <= top; k++) {
-                if (k > 1) {
-                    const double rx = ex * cs - ey * sn, ry = ex * sn + ey * cs;
-                    ex = rx;
-                    ey = ry;
-                }
-                T2 e, cj;
-                e.x = cj.x = (T)ex;
-                e.y = (T)ey;
-                cj.y = -e.y;
-                row[k] = e;
-                if (axis != 0) row[-k] = cj;
-            }
-            if (axis == 0) {
-                T2 zero;
-                zero.x = zero.y = 0;
-                for (int k = kmax > 1 ? kmax : 1; k < 16; k++) row[k] = zero;
-                qs[a] = (T)p.w;
-            }
-        }
-        __syncthreads();
-        const int abase = sub * per + (kk >> 1);
-        const T2* at0 = smem + abase * S;
-        // per = width / 4 is a multiple of 4: two atom pairs per trip
-        for (int p = 0; p < per; p += 4) {
-#pragma unroll
-            for (int u = 0; u < 4; u += 2) {
-                const T2* at = at0 + (p + u) * S;
-                const T2 x = at[c];
-                const T qa = qs[abase + p + u];
-                const T ar = qa * (comp ? -x.y : x.x);
-                const T ai = qa * (comp ? x.x : x.y);
-#pragma unroll
-                for (int t = 0; t < kRhoMfmaTpw; t++) {
-                    const T2 y = at[offy[t]], z = at[offz[t]];
-                    const T b = comp ? (y.x * z.y + y.y * z.x) : (y.x * z.x - y.y * z.y);
-                    are[t] = mfma16x16x4(ar, b, are[t]);
-                    aim[t] = mfma16x16x4(ai, b, aim[t]);
-                }
-            }
-        }
-    }
-    __syncthreads();  // staging reads done: the LDS now holds sub-wave tiles
-    T* red = reinterpret_cast<T*>(smem);
-    auto slot = [&](int s, int t, int part, int r) { return ((((half * 3 + s) * kRhoMfmaTpw + t) * 2 + part) * 4 + r) * 64 + lane; };
-    if (sub > 0) {
-#pragma unroll
-        for (int t = 0; t < kRhoMfmaTpw; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                red[slot(sub - 1, t, 0, r)] = are[t][r];
-                red[slot(sub - 1, t, 1, r)] = aim[t][r];
-            }
-    }
-    __syncthreads();
-    if (sub == 0) {
-#pragma unroll
-        for (int t = 0; t < kRhoMfmaTpw; t++) {
-            const int tt = t0 + t;
-            if (tt >= nt) continue;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int k = kmp[t][r];
-                double sr = (double)are[t][r], si = (double)aim[t][r];
-                for (int s2 = 0; s2 < 3; s2++) {
-                    sr += (double)red[slot(s2, t, 0, r)];
-                    si += (double)red[slot(s2, t, 1, r)];
-                }
-                if (k >= 0) ra.partial[(size_t)chunk * ra.nk + k] = make_double2(sr, si);
-            }
-        }
-    }
+    if (!xcd_block(ra.ngroups, ra.nchunks, grp, chunk)) return;
+    const int a0 = chunk * ra.width;
+    oct_rho_group<T>(ra, SA, grp, chunk, min(ra.width, n - a0), false, reinterpret_cast<T*>(oct_smem),
+                     [&](int at) { return pos[a0 + at]; });
 }
 
-template <typename T, typename T2>
-__global__ __launch_bounds__(512) void k_rho_mfma(RhoMfmaArgs<T, T2> ra) {
-    extern __shared__ __align__(16) unsigned char rho_smem[];
-    rho_mfma_block<T, T2>(ra, blockIdx.x, reinterpret_cast<T2*>(rho_smem));
-}
-
-// k_cells_rho with the matrix-core rho blocks; both parts use the one
-// dynamic LDS buffer (max of sizeof(CellsLds) and rho_mfma_lds).
-template <bool kMinImage, typename T, typename T2>
-__global__ __launch_bounds__(kCellBlock) void k_cells_rho_mfma(CellsArgs ca, RhoMfmaArgs<T, T2> ra, int ncb) {
-    extern __shared__ __align__(16) unsigned char rho_smem[];
+// The direct Verlet build in the first ncb blocks; any blocks past those run
+// the intra-molecular terms (forces only, kCellBlock terms per block), which
+// need only the positions of the first half-step (mixed form).
+template <bool kMinImage>
+__global__ __launch_bounds__(kCellBlock) void k_direct_intra(DirectArgs da, int ncb, IntraArgs ia) {
+    __shared__ DirectLds lds;
     if ((int)blockIdx.x < ncb)
-        nlist_cells_block<kMinImage>(ca, blockIdx.x, ncb, *reinterpret_cast<CellsLds*>(rho_smem));
+        nlist_direct_block<kMinImage>(da, blockIdx.x, ncb, lds);
     else
-        rho_mfma_block<T, T2>(ra, blockIdx.x - ncb, reinterpret_cast<T2*>(rho_smem));
+        intra_block<false>(ia, blockIdx.x - ncb);
 }
 
-// k-space forces: one lane per atom, rows of k-vectors (fixed ikx, iky;
+// k-space forces of the row form: one lane per atom, rows of k-vectors (fixed ikx, iky;
 // consecutive ikz) read uniformly; F_i += q_i / (4 pi eps0) *
 // sum_k Im(e^{ik.r_i} conj(rho_k)) field_k  (ewald.rs:699-719).
 struct KRow {
@@ -2758,13 +2401,6 @@ __global__ void k_phase32(const double4* __restrict__ pos, int n, int ld, Box b,
 // reference so that positions follow the reference's rounding.
 // ---------------------------------------------------------------------------------
 #pragma clang fp contract(off)
-// Neighbour-list displacement test of the new position.
-__device__ __forceinline__ bool moved_beyond(double4 p, const double4* __restrict__ ref, int i, double half_skin2) {
-    double4 r = ref[i];
-    double dx = p.x - r.x, dy = p.y - r.y, dz = p.z - r.z;
-    return dx * dx + dy * dy + dz * dz > half_skin2;
-}
-
 // Non-finite state of an atom after an integration step: flags[2] is set
 // (wave-level OR, one vector atomic per wave) so that the host can fail the
 // run instead of returning NaN positions as a result.
@@ -2776,202 +2412,146 @@ __device__ __forceinline__ void flag_nonfinite(bool bad, int* __restrict__ flags
 }
 
 // Berendsen factor (thermostats.rs:113-121) from the kinetic energy
-// partials of the previous step, dof = 3N (system.rs:249-255): the block sums
-// the partials in a fixed order (thread-strided, waves, then wave order), so
-// every block of a launch, and k_berendsen, get the same bits.
+// partials of the previous step, dof = 3N (system.rs:249-255).  Up to
+// kThermoParts partials are added by every block that needs the factor, in a
+// fixed order (thread-strided, then the wave sum) and by one wave, so every
+// block of a launch, and k_berendsen, get the same bits; more of them (large
+// systems) are added once, by k_berendsen, and the blocks read its factor.
+constexpr int kThermoParts = 1024;
 struct Thermo {
     const double* ke_part;  // null: no pending scale
     int nparts;
     double dof, T0, tau;
+    const double* lambda;   // the factor of k_berendsen (nparts > kThermoParts)
 };
 
-// The sum runs over the first 256 threads whatever the block size, so that
-// every kernel computes the same lambda bit for bit.
+// Any block size (a multiple of 64), all threads.
 __device__ __forceinline__ double berendsen_lambda(const Thermo& th) {
-    __shared__ double red[4];
-    __shared__ double lam;
+    __shared__ double red[16];
     double t = 0.0;
-    if (threadIdx.x < 256)
-        for (int p = threadIdx.x; p < th.nparts; p += 256) t += th.ke_part[p];
+#pragma unroll 4
+    for (int p = threadIdx.x; p < th.nparts; p += blockDim.x) t += th.ke_part[p];
     t = wave_sum(t);
-    if ((threadIdx.x & 63) == 0 && threadIdx.x < 256) red[threadIdx.x >> 6] = t;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double kin = red[0] + red[1] + red[2] + red[3];
-        double T = 2.0 * kin / (th.dof * kBoltzmann);
-        lam = sqrt(1.0 + (th.T0 / T - 1.0) / th.tau);
-    }
-    __syncthreads();
-    return lam;
+    double kin = red[0];
+    for (int w = 1; w < (int)(blockDim.x >> 6); w++) kin += red[w];
+    const double T = 2.0 * kin / (th.dof * kBoltzmann);
+    return sqrt(1.0 + (th.T0 / T - 1.0) / th.tau);
 }
 
-// Phase-table part of a first half-step: role r (1..3) of the block writes
-// the rows of axis r - 1 for the block's 64 new positions, staged in LDS by
-// role 0 (charges with axis 0).  Padding atoms (n <= i < ld) get x = 0 and
-// q = 0, as k_phase.
-// FP64 table: roles 1-3, one axis each (the recursion runs along k).
-// FP32 table (every k reduced and evaluated on its own): with 8 waves per
-// block, roles 1-6 write (axis, half of the k range), role 7 idles.
-__device__ __forceinline__ void phase_roles(const PhaseOut& ph, int i, int n, int role, int lane,
-                                            const double (&px)[4][64]) {
-    if (role == 0 || i >= ph.ld) return;
-    if (ph.mode == 1) {
-        if (role > 3) return;
-        const int axis = role - 1;
-        const double x = i < n ? px[axis][lane] : 0.0;
-        phase_axis64(x, ph.box.inv[axis], axis, ph.kmax, ph.tab, ph.ld, i);
-        if (axis == 0) ph.q[i] = i < n ? px[3][lane] : 0.0;
-    } else {
-        const int nsp = ((int)blockDim.x / 64 - 1) / 3;  // 1 (4 waves) or 2 (8 waves)
-        const int r = role - 1;
-        if (r >= 3 * nsp) return;
-        const int axis = r % 3, part = r / 3;
-        const int k0 = part * ph.kmax / nsp + 1, k1 = (part + 1) * ph.kmax / nsp;
-        const double x = i < n ? px[axis][lane] : 0.0;
-        phase_axis32(x, ph.box.inv[axis], axis, ph.kmax, ph.tab32, ph.ld, i, k0, k1);
-        if (axis == 0 && part == 0) ph.q32[i] = i < n ? (float)px[3][lane] : 0.f;
-    }
-}
-
-// VelocityVerlet first half (integrators.rs:47-53): the pending Berendsen
-// scale of the previous step (th.ke_part != null), then v += (dt/2) a;
-// x += v dt; the displacement test of the neighbour list (sets flags[0]);
-// and the phase table of the new position when `ph.mode` != 0.
-// Block = 64 atoms x 4 roles (FP64 table) or 8 roles (FP32 table): role 0
-// integrates, the others write the phase rows (phase_roles), so that the
-// trigonometry of an atom runs on three or six waves.  Grid:
-// ceil(max(n, ld) / 64).
-__global__ __launch_bounds__(512) void k_vv_first(double4* __restrict__ pos, double4* __restrict__ vel,
-                                                  const double4* __restrict__ acc, int n, double dt, Thermo th,
-                                                  const double4* __restrict__ ref, double half_skin2,
-                                                  int* __restrict__ flags, PhaseOut ph, CellTag tg) {
-    __shared__ double px[4][64];
-    const int lane = threadIdx.x & 63, role = threadIdx.x >> 6;
-    const int i = blockIdx.x * 64 + lane;
-    double l = th.ke_part ? berendsen_lambda(th) : 1.0;
-    if (role == 0) {
-        bool moved = false, bad = false;
-        double4 p = make_double4(0, 0, 0, 0);
-        if (i < n) {
-            double4 v = vel[i];
-            if (th.ke_part) {
-                v.x = v.x * l;
-                v.y = v.y * l;
-                v.z = v.z * l;
-            }
-            double4 a = acc[i];
-            double h = 0.5 * dt;
-            v.x += h * a.x;
-            v.y += h * a.y;
-            v.z += h * a.z;
-            p = pos[i];
-            p.x += v.x * dt;
-            p.y += v.y * dt;
-            p.z += v.z * dt;
-            vel[i] = v;
-            pos[i] = p;
-            moved = moved_beyond(p, ref, i, half_skin2);
-            bad = nonfinite3(p.x, p.y, p.z) || nonfinite3(v.x, v.y, v.z);
-            if (tg.tag) tg.tag[i] = cell_tag(tg, p);
-            if (tg.frac) tg.frac[i] = frac_pos(tg.b, tg.fo, p);
-        }
-        if (__any(moved) && lane == 0) atomicOr(flags, 1);
-        flag_nonfinite(bad, flags);
-        px[0][lane] = p.x;
-        px[1][lane] = p.y;
-        px[2][lane] = p.z;
-        px[3][lane] = p.w;
-    }
-    if (!ph.mode) return;  // uniform: a kernel argument
-    __syncthreads();
-    phase_roles(ph, i, n, role, lane, px);
-}
-
-// LeapFrog (integrators.rs:150-168), position part, after the pending
-// Berendsen scale of the previous step, with the displacement test and the
-// phase table as k_vv_first (same block layout).
-__global__ __launch_bounds__(512) void k_lf_first(double4* __restrict__ pos, double4* __restrict__ vel,
-                                                  const double4* __restrict__ acc, int n, double dt, Thermo th,
-                                                  const double4* __restrict__ ref, double half_skin2,
-                                                  int* __restrict__ flags, PhaseOut ph, CellTag tg) {
-    __shared__ double px[4][64];
-    const int lane = threadIdx.x & 63, role = threadIdx.x >> 6;
-    const int i = blockIdx.x * 64 + lane;
-    double l = th.ke_part ? berendsen_lambda(th) : 1.0;
-    if (role == 0) {
-        bool moved = false, bad = false;
-        double4 p = make_double4(0, 0, 0, 0);
-        if (i < n) {
-            double4 v = vel[i];
-            if (th.ke_part) {
-                v.x = v.x * l;
-                v.y = v.y * l;
-                v.z = v.z * l;
-                vel[i] = v;
-            }
-            double4 a = acc[i];
-            double dt2 = dt * dt;
-            p = pos[i];
-            p.x += v.x * dt + (0.5 * a.x) * dt2;
-            p.y += v.y * dt + (0.5 * a.y) * dt2;
-            p.z += v.z * dt + (0.5 * a.z) * dt2;
-            pos[i] = p;
-            moved = moved_beyond(p, ref, i, half_skin2);
-            bad = nonfinite3(p.x, p.y, p.z) || nonfinite3(v.x, v.y, v.z);
-            if (tg.tag) tg.tag[i] = cell_tag(tg, p);
-            if (tg.frac) tg.frac[i] = frac_pos(tg.b, tg.fo, p);
-        }
-        if (__any(moved) && lane == 0) atomicOr(flags, 1);
-        flag_nonfinite(bad, flags);
-        px[0][lane] = p.x;
-        px[1][lane] = p.y;
-        px[2][lane] = p.z;
-        px[3][lane] = p.w;
-    }
-    if (!ph.mode) return;
-    __syncthreads();
-    phase_roles(ph, i, n, role, lane, px);
-}
+// What a step's kernels read and write per atom.
+struct MdArgs {
+    double4* pos;
+    double4* vel;
+    double4* acc;
+    int n, lf;  // lf: LeapFrog, else VelocityVerlet
+    double dt;
+    const double4* ref;
+    double half_skin2;
+    int* flags;
+    CellTag tg;
+};
 
 // Second half of VelocityVerlet (integrators.rs:55-68) or LeapFrog
-// (:160-167).  The total force is the pair/intra-molecular force plus the
-// k-space partials q_i / (4 pi eps0) sum_g fk[g][i] (ewald.rs:716-719).
-// With a thermostat (ke_part != null), block partials of the kinetic energy
-// are written for k_berendsen.  Blocks of 64 atoms (one wave), so that the
-// loads of a small system spread over many CUs.
-template <bool kLeapFrog>
-__global__ __launch_bounds__(64) void k_md_second(const double4* __restrict__ force, const double4* __restrict__ pos,
-                                                   const double4* __restrict__ contrib,
-                                                   const int* __restrict__ slot_start,
-                                                   const double4* __restrict__ fk, int ksplit,
-                                                   double4* __restrict__ vel, double4* __restrict__ acc, int n,
-                                                   double dt, double* __restrict__ ke_part,
-                                                   int* __restrict__ flags) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+// (:160-167) from the total force f: new velocity and acceleration.
+__device__ __forceinline__ void md_kick(const MdArgs& m, double4 f, double4 a, double4& v, double4& na) {
+    const double ms = v.w;
+    na = make_double4(f.x / ms, f.y / ms, f.z / ms, 0.0);
+    if (m.lf) {
+        v.x += (0.5 * (a.x + na.x)) * m.dt;
+        v.y += (0.5 * (a.y + na.y)) * m.dt;
+        v.z += (0.5 * (a.z + na.z)) * m.dt;
+    } else {
+        const double h = 0.5 * m.dt;
+        v.x += h * na.x;
+        v.y += h * na.y;
+        v.z += h * na.z;
+    }
+}
+
+// First half: VelocityVerlet (integrators.rs:47-53) v += (dt/2) a, x += v dt;
+// LeapFrog (:150-158) x += v dt + (a/2) dt^2.
+__device__ __forceinline__ void md_drift(const MdArgs& m, double4 a, double4& v, double4& p) {
+    if (m.lf) {
+        const double dt2 = m.dt * m.dt;
+        p.x += v.x * m.dt + (0.5 * a.x) * dt2;
+        p.y += v.y * m.dt + (0.5 * a.y) * dt2;
+        p.z += v.z * m.dt + (0.5 * a.z) * dt2;
+    } else {
+        const double h = 0.5 * m.dt;
+        v.x += h * a.x;
+        v.y += h * a.y;
+        v.z += h * a.z;
+        p.x += v.x * m.dt;
+        p.y += v.y * m.dt;
+        p.z += v.z * m.dt;
+    }
+}
+
+// The new position and what goes beside it: the cell tag, the mixed form's
+// fractions, the displacement test of the neighbour list (flags[0]) and the
+// non-finite test.  All lanes of the wave; `live` lanes write.
+__device__ __forceinline__ void md_place(const MdArgs& m, int i, bool live, double4 p, double4 v, double4 r) {
+    bool moved = false, bad = false;
+    if (live) {
+        m.pos[i] = p;
+        const double dx = p.x - r.x, dy = p.y - r.y, dz = p.z - r.z;
+        moved = dx * dx + dy * dy + dz * dz > m.half_skin2;
+        bad = nonfinite3(p.x, p.y, p.z) || nonfinite3(v.x, v.y, v.z);
+        if (m.tg.tag) m.tg.tag[i] = cell_tag(m.tg, p);
+        if (m.tg.frac) m.tg.frac[i] = frac_pos(m.tg.b, m.tg.fo, p);
+    }
+    if (__any(moved) && (threadIdx.x & 63) == 0) atomicOr(m.flags, 1);
+    flag_nonfinite(bad, m.flags);
+}
+
+// First half of a step alone: the pending Berendsen scale of the previous
+// step (th.ke_part != null), then md_drift and md_place.
+constexpr int kMdBlock = 64;  // one wave: the loads of a small system spread over many CUs
+__global__ __launch_bounds__(kMdBlock) void k_md_first(MdArgs m, Thermo th) {
+    const int i = blockIdx.x * kMdBlock + threadIdx.x;
+    const bool live = i < m.n;
+    double4 p = make_double4(0, 0, 0, 0), v = p, a = p, r = p;
+    if (live) {
+        v = m.vel[i];
+        a = m.acc[i];
+        p = m.pos[i];
+        r = m.ref[i];
+    }
+    if (th.ke_part) {
+        const double l = th.lambda ? *th.lambda : berendsen_lambda(th);
+        v.x = v.x * l;
+        v.y = v.y * l;
+        v.z = v.z * l;
+    }
+    md_drift(m, a, v, p);
+    if (live && (!m.lf || th.ke_part)) m.vel[i] = v;
+    md_place(m, i, live, p, v, r);
+}
+
+// Second half alone.  The total force is the pair/intra-molecular force plus
+// the k-space partials (row form) q_i / (4 pi eps0) sum_g fk[g][i]
+// (ewald.rs:716-719).  With a thermostat (ke_part != null), block partials of
+// the kinetic energy are written for berendsen_lambda.
+__global__ __launch_bounds__(kMdBlock) void k_md_second(MdArgs m, const double4* __restrict__ force,
+                                                        const double4* __restrict__ contrib,
+                                                        const int* __restrict__ slot_start,
+                                                        const double4* __restrict__ fk, int ksplit,
+                                                        double* __restrict__ ke_part) {
+    const int i = blockIdx.x * kMdBlock + threadIdx.x;
     double ke = 0.0;
     bool bad = false;
-    if (i < n) {
-        double4 f = total_force(i, n, force, contrib, slot_start, fk, ksplit, pos);
-        double4 v = vel[i];
-        double m = v.w;
-        double4 na = make_double4(f.x / m, f.y / m, f.z / m, 0.0);
-        if (kLeapFrog) {
-            double4 a = acc[i];
-            v.x += (0.5 * (a.x + na.x)) * dt;
-            v.y += (0.5 * (a.y + na.y)) * dt;
-            v.z += (0.5 * (a.z + na.z)) * dt;
-        } else {
-            double h = 0.5 * dt;
-            v.x += h * na.x;
-            v.y += h * na.y;
-            v.z += h * na.z;
-        }
-        acc[i] = na;
-        vel[i] = v;
-        ke = 0.5 * m * (v.x * v.x + v.y * v.y + v.z * v.z);
+    if (i < m.n) {
+        const double4 f = total_force(i, m.n, force, contrib, slot_start, fk, ksplit, m.pos);
+        double4 v = m.vel[i], na;
+        md_kick(m, f, m.lf ? m.acc[i] : v, v, na);
+        m.acc[i] = na;
+        m.vel[i] = v;
+        ke = 0.5 * v.w * (v.x * v.x + v.y * v.y + v.z * v.z);
         bad = nonfinite3(v.x, v.y, v.z) || nonfinite3(na.x, na.y, na.z);
     }
-    flag_nonfinite(bad, flags);
+    flag_nonfinite(bad, m.flags);
     if (!ke_part) return;
     double s = wave_sum(ke);
     if (threadIdx.x == 0) ke_part[blockIdx.x] = s;
@@ -2980,80 +2560,32 @@ __global__ __launch_bounds__(64) void k_md_second(const double4* __restrict__ fo
 // The second half of step k and the first half of step k + 1 in one launch
 // (inside lg_md_run, without a thermostat: the first half then needs no
 // global kinetic energy).  The arithmetic of k_md_second followed by
-// k_vv_first / k_lf_first, in the same order, on the values those kernels
-// pass through memory: the same bits, one launch fewer per step.  Block
-// layout of the first-half kernels (64 atoms; the other waves write the
-// phase table).
-template <bool kLeapFrog>
-__global__ __launch_bounds__(512) void k_md_fused(const double4* __restrict__ force, double4* __restrict__ pos,
-                                                  const double4* __restrict__ contrib,
-                                                  const int* __restrict__ slot_start,
-                                                  const double4* __restrict__ fk, int ksplit,
-                                                  double4* __restrict__ vel, double4* __restrict__ acc, int n,
-                                                  double dt, const double4* __restrict__ ref, double half_skin2,
-                                                  int* __restrict__ flags, PhaseOut ph, CellTag tg) {
-    __shared__ double px[4][64];
-    const int lane = threadIdx.x & 63, role = threadIdx.x >> 6;
-    const int i = blockIdx.x * 64 + lane;
-    if (role == 0) {
-        bool moved = false, bad = false;
-        double4 p = make_double4(0, 0, 0, 0);
-        if (i < n) {
-            // second half of step k
-            double4 f = total_force(i, n, force, contrib, slot_start, fk, ksplit, pos);
-            double4 v = vel[i];
-            double m = v.w;
-            double4 na = make_double4(f.x / m, f.y / m, f.z / m, 0.0);
-            if (kLeapFrog) {
-                double4 a = acc[i];
-                v.x += (0.5 * (a.x + na.x)) * dt;
-                v.y += (0.5 * (a.y + na.y)) * dt;
-                v.z += (0.5 * (a.z + na.z)) * dt;
-            } else {
-                double h = 0.5 * dt;
-                v.x += h * na.x;
-                v.y += h * na.y;
-                v.z += h * na.z;
-            }
-            acc[i] = na;
-            // first half of step k + 1
-            p = pos[i];
-            if (kLeapFrog) {
-                double dt2 = dt * dt;
-                p.x += v.x * dt + (0.5 * na.x) * dt2;
-                p.y += v.y * dt + (0.5 * na.y) * dt2;
-                p.z += v.z * dt + (0.5 * na.z) * dt2;
-            } else {
-                double h = 0.5 * dt;
-                v.x += h * na.x;
-                v.y += h * na.y;
-                v.z += h * na.z;
-                p.x += v.x * dt;
-                p.y += v.y * dt;
-                p.z += v.z * dt;
-            }
-            vel[i] = v;
-            pos[i] = p;
-            moved = moved_beyond(p, ref, i, half_skin2);
-            bad = nonfinite3(p.x, p.y, p.z) || nonfinite3(v.x, v.y, v.z);
-            if (tg.tag) tg.tag[i] = cell_tag(tg, p);
-            if (tg.frac) tg.frac[i] = frac_pos(tg.b, tg.fo, p);
-        }
-        if (__any(moved) && lane == 0) atomicOr(flags, 1);
-        flag_nonfinite(bad, flags);
-        px[0][lane] = p.x;
-        px[1][lane] = p.y;
-        px[2][lane] = p.z;
-        px[3][lane] = p.w;
+// k_md_first, in the same order, on the values those kernels pass through
+// memory: the same bits, one launch fewer per step.
+__global__ __launch_bounds__(kMdBlock) void k_md_fused(MdArgs m, const double4* __restrict__ force,
+                                                       const double4* __restrict__ contrib,
+                                                       const int* __restrict__ slot_start,
+                                                       const double4* __restrict__ fk, int ksplit) {
+    const int i = blockIdx.x * kMdBlock + threadIdx.x;
+    const bool live = i < m.n;
+    double4 p = make_double4(0, 0, 0, 0), v = p, r = p;
+    if (live) {
+        const double4 f = total_force(i, m.n, force, contrib, slot_start, fk, ksplit, m.pos);
+        double4 na;
+        v = m.vel[i];
+        p = m.pos[i];
+        r = m.ref[i];
+        md_kick(m, f, m.lf ? m.acc[i] : v, v, na);
+        m.acc[i] = na;
+        md_drift(m, na, v, p);
+        m.vel[i] = v;
     }
-    if (!ph.mode) return;  // uniform: a kernel argument
-    __syncthreads();
-    phase_roles(ph, i, n, role, lane, px);
+    md_place(m, i, live, p, v, r);
 }
 
-// Berendsen factor of the last step of a run into *lambda (one block, same
-// sum as berendsen_lambda).
-__global__ __launch_bounds__(256) void k_berendsen(Thermo th, double* __restrict__ lambda) {
+// Berendsen factor of the last step into *lambda (one block: one wave up to
+// kThermoParts partials, as every block of k_md_first, else 1024 threads).
+__global__ __launch_bounds__(1024) void k_berendsen(Thermo th, double* __restrict__ lambda) {
     double l = berendsen_lambda(th);
     if (threadIdx.x == 0) *lambda = l;
 }
@@ -3067,6 +2599,141 @@ __global__ void k_scale_vel(double4* __restrict__ vel, int n, const double* __re
     v.y = v.y * l;
     v.z = v.z * l;
     vel[i] = v;
+}
+
+// ---- the octant form's part of a step -----------------------------------------------
+// Block = C atoms (a multiple of 16), 512 threads.  By `what`:
+//   OCT_FORCE   the k-space forces of the current positions (oct_force_sums)
+//               and, by one lane per atom, the total force; then `then`:
+//     OCT_COMBINE  force[i] = total force (and the k-space sums to fk)
+//     OCT_SECOND   the second half of a step (k_md_second)
+//     OCT_FUSED    the second half and the next first half (k_md_fused)
+//   OCT_FIRST   the first half of a step alone (k_md_first)
+//   OCT_RHO     the rho(k) partials of the positions that result (chunk =
+//               block), for the next evaluation
+// in the arithmetic of those kernels: an Ewald step has neither launches of
+// its own for the k-space forces and rho(k) nor a phase table in memory.  The
+// atoms' state is loaded while the phases are formed.  Bound by the matrix
+// cores from a few ten thousand atoms on, below by the latencies of its
+// stages, so the atoms are dealt to one block per CU (see oct_step_atoms).
+// Against the complex row recursion it replaces (phase table in HBM, rho
+// beside the list build, k-space forces and integrator apart), time per MD
+// step: SPC/E 9000 atoms, kmax 10: 55 -> 48 us mixed, 85 -> 73 us FP64; 36 000
+// atoms, kmax 16: 328 -> 151 us mixed (this kernel 79 us where the old ones
+// took 259); NaCl 4096 ions NVT, kmax 9: level.
+enum : int { OCT_COMBINE = 0, OCT_SECOND = 1, OCT_FUSED = 2 };
+enum : int { OCT_FORCE = 1, OCT_FIRST = 2, OCT_RHO = 4 };
+struct OctStep {
+    int what, then;
+    double4* force;
+    const double4* contrib;
+    const int* slot_start;
+    double4* fk;
+    double* ke_part;
+    MdArgs m;
+    Thermo th;
+};
+
+template <typename T>
+__host__ __device__ __forceinline__ size_t oct_step_rows(int kmax, int zcols, int C) {
+    const size_t b = (oct_lds<T>(kmax, zcols, C) + 31) / 32 * 32;
+    return b > kOctRed ? b : kOctRed;
+}
+template <typename T>
+__host__ __device__ __forceinline__ size_t oct_step_lds(int kmax, int zcols, int C) {
+    return oct_step_rows<T>(kmax, zcols, C) + size_t(24 + 32) * C;
+}
+
+template <typename T, int NST>
+__global__ __launch_bounds__(512, 2) void k_oct_step(OctForce a, OctStep s, OctRho ra, int C) {
+    // dynamic LDS: the rows (at least kOctRed), then res[3 C], then the
+    // current and later the new positions [C]
+    extern __shared__ __align__(16) unsigned char oct_smem[];
+    __shared__ double red[8][3][3][16];
+    T* sm = reinterpret_cast<T*>(oct_smem);
+    const size_t rows = oct_step_rows<T>(ra.kmax, ra.zcols, C);
+    double* res = reinterpret_cast<double*>(oct_smem + rows);
+    double4* pos_s = reinterpret_cast<double4*>(oct_smem + rows + size_t(24) * C);
+    const int blk = blockIdx.x, tid = threadIdx.x, n = s.m.n;
+    const int a0 = blk * C, na = min(C, n - a0);
+    const int i = a0 + tid;
+    const bool live = tid < na;
+    const bool whole = tid < (C + 63) / 64 * 64;  // the waves that hold the atoms' lanes
+    // one lane per atom holds its state; every load is issued before the
+    // first is waited for
+    double4 p = make_double4(0, 0, 0, 0), v = p, f = p, r = p, ac = p;
+    OctUnit<T, NST> first;
+    if (s.what & OCT_FORCE)
+        oct_load_unit<T, NST>(a, oct_unit0((C >> 4) * a.nrt, __builtin_amdgcn_readfirstlane(tid >> 6)) % a.nrt, first);
+    if (live) {
+        p = s.m.pos[i];
+        if ((s.what & OCT_FIRST) || ((s.what & OCT_FORCE) && s.then != OCT_COMBINE)) v = s.m.vel[i];
+        if ((s.what & OCT_FIRST) || s.then == OCT_FUSED) r = s.m.ref[i];
+        if ((s.what & OCT_FIRST) || ((s.what & OCT_FORCE) && s.m.lf)) ac = s.m.acc[i];
+        if (s.what & OCT_FORCE) f = total_force(i, n, s.force, s.contrib, s.slot_start, nullptr, 0, nullptr);
+    }
+    if (s.what & OCT_FIRST) {
+        if (s.th.ke_part) {
+            const double l = s.th.lambda ? *s.th.lambda : berendsen_lambda(s.th);
+            v.x = v.x * l;
+            v.y = v.y * l;
+            v.z = v.z * l;
+        }
+        if (whole) {
+            if (live) {
+                md_drift(s.m, ac, v, p);
+                if (!s.m.lf || s.th.ke_part) s.m.vel[i] = v;
+            }
+            md_place(s.m, i, live, p, v, r);
+        }
+    }
+    if (tid < C) pos_s[tid] = p;
+    __syncthreads();
+    if (s.what & OCT_FORCE) {
+        oct_stage_rows<T>(sm, ra.inv, ra.kmax, ra.zcols, C, na, [&](int at) { return pos_s[at]; });
+        __syncthreads();
+        oct_force_sums<T, NST>(a, ra.kmax, C, sm, red, res, first);
+        if (live) {
+            f.x += res[tid] / kFourPiEps0;
+            f.y += res[C + tid] / kFourPiEps0;
+            f.z += res[2 * C + tid] / kFourPiEps0;
+        }
+        if (s.then == OCT_COMBINE) {
+            if (live) {
+                s.force[i] = f;
+                if (s.fk) s.fk[i] = make_double4(res[tid], res[C + tid], res[2 * C + tid], 0.0);
+            }
+        } else if (whole) {
+            double4 na4 = make_double4(0, 0, 0, 0);
+            if (live) {
+                md_kick(s.m, f, ac, v, na4);
+                s.m.acc[i] = na4;
+            }
+            if (s.then == OCT_FUSED) {
+                if (live) {
+                    md_drift(s.m, na4, v, p);
+                    s.m.vel[i] = v;
+                    pos_s[tid] = p;
+                }
+                md_place(s.m, i, live, p, v, r);
+            } else {
+                if (live) s.m.vel[i] = v;
+                flag_nonfinite(live && (nonfinite3(v.x, v.y, v.z) || nonfinite3(na4.x, na4.y, na4.z)), s.m.flags);
+                if (s.ke_part) {
+                    const double ke = wave_sum(live ? 0.5 * v.w * (v.x * v.x + v.y * v.y + v.z * v.z) : 0.0);
+                    if ((tid & 63) == 0) s.ke_part[blk * ((C + 63) / 64) + (tid >> 6)] = ke;
+                }
+            }
+        }
+        __syncthreads();  // the new positions are in LDS, the old rows read
+    }
+    if (!(s.what & OCT_RHO)) return;
+    for (int grp = 0; grp < ra.ngroups; grp++) {
+        // one stage holds the chunk: its rows stand for every group, unless
+        // the sums over asplit take their LDS
+        if (grp > 0 && ra.asplit > 1) __syncthreads();
+        oct_rho_group<T>(ra, C, grp, blk, na, grp > 0 && ra.asplit == 1, sm, [&](int at) { return pos_s[at]; });
+    }
 }
 #pragma clang fp contract(on)
 

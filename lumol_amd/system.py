@@ -466,12 +466,13 @@ class System:
 
     def set_tuning(self, pair_lanes=0, kspace_split=0, rho_width=0, nlist_build=0, md_graph=0, rho_kind=0):
         """Launch knobs of the device kernels (0 = built-in choice); see
-        lumol_amd.tuning.autotune.  rho_width: atoms per block of the row form
-        of the rho(k) kernel; nlist_build: 1 lanes per atom, 2 one workgroup
-        per cell over the cell list, 3 direct (workgroups per cell over the
-        atoms' cell tags, up to 32768 atoms); md_graph: 1 eager launches (default), 2 HIP-graph replay of
-        MD chunks; rho_kind: 1 row form (phase rows staged in LDS), 2
-        matrix-core form (kmax <= 16), 3 row form without the staging."""
+        lumol_amd.tuning.autotune.  rho_width: atoms per block of the rho(k)
+        kernel (a quarter of it where the half-steps form rho); nlist_build: 1
+        lanes per atom, 2 one workgroup per cell over the cell list, 3 direct
+        (workgroups per cell over the atoms' cell tags, up to 32768 atoms);
+        md_graph: 1 eager launches (default), 2 HIP-graph replay of MD chunks;
+        rho_kind: 1, 2 or 3, one and the same octant form on the matrix cores
+        now (kept for saved choices)."""
         self.tuning_ = (int(pair_lanes), int(kspace_split), int(rho_width), int(nlist_build), int(md_graph),
                         int(rho_kind))
         if self._handle is not None and not self._dirty:

@@ -24,7 +24,7 @@ PAIR_LANES = (8, 16, 32, 64)
 KSPACE_SPLITS = (2, 4, 8, 16, 32)
 RHO_WIDTHS = (64, 128, 192, 256, 512)
 NLIST_BUILDS = (0, 2)  # automatic, cell list (lg_tuning.nlist_build)
-RHO_KINDS = (1, 2, 3)  # rows staged in LDS, matrix cores, rows from the table (lg_tuning.rho_kind)
+RHO_KINDS = (1, 2, 3)  # one octant form now (lg_tuning.rho_kind); timed as before for saved choices
 
 _cache = {}
 _lock = threading.Lock()
