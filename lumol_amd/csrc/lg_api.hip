@@ -420,6 +420,7 @@ struct lg_system {
     // h(r) = erfc(alpha r) + (2 alpha / sqrt(pi)) r exp(-alpha^2 r^2) on
     // [0, rc], FP32 pieces (hforce_ld); hf_ok when the fit met 1e-7
     DevBuf<float> hf32;
+    DevBuf<double> hf64;  // the same in FP64 pieces
     double hf_inv_h = 0.0;
     bool hf_ok = false;
     bool ecx_ok = false;
@@ -777,12 +778,12 @@ int prepare_meta(lg_system* s) {
 // A function f on [0, xmax] as kErfcxPieces polynomials of degree `deg` in
 // t in [-1, 1] per piece: the piece's Chebyshev interpolant (deg + 1
 // Chebyshev nodes, long double), expanded in powers of t.  Returns the
-// largest relative error against f (long double) over 64 points per piece.
+// largest relative (or absolute) error against f (long double) over 64 points per piece.
 // Used for erfcx(x) = exp(x^2) erfc(x) and for the real-space force factor
 // of the mixed pair kernel (hforce_ld).
 static long double erfcx_ld(long double x) { return erfcl(x) * expl(x * x); }
 template <typename T, typename F>
-static double fit_pieces(double xmax, int deg, F fn, std::vector<T>& out) {
+static double fit_pieces(double xmax, int deg, F fn, std::vector<T>& out, bool absolute = false) {
     const int M = kErfcxPieces, D = deg;
     const long double pi = 3.141592653589793238462643383279502884L;
     const long double h = (long double)xmax / M;
@@ -822,7 +823,7 @@ static double fit_pieces(double xmax, int deg, F fn, std::vector<T>& out) {
             long double p = (long double)out[size_t(k) * (D + 1) + D];
             for (int q = D - 1; q >= 0; q--) p = p * t + (long double)out[size_t(k) * (D + 1) + q];
             const long double ref = fn(mid + half * t);
-            worst = std::max(worst, double(fabsl(p - ref) / ref));
+            worst = std::max(worst, double(fabsl(p - ref) / (absolute ? 1.0L : ref)));
         }
     }
     return worst;
@@ -832,7 +833,8 @@ static double fit_pieces(double xmax, int deg, F fn, std::vector<T>& out) {
 // stream of one water model) fit once.  A fit is a pure function of the key,
 // so a cached table is the table the fit would return.
 template <typename T, typename F>
-static double fit_cached(int fn_id, double param, double xmax, int deg, F fn, std::vector<T>& out) {
+static double fit_cached(int fn_id, double param, double xmax, int deg, F fn, std::vector<T>& out,
+                         bool absolute = false) {
     using Key = std::tuple<int, uint64_t, uint64_t, int>;
     static std::mutex mu;
     static std::map<Key, std::pair<std::vector<T>, double>> cache;
@@ -848,7 +850,7 @@ static double fit_cached(int fn_id, double param, double xmax, int deg, F fn, st
             return it->second.second;
         }
     }
-    const double err = fit_pieces(xmax, deg, fn, out);
+    const double err = fit_pieces(xmax, deg, fn, out, absolute);
     std::lock_guard<std::mutex> lk(mu);
     cache.emplace(key, std::make_pair(out, err));
     return err;
@@ -859,10 +861,21 @@ static double fit_erfcx(double xmax, int deg, std::vector<T>& out) {
 }
 
 
+// Least double x with sqrt(x) >= rc (sqrt(x) > rc when `beyond`): the square
+// root rounds monotonically, so the reference's cutoff tests on r = sqrt(x)
+// are tests of x.
+double r2_bound(double rc, bool beyond) {
+    auto out = [&](double x) { return beyond ? std::sqrt(x) > rc : std::sqrt(x) >= rc; };
+    double x = rc * rc;
+    while (out(x) && x > 0.0) x = std::nextafter(x, 0.0);
+    while (!out(x)) x = std::nextafter(x, INFINITY);
+    return x;
+}
+
 int prepare_params(lg_system* s) {
     uint32_t K = s->nkinds;
     if (K > uint32_t(kMaxKinds)) return fail(LG_E_UNSUPPORTED, "more than 16 particle kinds");
-    s->h_table.assign(size_t(K) * K, PairParam{POT_NONE, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0});
+    s->h_table.assign(size_t(K) * K, PairParam{POT_NONE, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0});
     std::vector<int> restr(size_t(K) * K, 0);
     std::vector<double> s14(size_t(K) * K, 1.0);
     std::vector<double> tabs;
@@ -889,6 +902,7 @@ int prepare_params(lg_system* s) {
             pp.p3 = p.v.p[3];
             pp.p4 = p.v.p[4];
             pp.rc = p.rc;
+            pp.r2c = r2_bound(p.rc, false);
             pp.tab_n = int(p.v.tab_n);
             pp.tab_off = tab_off;
             pp.tab_delta = p.v.tab_n > 0 ? p.v.tab_max / double(p.v.tab_n) : 0.0;
@@ -908,6 +922,7 @@ int prepare_params(lg_system* s) {
     c.kind = s->coul_kind;
     c.inter_excl = s->coul_restr == LG_RESTRICT_INTRA ? 1 : 0;
     c.rc = s->coul_rc;
+    c.r2c = r2_bound(s->coul_rc, true);
     if (s->coul_kind == COUL_EWALD) {
         c.alpha = s->coul_alpha;
     } else if (s->coul_kind == COUL_WOLF) {
@@ -943,9 +958,14 @@ int prepare_params(lg_system* s) {
         const double rmax = c.rc * (1.0 + 1e-9);
         std::vector<float> th;
         const double eh = fit_cached(1, c.alpha, rmax, kErfcxDeg32, hforce_ld, th);
+        // FP64: the largest error against h itself, whose tail (5e-5 at the
+        // cutoff) a relative bound would overrate
+        std::vector<double> th64;
+        const double eh64 = fit_cached(2, c.alpha, rmax, kErfcxDeg64, hforce_ld, th64, true);
         s->hf_ok = false;
-        if (s->ecx_ok && eh < 1e-7) {
+        if (s->ecx_ok && eh < 1e-7 && eh64 < 2e-15) {
             LG_TRY(upload(s->hf32, th, S(s)));
+            LG_TRY(upload(s->hf64, th64, S(s)));
             s->hf_inv_h = kErfcxPieces / rmax;
             s->hf_ok = true;
         }
@@ -1418,11 +1438,17 @@ static OctRho oct_rho_args(const lg_system* s, bool mixed) {
     return a;
 }
 template <typename T>
-static void launch_rho_oct(lg_system* s, const OctRho& ra, int grid) {
+static void launch_rho_oct(lg_system* s, const OctRho& ra, int grid, bool energy, int intra_blocks,
+                           const IntraArgs& ia) {
     int sa = std::min(128, ra.width);
     while (sa > 16 && oct_lds<T>(ra.kmax, ra.zcols, sa) > kOctRhoLds) sa -= 16;
-    const size_t lds = std::max(kOctRed, oct_lds<T>(ra.kmax, ra.zcols, sa));
-    launch_timed(s, LG_KERNEL_KSPACE_RHO, k_rho_oct<T>, grid, 512, uint32_t(lds), ra, sa, s->pos.p, int(s->n));
+    const uint32_t lds = uint32_t(std::max(kOctRed, oct_lds<T>(ra.kmax, ra.zcols, sa)));
+    auto go = [&](auto kernel) {
+        launch_timed(s, LG_KERNEL_KSPACE_RHO, kernel, grid + intra_blocks, 512, lds, ra, sa, s->pos.p, int(s->n),
+                     grid, ia);
+    };
+    if (energy) go(k_rho_oct<T, true>);
+    else go(k_rho_oct<T, false>);
 }
 
 // k_oct_step: NST by the steps of the longest row (0 above eight steps).
@@ -1539,9 +1565,9 @@ int launch_nlist(lg_system* s, bool check, bool energy) {
                       s->nbr.p, s->nnbr.p, s->ref.p, s->sorted.p, flag, direct_split(s)};
         const bool nearest = s->periodic && (g.reach[0] == 0 || g.reach[1] == 0 || g.reach[2] == 0);
         prof_stop(s, prof);
-        // mixed form, forces only: the intra-molecular terms ride as the last
-        // blocks of this launch, which most steps leave empty
-        s->intra_done = !energy && s->precision == LG_PRECISION_MIXED && !s->gen_pairs && s->nterms > 0;
+        // forces only: the intra-molecular terms ride as the last blocks of
+        // this launch, which most steps leave empty
+        s->intra_done = !energy && !s->gen_pairs && s->nterms > 0;
         if (s->intra_done) {
             const int ncb = direct_blocks(s), fib = blocks_for(s->nterms, kCellBlock);
             auto go = [&](auto kernel) {
@@ -1629,8 +1655,11 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
             const OctRho ra = oct_rho_args(s, mixed);
             const int grid = int(xcd_grid(ra.ngroups, ra.nchunks));
             s->rho_nchunks = ra.nchunks;
-            if (mixed) launch_rho_oct<float>(s, ra, grid);
-            else launch_rho_oct<double>(s, ra, grid);
+            // the intra-molecular terms ride along, unless the list launch ran them
+            const int ib = s->nterms > 0 && !s->gen_pairs && !s->intra_done ? blocks_for(s->nterms, 512) : 0;
+            if (mixed) launch_rho_oct<float>(s, ra, grid, energy, ib, intra_args(s));
+            else launch_rho_oct<double>(s, ra, grid, energy, ib, intra_args(s));
+            if (ib > 0) s->intra_done = true;
         }
         nchunks = s->rho_nchunks;
     } else if (kspace) {
@@ -1671,6 +1700,8 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
     pa.ecx32 = s->ecx_ok ? s->ecx32.p : nullptr;
     pa.ecx_inv_h = s->ecx_inv_h;
     pa.hf32 = s->hf_ok ? s->hf32.p : nullptr;
+    pa.hf64 = s->hf_ok ? s->hf64.p : nullptr;
+    pa.tie = s->periodic && max_cutoff(s) > (0.5 - 1e-6) * std::min(s->L[0], std::min(s->L[1], s->L[2]));
     pa.hf_inv_h = s->hf_inv_h;
     pa.frac = s->frac.p;
     if (mixed && !s->gen_pairs && !frac_done) {
@@ -1679,9 +1710,9 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
         launch_timed(s, LG_KERNEL_PAIRS, k_frac, blocks_for(n, 256), 256, 0, s->pos.p, n, s->box, s->frac_origin,
                      s->frac.p);
     }
-    // the intra-molecular terms run as the last blocks of the pair launch
-    // (FP64 form), of the list launch (mixed form, forces only, direct build:
-    // intra_done) or in a launch of their own
+    // the intra-molecular terms run as the last blocks of the list launch
+    // (forces only, direct build) or of the rho(k) launch (intra_done), of
+    // the general pair launch, or in a launch of their own
     IntraArgs& ia = pa.intra;
     ia = intra_args(s);
     const int iblocks = s->nterms > 0 ? blocks_for(s->nterms, 256) : 0;
@@ -1718,9 +1749,7 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
         rr.vfac = s->vfac.p;
         rr.epart = epk;
     }
-    // the mixed instance leaves the intra-molecular terms to a launch of
-    // their own (see k_pairs_mixed)
-    const bool intra_apart = mixed && !s->gen_pairs;
+    const bool intra_apart = !s->gen_pairs;
     if (intra_apart && iblocks > 0 && !s->intra_done) {
         if (energy)
             launch_timed(s, LG_KERNEL_MOLECULES, k_intra_terms<true>, iblocks, 256, 0, ia);
@@ -1732,37 +1761,38 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
     pa.intra_blocks = intra_apart ? 0 : iblocks;
     const int nblocks = pblocks + pa.intra_blocks + rblocks;
     const int ck = coulomb_variant(s->coul);
-#define LG_PAIRS_CK(T, CK)                                                      \
+    const bool lib = !s->hf_ok;  // FP64: the tables of h and erfcx missed their bound
+#define LG_PAIRS_CK(T, CK, LIB)                                                 \
     if (ck == CK) {                                                             \
         if (mixed && energy)                                                    \
             launch_timed(s, LG_KERNEL_PAIRS, k_pairs_mixed<true, T, CK>, nblocks, kPairBlock, 0, pa);     \
         else if (mixed)                                                         \
             launch_timed(s, LG_KERNEL_PAIRS, k_pairs_mixed<false, T, CK>, nblocks, kPairBlock, 0, pa);    \
         else if (energy)                                                        \
-            launch_timed(s, LG_KERNEL_PAIRS, k_pairs<true, T, CK>, nblocks, kPairBlock, 0, pa);           \
+            launch_timed(s, LG_KERNEL_PAIRS, lib ? k_pairs<true, T, LIB> : k_pairs<true, T, CK>, nblocks, kPairBlock, 0, pa);   \
         else                                                                    \
-            launch_timed(s, LG_KERNEL_PAIRS, k_pairs<false, T, CK>, nblocks, kPairBlock, 0, pa);          \
+            launch_timed(s, LG_KERNEL_PAIRS, lib ? k_pairs<false, T, LIB> : k_pairs<false, T, CK>, nblocks, kPairBlock, 0, pa); \
     }
 #define LG_PAIRS_CASE(T)                 \
     case T:                              \
-        LG_PAIRS_CK(T, CK_NONE)          \
-        LG_PAIRS_CK(T, CK_EWALD)         \
-        LG_PAIRS_CK(T, CK_EWALD_ERF)     \
-        LG_PAIRS_CK(T, CK_WOLF)          \
+        LG_PAIRS_CK(T, CK_NONE, CK_NONE)          \
+        LG_PAIRS_CK(T, CK_EWALD, CK_EWALD_LIB)         \
+        LG_PAIRS_CK(T, CK_EWALD_ERF, CK_EWALD_ERF)     \
+        LG_PAIRS_CK(T, CK_WOLF, CK_WOLF_LIB)          \
         break;
     if (s->gen_pairs) {
         // any pair potential kind or a table: the general FP64 instance, in
         // both forms
         if (energy) {
-            if (ck == CK_NONE) launch_timed(s, LG_KERNEL_PAIRS, k_pairs<true, 16, CK_NONE, true>, nblocks, kPairBlock, 0, pa);
-            if (ck == CK_EWALD) launch_timed(s, LG_KERNEL_PAIRS, k_pairs<true, 16, CK_EWALD, true>, nblocks, kPairBlock, 0, pa);
-            if (ck == CK_EWALD_ERF) launch_timed(s, LG_KERNEL_PAIRS, k_pairs<true, 16, CK_EWALD_ERF, true>, nblocks, kPairBlock, 0, pa);
-            if (ck == CK_WOLF) launch_timed(s, LG_KERNEL_PAIRS, k_pairs<true, 16, CK_WOLF, true>, nblocks, kPairBlock, 0, pa);
+            if (ck == CK_NONE) launch_timed(s, LG_KERNEL_PAIRS, k_pairs_gen<true, 16, CK_NONE>, nblocks, kPairBlock, 0, pa);
+            if (ck == CK_EWALD) launch_timed(s, LG_KERNEL_PAIRS, k_pairs_gen<true, 16, CK_EWALD>, nblocks, kPairBlock, 0, pa);
+            if (ck == CK_EWALD_ERF) launch_timed(s, LG_KERNEL_PAIRS, k_pairs_gen<true, 16, CK_EWALD_ERF>, nblocks, kPairBlock, 0, pa);
+            if (ck == CK_WOLF) launch_timed(s, LG_KERNEL_PAIRS, k_pairs_gen<true, 16, CK_WOLF>, nblocks, kPairBlock, 0, pa);
         } else {
-            if (ck == CK_NONE) launch_timed(s, LG_KERNEL_PAIRS, k_pairs<false, 16, CK_NONE, true>, nblocks, kPairBlock, 0, pa);
-            if (ck == CK_EWALD) launch_timed(s, LG_KERNEL_PAIRS, k_pairs<false, 16, CK_EWALD, true>, nblocks, kPairBlock, 0, pa);
-            if (ck == CK_EWALD_ERF) launch_timed(s, LG_KERNEL_PAIRS, k_pairs<false, 16, CK_EWALD_ERF, true>, nblocks, kPairBlock, 0, pa);
-            if (ck == CK_WOLF) launch_timed(s, LG_KERNEL_PAIRS, k_pairs<false, 16, CK_WOLF, true>, nblocks, kPairBlock, 0, pa);
+            if (ck == CK_NONE) launch_timed(s, LG_KERNEL_PAIRS, k_pairs_gen<false, 16, CK_NONE>, nblocks, kPairBlock, 0, pa);
+            if (ck == CK_EWALD) launch_timed(s, LG_KERNEL_PAIRS, k_pairs_gen<false, 16, CK_EWALD>, nblocks, kPairBlock, 0, pa);
+            if (ck == CK_EWALD_ERF) launch_timed(s, LG_KERNEL_PAIRS, k_pairs_gen<false, 16, CK_EWALD_ERF>, nblocks, kPairBlock, 0, pa);
+            if (ck == CK_WOLF) launch_timed(s, LG_KERNEL_PAIRS, k_pairs_gen<false, 16, CK_WOLF>, nblocks, kPairBlock, 0, pa);
         }
     } else switch (s->tpa) {
         LG_PAIRS_CASE(4)
@@ -2186,6 +2216,7 @@ int lg_system_destroy(lg_system* s) {
     s->ecx64.release();
     s->ecx32.release();
     s->hf32.release();
+    s->hf64.release();
     s->phase_tab.release();
     s->phase_q.release();
     s->phase_tab32.release();

@@ -58,6 +58,7 @@ struct PairParam {
     double p2, p3, p4;
     int tab_n, tab_off;
     double tab_delta;
+    double r2c;        // least double whose square root is >= rc: r < rc as r^2 < r2c
 };
 
 // The fields of PairParam that the LJ/Harmonic/Null pair kernels read
@@ -92,6 +93,7 @@ struct CoulParam {
     int inter_excl;    // restriction excludes inter-molecular pairs
     double alpha, rc;
     double e_const, f_const;  // Wolf energy_constant / force_constant
+    double r2c;               // least double whose square root is > rc: r <= rc as r^2 < r2c
 };
 
 // Orthorhombic cell: lengths and reciprocal lengths.
@@ -122,6 +124,9 @@ __device__ __forceinline__ void min_image(const Box& b, double& dx, double& dy, 
         dz = image1(dz, b.L[2], b.inv[2]);
     }
 }
+
+// image1 without its check of near-halves (see PairArgs.tie).
+__device__ __forceinline__ double image_rint(double d, double L, double inv) { return d - rint(d * inv) * L; }
 
 // Minimum image for the mixed form, whose distance is rounded to FP32 next:
 // d - rint(d / a) a with the reciprocal, 3 operations per axis.  It differs

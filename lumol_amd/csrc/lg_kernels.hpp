@@ -1051,11 +1051,12 @@ struct IntraArgs {
     double* epart;     // per block: pairs, coul, bonds, angles, dihedrals, w6
 };
 
-// One block (256 threads) of intra-molecular terms, block index `blk`: run as
-// its own kernel or as the extra blocks of a pair-kernel launch.
+// One block of intra-molecular terms, block index `blk`: run as its own kernel
+// or as extra blocks of another launch.  Energy partials: one set per 256
+// terms (blocks of 256 or 512 threads).
 template <bool kEnergy>
 __device__ __forceinline__ void intra_block(const IntraArgs& a, int blk) {
-    __shared__ double red[4][11];
+    __shared__ double red[8][11];
     int t = blk * blockDim.x + threadIdx.x;
     double acc[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     if (t < a.nterms) {
@@ -1212,10 +1213,12 @@ __device__ __forceinline__ void intra_block(const IntraArgs& a, int blk) {
             if (lane == 0) red[wid][q] = sum;
         }
         __syncthreads();
-        if (threadIdx.x < 11) {
+        const int set = threadIdx.x >> 8, q = threadIdx.x & 255;
+        const int at = blk * (int)(blockDim.x >> 8) + set;
+        if (q < 11 && at * 256 < a.nterms) {
             double sum = 0;
-            for (int w = 0; w < 4; w++) sum += red[w][threadIdx.x];
-            a.epart[blk * 11 + threadIdx.x] = sum;
+            for (int w = 0; w < 4; w++) sum += red[4 * set + w][q];
+            a.epart[at * 11 + q] = sum;
         }
     }
 }
@@ -1261,11 +1264,11 @@ struct RhoReduceArgs {
 // One block (256 threads) of the reduction, block index `blk`: run as its
 // own kernel or as the last blocks of a pair-kernel launch.
 template <bool kEnergy>
-__device__ __forceinline__ void rho_reduce_block(const RhoReduceArgs& a, int blk) {
+__device__ __forceinline__ void rho_reduce_block(const RhoReduceArgs& a, int blk, unsigned char* lds) {
     const double2* __restrict__ partial = a.partial;
     const int nchunks = a.nchunks, nslot = a.nslot, nk = a.nk;
     constexpr int G = 256 / kRhoReduceK;
-    __shared__ double2 part[G][kRhoReduceK];
+    double2(*part)[kRhoReduceK] = reinterpret_cast<double2(*)[kRhoReduceK]>(lds);
     int g = threadIdx.x / kRhoReduceK, kl = threadIdx.x % kRhoReduceK;
     int k = blk * kRhoReduceK + kl;
     double re = 0.0, im = 0.0;
@@ -1312,11 +1315,6 @@ __device__ __forceinline__ void rho_reduce_block(const RhoReduceArgs& a, int blk
     }
 }
 
-template <bool kEnergy>
-__global__ __launch_bounds__(256) void k_rho_reduce(RhoReduceArgs a) {
-    rho_reduce_block<kEnergy>(a, blockIdx.x);
-}
-
 // ---------------------------------------------------------------------------------
 // Non-bonded pair kernel: inter-molecular pairs, Lennard-Jones family + Ewald
 // real space or Wolf, one lane per atom i over its neighbour list.
@@ -1351,6 +1349,8 @@ struct PairArgs {
     const double* ecx64;
     const float* ecx32;
     double ecx_inv_h;
+    const double* hf64;  // h(r) as hf32 below, in FP64 pieces, or null
+    int tie;             // a cutoff reaches half the box: images within 1e-9 of a tie are checked
     const double* tabs;  // TableComputation tables (general instance)
     const float4* frac;  // positions as frac_pos (mixed instance)
     // the real-space force factor h(r) = erfc(alpha r) + g0 r exp(-alpha^2 r^2)
@@ -1360,11 +1360,11 @@ struct PairArgs {
 };
 
 template <bool kEnergy>
-__device__ __forceinline__ void kspace_reduce_block(const PairArgs& a, int blk) {
+__device__ __forceinline__ void kspace_reduce_block(const PairArgs& a, int blk, unsigned char* lds) {
     if (a.oct)
-        oct_reduce_block<kEnergy>(a.orr, blk);
+        oct_reduce_block<kEnergy>(a.orr, blk, lds);
     else
-        rho_reduce_block<kEnergy>(a.rr, blk);
+        rho_reduce_block<kEnergy>(a.rr, blk, lds);
 }
 
 constexpr int kMaxKinds = 16;
@@ -1384,7 +1384,8 @@ __device__ __forceinline__ int xcd_contiguous(int b, int P) { return (b & 7) * (
 // excludes (the -erf removal term only), Wolf.  A Wolf system whose
 // restriction excludes the pairs uses CK_NONE.  One variant per instance
 // keeps the registers of the unused paths out of the kernel.
-enum : int { CK_NONE = 0, CK_EWALD = 1, CK_EWALD_ERF = 2, CK_WOLF = 3 };
+// The last two: Ewald and Wolf whose tables missed their bound (FP64 form).
+enum : int { CK_NONE = 0, CK_EWALD = 1, CK_EWALD_ERF = 2, CK_WOLF = 3, CK_EWALD_LIB = 4, CK_WOLF_LIB = 5 };
 
 __host__ __forceinline__ int coulomb_variant(const CoulParam& c) {
     if (c.kind == COUL_EWALD) return c.inter_excl ? CK_EWALD_ERF : CK_EWALD;
@@ -1392,18 +1393,214 @@ __host__ __forceinline__ int coulomb_variant(const CoulParam& c) {
     return CK_NONE;
 }
 
-// TPA lanes share one atom i and stride through its neighbour row; the
-// group's partial forces are combined with xor-shuffles (TPA divides 64).
-// Held to 128 VGPRs (four waves per SIMD instead of three): the kernel waits
-// on its gathers most of the time, and the extra resident wave outweighs the
-// few spilled registers (SPC/E FP64 pairs 44 -> 40 us per launch).
-// kGen: the general instance for systems with a pair potential other than
-// LJ/Harmonic/Null or a TableComputation (any kind, FP64, both forms); the
-// fast instances stage only the LJ/Harmonic fields.
-template <bool kEnergy, int TPA, int CK, bool kGen = false>
-__global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_pairs(PairArgs a) {
-    using TabEntry = typename std::conditional<kGen, PairParam, PairFast>::type;
-    __shared__ TabEntry tab[kMaxKinds * kMaxKinds];
+// 1 / sqrt(x) to about an ulp: the hardware estimate and two Newton steps.
+__device__ __forceinline__ double rsqrt_newton(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    double t = x * y;
+    double e = 0.5 - 0.5 * t * y;
+    y = y + y * e;
+    t = x * y;
+    e = 0.5 - 0.5 * t * y;
+    return y + y * e;
+}
+
+// The pair kernel of LJ/Harmonic/Null systems, FP64.  TPA lanes share one
+// atom i and stride through its neighbour row; the group's partial forces
+// are combined with xor-shuffles (TPA divides 64).
+//
+// Bound by the vector ALU, so it is written for few FP64 instructions per
+// list entry:
+// * the minimum image by rint(d / L) (image1's check of near-halves only
+//   where a cutoff reaches half the box, a.tie: elsewhere a component within
+//   1e-9 of a tie puts the pair beyond every cutoff, whichever image), with
+//   the difference and the norm unfused as the reference rounds them;
+// * the cutoffs as tests of r^2 against the least double whose square root
+//   fails the reference's test (`r < rc`, `r <= rc`; the square root rounds
+//   monotonically), so the pair set stays the reference's without a root;
+// * 1 / r by the hardware estimate and Newton steps, no root or division;
+// * Lennard-Jones as (A r^-6 - B) r^-8, formed for every pair and selected;
+// * the real-space Ewald or Wolf force as h(r) r^-3 with h(r) = erfc(alpha r)
+//   + (2 alpha / sqrt(pi)) r exp(-alpha^2 r^2) from a table of polynomial
+//   pieces (no exponential); energies keep exp(-x^2) erfcx(x).
+// SPC/E, 9000 atoms: 41 -> 21 us per launch against the reference's order with
+// library root, division and exponential.
+template <bool kEnergy, int TPA, int CK>
+__global__ __launch_bounds__(kPairBlock) void k_pairs(PairArgs a) {
+    struct alignas(16) Lj {
+        double A, B, r2c, shift;  // 48 eps s^12, 24 eps s^6, cutoff test (0: no term), energy shift
+    };
+    // the reduction blocks use the tables' LDS (residency is set by it)
+    __shared__ __align__(32) unsigned char lds[(sizeof(Lj) + sizeof(double2)) * kMaxKinds * kMaxKinds];
+    Lj* const ljt = reinterpret_cast<Lj*>(lds);
+    double2* const hmt = reinterpret_cast<double2*>(lds + sizeof(Lj) * kMaxKinds * kMaxKinds);  // Harmonic {k, x0}, k = 0 otherwise
+    __shared__ double red[kPairBlock / 64][8];
+    constexpr bool kTab = CK == CK_EWALD || CK == CK_WOLF;
+    __shared__ __align__(16) double hft[kTab ? kErfcxPieces * (kErfcxDeg64 + 1) : 2];
+    __shared__ __align__(16) double ecx[kTab && kEnergy ? kErfcxPieces * (kErfcxDeg64 + 1) : 2];
+    if ((int)blockIdx.x >= a.pair_blocks) {  // uniform over the block
+        kspace_reduce_block<kEnergy>(a, blockIdx.x - a.pair_blocks, lds);
+        return;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.rebuild) *a.rebuild = 0;
+    const int nk2 = a.nkinds * a.nkinds;
+    int harmonic = 0;
+    for (int x = threadIdx.x; x < nk2; x += blockDim.x) {
+        const PairParam pp = a.table[x];
+        const bool on = pp.pot > POT_NULL && !pp.inter_excl, lj = pp.pot == POT_LJ;
+        const double s2 = pp.p0 * pp.p0, s6 = lj ? s2 * s2 * s2 : 0.0;
+        ljt[x] = Lj{lj ? 48.0 * pp.p1 * (s6 * s6) : 0.0, lj ? 24.0 * pp.p1 * s6 : 0.0, on ? pp.r2c : 0.0, pp.shift};
+        const bool hm = on && pp.pot == POT_HARMONIC;
+        hmt[x] = make_double2(hm ? pp.p0 : 0.0, hm ? pp.p1 : 0.0);
+        harmonic |= hm;
+    }
+    if (kTab) {
+        constexpr int n2 = kErfcxPieces * (kErfcxDeg64 + 1) / 2;
+        for (int x = threadIdx.x; x < n2; x += blockDim.x) {
+            reinterpret_cast<double2*>(hft)[x] = reinterpret_cast<const double2*>(a.hf64)[x];
+            if (kEnergy) reinterpret_cast<double2*>(ecx)[x] = reinterpret_cast<const double2*>(a.ecx64)[x];
+        }
+    }
+    harmonic = __syncthreads_or(harmonic);  // also the barrier of the LDS tables
+
+    // XCD-contiguous order of the pair blocks (the launch has a multiple of 8)
+    const int g = xcd_contiguous(blockIdx.x, a.pair_blocks) * blockDim.x + threadIdx.x;
+    const int t = g / TPA, sub = g % TPA;
+    double fx = 0, fy = 0, fz = 0;
+    double e_pair = 0, e_coul = 0;
+    double wxx = 0, wyy = 0, wzz = 0, wxy = 0, wxz = 0, wyz = 0;
+    int i = -1;
+    if (t < a.n) {
+        i = a.sorted[t];
+        const double4 pi = a.pos[i];
+        const int ki = a.meta[i].x;
+        const double qi = pi.w / kFourPiEps0;
+        const int nn = a.nnbr[t];
+        const CoulParam& c = a.coul;
+        const int* row = a.nbr + (size_t)t * a.cap;
+        const Lj* ljrow = ljt + ki * a.nkinds;
+        const double2* hmrow = hmt + ki * a.nkinds;
+        const double Lx = a.box.L[0], Ly = a.box.L[1], Lz = a.box.L[2];
+        const double ix = a.box.inv[0], iy = a.box.inv[1], iz = a.box.inv[2];  // 0 in an infinite cell
+        // Software pipeline over the row: the row entries two passes ahead
+        // and the next pass's neighbour positions are loaded while the
+        // current pair is evaluated, unrolled by two on alternating
+        // registers (A, B); an entry carries the neighbour's kind.  Entries
+        // past the row end read a clamped index and stand for atom i
+        // itself, never evaluated.
+        auto jat = [&](int k) {
+            int v = row[min(k, max(nn - 1, 0))];
+            return k < nn ? v : nbr_entry(i, ki);
+        };
+        auto pair = [&](int j, const double4& pj, int kj) {
+            double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
+            if (a.tie) {  // uniform
+                min_image(a.box, dx, dy, dz);
+            } else {
+                dx = image_rint(dx, Lx, ix);
+                dy = image_rint(dy, Ly, iy);
+                dz = image_rint(dz, Lz, iz);
+            }
+            const double r2 = norm2_ordered(dx, dy, dz);
+            const double inv_r = rsqrt_newton(r2), i2 = inv_r * inv_r, i6 = i2 * i2 * i2;
+            const Lj P = ljrow[kj];
+            const bool in_pair = r2 < P.r2c;
+            double fp = (P.A * i6 - P.B) * (i6 * i2), e_p = 0.0, e_c = 0.0;
+            if (kEnergy) e_p = i6 * (P.A * (1.0 / 12.0) * i6 - P.B * (1.0 / 6.0));
+            if (harmonic) {  // uniform
+                const double2 H = hmrow[kj];
+                const double r = r2 * inv_r;
+                fp += H.x * (H.y - r) * inv_r;
+                if (kEnergy) e_p += 0.5 * H.x * (r - H.y) * (r - H.y);
+            }
+            double fs = in_pair ? fp : 0.0;
+            if (kEnergy) e_p = in_pair ? e_p - P.shift : 0.0;
+            if (CK != CK_NONE) {
+                const double pref = qi * pj.w;  // 0 adds an exact 0
+                const bool in_coul = r2 < c.r2c;
+                const double r = r2 * inv_r;
+                double fc, ec = 0.0;
+                if constexpr (kTab) {
+                    const double h3 = erfcx_tab(hft, r, a.hf_inv_h) * (inv_r * i2);
+                    fc = CK == CK_EWALD ? pref * h3 : pref * (h3 - c.f_const * inv_r);
+                    if (kEnergy) {
+                        const double x = c.alpha * r;
+                        const double er = exp(-x * x) * erfcx_tab(ecx, x, a.ecx_inv_h) * inv_r;
+                        ec = CK == CK_EWALD ? pref * er : pref * (er - c.e_const);
+                    }
+                } else if (in_coul) {
+                    // the library's erf and erfc
+                    if (CK == CK_WOLF_LIB)
+                        wolf_pair(c, qi * kFourPiEps0 * pj.w, r, inv_r, ec, fc);
+                    else
+                        ewald_real(c.alpha, qi * kFourPiEps0 * pj.w, r, inv_r, CK == CK_EWALD_ERF, ec, fc);
+                } else {
+                    fc = 0.0;
+                }
+                const bool on = in_coul && pref != 0.0;
+                fs += on ? fc : 0.0;
+                if (kEnergy) e_c = on ? ec : 0.0;
+            }
+            fx += fs * dx;
+            fy += fs * dy;
+            fz += fs * dz;
+            if (kEnergy && j > i) {
+                e_pair += e_p;
+                e_coul += e_c;
+                wxx += fs * dx * dx;
+                wyy += fs * dy * dy;
+                wzz += fs * dz * dz;
+                wxy += fs * dx * dy;
+                wxz += fs * dx * dz;
+                wyz += fs * dy * dz;
+            }
+        };
+        int k = sub;
+        int eA = jat(k), eB = jat(k + TPA);  // list entries: atom and kind
+        double4 pA = a.pos[nbr_atom(eA)], pB = a.pos[nbr_atom(eB)];
+        for (; k < nn; k += 2 * TPA) {
+            const int eA2 = jat(k + 2 * TPA), eB2 = jat(k + 3 * TPA);
+            pair(nbr_atom(eA), pA, nbr_kind(eA));
+            pA = a.pos[nbr_atom(eA2)];
+            if (k + TPA < nn) pair(nbr_atom(eB), pB, nbr_kind(eB));
+            pB = a.pos[nbr_atom(eB2)];
+            eA = eA2;
+            eB = eB2;
+        }
+    }
+#pragma unroll
+    for (int off = TPA / 2; off > 0; off >>= 1) {
+        fx += __shfl_xor(fx, off, 64);
+        fy += __shfl_xor(fy, off, 64);
+        fz += __shfl_xor(fz, off, 64);
+    }
+    if (t < a.n && sub == 0) a.force[i] = make_double4(fx, fy, fz, 0.0);
+    if (kEnergy) {
+        double v[8] = {e_pair, e_coul, wxx, wyy, wzz, wxy, wxz, wyz};
+        int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            double sum = wave_sum(v[q]);
+            if (lane == 0) red[wid][q] = sum;
+        }
+        __syncthreads();
+        if (threadIdx.x < 8) {
+            double sum = 0;
+            for (int w = 0; w < kPairBlock / 64; w++) sum += red[w][threadIdx.x];
+            a.epart[blockIdx.x * 8 + threadIdx.x] = sum;
+        }
+    }
+}
+
+// The general pair kernel, for systems with a pair potential other than
+// LJ/Harmonic/Null or a TableComputation (any kind, FP64, both forms), in
+// the reference's operation order.  TPA lanes share one atom i and stride
+// through its neighbour row; the group's partial forces are combined with
+// xor-shuffles (TPA divides 64).
+template <bool kEnergy, int TPA, int CK>
+__global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_pairs_gen(PairArgs a) {
+    using TabEntry = PairParam;
+    __shared__ __align__(32) unsigned char tab_lds[sizeof(TabEntry) * kMaxKinds * kMaxKinds];
+    TabEntry* const tab = reinterpret_cast<TabEntry*>(tab_lds);
     __shared__ double red[kPairBlock / 64][8];
     constexpr bool kTab = CK == CK_EWALD || CK == CK_WOLF;
     __shared__ double ecx[kTab ? kErfcxPieces * (kErfcxDeg64 + 1) : 1];
@@ -1412,16 +1609,13 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(4)))
         if (b < a.intra_blocks)
             intra_block<kEnergy>(a.intra, b);
         else
-            kspace_reduce_block<kEnergy>(a, b - a.intra_blocks);
+            kspace_reduce_block<kEnergy>(a, b - a.intra_blocks, reinterpret_cast<unsigned char*>(tab));
         return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.rebuild) *a.rebuild = 0;
     int nk2 = a.nkinds * a.nkinds;
     for (int x = threadIdx.x; x < nk2; x += blockDim.x) {
-        if constexpr (kGen)
-            tab[x] = a.table[x];
-        else
-            tab[x] = pair_fast(a.table[x]);
+        tab[x] = a.table[x];
     }
     const bool use_tab = kTab && a.ecx64 != nullptr;  // uniform
     if (use_tab)
@@ -1465,10 +1659,7 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(4)))
             const TabEntry& pp = tab[ki * a.nkinds + kj];
             if (pp.pot > POT_NULL && !pp.inter_excl && r < pp.rc) {
                 double e, f;
-                if constexpr (kGen)
-                    pot_eval_any(pp, a.tabs, r, inv_r, e, f);
-                else
-                    pot_eval(pp.pot, pp.p0, pp.p1, r, inv_r, e, f);
+                pot_eval_any(pp, a.tabs, r, inv_r, e, f);
                 fs += f;
                 e_p = e - pp.shift;
             }
@@ -1574,21 +1765,28 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(4)))
 // energies keep exp(-x^2) erfcx(x).  1/r is the hardware reciprocal square
 // root (1 ulp).
 //
-// The launch carries the rho(k) reduction blocks but not the
-// intra-molecular terms (k_intra_terms, a launch of its own): their code
-// needs 104 VGPRs, which would hold every pair block of the launch to four
-// waves per SIMD, against eight for the pair code alone.
+// The launch carries the rho(k) reduction blocks but not the intra-molecular
+// terms: their code needs 104 VGPRs, which would hold every pair block of the
+// launch to four waves per SIMD, against eight for the pair code alone.
 template <bool kEnergy, int TPA, int CK>
 __global__ __launch_bounds__(kPairBlock) void k_pairs_mixed(PairArgs a) {
-    __shared__ float4 ljt[kMaxKinds * kMaxKinds];
-    __shared__ float2 hmt[kMaxKinds * kMaxKinds];  // Harmonic {k, x0}, k = 0 otherwise
     __shared__ double red[kPairBlock / 64][8];
     constexpr bool kTab = CK == CK_EWALD || CK == CK_WOLF;
-    // erfcx pieces (energies, and forces without the h table) and h pieces
-    __shared__ __align__(16) float ecx[kTab ? kErfcxPieces * (kErfcxDeg32 + 1) : 4];
-    __shared__ __align__(16) float hft[kTab ? kErfcxPieces * (kErfcxDeg32 + 1) : 4];
+    struct Tables {
+        float4 ljt[kMaxKinds * kMaxKinds];
+        float2 hmt[kMaxKinds * kMaxKinds];  // Harmonic {k, x0}, k = 0 otherwise
+        // erfcx pieces (energies, and forces without the h table) and h pieces
+        float4 ecx[kTab ? kErfcxPieces : 1], hft[kTab ? kErfcxPieces : 1];
+    };
+    // the reduction blocks use the tables' LDS (residency is set by it)
+    __shared__ __align__(32) unsigned char lds[sizeof(Tables) > 8192 ? sizeof(Tables) : 8192];
+    Tables& tb = *reinterpret_cast<Tables*>(lds);
+    float4* const ljt = tb.ljt;
+    float2* const hmt = tb.hmt;
+    float* const ecx = reinterpret_cast<float*>(tb.ecx);
+    float* const hft = reinterpret_cast<float*>(tb.hft);
     if ((int)blockIdx.x >= a.pair_blocks) {  // uniform over the block
-        kspace_reduce_block<kEnergy>(a, blockIdx.x - a.pair_blocks);
+        kspace_reduce_block<kEnergy>(a, blockIdx.x - a.pair_blocks, lds);
         return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.rebuild) *a.rebuild = 0;
@@ -2196,9 +2394,15 @@ __global__ __launch_bounds__(512) void k_rho_rows(RhoRowsArgs<T, T2> ra) {
 // For evaluations outside MD steps and systems of too many chunks for
 // k_oct_step: blocks of a.width atoms (several stages of SA) x item groups.
 // Dynamic LDS: the rows of SA atoms, at least kOctRed.
-template <typename T>
-__global__ __launch_bounds__(512, 2) void k_rho_oct(OctRho ra, int SA, const double4* __restrict__ pos, int n) {
+// Blocks past nrho run the intra-molecular terms (512 per block).
+template <typename T, bool kEnergy>
+__global__ __launch_bounds__(512, 2) void k_rho_oct(OctRho ra, int SA, const double4* __restrict__ pos, int n,
+                                                    int nrho, IntraArgs ia) {
     extern __shared__ __align__(16) unsigned char oct_smem[];
+    if ((int)blockIdx.x >= nrho) {
+        intra_block<kEnergy>(ia, blockIdx.x - nrho);
+        return;
+    }
     int grp, chunk;
     if (!xcd_block(ra.ngroups, ra.nchunks, grp, chunk)) return;
     const int a0 = chunk * ra.width;

@@ -296,9 +296,10 @@ struct OctReduce {
     double* coef64;
 };
 
+// lds: 8 KB.
 template <bool kEnergy>
-__device__ __forceinline__ void oct_reduce_block(const OctReduce& a, int blk) {
-    __shared__ double4 part[16][16];
+__device__ __forceinline__ void oct_reduce_block(const OctReduce& a, int blk, unsigned char* lds) {
+    double4(*part)[16] = reinterpret_cast<double4(*)[16]>(lds);
     const int g = threadIdx.x >> 4, col = threadIdx.x & 15;
     const int4 sl = a.slots[blk >> 2];
     const int pair = blk & 3;
@@ -382,11 +383,6 @@ __device__ __forceinline__ void oct_reduce_block(const OctReduce& a, int blk) {
             if (threadIdx.x == 0) a.epart[blk * 7 + x] = sum;
         }
     }
-}
-
-template <bool kEnergy>
-__global__ __launch_bounds__(256) void k_oct_reduce(OctReduce a) {
-    oct_reduce_block<kEnergy>(a, blockIdx.x);
 }
 
 // ---- forces -------------------------------------------------------------------------
