@@ -2182,7 +2182,7 @@ int lg_system_create(lg_context* ctx, size_t natoms, lg_system** out) {
     int r;
     if ((r = s->pos.ensure(natoms)) || (r = s->vel.ensure(natoms)) || (r = s->acc.ensure(natoms)) ||
         (r = s->force.ensure(natoms)) || (r = s->lambda.ensure(1)) ||
-        (r = s->ke_part.ensure(size_t(blocks_for(natoms, 16))))) {
+        (r = s->ke_part.ensure(size_t(std::max(blocks_for(natoms, 16), 1024))))) {
         delete s;
         return r;
     }
@@ -2607,6 +2607,96 @@ __global__ void k_energy_gather(const double* __restrict__ pp, int nbp, const do
 }
 }  // namespace
 
+// Whether lg_md_run takes whole steps without a neighbour list (k_small_step):
+// point particles of fast potentials without k-space, Wolf only with its
+// tables, of at most small_max atoms.  A set knob of the list kernels keeps
+// the list.
+static bool small_steps(const lg_system* s) {
+    return s->n <= size_t(small_max(s->precision == LG_PRECISION_MIXED)) && !s->gen_pairs && s->nterms == 0 &&
+           s->nmol == int(s->n) &&
+           (s->coul_kind == COUL_NONE || (s->coul_kind == COUL_WOLF && (s->hf_ok || s->coul.inter_excl))) &&
+           s->tune.nlist_build == 0 && s->tune.pair_lanes == 0;
+}
+template <bool kMixed>
+static void launch_small(lg_system* s, const SmallArgs& a, bool loop) {
+    const bool wolf = coulomb_variant(s->coul) == CK_WOLF;
+    if (loop)
+        launch_timed(s, LG_KERNEL_INTEGRATE, wolf ? k_small_step<kMixed, CK_WOLF, true> : k_small_step<kMixed, CK_NONE, true>,
+                     1, 1024, 0, a);
+    else
+        launch_timed(s, LG_KERNEL_INTEGRATE,
+                     wolf ? k_small_step<kMixed, CK_WOLF, false> : k_small_step<kMixed, CK_NONE, false>,
+                     blocks_for(s->n, 4), 256, 0, a);
+}
+// The current state back from the second set of arrays.
+__global__ void k_state_back(double4* __restrict__ p, double4* __restrict__ v, double4* __restrict__ a,
+                             const double4* __restrict__ p2, const double4* __restrict__ v2,
+                             const double4* __restrict__ a2, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    p[i] = p2[i];
+    v[i] = v2[i];
+    a[i] = a2[i];
+}
+static int small_chunk(lg_system* s, uint64_t todo) {
+    const bool mixed = s->precision == LG_PRECISION_MIXED, thermo = s->thermostat;
+    const int n = int(s->n);
+    SmallArgs a{};
+    a.meta = s->meta.p;
+    a.n = n;
+    a.lf = s->integrator != LG_INTEGRATOR_VELOCITY_VERLET;
+    a.dt = s->dt;
+    a.thermostat = thermo;
+    a.flags = s->flags.p;
+    a.table = s->table.p;
+    a.nkinds = int(s->nkinds);
+    a.coul = s->coul;
+    a.box = s->box;
+    a.fo = s->frac_origin;
+    a.hf64 = s->hf64.p;
+    a.hf32 = s->hf32.p;
+    a.hf_inv_h = s->hf_inv_h;
+    a.tie = s->periodic && max_cutoff(s) > (0.5 - 1e-6) * std::min(s->L[0], std::min(s->L[1], s->L[2]));
+    a.th = Thermo{nullptr, 0, double(3 * s->n), s->berendsen_T, s->berendsen_tau, nullptr};
+    if (n <= small_loop_max(mixed)) {
+        a.pos = a.pos2 = s->pos.p;
+        a.vel = a.vel2 = s->vel.p;
+        a.acc = a.acc2 = s->acc.p;
+        a.nsteps = int(todo);
+        if (mixed) launch_small<true>(s, a, true);
+        else launch_small<false>(s, a, true);
+        LG_HIP(hipGetLastError());
+        return LG_OK;
+    }
+    const int grid = blocks_for(n, 4);
+    a.nsteps = 1;
+    a.th.nparts = grid;
+    double4* const set[2][3] = {{s->pos.p, s->vel.p, s->acc.p}, {s->snap_pos.p, s->snap_vel.p, s->snap_acc.p}};
+    for (uint64_t k = 0; k < todo; k++) {
+        // two sets of partials: a launch reads the one before while it writes its own
+        a.th.ke_part = thermo && k > 0 ? s->ke_part.p + (k & 1 ? 0 : grid) : nullptr;
+        a.ke_part = thermo ? s->ke_part.p + (k & 1 ? grid : 0) : nullptr;
+        a.pos = set[k & 1][0];
+        a.vel = set[k & 1][1];
+        a.acc = set[k & 1][2];
+        a.pos2 = set[(k + 1) & 1][0];
+        a.vel2 = set[(k + 1) & 1][1];
+        a.acc2 = set[(k + 1) & 1][2];
+        if (mixed) launch_small<true>(s, a, false);
+        else launch_small<false>(s, a, false);
+    }
+    if (todo & 1)
+        k_state_back<<<blocks_for(n, 256), 256, 0, S(s)>>>(s->pos.p, s->vel.p, s->acc.p, s->snap_pos.p, s->snap_vel.p,
+                                                           s->snap_acc.p, n);
+    if (thermo) {
+        a.th.ke_part = s->ke_part.p + (todo & 1 ? 0 : grid);
+        k_berendsen<<<1, 256, 0, S(s)>>>(a.th, s->lambda.p);
+        k_scale_vel<<<blocks_for(n, 256), 256, 0, S(s)>>>(s->vel.p, n, s->lambda.p);
+    }
+    LG_HIP(hipGetLastError());
+    return LG_OK;
+}
+
 extern "C" {
 
 int lg_potential_energy(lg_system* s, lg_energy_terms* out) {
@@ -2842,6 +2932,7 @@ int lg_md_setup(lg_system* s, int integrator, double timestep, double bT, double
 // scale at the end: launched eagerly, or captured into a HIP graph by
 // lg_md_run.  No allocation, copy, memset or synchronisation in between.
 static int md_chunk(lg_system* s, uint64_t todo) {
+    if (small_steps(s)) return small_chunk(s, todo);
     hipStream_t st = S(s);
     const int n = int(s->n);
     const bool thermo = s->thermostat;
@@ -2924,9 +3015,14 @@ int lg_md_run(lg_system* s, uint64_t nsteps) {
     LG_HIP(hipMemsetAsync(s->flags.p + 2, 0, sizeof(int), st));
     while (done < nsteps) {
         uint64_t todo = std::min<uint64_t>(chunk, nsteps - done);
-        LG_HIP(hipMemcpyAsync(s->snap_pos.p, s->pos.p, s->n * sizeof(double4), hipMemcpyDeviceToDevice, st));
-        LG_HIP(hipMemcpyAsync(s->snap_vel.p, s->vel.p, s->n * sizeof(double4), hipMemcpyDeviceToDevice, st));
-        LG_HIP(hipMemcpyAsync(s->snap_acc.p, s->acc.p, s->n * sizeof(double4), hipMemcpyDeviceToDevice, st));
+        // the state of before the chunk, for a list that overflows (without a
+        // list, the snapshot arrays are the steps' second set)
+        const bool listed = !small_steps(s);
+        if (listed) {
+            LG_HIP(hipMemcpyAsync(s->snap_pos.p, s->pos.p, s->n * sizeof(double4), hipMemcpyDeviceToDevice, st));
+            LG_HIP(hipMemcpyAsync(s->snap_vel.p, s->vel.p, s->n * sizeof(double4), hipMemcpyDeviceToDevice, st));
+            LG_HIP(hipMemcpyAsync(s->snap_acc.p, s->acc.p, s->n * sizeof(double4), hipMemcpyDeviceToDevice, st));
+        }
         const bool graph = s->tune.md_graph == 2 && s->prof_mask == 0;
         if (graph) {
             // captured once per (chunk length, configuration, buffer set,
@@ -2962,7 +3058,7 @@ int lg_md_run(lg_system* s, uint64_t nsteps) {
         LG_HIP(hipGetLastError());
         bool ov = false, bad = false;
         LG_TRY(check_overflow(s, &ov, &bad));
-        if (ov) {
+        if (ov && listed) {
             if (++retries > 4) return fail(LG_E_DEVICE, "neighbour list overflow could not be resolved");
             LG_HIP(hipMemcpyAsync(s->pos.p, s->snap_pos.p, s->n * sizeof(double4), hipMemcpyDeviceToDevice, st));
             LG_HIP(hipMemcpyAsync(s->vel.p, s->snap_vel.p, s->n * sizeof(double4), hipMemcpyDeviceToDevice, st));

@@ -2787,6 +2787,295 @@ __global__ __launch_bounds__(kMdBlock) void k_md_fused(MdArgs m, const double4* 
     md_place(m, i, live, p, v, r);
 }
 
+// ---- whole steps of small atomic systems ---------------------------------------------
+// Below a few thousand atoms a step's kernels each take less time than their
+// launches.  For systems of point particles without k-space, one launch does
+// a whole step without a neighbour list: every block moves every atom by the
+// first half-step (from the step before, read from the `in` arrays), keeps
+// the new positions in LDS, evaluates all pairs of its own atoms there (the
+// pair kernels' arithmetic and cutoffs, so the same pair set) and finishes
+// the step for them; its atoms' new state goes to the `out` arrays, which
+// other blocks do not read until the next launch.  The Berendsen factor
+// comes from the previous launch's kinetic energies, as in k_md_first.
+// TPA lanes per atom, combined with xor-shuffles: a wave for each atom, so
+// that the pairs of even a few hundred atoms are spread over the card (32
+// lanes: 13.2 against 9.4 us at 1024 atoms FP64).  kLoop: one block holds the
+// system and runs `nsteps` steps without leaving the kernel.
+// Bound by the launch below 500 atoms and by pair arithmetic above.  Per
+// step, four launches with a list / one: 64 atoms mixed 13 / 2.5 us in the
+// loop, 500 atoms FP64 13.5 / 6.8 us.  Letting each block also take its
+// atoms' next first half (the others then read positions alone) gave nothing.
+struct SmallArgs {
+    const double4 *pos, *vel, *acc;
+    double4 *pos2, *vel2, *acc2;
+    const int2* meta;
+    int n, lf, nsteps;
+    double dt;
+    Thermo th;         // of the previous step (nsteps > 1: th.T0, th.tau, th.dof used inside)
+    int thermostat;
+    double* ke_part;   // per block, with a thermostat
+    int* flags;
+    const PairParam* table;
+    int nkinds, tie;
+    CoulParam coul;
+    Box box;
+    double3 fo;        // origin of the FP32 coordinates in an infinite cell
+    const double* hf64;
+    const float* hf32;
+    double hf_inv_h;
+};
+// Atoms of the largest system in each form; past them the all-pairs work
+// costs more than the list's launches.  us per step, list / one launch:
+// FP64 1024 atoms 13.6 / 9.4, 1200 13.9 / 18.1 (its blocks pass the 256
+// compute units); mixed 1500 13.8 / 11.3, 2048 13.8 / 13.7.
+constexpr int small_max(bool mixed) { return mixed ? 1536 : 1024; }
+// The same for the loop, one launch per step / loop: FP64 64 atoms 4.6 / 3.4,
+// 80 atoms 4.8 / 5.2; mixed 96 atoms 4.8 / 3.8, 112 atoms 4.9 / 4.8.
+constexpr int small_loop_max(bool mixed) { return mixed ? 96 : 64; }
+
+// Force over r of one pair at r2 (FP64; k_pairs without energies).
+template <int CK>
+__device__ __forceinline__ double small_pair(double4 P, double2 H, int harmonic, double r2, double pref,
+                                             const CoulParam& c, const double* hft, double hf_inv_h) {
+    const double inv_r = rsqrt_newton(r2), i2 = inv_r * inv_r, i6 = i2 * i2 * i2;
+    double fp = (P.x * i6 - P.y) * (i6 * i2);
+    if (harmonic) fp += H.x * (H.y - r2 * inv_r) * inv_r;  // uniform
+    double fs = r2 < P.z ? fp : 0.0;
+    if constexpr (CK == CK_WOLF) {
+        const double fc = pref * (erfcx_tab(hft, r2 * inv_r, hf_inv_h) * (inv_r * i2) - c.f_const * inv_r);
+        fs += r2 < c.r2c && pref != 0.0 ? fc : 0.0;
+    }
+    return fs;
+}
+// The same in FP32 (k_pairs_mixed without energies).
+template <int CK>
+__device__ __forceinline__ float small_pair(float4 P, float2 H, int harmonic, float r2, float pref, float rcc2,
+                                            float wf, const float* hft, float hf_inv_h) {
+    const float inv_r = __builtin_amdgcn_rsqf(r2), i2 = inv_r * inv_r, i6 = i2 * i2 * i2;
+    float fp = (P.x * i6 - P.y) * (i6 * i2);
+    if (harmonic) fp += H.x * (H.y - r2 * inv_r) * inv_r;
+    float fs = r2 < P.z ? fp : 0.f;
+    if constexpr (CK == CK_WOLF) {
+        const float fc = pref * (erfcx_tab(hft, r2 * inv_r, hf_inv_h) * (inv_r * i2) - wf * inv_r);
+        fs += r2 <= rcc2 ? fc : 0.f;
+    }
+    return fs;
+}
+
+template <bool kMixed, int CK, bool kLoop>
+__global__ __launch_bounds__(kLoop ? 1024 : 256) void k_small_step(SmallArgs a) {
+    typedef typename std::conditional<kMixed, float, double>::type T;
+    typedef typename std::conditional<kMixed, float4, double4>::type T4;
+    typedef typename std::conditional<kMixed, float2, double2>::type T2;
+    constexpr int BLOCK = kLoop ? 1024 : 256, TPA = kLoop ? (kMixed ? 8 : 16) : 64, OWN = BLOCK / TPA;
+    constexpr int NMAX = kLoop ? small_loop_max(kMixed) : small_max(kMixed);
+    // positions: fixed-point fractions (or FP32 coordinates) and charge in the
+    // mixed form, coordinates in FP64
+    __shared__ float4 xf[kMixed ? NMAX : 1];
+    __shared__ double xd[kMixed ? 1 : 3][kMixed ? 1 : NMAX];
+    __shared__ T qs[kMixed || CK == CK_NONE ? 1 : NMAX];
+    __shared__ unsigned char ks[NMAX];
+    __shared__ T4 ljt[kMaxKinds * kMaxKinds];
+    __shared__ T2 hmt[kMaxKinds * kMaxKinds];
+    __shared__ __align__(16) T hft[CK == CK_WOLF ? kErfcxPieces * ((kMixed ? kErfcxDeg32 : kErfcxDeg64) + 1) : 4];
+    __shared__ double4 own_p[OWN], own_v[OWN];
+    __shared__ double ke_red[16];
+    const int tid = threadIdx.x, n = a.n;
+    int harmonic = 0;
+    for (int x = tid; x < a.nkinds * a.nkinds; x += BLOCK) {
+        const PairParam pp = a.table[x];
+        const bool on = pp.pot > POT_NULL && !pp.inter_excl, lj = pp.pot == POT_LJ, hm = on && pp.pot == POT_HARMONIC;
+        const double s2 = pp.p0 * pp.p0, s6 = lj ? s2 * s2 * s2 : 0.0;
+        const float rcf = (float)pp.rc;
+        ljt[x].x = (T)(lj ? 48.0 * pp.p1 * (s6 * s6) : 0.0);
+        ljt[x].y = (T)(lj ? 24.0 * pp.p1 * s6 : 0.0);
+        ljt[x].z = on ? (kMixed ? (T)(rcf * rcf) : (T)pp.r2c) : (T)0;
+        hmt[x].x = (T)(hm ? pp.p0 : 0.0);
+        hmt[x].y = (T)(hm ? pp.p1 : 0.0);
+        harmonic |= hm;
+    }
+    if constexpr (CK == CK_WOLF) {
+        const T* src;
+        if constexpr (kMixed) src = a.hf32;
+        else src = a.hf64;
+        for (int x = tid; x < (int)(sizeof(hft) / sizeof(T)); x += BLOCK) hft[x] = src[x];
+    }
+    for (int j = tid; j < n; j += BLOCK) ks[j] = (unsigned char)a.meta[j].x;
+    harmonic = __syncthreads_or(harmonic);
+    // a home atom of this group of TPA lanes
+    const int a0 = blockIdx.x * OWN, sub = tid % TPA, ho = tid / TPA, i = a0 + ho;
+    const bool mine = i < n;
+    const double* invL = a.box.inv;
+    double lambda = 1.0;
+    if (a.th.ke_part) lambda = a.th.lambda ? *a.th.lambda : berendsen_lambda(a.th);
+    bool scale = a.th.ke_part != nullptr;
+    MdArgs m{};
+    m.lf = a.lf;
+    m.dt = a.dt;
+    double4 kp = make_double4(0, 0, 0, 0), kv = kp, ka = kp;  // kLoop: the state of atom tid between steps
+    if (kLoop && tid < n) {
+        kp = a.pos[tid];
+        kv = a.vel[tid];
+        ka = a.acc[tid];
+    }
+    for (int step = 0; step < (kLoop ? a.nsteps : 1); step++) {
+        for (int j = tid; j < n; j += BLOCK) {
+            double4 p, v, ac;
+            if (kLoop) {
+                p = kp;
+                v = kv;
+                ac = ka;
+            } else {
+                p = a.pos[j];
+                v = a.vel[j];
+                ac = a.acc[j];
+            }
+            if (scale) {
+                v.x = v.x * lambda;
+                v.y = v.y * lambda;
+                v.z = v.z * lambda;
+            }
+            md_drift(m, ac, v, p);
+            if (kMixed) {
+                xf[j] = frac_pos(a.box, a.fo, p);
+            } else {
+                xd[0][j] = p.x;
+                xd[kMixed ? 0 : 1][j] = p.y;
+                xd[kMixed ? 0 : 2][j] = p.z;
+                if (CK != CK_NONE) qs[j] = (T)p.w;
+            }
+            if (kLoop) {
+                kp = p;
+                kv = v;
+            } else if (j >= a0 && j < a0 + OWN) {
+                own_p[j - a0] = p;
+                own_v[j - a0] = v;
+            }
+        }
+        __syncthreads();
+        double fx = 0.0, fy = 0.0, fz = 0.0;
+        if (mine) {
+            const int ki = ks[i] * a.nkinds;
+            if constexpr (kMixed) {
+                const float4 pi = xf[i];
+                const bool periodic = a.box.periodic;  // uniform
+                const float Lx = (float)(a.box.L[0] * 0x1p-32), Ly = (float)(a.box.L[1] * 0x1p-32),
+                            Lz = (float)(a.box.L[2] * 0x1p-32);
+                const float qk = pi.w * (float)(1.0 / kFourPiEps0), rcc2 = (float)(a.coul.rc * a.coul.rc),
+                            wf = (float)a.coul.f_const, ih = (float)a.hf_inv_h;
+                auto pair = [&](int j, float& dx, float& dy, float& dz) {
+                    const float4 pj = xf[j];
+                    if (periodic) {
+                        dx = (float)(int)(__float_as_uint(pi.x) - __float_as_uint(pj.x)) * Lx;
+                        dy = (float)(int)(__float_as_uint(pi.y) - __float_as_uint(pj.y)) * Ly;
+                        dz = (float)(int)(__float_as_uint(pi.z) - __float_as_uint(pj.z)) * Lz;
+                    } else {
+                        dx = pi.x - pj.x;
+                        dy = pi.y - pj.y;
+                        dz = pi.z - pj.z;
+                    }
+                    const int kk = ki + ks[j];
+                    const float f = small_pair<CK>(ljt[kk], hmt[kk], harmonic, dx * dx + dy * dy + dz * dz, qk * pj.w,
+                                                   rcc2, wf, hft, ih);
+                    return j == i ? 0.f : f;
+                };
+                // two pairs at a time, added in FP32, then to the FP64 sums
+                for (int j = sub; j < n; j += 2 * TPA) {
+                    float ax, ay, az, bx, by, bz;
+                    const int j2 = j + TPA < n ? j + TPA : i;
+                    const float fa = pair(j, ax, ay, az), fb = pair(j2, bx, by, bz);
+                    // the pair with itself adds nothing (its force is not finite)
+                    const bool sa = j == i, sb = j2 == i;
+                    fx += (double)((sa ? 0.f : fa * ax) + (sb ? 0.f : fb * bx));
+                    fy += (double)((sa ? 0.f : fa * ay) + (sb ? 0.f : fb * by));
+                    fz += (double)((sa ? 0.f : fa * az) + (sb ? 0.f : fb * bz));
+                }
+            } else {
+                const double px = xd[0][i], py = xd[kMixed ? 0 : 1][i], pz = xd[kMixed ? 0 : 2][i];
+                const double qk = CK != CK_NONE ? (double)qs[i] / kFourPiEps0 : 0.0;
+                for (int j = sub; j < n; j += TPA) {
+                    double dx = px - xd[0][j], dy = py - xd[kMixed ? 0 : 1][j], dz = pz - xd[kMixed ? 0 : 2][j];
+                    if (a.tie) {
+                        min_image(a.box, dx, dy, dz);
+                    } else {
+                        dx = image_rint(dx, a.box.L[0], invL[0]);
+                        dy = image_rint(dy, a.box.L[1], invL[1]);
+                        dz = image_rint(dz, a.box.L[2], invL[2]);
+                    }
+                    const int kk = ki + ks[j];
+                    const double f = small_pair<CK>(ljt[kk], hmt[kk], harmonic, norm2_ordered(dx, dy, dz),
+                                                    CK != CK_NONE ? qk * (double)qs[j] : 0.0, a.coul, hft, a.hf_inv_h);
+                    const bool self = j == i;
+                    fx += self ? 0.0 : f * dx;
+                    fy += self ? 0.0 : f * dy;
+                    fz += self ? 0.0 : f * dz;
+                }
+            }
+        }
+#pragma unroll
+        for (int off = TPA / 2; off > 0; off >>= 1) {
+            fx += __shfl_xor(fx, off, 64);
+            fy += __shfl_xor(fy, off, 64);
+            fz += __shfl_xor(fz, off, 64);
+        }
+        double ke = 0.0;
+        bool bad = false;
+        if (kLoop) {
+            // the force to the thread that keeps the atom's state
+            if (mine && sub == 0) own_p[ho] = make_double4(fx, fy, fz, 0.0);
+            __syncthreads();
+            if (tid < n) {
+                const double4 f = own_p[tid];
+                double4 na;
+                md_kick(m, f, ka, kv, na);
+                ka = na;
+                ke = 0.5 * kv.w * (kv.x * kv.x + kv.y * kv.y + kv.z * kv.z);
+                bad = nonfinite3(kp.x, kp.y, kp.z) || nonfinite3(kv.x, kv.y, kv.z) || nonfinite3(na.x, na.y, na.z);
+            }
+            flag_nonfinite(bad, a.flags);
+            if (a.thermostat) {
+                // as berendsen_lambda from one partial per wave, in wave order
+                ke = wave_sum(ke);
+                if ((tid & 63) == 0) ke_red[tid >> 6] = ke;
+                __syncthreads();
+                double kin = 0.0;
+                for (int w = 0; w < BLOCK / 64; w++) kin += ke_red[w];
+                const double temp = 2.0 * kin / (a.th.dof * kBoltzmann);
+                lambda = sqrt(1.0 + (a.th.T0 / temp - 1.0) / a.th.tau);
+                scale = true;
+            }
+        } else {
+            if (mine && sub == 0) {
+                const double4 p = own_p[ho];
+                double4 v = own_v[ho], na;
+                md_kick(m, make_double4(fx, fy, fz, 0.0), a.lf ? a.acc[i] : v, v, na);
+                a.pos2[i] = p;
+                a.vel2[i] = v;
+                a.acc2[i] = na;
+                ke = 0.5 * v.w * (v.x * v.x + v.y * v.y + v.z * v.z);
+                bad = nonfinite3(p.x, p.y, p.z) || nonfinite3(v.x, v.y, v.z) || nonfinite3(na.x, na.y, na.z);
+            }
+            flag_nonfinite(bad, a.flags);
+            if (a.ke_part) {
+                ke = wave_sum(ke);
+                if ((tid & 63) == 0) ke_red[tid >> 6] = ke;
+                __syncthreads();
+                if (tid == 0) a.ke_part[blockIdx.x] = ((ke_red[0] + ke_red[1]) + ke_red[2]) + ke_red[3];
+            }
+        }
+    }
+    if (kLoop && tid < n) {
+        if (a.thermostat) {  // the last step's scale
+            kv.x = kv.x * lambda;
+            kv.y = kv.y * lambda;
+            kv.z = kv.z * lambda;
+        }
+        a.pos2[tid] = kp;
+        a.vel2[tid] = kv;
+        a.acc2[tid] = ka;
+    }
+}
+
 // Berendsen factor of the last step into *lambda (one block: one wave up to
 // kThermoParts partials, as every block of k_md_first, else 1024 threads).
 __global__ __launch_bounds__(1024) void k_berendsen(Thermo th, double* __restrict__ lambda) {
