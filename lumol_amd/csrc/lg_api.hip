@@ -2082,6 +2082,18 @@ int mc_prepare_cells(lg_system* s, bool full) {
     return LG_OK;
 }
 
+// Whether a chain runs k_mc_atoms: single atoms with Lennard-Jones or no
+// potential, no Coulomb term, no cutoff that reaches half the box (there the
+// nearest-integer image could differ), and a state that fits the LDS (4600
+// atoms; k_mc_chains with its cell list beyond).
+bool mc_atoms(lg_system* s) {
+    if (s->nmol != int(s->n) || s->coul_kind != COUL_NONE || s->gen_pairs) return false;
+    for (auto& [k, p] : s->pairs)
+        if (p.v.pot != LG_POT_NULL && p.v.pot != LG_POT_LJ) return false;
+    if (s->periodic && max_cutoff(s) > (0.5 - 1e-6) * std::min(s->L[0], std::min(s->L[1], s->L[2]))) return false;
+    return s->n <= kMcAtomMax && kMcAtomStatic + mc_atoms_lds(s->n) <= s->ctx->max_shared;
+}
+
 McChain mc_chain(lg_system* s, bool cells) {
     McChain c{};
     c.pos = s->pos.p;
@@ -3209,7 +3221,10 @@ int lg_mc_run_batch(lg_system* const* systems, size_t count, const uint64_t* see
         LG_TRY(prepare(s));
         if (!s->mc_ready) LG_TRY(mc_init(s));
         if (s->max_mol > kMcMaxMol) return fail(LG_E_UNSUPPORTED, "molecule too large for a device Monte Carlo move");
-        if (!s->mc_cells_valid) LG_TRY(mc_prepare_cells(s, false));
+        if (mc_atoms(s))
+            s->mc_cells_valid = false;  // its kernel keeps no cell list
+        else if (!s->mc_cells_valid)
+            LG_TRY(mc_prepare_cells(s, false));
         shmem = std::max(shmem, mc_phase_bytes(s));
         next[b] = attempt0[b];
         end[b] = attempt0[b] + nattempts[b];
@@ -3224,14 +3239,20 @@ int lg_mc_run_batch(lg_system* const* systems, size_t count, const uint64_t* see
     for (int round = 0; !active.empty(); round++) {
         if (round > 8) return fail(LG_E_DEVICE, "Monte Carlo cell list overflow could not be resolved");
         desc.clear();
-        // chains with a Coulomb potential first: they run the kCoul kernel
-        std::stable_partition(active.begin(), active.end(),
-                              [&](size_t b) { return systems[b]->coul_kind != COUL_NONE; });
-        size_t ncoul = 0;
-        for (size_t b : active) ncoul += systems[b]->coul_kind != COUL_NONE;
+        // chains with a Coulomb potential first: they run the kCoul kernel;
+        // those of single Lennard-Jones sites last (k_mc_atoms)
+        auto kind = [&](size_t b) { return systems[b]->coul_kind != COUL_NONE ? 0 : mc_atoms(systems[b]) ? 2 : 1; };
+        std::stable_sort(active.begin(), active.end(), [&](size_t a, size_t b) { return kind(a) < kind(b); });
+        size_t ncoul = 0, natoms = 0, atoms_lds = 0;
+        for (size_t b : active) {
+            ncoul += kind(b) == 0;
+            if (kind(b) != 2) continue;
+            natoms++;
+            atoms_lds = std::max(atoms_lds, mc_atoms_lds(systems[b]->n));
+        }
         for (size_t b : active) {
             lg_system* s = systems[b];
-            McChain c = mc_chain(s, true);
+            McChain c = mc_chain(s, kind(b) != 2);
             c.key = make_uint2(uint32_t(seeds[b]), uint32_t(seeds[b] >> 32));
             c.attempt0 = next[b];
             c.nattempts = end[b] - next[b];
@@ -3252,7 +3273,10 @@ int lg_mc_run_batch(lg_system* const* systems, size_t count, const uint64_t* see
         LG_HIP(hipMemcpyAsync(ctx->mc_desc.p, desc.data(), na * sizeof(McChain), hipMemcpyHostToDevice, st));
         LG_HIP(hipMemsetAsync(ctx->mc_cnt.p, 0, na * 2 * sizeof(unsigned long long), st));
         if (ncoul > 0) k_mc_chains<true><<<unsigned(ncoul), kMcBlock, shmem, st>>>(ctx->mc_desc.p);
-        if (na > ncoul) k_mc_chains<false><<<unsigned(na - ncoul), kMcBlock, shmem, st>>>(ctx->mc_desc.p + ncoul);
+        if (na > ncoul + natoms)
+            k_mc_chains<false><<<unsigned(na - ncoul - natoms), kMcBlock, shmem, st>>>(ctx->mc_desc.p + ncoul);
+        if (natoms > 0)
+            k_mc_atoms<<<unsigned(natoms), kMcAtomBlock, atoms_lds, st>>>(ctx->mc_desc.p + (na - natoms));
         LG_HIP(hipGetLastError());
         cnt.resize(na * 2);
         LG_HIP(hipMemcpyAsync(cnt.data(), ctx->mc_cnt.p, na * 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,

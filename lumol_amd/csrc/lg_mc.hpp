@@ -660,6 +660,297 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_chains(const McChain* __restric
 }
 #pragma clang fp contract(on)
 
+// ---- chains of single Lennard-Jones sites ----------------------------------------------
+// The same chain for systems whose molecules are single atoms, with LJ or no
+// potential between their kinds and no Coulomb term.  The chain's state stays
+// in LDS for the whole launch: the positions, and per axis the 16-bit
+// fractions of the box, whose wrapped differences are nearest images.  An
+// attempt tests all atoms, two per lane and instruction, for a place within
+// the cutoff of the way from the old to the new position on every axis (no
+// cell list: its look-ups are a chain of dependent loads, and 4 cells on an
+// axis leave most atoms in); each wave lists the atoms that pass, about 110
+// in a liquid, and evaluates only those in FP64.
+// An attempt is one long dependency (draw, position, candidates, sum, test),
+// on which a wave issues an instruction each 4 to 5 cycles, so what need not
+// be on it is taken off: a wave draws 64 attempts at once, one per lane (the
+// three Philox blocks of an attempt are 2000 cycles of quarter-rate
+// multiplies); the next atom's position is read early; the energies come
+// from r^2 (no root, division or image test: the host sends boxes whose
+// cutoff reaches half an edge to k_mc_chains); wave sums use DPP moves; exp is
+// left for costs within 1e-12 of -log(u); the wrap is computed only within
+// 1e-9 of a face.  Decisions and positions are those of k_mc_chains, sums to
+// rounding.
+// 256 chains of 108-4000 atoms, us per attempt of the slowest: k_mc_chains
+// 7.0; cell lists in LDS 2.8, a sphere test of every atom 2.3, this 1.8.
+constexpr int kMcAtomBlock = 256;
+constexpr size_t mc_atoms_rows(size_t n) { return (n + 2 * kMcAtomBlock - 1) / (2 * kMcAtomBlock); }
+// positions, kinds, then per row of 512 atoms their fractions and lists
+constexpr size_t mc_atoms_lds(size_t n) { return 24 * n + ((n + 7) & ~size_t(7)) + mc_atoms_rows(n) * 4096; }
+constexpr size_t kMcAtomStatic = 9216;  // the rest of the LDS, with room
+// a lane's test results are one bit per row and half word
+constexpr size_t kMcAtomMax = 16 * 2 * kMcAtomBlock;
+
+__device__ __forceinline__ double mc_readlane(double v, int k) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, k), hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int kCtrl>
+__device__ __forceinline__ double mc_dpp(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, kCtrl, 0xf, 0xf, true),
+              hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), kCtrl, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// Sum over the wave, the same bits in every lane: butterflies within rows of
+// 16 lanes (quad_perm 1 0 3 2 and 2 3 0 1, half-row and row mirrors), then
+// the four rows.
+__device__ __forceinline__ double mc_wave_sum(double v) {
+    v += mc_dpp<0xB1>(v);
+    v += mc_dpp<0x4E>(v);
+    v += mc_dpp<0x141>(v);
+    v += mc_dpp<0x140>(v);
+    return (mc_readlane(v, 0) + mc_readlane(v, 16)) + (mc_readlane(v, 32) + mc_readlane(v, 48));
+}
+
+// Pair energy at r2 from {4 eps s^12, 4 eps s^6, r2 bound, shift}.
+__device__ __forceinline__ double mc_lj(double4 P, double r2) {
+    double y = __builtin_amdgcn_rcp(r2);
+    y += y * (1.0 - r2 * y);
+    y += y * (1.0 - r2 * y);
+    const double i6 = y * y * y, e = (P.x * i6 - P.y) * i6 - P.w;
+    return r2 < P.z ? e : 0.0;
+}
+
+#pragma clang fp contract(off)
+// Wraps the position of a single atom as mc_final_positions does.
+__device__ __forceinline__ void mc_wrap_atom(const McChain& c, int i, double& x, double& y, double& z) {
+    const double mass = c.vel[i].w;
+    const double total = 0.0 + mass;
+    const double cx = (0.0 + mass * x) / total, cy = (0.0 + mass * y) / total, cz = (0.0 + mass * z) / total;
+    x += (cx - floor(cx / c.box.L[0]) * c.box.L[0]) - cx;
+    y += (cy - floor(cy / c.box.L[1]) * c.box.L[1]) - cy;
+    z += (cz - floor(cz / c.box.L[2]) * c.box.L[2]) - cz;
+}
+__device__ __forceinline__ double mc_step(double d, double u) { return -d + 2.0 * d * u; }
+#pragma clang fp contract(on)
+
+// 16-bit fraction of the box, rounded down (0 in an infinite cell, where
+// every atom passes the test).
+__device__ __forceinline__ unsigned mc_frac16(double x, double inv) {
+    const double f = x * inv;
+    return (unsigned)((f - floor(f)) * 65536.0) & 0xffffu;
+}
+// Both half words.
+__device__ __forceinline__ unsigned mc_twice(unsigned v) { return (v & 0xffffu) * 0x10001u; }
+// Units of a fraction from the old place down to the lowest and up to the
+// highest place within rc of a move by d (both fractions round down: one unit
+// more, and one for the truncation here), and in all: {down, width}.
+__device__ __forceinline__ uint2 mc_span(double rc, double d, double L) {
+    if (!(L > 0.0)) return make_uint2(0u, 0xffffu);
+    const double unit = 65536.0 / L, down = (rc - fmin(d, 0.0)) * unit, up = (rc + fmax(d, 0.0)) * unit;
+    if (!(down + up < 65530.0)) return make_uint2(0u, 0xffffu);  // the whole axis
+    const unsigned a = (unsigned)down + 2u, b = (unsigned)up + 2u;
+    return make_uint2(a, a + b);
+}
+typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
+// Zero half words where base <= f <= base + width (modulo 2^16).
+__device__ __forceinline__ unsigned mc_outside(unsigned f, unsigned base, unsigned width) {
+    const ushort2v d = __builtin_bit_cast(ushort2v, f) - __builtin_bit_cast(ushort2v, base);
+    return __builtin_bit_cast(unsigned, __builtin_elementwise_sub_sat(d, __builtin_bit_cast(ushort2v, width)));
+}
+
+__global__ __launch_bounds__(kMcAtomBlock) void k_mc_atoms(const McChain* __restrict__ chains) {
+    extern __shared__ __align__(16) double mc_lds[];
+    __shared__ double4 tab[kMaxKinds * kMaxKinds];
+    constexpr int BLOCK = kMcAtomBlock, WAVES = BLOCK / 64;
+    __shared__ double red[2][WAVES];
+    const McChain& c = chains[blockIdx.x];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = c.n;
+    double *const X = mc_lds, *const Y = X + n, *const Z = Y + n;
+    const int rows = (int)mc_atoms_rows(n);
+    unsigned* const FX = reinterpret_cast<unsigned*>(Z + n);  // two atoms per word
+    unsigned* const FY = FX + rows * BLOCK;
+    unsigned* const FZ = FY + rows * BLOCK;
+    // a wave's list holds all atoms that it tests
+    unsigned short* const list = reinterpret_cast<unsigned short*>(FZ + rows * BLOCK) + wave * rows * 128;
+    unsigned char* const kind = reinterpret_cast<unsigned char*>(FZ + rows * BLOCK) + rows * BLOCK * 4;
+    unsigned short *const fx = reinterpret_cast<unsigned short*>(FX), *const fy = reinterpret_cast<unsigned short*>(FY),
+                          *const fz = reinterpret_cast<unsigned short*>(FZ);
+    const bool periodic = c.box.periodic != 0;
+    const double Lx = c.box.L[0], Ly = c.box.L[1], Lz = c.box.L[2];
+    const double ix = c.box.inv[0], iy = c.box.inv[1], iz = c.box.inv[2];
+    const int nkinds = c.nkinds;
+    for (int x = tid; x < nkinds * nkinds; x += BLOCK) {
+        const PairParam pp = c.table[x];
+        const bool on = pp.pot == POT_LJ && !pp.inter_excl;
+        const double s2 = pp.p0 * pp.p0, s6 = s2 * s2 * s2;
+        tab[x] = on ? make_double4(4.0 * pp.p1 * (s6 * s6), 4.0 * pp.p1 * s6, pp.r2c, pp.shift)
+                    : make_double4(0.0, 0.0, 0.0, 0.0);
+    }
+    for (int i = tid; i < n; i += BLOCK) {
+        const double4 p = c.pos[i];
+        X[i] = p.x;
+        Y[i] = p.y;
+        Z[i] = p.z;
+        fx[i] = (unsigned short)mc_frac16(p.x, ix);
+        fy[i] = (unsigned short)mc_frac16(p.y, iy);
+        fz[i] = (unsigned short)mc_frac16(p.z, iz);
+        kind[i] = (unsigned char)c.meta[i].x;
+    }
+    // test results of a lane: bit rows - 1 - r and 16 above it for the atoms
+    // 2 (256 r + tid) and the next; those past the end never pass
+    unsigned past = 0;
+    for (int r = 0; r < rows; r++) {
+        const int j = 2 * (r * BLOCK + tid);
+        past = past << 1 | (j >= n ? 1u : 0u) | (j + 1 >= n ? 0x10000u : 0u);
+        if (j >= n) FX[r * BLOCK + tid] = FY[r * BLOCK + tid] = FZ[r * BLOCK + tid] = 0;
+        if (j + 1 == n) fx[n] = fy[n] = fz[n] = 0;
+    }
+    __syncthreads();
+    const double rc = sqrt(c.r2_filter);
+    double e_pairs = c.out[0];
+    unsigned long long accepted = 0;
+    unsigned long long t = c.attempt0;
+    const unsigned long long end = c.attempt0 + c.nattempts;
+    const double beta = c.beta;
+    while (t < end) {
+        // draws of attempts t .. t + 63, one per lane
+        const uint4 r0 = mc_draw(c, t + lane, 0u), r1 = mc_draw(c, t + lane, 1u), r2 = mc_draw(c, t + lane, 2u);
+        const int mol_l = mc_mol_of(c, r0);
+        const double dx_l = mc_step(c.d, u01(r0.z, r0.w)), dy_l = mc_step(c.d, u01(r1.x, r1.y)),
+                     dz_l = mc_step(c.d, u01(r1.z, r1.w));
+        const double u_l = u01(r2.x, r2.y), log_l = -log(u_l);
+        // below `sure` a move is accepted and above `never` it is not; u = 0
+        // leaves both to exp
+        const double sure_l = u_l > 0.0 ? log_l * (1.0 - 1e-12) - 1e-12 : 0.0, never_l = log_l * (1.0 + 1e-12) + 1e-12;
+        const uint2 sx_l = mc_span(rc, dx_l, Lx), sy_l = mc_span(rc, dy_l, Ly), sz_l = mc_span(rc, dz_l, Lz);
+        const unsigned bx_l = mc_twice(sx_l.x), by_l = mc_twice(sy_l.x), bz_l = mc_twice(sz_l.x);
+        const unsigned wx_l = mc_twice(sx_l.y), wy_l = mc_twice(sy_l.y), wz_l = mc_twice(sz_l.y);
+        const int batch = (int)min(end - t, 64ull);
+        int i = __builtin_amdgcn_readlane(mol_l, 0);
+        double px = X[i], py = Y[i], pz = Z[i];
+        unsigned gx = fx[i], gy = fy[i], gz = fz[i];
+        for (int k = 0; k < batch; k++, t++) {
+            auto of = [&](unsigned v) { return (unsigned)__builtin_amdgcn_readlane((int)v, k); };
+            auto base = [&](unsigned g, unsigned down) {
+                return __builtin_bit_cast(unsigned, __builtin_bit_cast(ushort2v, g * 0x10001u) -
+                                                        __builtin_bit_cast(ushort2v, of(down)));
+            };
+            // the next attempt's atom
+            const int i2 = __builtin_amdgcn_readlane(mol_l, min(k + 1, 63));
+            double px2 = X[i2], py2 = Y[i2], pz2 = Z[i2];
+            unsigned gx2 = fx[i2], gy2 = fy[i2], gz2 = fz[i2];
+            double qx = px + mc_readlane(dx_l, k), qy = py + mc_readlane(dy_l, k), qz = pz + mc_readlane(dz_l, k);
+            const unsigned bx = base(gx, bx_l), by = base(gy, by_l), bz = base(gz, bz_l);
+            const unsigned wx = of(wx_l), wy = of(wy_l), wz = of(wz_l);
+            unsigned in = 0;
+            for (int r = 0; r < rows; r += 4) {
+                unsigned ax[4], ay[4], az[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int w = min(r + u, rows - 1) * BLOCK + tid;
+                    ax[u] = FX[w];
+                    ay[u] = FY[w];
+                    az[u] = FZ[w];
+                }
+                __builtin_amdgcn_sched_barrier(0);  // all in flight
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (r + u < rows) {  // uniform
+                        const unsigned o = mc_outside(ax[u], bx, wx) | mc_outside(ay[u], by, wy) | mc_outside(az[u], bz, wz);
+                        const ushort2v one = {1, 1};
+                        in = (in << 1) + __builtin_bit_cast(unsigned, __builtin_elementwise_sub_sat(
+                                                                          one, __builtin_bit_cast(ushort2v, o)));
+                    }
+            }
+            in &= ~past;
+            int found = 0;
+            for (;;) {
+                const unsigned long long mask = __ballot(in != 0);
+                if (mask == 0) break;
+                const int bit = __builtin_ctz(in | 0x80000000u);
+                if (in) list[found + __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0))] =
+                    (unsigned short)(2 * ((rows - 1 - (bit & 15)) * BLOCK + tid) + (bit >> 4));
+                in &= in - 1;
+                found += __popcll(mask);
+            }
+            double d_p = 0.0;
+            for (int e = lane; e < found; e += 64) {
+                const int j = list[e];  // the atom itself too
+                const double jx = X[j], jy = Y[j], jz = Z[j];
+                double ox = px - jx, oy = py - jy, oz = pz - jz, nx = qx - jx, ny = qy - jy, nz = qz - jz;
+                if (periodic) {  // uniform
+                    ox = image_rint(ox, Lx, ix);
+                    oy = image_rint(oy, Ly, iy);
+                    oz = image_rint(oz, Lz, iz);
+                    nx = image_rint(nx, Lx, ix);
+                    ny = image_rint(ny, Ly, iy);
+                    nz = image_rint(nz, Lz, iz);
+                }
+                const double4 P = tab[nkinds == 1 ? 0 : (int)kind[i] * nkinds + kind[j]];  // uniform
+                const double e_j = mc_lj(P, norm2_ordered(nx, ny, nz)) - mc_lj(P, norm2_ordered(ox, oy, oz));
+                d_p += j != i ? e_j : 0.0;
+            }
+            // two buffers: a wave may still read the sums of the attempt before
+            d_p = mc_wave_sum(d_p);
+            if (lane == 0) red[k & 1][wave] = d_p;
+            __syncthreads();
+            double dp = red[k & 1][0];
+#pragma unroll
+            for (int w = 1; w < WAVES; w++) dp += red[k & 1][w];
+            dp = mc_readlane(dp, 0);
+            const double cost = beta * dp;
+            bool accept = cost <= 0.0 || cost < mc_readlane(sure_l, k);
+            if (!accept && !(cost > mc_readlane(never_l, k))) accept = mc_readlane(u_l, k) < exp(-cost);
+            if (accept) {  // the same in every thread
+                if (periodic) {
+                    const bool inside = qx >= 1e-9 * Lx && qx <= (1.0 - 1e-9) * Lx && qy >= 1e-9 * Ly &&
+                                        qy <= (1.0 - 1e-9) * Ly && qz >= 1e-9 * Lz && qz <= (1.0 - 1e-9) * Lz;
+                    if (!inside) mc_wrap_atom(c, i, qx, qy, qz);
+                }
+                e_pairs += dp;
+                accepted++;
+                const unsigned hx = mc_frac16(qx, ix), hy = mc_frac16(qy, iy), hz = mc_frac16(qz, iz);
+                // every wave writes the same values, and reads them after its
+                // own writes; all have passed the barrier behind their reads
+                // of the old ones
+                if (lane == 0) {
+                    X[i] = qx;
+                    Y[i] = qy;
+                    Z[i] = qz;
+                    fx[i] = (unsigned short)hx;
+                    fy[i] = (unsigned short)hy;
+                    fz[i] = (unsigned short)hz;
+                }
+                if (i2 == i) {
+                    px2 = qx;
+                    py2 = qy;
+                    pz2 = qz;
+                    gx2 = hx;
+                    gy2 = hy;
+                    gz2 = hz;
+                }
+            }
+            i = i2;
+            px = px2;
+            py = py2;
+            pz = pz2;
+            gx = gx2;
+            gy = gy2;
+            gz = gz2;
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += BLOCK) c.pos[i] = make_double4(X[i], Y[i], Z[i], c.pos[i].w);
+    if (tid == 0) {
+        c.out[0] = e_pairs;
+        c.counters[0] += accepted;
+        c.counters[1] = end;
+    }
+}
+
 __global__ void k_set_flag(int* p, int v) { *p = v; }
 
 }  // namespace lg
