@@ -106,6 +106,7 @@ struct McChain {
     // (attempt0 + nattempts when complete)
     double* out;
     unsigned long long* counters;
+    int* rebuild;           // set for the neighbour list, or null
 };
 
 // Pair energy of an inter-molecular pair at distance r: the pair potential
@@ -656,6 +657,7 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_chains(const McChain* __restric
         c.out[1] = e_coul;
         c.counters[0] += accepted;
         c.counters[1] = t;
+        if (c.rebuild) *c.rebuild = 1;
     }
 }
 #pragma clang fp contract(on)
@@ -948,6 +950,7 @@ __global__ __launch_bounds__(kMcAtomBlock) void k_mc_atoms(const McChain* __rest
         c.out[0] = e_pairs;
         c.counters[0] += accepted;
         c.counters[1] = end;
+        if (c.rebuild) *c.rebuild = 1;
     }
 }
 

@@ -490,37 +490,53 @@ class System:
     # -- state -----------------------------------------------------------------
     @property
     def positions(self):
-        self._pull()
+        self._pull_positions()
         return self._positions
 
     @positions.setter
     def positions(self, value):
-        self._pull()
         self._positions = np.array(value, dtype=float).reshape(-1, 3)
+        self._stale_positions = False
         if self._handle is not None:
             nat.check(nat.lib().lg_system_set_positions(self._handle, nat.dptr(self._positions)))
 
     @property
     def velocities(self):
-        self._pull()
+        self._pull_velocities()
         return self._velocities
 
     @velocities.setter
     def velocities(self, value):
-        self._pull()
         self._velocities = np.array(value, dtype=float).reshape(-1, 3)
+        self._stale_velocities = False
         if self._handle is not None:
             nat.check(nat.lib().lg_system_set_velocities(self._handle, nat.dptr(self._velocities)))
 
+    # Whether the device holds newer positions or velocities.  Each is read
+    # when it is asked for: Monte Carlo leaves the velocities alone.
+    @property
+    def _device_state(self):
+        return self._stale_positions or self._stale_velocities
+
+    @_device_state.setter
+    def _device_state(self, value):
+        self._stale_positions = self._stale_velocities = value
+
+    def _pull_positions(self):
+        if self._handle is not None and self._stale_positions:
+            pos = np.empty((self.size(), 3))
+            nat.check(nat.lib().lg_system_get_positions(self._handle, nat.dptr(pos)))
+            self._positions, self._stale_positions = pos, False
+
+    def _pull_velocities(self):
+        if self._handle is not None and self._stale_velocities:
+            vel = np.empty((self.size(), 3))
+            nat.check(nat.lib().lg_system_get_velocities(self._handle, nat.dptr(vel)))
+            self._velocities, self._stale_velocities = vel, False
+
     def _pull(self):
-        if self._handle is not None and self._device_state:
-            L = nat.lib()
-            pos = np.zeros((self.size(), 3))
-            vel = np.zeros((self.size(), 3))
-            nat.check(L.lg_system_get_positions(self._handle, nat.dptr(pos)))
-            nat.check(L.lg_system_get_velocities(self._handle, nat.dptr(vel)))
-            self._positions, self._velocities = pos, vel
-            self._device_state = False
+        self._pull_positions()
+        self._pull_velocities()
 
     def particles_changed(self):
         """Push host-side edits of charges or masses to the device."""
@@ -799,7 +815,7 @@ class System:
         """EnergyCache::update (cache.rs:118-127) and the COM wrap of
         Translate::apply (translate.rs:115-127)."""
         nat.check(nat.lib().lg_move_commit(self._sync(), int(bool(wrap))))
-        self._device_state = True
+        self._stale_positions = True
 
     def move_discard(self):
         nat.check(nat.lib().lg_move_discard(self._sync()))
@@ -810,7 +826,7 @@ class System:
         acc = ctypes.c_uint64()
         nat.check(nat.lib().lg_mc_run(self._sync(), int(seed), int(attempt0), int(nattempts), float(beta),
                                       float(delta), ctypes.byref(acc)))
-        self._device_state = True
+        self._stale_positions = True
         return acc.value
 
 
@@ -831,7 +847,7 @@ def mc_run_batch(systems, seeds, attempt0, nattempts, beta, delta):
     nat.check(nat.lib().lg_mc_run_batch(handles, count, u64(seeds), u64(a0), u64(na), nat.dptr(beta),
                                         nat.dptr(delta), u64(acc)))
     for s in systems:
-        s._device_state = True
+        s._stale_positions = True
     return acc
 
 
