@@ -1261,6 +1261,9 @@ double max_cutoff(lg_system* s) {
     return rc;
 }
 
+constexpr size_t kDirectMax = 32768;  // atoms of the direct list build
+constexpr int kDenseCells = 27;       // cells of the per-cell list builds
+
 int prepare_nlist(lg_system* s) {
     size_t n = s->n;
     double rc = max_cutoff(s);
@@ -1299,7 +1302,18 @@ int prepare_nlist(lg_system* s) {
     };
     layout(true);
     double cells = double(g.n[0]) * g.n[1] * g.n[2];
-    if (cells > std::min(8.0 * double(n) + 4096.0, double(1 << 22))) layout(false);
+    if (cells > std::min(8.0 * double(n) + 4096.0, double(1 << 22))) {
+        layout(false);
+    } else if (n <= kDirectMax && (s->tune.nlist_build == 0 || s->tune.nlist_build == 3) && double(n) < 8.0 * cells) {
+        // short cutoffs leave 2 or 3 atoms in a half cell; full cells, if
+        // they hold 8, let the direct build run (cells_dense): its one launch
+        // replaces the cell list's and the lanes' build.  Lennard-Jones
+        // argon, rc 8.5 A, us per step with half / full cells: 4500 atoms
+        // 18.6 / 14.3, 20 000 32.1 / 17.2, 32 000 33.4 / 20.8
+        layout(false);
+        const double full = double(g.n[0]) * g.n[1] * g.n[2];
+        if (full < kDenseCells || double(n) < 8.0 * full) layout(true);
+    }
     g.ncell = g.n[0] * g.n[1] * g.n[2];
     // capacity from the mean density, with margin; exact sizes are checked
     // after every build (overflow flag) and grown on demand.
@@ -1328,6 +1342,10 @@ int prepare_nlist(lg_system* s) {
     // lists; not fewer than 8 (1M-atom Kob-Andersen: 4 lanes 660/720 us per
     // mixed/FP64 step, 8 lanes 562/625 us; lumol_amd.tuning picks per bucket)
     s->tpa = n <= 8192 ? 64 : n <= 32768 ? 32 : n <= 131072 ? 16 : 8;
+    // lists without Coulomb pairs are short (75 entries in liquid argon), and
+    // half of 64 lanes would idle: 16 against 64 lanes 14.2 / 15.8 us per
+    // step at 7919 atoms, 20.8 / 30.4 at 32 000 (8 lanes 14.9 / 20.7)
+    if (s->coul_kind == COUL_NONE) s->tpa = std::min(s->tpa, 16);
     if (s->tune.pair_lanes > 0) s->tpa = s->tune.pair_lanes;
     if (s->gen_pairs) s->tpa = 16;  // the general pair kernel has one instance
     LG_TRY(s->epart_pairs.ensure(size_t(pair_blocks_of(n, s->tpa)) * 8));
@@ -1376,13 +1394,14 @@ int prepare(lg_system* s) {
 // Verlet build: 1 lanes per atom over the cell list, 2 one workgroup per
 // cell over the cell list, 3 workgroups per cell (direct_split) over the
 // atoms' cell tags (no cell list; up to 32768 atoms and 1023 cells per axis).  Default:
-// the per-cell builds when there are >= 128 cells and >= 8 atoms per cell,
-// the direct one where it applies.
+// the per-cell builds when there are >= 27 cells (kDenseCells; argon of 1600
+// atoms in 64 cells: 18.0 us per step by lanes, 13.8 direct) and >= 8 atoms
+// per cell, the direct one where it applies.
 static bool direct_fits(const lg_system* s) {
-    return s->n <= 32768 && s->grid.n[0] <= 1023 && s->grid.n[1] <= 1023 && s->grid.n[2] <= 1023;
+    return s->n <= kDirectMax && s->grid.n[0] <= 1023 && s->grid.n[1] <= 1023 && s->grid.n[2] <= 1023;
 }
 static bool cells_dense(const lg_system* s) {
-    return s->grid.ncell >= 128 && s->n >= size_t(8) * s->grid.ncell;
+    return s->grid.ncell >= kDenseCells && s->n >= size_t(8) * s->grid.ncell;
 }
 static bool direct_build(const lg_system* s) {
     if (!direct_fits(s)) return false;
