@@ -380,6 +380,10 @@ struct lg_system {
     int cap = 0;
     DevBuf<int> cellid, slot, count, start, tmp, sorted, nbr, nnbr, flags;  // flags[0] rebuild, [1] overflow
     DevBuf<float4> cpos;  // list-build candidate records in sorted order
+    int listed_precision = 0;  // of the copies below
+    bool slot_rows = false;  // list entries name sorted places (slot_form), and
+    DevBuf<int> rank;        // where each atom is
+    DevBuf<double4> spos;    // FP64: the positions in that order
     DevBuf<float4> frac;  // positions as the mixed pair kernel reads them (frac_pos)
     double3 frac_origin = make_double3(0.0, 0.0, 0.0);  // infinite cells: atom 0 at the last set
     // parameters
@@ -1264,6 +1268,47 @@ double max_cutoff(lg_system* s) {
 constexpr size_t kDirectMax = 32768;  // atoms of the direct list build
 constexpr int kDenseCells = 27;       // cells of the per-cell list builds
 
+// Neighbour-list maintenance.  `check` runs the displacement test here; the
+// MD step does it inside the integrator's first half instead.  Every kernel
+// returns at once when flags[0] (rebuild) is clear; the build kernel clears
+// it again.
+// Which list-build kernel runs: one workgroup per cell (k_nlist_cells) when
+// there are enough cells to fill the device and enough atoms per cell to keep
+// its waves busy, else TPA lanes per atom (k_nlist_build); the tuning knob
+// nlist_build overrides (1 lanes per atom, 2 cells).
+// Verlet build: 1 lanes per atom over the cell list, 2 one workgroup per
+// cell over the cell list, 3 workgroups per cell (direct_split) over the
+// atoms' cell tags (no cell list; up to 32768 atoms and 1023 cells per axis).  Default:
+// the per-cell builds when there are >= 27 cells (kDenseCells; argon of 1600
+// atoms in 64 cells: 18.0 us per step by lanes, 13.8 direct) and >= 8 atoms
+// per cell, the direct one where it applies.
+static bool direct_fits(const lg_system* s) {
+    return s->n <= kDirectMax && s->grid.n[0] <= 1023 && s->grid.n[1] <= 1023 && s->grid.n[2] <= 1023;
+}
+static bool cells_dense(const lg_system* s) {
+    return s->grid.ncell >= kDenseCells && s->n >= size_t(8) * s->grid.ncell;
+}
+static bool direct_build(const lg_system* s) {
+    if (!direct_fits(s)) return false;
+    if (s->tune.nlist_build == 3) return true;
+    return s->tune.nlist_build == 0 && cells_dense(s);
+}
+static bool cell_build(const lg_system* s) {
+    if (s->tune.nlist_build == 1) return false;
+    if (s->tune.nlist_build == 2 || s->tune.nlist_build == 3) return true;
+    return cells_dense(s);
+}
+// Whether one workgroup makes the cell list (k_cell_small).
+static size_t cells_small_lds(const lg_system* s) { return size_t(8) * s->grid.ncell + 4 + size_t(8) * s->n; }
+static bool cells_small(const lg_system* s) {
+    return s->grid.ncell < 65536 && s->n <= 32768 && cells_small_lds(s) <= s->ctx->max_shared;
+}
+// Whether list entries name sorted places and the pair kernels' positions are
+// kept in that order (k_cell_rank): where the cell list is made by the chain
+// of kernels, that is above about 16 000 atoms unless the direct build runs.
+// Smaller systems' positions fit the caches in any order.
+static bool slot_form(const lg_system* s) { return !s->gen_pairs && !direct_build(s) && !cells_small(s); }
+
 int prepare_nlist(lg_system* s) {
     size_t n = s->n;
     double rc = max_cutoff(s);
@@ -1328,8 +1373,9 @@ int prepare_nlist(lg_system* s) {
     s->cap = int(std::max<size_t>(capacity, 1));
     LG_TRY(s->cellid.ensure(n));
     LG_TRY(s->slot.ensure(n));
-    LG_TRY(s->count.ensure(g.ncell));
-    LG_TRY(s->start.ensure(g.ncell + 1));
+    const size_t scan_cells = (size_t(g.ncell) + kScanCells) / kScanCells * kScanCells;  // k_cell_scan, with start[ncell]
+    LG_TRY(s->count.ensure(scan_cells));
+    LG_TRY(s->start.ensure(scan_cells));
     LG_TRY(s->tmp.ensure(n));
     LG_TRY(s->sorted.ensure(n));
     LG_TRY(s->cpos.ensure(n));
@@ -1344,14 +1390,23 @@ int prepare_nlist(lg_system* s) {
     s->tpa = n <= 8192 ? 64 : n <= 32768 ? 32 : n <= 131072 ? 16 : 8;
     // lists without Coulomb pairs are short (75 entries in liquid argon), and
     // half of 64 lanes would idle: 16 against 64 lanes 14.2 / 15.8 us per
-    // step at 7919 atoms, 20.8 / 30.4 at 32 000 (8 lanes 14.9 / 20.7)
-    if (s->coul_kind == COUL_NONE) s->tpa = std::min(s->tpa, 16);
+    // step at 7919 atoms, 20.8 / 30.4 at 32 000 (8 lanes 14.9 / 20.7); above, 8
+    // against 16 lanes 48.3 / 53.9 at 100 000
+    if (s->coul_kind == COUL_NONE) s->tpa = n <= 32768 ? std::min(s->tpa, 16) : 8;
     if (s->tune.pair_lanes > 0) s->tpa = s->tune.pair_lanes;
     if (s->gen_pairs) s->tpa = 16;  // the general pair kernel has one instance
     LG_TRY(s->epart_pairs.ensure(size_t(pair_blocks_of(n, s->tpa)) * 8));
     int init[4] = {1, 0, 0, 0};  // force a rebuild; clear overflow
     LG_HIP(hipMemcpyAsync(s->flags.p, init, sizeof(init), hipMemcpyHostToDevice, S(s)));
     LG_HIP(hipMemsetAsync(s->count.p, 0, g.ncell * sizeof(int), S(s)));
+    s->slot_rows = slot_form(s);
+    s->listed_precision = s->precision;
+    if (s->slot_rows) {
+        // any valid place until the first build sets them
+        LG_TRY(s->rank.ensure(n));
+        LG_HIP(hipMemsetAsync(s->rank.p, 0, n * sizeof(int), S(s)));
+        if (s->precision != LG_PRECISION_MIXED) LG_TRY(s->spos.ensure(n));
+    }
     s->nlist_dirty = false;
     return LG_OK;
 }
@@ -1359,6 +1414,9 @@ int prepare_nlist(lg_system* s) {
 
 int prepare(lg_system* s) {
     if (s->n == 0) return fail(LG_E_INVALID, "empty system");
+    // the lists hold another form of entries, or lack the copies that the
+    // other precision reads
+    if (s->listed_precision != s->precision && s->slot_rows) s->nlist_dirty = true;
     if (s->topo_dirty || s->meta_dirty || s->params_dirty || s->kspace_dirty || s->nlist_dirty) {
         s->cfg_epoch++;
         s->mc_ready = false;
@@ -1378,46 +1436,19 @@ int prepare(lg_system* s) {
         if (s->coul_kind != COUL_NONE && s->coul_rc > half)
             return fail(LG_E_INVALID, "The cutoff for the coulomb potential is bigger than half the cell length");
     }
+    if (slot_form(s) != s->slot_rows) s->nlist_dirty = true;  // gen_pairs may have changed
     if (s->nlist_dirty) LG_TRY(prepare_nlist(s));
     return LG_OK;
 }
 
 // ---- kernel sequences --------------------------------------------------------------------
-// Neighbour-list maintenance.  `check` runs the displacement test here; the
-// MD step does it inside the integrator's first half instead.  Every kernel
-// returns at once when flags[0] (rebuild) is clear; the build kernel clears
-// it again.
-// Which list-build kernel runs: one workgroup per cell (k_nlist_cells) when
-// there are enough cells to fill the device and enough atoms per cell to keep
-// its waves busy, else TPA lanes per atom (k_nlist_build); the tuning knob
-// nlist_build overrides (1 lanes per atom, 2 cells).
-// Verlet build: 1 lanes per atom over the cell list, 2 one workgroup per
-// cell over the cell list, 3 workgroups per cell (direct_split) over the
-// atoms' cell tags (no cell list; up to 32768 atoms and 1023 cells per axis).  Default:
-// the per-cell builds when there are >= 27 cells (kDenseCells; argon of 1600
-// atoms in 64 cells: 18.0 us per step by lanes, 13.8 direct) and >= 8 atoms
-// per cell, the direct one where it applies.
-static bool direct_fits(const lg_system* s) {
-    return s->n <= kDirectMax && s->grid.n[0] <= 1023 && s->grid.n[1] <= 1023 && s->grid.n[2] <= 1023;
-}
-static bool cells_dense(const lg_system* s) {
-    return s->grid.ncell >= kDenseCells && s->n >= size_t(8) * s->grid.ncell;
-}
-static bool direct_build(const lg_system* s) {
-    if (!direct_fits(s)) return false;
-    if (s->tune.nlist_build == 3) return true;
-    return s->tune.nlist_build == 0 && cells_dense(s);
-}
-static bool cell_build(const lg_system* s) {
-    if (s->tune.nlist_build == 1) return false;
-    if (s->tune.nlist_build == 2 || s->tune.nlist_build == 3) return true;
-    return cells_dense(s);
-}
 // Where the displacement tests write the atoms' cell tags: only for the
 // direct build.
 static CellTag cell_tags(lg_system* s) {
     return CellTag{direct_build(s) ? s->cellid.p : nullptr, s->grid, s->box,
-                   s->precision == LG_PRECISION_MIXED ? s->frac.p : nullptr, s->frac_origin};
+                   s->precision == LG_PRECISION_MIXED ? s->frac.p : nullptr, s->frac_origin,
+                   s->slot_rows ? s->rank.p : nullptr,
+                   s->slot_rows && s->precision != LG_PRECISION_MIXED ? s->spos.p : nullptr};
 }
 static MdArgs md_args(lg_system* s) {
     const double hs = 0.5 * s->skin;
@@ -1616,9 +1647,8 @@ int launch_nlist(lg_system* s, bool check, bool energy) {
     }
     if (prof < 0) prof = prof_start(s, LG_KERNEL_NLIST);
     // small systems: the whole cell list in one workgroup
-    size_t small_lds = size_t(8) * g.ncell + 4 + size_t(8) * n;
-    if (g.ncell < 65536 && n <= 32768 && small_lds <= s->ctx->max_shared) {
-        k_cell_small<<<1, 1024, small_lds, st>>>(s->pos.p, s->meta.p, n, g, s->box, s->cellid.p, s->start.p,
+    if (cells_small(s)) {
+        k_cell_small<<<1, 1024, cells_small_lds(s), st>>>(s->pos.p, s->meta.p, n, g, s->box, s->cellid.p, s->start.p,
                                                  s->sorted.p, s->cpos.p, flag);
     } else {
         k_cell_count<<<blocks_for(n, 256), 256, 0, st>>>(s->pos.p, n, g, s->box, s->cellid.p, s->slot.p,
@@ -1627,14 +1657,19 @@ int launch_nlist(lg_system* s, bool check, bool energy) {
         k_cell_scatter<<<blocks_for(n, 256), 256, 0, st>>>(s->cellid.p, s->slot.p, s->start.p, s->tmp.p, n,
                                                             flag);
         k_cell_rank<<<std::min(blocks_for(g.ncell, 4), kRankBlocks), 256, 0, st>>>(
-            s->tmp.p, s->start.p, s->sorted.p, s->cpos.p, s->pos.p, s->meta.p, s->box, g.ncell, flag);
+            s->tmp.p, s->start.p, s->sorted.p, s->cpos.p, s->pos.p, s->meta.p, s->box, g.ncell, flag,
+            s->slot_rows ? s->rank.p : nullptr, cell_tags(s));
     }
-    int nb = blocks_for(size_t(n) * s->tpa, 256);
+    // the build by lanes pays for each run of cells once per lane group: 4
+    // lanes against 8, 10^6 Kob-Andersen atoms: 314 / 328 us per step, 36 000
+    // atoms (too few waves) 28.3 / 27.9
+    const int lanes = s->tune.pair_lanes == 0 && n > 131072 ? std::min(s->tpa, 4) : s->tpa;
+    int nb = blocks_for(size_t(n) * lanes, 256);
     // FP32 candidate test with a 1e-4 relative margin on rlist
     float rl2f = (!s->periodic || s->rlist <= 0) ? INFINITY : float(s->rlist * (1.0 + 1e-4) * s->rlist * (1.0 + 1e-4));
     if (cell_build(s)) {
         CellsArgs ca{s->meta.p, s->cpos.p, s->sorted.p, s->start.p, s->count.p, g, s->box, rl2f, s->cap,
-                     s->nbr.p, s->nnbr.p, s->pos.p, s->ref.p, flag};
+                     s->nbr.p, s->nnbr.p, s->pos.p, s->ref.p, flag, s->slot_rows};
         const bool nearest = s->periodic && (g.reach[0] == 0 || g.reach[1] == 0 || g.reach[2] == 0);
         prof_stop(s, prof);
         long p2 = prof_start(s, LG_KERNEL_NLIST);
@@ -1646,12 +1681,12 @@ int launch_nlist(lg_system* s, bool check, bool energy) {
         LG_HIP(hipGetLastError());
         return LG_OK;
     }
-    switch (s->tpa) {
+    switch (lanes) {
 #define LG_BUILD_CASE(T)                                                                                   \
     case T:                                                                                                \
         k_nlist_build<T><<<nb, 256, 0, st>>>(s->cpos.p, s->sorted.p, s->cellid.p, s->start.p, s->count.p, g,  \
                                              s->box, rl2f, n, s->cap, s->nbr.p, s->nnbr.p, s->pos.p, s->ref.p,  \
-                                             flag, s->meta.p);                                                \
+                                             flag, s->meta.p, s->slot_rows);                                  \
         break;
         LG_BUILD_CASE(4)
         LG_BUILD_CASE(8)
@@ -1732,11 +1767,12 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
     pa.tie = s->periodic && max_cutoff(s) > (0.5 - 1e-6) * std::min(s->L[0], std::min(s->L[1], s->L[2]));
     pa.hf_inv_h = s->hf_inv_h;
     pa.frac = s->frac.p;
-    if (mixed && !s->gen_pairs && !frac_done) {
-        // the MD half-steps write the FP32 positions beside the new ones;
+    pa.slots = s->slot_rows;
+    pa.ppos = s->slot_rows ? s->spos.p : s->pos.p;
+    if ((mixed || s->slot_rows) && !s->gen_pairs && !frac_done) {
+        // the MD half-steps write these copies beside the new positions;
         // any other caller converts the current positions here
-        launch_timed(s, LG_KERNEL_PAIRS, k_frac, blocks_for(n, 256), 256, 0, s->pos.p, n, s->box, s->frac_origin,
-                     s->frac.p);
+        launch_timed(s, LG_KERNEL_PAIRS, k_frac, blocks_for(n, 256), 256, 0, s->pos.p, n, cell_tags(s));
     }
     // the intra-molecular terms run as the last blocks of the list launch
     // (forces only, direct build) or of the rho(k) launch (intra_done), of
@@ -2334,6 +2370,8 @@ int lg_system_destroy(lg_system* s) {
     s->mc_cell_pos.release();
     s->cpos.release();
     s->frac.release();
+    s->rank.release();
+    s->spos.release();
     s->mc_cell_ids.release();
     s->bparam.release();
     s->aparam.release();
@@ -2901,6 +2939,7 @@ int lg_molecular_virial(lg_system* s, double* w9) {
     a.pos = s->pos.p;
     a.meta = s->meta.p;
     a.sorted = s->sorted.p;
+    a.slots = s->slot_rows;
     a.nbr = s->nbr.p;
     a.nnbr = s->nnbr.p;
     a.cap = s->cap;
@@ -2974,7 +3013,7 @@ int lg_pairs_within(lg_system* s, double cutoff, uint32_t* pairs, uint64_t capac
     LG_HIP(hipMemsetAsync(cnt.p, 0, sizeof(unsigned long long), S(s)));
     int n = int(s->n);
     k_pairs_within<<<blocks_for(n, 256), 256, 0, S(s)>>>(s->pos.p, s->sorted.p, s->nbr.p, s->nnbr.p, n, s->cap,
-                                                         s->box, cutoff, out.p, capacity, cnt.p);
+                                                         s->box, cutoff, int(s->slot_rows), out.p, capacity, cnt.p);
     LG_HIP(hipGetLastError());
     unsigned long long c = 0;
     LG_HIP(hipMemcpyAsync(&c, cnt.p, sizeof(c), hipMemcpyDeviceToHost, S(s)));

@@ -40,6 +40,9 @@ struct Grid {
 __host__ __device__ __forceinline__ int nbr_entry(int j, int kind) { return j | (kind << 24); }
 __host__ __device__ __forceinline__ int nbr_atom(int e) { return e & 0xffffff; }
 __host__ __device__ __forceinline__ int nbr_kind(int e) { return e >> 24; }
+// Molecule and kind of a candidate record of the list builds, so that a build
+// reads nothing else per candidate.
+__host__ __device__ __forceinline__ int mol_kind(int2 meta) { return meta.y | (meta.x << 24); }
 
 // Rebuild protocol: a displacement test (here, or in the MD first half-step)
 // sets *flag when an atom moved more than skin/2 since the last build; the
@@ -87,6 +90,10 @@ struct CellTag {
     Box b;
     float4* frac;
     double3 fo;  // origin of the FP32 Cartesian coordinates in an infinite cell
+    // slot form of the lists (see k_cell_rank): where atom i is kept in frac,
+    // or in spos for the FP64 kernel; else null
+    const int* rank;
+    double4* spos;
 };
 __host__ __device__ __forceinline__ int cell_tag(const CellTag& t, double4 p) {
     const int cx = cell_coord(p.x, t.b.L[0], t.b.inv[0], t.g.n[0], t.g.inv_size[0], t.b.periodic);
@@ -118,9 +125,16 @@ __device__ __forceinline__ float4 frac_pos(const Box& b, double3 fo, double4 p) 
                        __uint_as_float(fixed_frac(p.z, b.inv[2])), (float)p.w);
 }
 
-__global__ void k_frac(const double4* __restrict__ pos, int n, Box b, double3 fo, float4* __restrict__ frac) {
+// Writes the copies that the pair kernels read (frac, spos), if any.
+__device__ __forceinline__ void place_copies(const CellTag& tg, int i, double4 p) {
+    const int r = tg.rank ? tg.rank[i] : i;
+    if (tg.frac) tg.frac[r] = frac_pos(tg.b, tg.fo, p);
+    if (tg.spos) tg.spos[r] = p;
+}
+
+__global__ void k_frac(const double4* __restrict__ pos, int n, CellTag tg) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) frac[i] = frac_pos(b, fo, pos[i]);
+    if (i < n) place_copies(tg, i, pos[i]);
 }
 
 __global__ void k_nlist_check(const double4* __restrict__ pos, const double4* __restrict__ ref, int n,
@@ -151,57 +165,62 @@ __global__ void k_cell_count(const double4* __restrict__ pos, int n, Grid g, Box
     slot[i] = atomicAdd(&count[c], 1);
 }
 
-// Exclusive scan of the per-cell counts (one block, 1024 threads), chunk by
-// chunk of blockDim cells with a running carry; the counts of kScanBatch
-// chunks are loaded together, so that the chunks wait for memory once per
-// batch (at 50k cells, one wait per chunk cost ~300 us per rebuild).
-constexpr int kScanBatch = 8;
-__global__ void k_cell_scan(const int* __restrict__ count, int* __restrict__ start, int ncell, const int* __restrict__ flag) {
+// Exclusive scan of the per-cell counts (one block, 1024 threads): a thread
+// takes 32 consecutive cells, their loads in flight together, so that 32768
+// cells cost one wait for memory and one block scan (a cell per thread and
+// four barriers for each 1024 cells cost 268 us per rebuild at 339 000 cells,
+// this 109).  The arrays are padded to a multiple of 32 cells.
+constexpr int kScanCells = 32;
+__global__ __launch_bounds__(1024) void k_cell_scan(const int* __restrict__ count, int* __restrict__ start, int ncell,
+                                                    const int* __restrict__ flag) {
     if (*flag == 0) return;
-    __shared__ int warp_sums[16];
-    __shared__ int carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    for (int base0 = 0; base0 < ncell; base0 += kScanBatch * blockDim.x) {
-        int vb[kScanBatch];
+    __shared__ int wsum[2][16];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    int carry = 0;
+    for (int base = 0, it = 0; base < ncell; base += 1024 * kScanCells, it ^= 1) {
+        const int c0 = base + tid * kScanCells;
+        int4 v[kScanCells / 4];
 #pragma unroll
-        for (int u = 0; u < kScanBatch; u++) {
-            const int c = base0 + u * blockDim.x + threadIdx.x;
-            vb[u] = c < ncell ? count[c] : 0;
-        }
+        for (int u = 0; u < kScanCells / 4; u++)
+            v[u] = c0 < ncell ? reinterpret_cast<const int4*>(count + c0)[u] : make_int4(0, 0, 0, 0);
+        int local = 0;
 #pragma unroll
-        for (int u = 0; u < kScanBatch; u++) {
-            const int base = base0 + u * blockDim.x;
-            if (base >= ncell) break;  // uniform
-            const int c = base + threadIdx.x;
-            const int v = vb[u];
-            // inclusive scan within the wave
-            int x = v;
-            for (int off = 1; off < 64; off <<= 1) {
-                int y = __shfl_up(x, off, 64);
-                if (lane >= off) x += y;
-            }
-            if (lane == 63) warp_sums[wid] = x;
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                int s = 0;
-                int nw = blockDim.x >> 6;
-                for (int w = 0; w < nw; w++) {
-                    int t = warp_sums[w];
-                    warp_sums[w] = s;
-                    s += t;
-                }
-            }
-            __syncthreads();
-            int excl = carry + warp_sums[wid] + x - v;
-            if (c < ncell) start[c] = excl;
-            __syncthreads();
-            if (threadIdx.x == blockDim.x - 1) carry = excl + v;
-            __syncthreads();
+        for (int u = 0; u < kScanCells / 4; u++) {
+            // cells past the last are whatever the padding holds
+            const int c = c0 + 4 * u;
+            v[u].x = c < ncell ? v[u].x : 0;
+            v[u].y = c + 1 < ncell ? v[u].y : 0;
+            v[u].z = c + 2 < ncell ? v[u].z : 0;
+            v[u].w = c + 3 < ncell ? v[u].w : 0;
+            local += (v[u].x + v[u].y) + (v[u].z + v[u].w);
         }
+        int x = local;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(x, off, 64);
+            if (lane >= off) x += y;
+        }
+        if (lane == 63) wsum[it][wid] = x;
+        __syncthreads();
+        int run = carry + x - local;
+        for (int w = 0; w < 16; w++) {
+            if (w < wid) run += wsum[it][w];
+            carry += wsum[it][w];
+        }
+        if (c0 < ncell)
+#pragma unroll
+            for (int u = 0; u < kScanCells / 4; u++) {
+                int4 o;
+                o.x = run;
+                o.y = o.x + v[u].x;
+                o.z = o.y + v[u].y;
+                o.w = o.z + v[u].z;
+                run = o.w + v[u].w;
+                reinterpret_cast<int4*>(start + c0)[u] = o;
+            }
     }
-    if (threadIdx.x == 0) start[ncell] = carry;
+    // after the padding's values, which a thread of another wave may write
+    __syncthreads();
+    if (tid == 0) start[ncell] = carry;
 }
 
 __global__ void k_cell_scatter(const int* __restrict__ cellid, const int* __restrict__ slot,
@@ -219,11 +238,19 @@ __global__ void k_cell_scatter(const int* __restrict__ cellid, const int* __rest
 // on every step, rebuild or not, in block dispatch alone.  Also writes the
 // candidate record of the list build in sorted order: FP32 wrapped position
 // (the binning's own wrap) and the molecule id.
+// Slot form (tg.rank): large systems keep the copies of the positions that
+// the pair kernel gathers in sorted order, and list entries name places in
+// that order.  The atoms of a run of cells then lie in a row, and a wave's
+// gather touches a few cache lines instead of one per lane: 10^6 Kob-Andersen
+// atoms, mixed, pair kernel 363 -> 215 us (its
+// address units are busy 80% of that, its arithmetic 60%).  The copies and the atoms'
+// places (rank) are rewritten here with the order.
 constexpr int kRankBlocks = 4096;
 __global__ __launch_bounds__(256) void k_cell_rank(const int* __restrict__ tmp, const int* __restrict__ start,
                                                    int* __restrict__ sorted, float4* __restrict__ cpos,
                                                    const double4* __restrict__ pos, const int2* __restrict__ meta,
-                                                   Box b, int ncell, const int* __restrict__ flag) {
+                                                   Box b, int ncell, const int* __restrict__ flag,
+                                                   int* __restrict__ rank_out, CellTag tg) {
     if (*flag == 0) return;
     const int lane = threadIdx.x & 63;
     const int wid = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), nw = (int)((gridDim.x * blockDim.x) >> 6);
@@ -238,7 +265,12 @@ __global__ __launch_bounds__(256) void k_cell_rank(const int* __restrict__ tmp, 
             cpos[s + rank] = make_float4((float)wrap_coord(p.x, b.L[0], b.inv[0], b.periodic),
                                          (float)wrap_coord(p.y, b.L[1], b.inv[1], b.periodic),
                                          (float)wrap_coord(p.z, b.L[2], b.inv[2], b.periodic),
-                                         __int_as_float(meta[v].y));
+                                         __int_as_float(mol_kind(meta[v])));
+            if (rank_out) {
+                rank_out[v] = s + rank;
+                if (tg.frac) tg.frac[s + rank] = frac_pos(tg.b, tg.fo, p);
+                if (tg.spos) tg.spos[s + rank] = p;
+            }
         }
     }
 }
@@ -354,7 +386,7 @@ __global__ __launch_bounds__(1024) void k_cell_small(const double4* __restrict__
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             pv[u] = pos[vv[u]];
-            mv[u] = meta[vv[u]].y;
+            mv[u] = mol_kind(meta[vv[u]]);
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -388,7 +420,8 @@ __global__ __launch_bounds__(256) void k_nlist_build(const float4* __restrict__ 
                                                      int* __restrict__ count_zero, Grid g, Box b, float rl2f,
                                                      int n, int cap, int* __restrict__ nbr, int* __restrict__ nnbr,
                                                      const double4* __restrict__ pos, double4* __restrict__ ref,
-                                                     int* __restrict__ flags, const int2* __restrict__ meta) {
+                                                     int* __restrict__ flags, const int2* __restrict__ meta,
+                                                     int slots) {
     if (flags[0] == 0) return;
     int gid = blockIdx.x * blockDim.x + threadIdx.x;
     for (int c = gid; c < g.ncell; c += gridDim.x * blockDim.x) count_zero[c] = 0;
@@ -398,7 +431,7 @@ __global__ __launch_bounds__(256) void k_nlist_build(const float4* __restrict__ 
     if (t < n) {
         int i = sorted[t];
         float4 pi = cpos[t];
-        int mi = __float_as_int(pi.w);
+        int mi = __float_as_int(pi.w) & 0xffffff;
         int c = cellid[i];
         int cx = c % g.n[0];
         int cy = (c / g.n[0]) % g.n[1];
@@ -481,7 +514,8 @@ __global__ __launch_bounds__(256) void k_nlist_build(const float4* __restrict__ 
             // a ballot prefix count
             auto pass = [&](int q, float4 cj, int jj) {
                 bool accept = false;
-                if (q < cur.e0 && __float_as_int(cj.w) != mi) {
+                const int mk = __float_as_int(cj.w);
+                if (q < cur.e0 && (mk & 0xffffff) != mi) {
                     float ddx = ddx0 - cj.x, ddy = ddy0 - cj.y, ddz = ddz0 - cj.z;
                     if (nx1) ddx -= rintf(ddx * ix) * Lx;
                     if (ny1) ddy -= rintf(ddy * iy) * Ly;
@@ -491,7 +525,7 @@ __global__ __launch_bounds__(256) void k_nlist_build(const float4* __restrict__ 
                 unsigned long long bal = __ballot(accept);
                 unsigned long long gm = TPA == 64 ? bal : ((bal >> gbase) & ((1ull << (TPA & 63)) - 1ull));
                 int slot = count + __popcll(gm & ((1ull << sub) - 1ull));
-                if (accept && slot < cap) row[slot] = nbr_entry(jj, meta[jj].x);
+                if (accept && slot < cap) row[slot] = nbr_entry(slots ? q : jj, mk >> 24);
                 count += __popcll(gm);
             };
             // two passes per iteration on alternating registers, each
@@ -500,13 +534,13 @@ __global__ __launch_bounds__(256) void k_nlist_build(const float4* __restrict__ 
             auto clampq = [&](int q) { return q < n ? q : n - 1; };
             int q = cur.s0 + sub;
             float4 cA = cpos[clampq(q)];
-            int jA = sorted[clampq(q)];
+            int jA = slots ? 0 : sorted[clampq(q)];
             for (int q0 = cur.s0; q0 < cur.e0; q0 += 2 * TPA) {
                 float4 cB = cpos[clampq(q + TPA)];
-                int jB = sorted[clampq(q + TPA)];
+                int jB = slots ? 0 : sorted[clampq(q + TPA)];
                 pass(q, cA, jA);
                 cA = cpos[clampq(q + 2 * TPA)];
-                jA = sorted[clampq(q + 2 * TPA)];
+                if (!slots) jA = sorted[clampq(q + 2 * TPA)];
                 if (q0 + TPA < cur.e0) pass(q + TPA, cB, jB);
                 q += 2 * TPA;
             }
@@ -612,6 +646,7 @@ struct CellsArgs {
     const double4* pos;
     double4* ref;
     int* flags;
+    int slots;  // entries name sorted places (k_cell_rank)
 };
 
 // kMinImage: some axis has a single cell (nearest image along it).  Block
@@ -726,7 +761,9 @@ __device__ __forceinline__ void nlist_cells_block(const CellsArgs& args, int blk
         for (int h0 = 0; h0 < H; h0 += kCellHome) {
             const int hn = min(kCellHome, H - h0);
             if (tid < hn) {
-                home[tid] = cpos[hs + h0 + tid];
+                float4 hp = cpos[hs + h0 + tid];
+                hp.w = __int_as_float(__float_as_int(hp.w) & 0xffffff);
+                home[tid] = hp;
                 home_row[tid] = hs + h0 + tid;
                 home_cnt[tid] = 0;
             }
@@ -747,22 +784,21 @@ __device__ __forceinline__ void nlist_cells_block(const CellsArgs& args, int blk
                     qv[r] = seg_s0[k] + (mm - seg_base[k]);
                 }
                 float4 cv[R];
-                int jv[R], kv2[R];
+                int jv[R];
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     cv[r] = cpos[qv[r]];
-                    jv[r] = sorted[qv[r]];
+                    jv[r] = args.slots ? qv[r] : sorted[qv[r]];
                 }
-#pragma unroll
-                for (int r = 0; r < R; r++) kv2[r] = args.meta[jv[r]].x;
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     int e = tid + r * kCellBlock;
                     if (e < tl) {
                         int k = kv[r];
+                        const int mk = __float_as_int(cv[r].w);
                         tile[e] = make_float4(cv[r].x + seg_sh[k][0], cv[r].y + seg_sh[k][1],
-                                              cv[r].z + seg_sh[k][2], cv[r].w);
-                        tidx[e] = nbr_entry(jv[r], kv2[r]);
+                                              cv[r].z + seg_sh[k][2], __int_as_float(mk & 0xffffff));
+                        tidx[e] = nbr_entry(jv[r], mk >> 24);
                     }
                 }
                 __syncthreads();
@@ -1320,7 +1356,8 @@ __device__ __forceinline__ void rho_reduce_block(const RhoReduceArgs& a, int blk
 // real space or Wolf, one lane per atom i over its neighbour list.
 // Forces are written for every i (full list, both directions), so no atomics
 // are needed and the per-atom sums are deterministic.  Energies and the
-// virial are accumulated for j > i only, the reference's i < j pair set.
+// virial are accumulated for j > i only (in the slot form by sorted place):
+// each pair of the reference's i < j set once.
 // ---------------------------------------------------------------------------------
 struct PairArgs {
     const double4* pos;
@@ -1353,6 +1390,10 @@ struct PairArgs {
     int tie;             // a cutoff reaches half the box: images within 1e-9 of a tie are checked
     const double* tabs;  // TableComputation tables (general instance)
     const float4* frac;  // positions as frac_pos (mixed instance)
+    // positions as the fast FP64 instance reads them, by atom, or with `slots`
+    // by sorted place (frac too); list entries name the same
+    const double4* ppos;
+    int slots;
     // the real-space force factor h(r) = erfc(alpha r) + g0 r exp(-alpha^2 r^2)
     // in FP32 pieces over [0, rc] (mixed instance, Ewald and Wolf), or null
     const float* hf32;
@@ -1471,7 +1512,8 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs(PairArgs a) {
     int i = -1;
     if (t < a.n) {
         i = a.sorted[t];
-        const double4 pi = a.pos[i];
+        const int self = a.slots ? t : i;
+        const double4 pi = a.ppos[self];
         const int ki = a.meta[i].x;
         const double qi = pi.w / kFourPiEps0;
         const int nn = a.nnbr[t];
@@ -1489,7 +1531,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs(PairArgs a) {
         // itself, never evaluated.
         auto jat = [&](int k) {
             int v = row[min(k, max(nn - 1, 0))];
-            return k < nn ? v : nbr_entry(i, ki);
+            return k < nn ? v : nbr_entry(self, ki);
         };
         auto pair = [&](int j, const double4& pj, int kj) {
             double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
@@ -1543,7 +1585,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs(PairArgs a) {
             fx += fs * dx;
             fy += fs * dy;
             fz += fs * dz;
-            if (kEnergy && j > i) {
+            if (kEnergy && j > self) {
                 e_pair += e_p;
                 e_coul += e_c;
                 wxx += fs * dx * dx;
@@ -1556,13 +1598,13 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs(PairArgs a) {
         };
         int k = sub;
         int eA = jat(k), eB = jat(k + TPA);  // list entries: atom and kind
-        double4 pA = a.pos[nbr_atom(eA)], pB = a.pos[nbr_atom(eB)];
+        double4 pA = a.ppos[nbr_atom(eA)], pB = a.ppos[nbr_atom(eB)];
         for (; k < nn; k += 2 * TPA) {
             const int eA2 = jat(k + 2 * TPA), eB2 = jat(k + 3 * TPA);
             pair(nbr_atom(eA), pA, nbr_kind(eA));
-            pA = a.pos[nbr_atom(eA2)];
+            pA = a.ppos[nbr_atom(eA2)];
             if (k + TPA < nn) pair(nbr_atom(eB), pB, nbr_kind(eB));
-            pB = a.pos[nbr_atom(eB2)];
+            pB = a.ppos[nbr_atom(eB2)];
             eA = eA2;
             eB = eB2;
         }
@@ -1841,7 +1883,8 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs_mixed(PairArgs a) {
     int i = -1;
     if (t < a.n) {
         i = a.sorted[t];
-        const float4 pi = frac[i];
+        const int self = a.slots ? t : i;
+        const float4 pi = frac[self];
         const int ki = a.meta[i].x;
         const float qi = pi.w;
         // the home charge with 1 / (4 pi eps0): one product per pair fewer
@@ -1858,7 +1901,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs_mixed(PairArgs a) {
         // itself, never evaluated.
         auto jat = [&](int k) {
             int v = row[min(k, max(nn - 1, 0))];
-            return k < nn ? v : nbr_entry(i, ki);
+            return k < nn ? v : nbr_entry(self, ki);
         };
         // one list entry: returns the force factor f/r, with the difference
         // vector in dx, dy, dz (the energies and virial, in energy mode,
@@ -1932,7 +1975,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs_mixed(PairArgs a) {
                 fs += in_coul ? fc : 0.f;
                 if (kEnergy) e_c = in_coul ? e_c : 0.f;
             }
-            if (kEnergy && j > i) {
+            if (kEnergy && j > self) {
                 e_pair += e_p;
                 e_coul += e_c;
                 const double f = fs, ddx = dx, ddy = dy, ddz = dz;
@@ -2000,7 +2043,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs_mixed(PairArgs a) {
 // same distance code as k_pairs.
 __global__ void k_pairs_within(const double4* __restrict__ pos, const int* __restrict__ sorted,
                                const int* __restrict__ nbr, const int* __restrict__ nnbr, int n, int cap, Box box,
-                               double rc,
+                               double rc, int slots,
                                uint2* __restrict__ out, unsigned long long out_cap,
                                unsigned long long* __restrict__ count) {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2010,6 +2053,7 @@ __global__ void k_pairs_within(const double4* __restrict__ pos, const int* __res
     int nn = nnbr[t];
     for (int k = 0; k < nn; k++) {
         int j = nbr_atom(nbr[(size_t)t * cap + k]);
+        if (slots) j = sorted[j];
         if (j <= i) continue;
         double4 pj = pos[j];
         double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
@@ -2097,6 +2141,7 @@ __global__ void k_mol_com(const double4* __restrict__ pos, const double4* __rest
 }
 
 struct MolVirialArgs {
+    int slots;  // list entries name sorted places
     const double4* pos;
     const int2* meta;
     const int* sorted;
@@ -2138,7 +2183,7 @@ __global__ __launch_bounds__(256) void k_mol_pairs(MolVirialArgs a) {
         const int nn = a.nnbr[t];
         for (int k = 0; k < nn; k++) {
             const int e = row[k];
-            const int j = nbr_atom(e);
+            const int j = a.slots ? a.sorted[nbr_atom(e)] : nbr_atom(e);
             const int mj = a.meta[j].y;
             if (mj <= mi.y) continue;
             const double4 pj = a.pos[j];
@@ -2704,7 +2749,7 @@ __device__ __forceinline__ void md_place(const MdArgs& m, int i, bool live, doub
         moved = dx * dx + dy * dy + dz * dz > m.half_skin2;
         bad = nonfinite3(p.x, p.y, p.z) || nonfinite3(v.x, v.y, v.z);
         if (m.tg.tag) m.tg.tag[i] = cell_tag(m.tg, p);
-        if (m.tg.frac) m.tg.frac[i] = frac_pos(m.tg.b, m.tg.fo, p);
+        place_copies(m.tg, i, p);
     }
     if (__any(moved) && (threadIdx.x & 63) == 0) atomicOr(m.flags, 1);
     flag_nonfinite(bad, m.flags);
@@ -2780,7 +2825,8 @@ __global__ __launch_bounds__(kMdBlock) void k_md_fused(MdArgs m, const double4* 
         p = m.pos[i];
         r = m.ref[i];
         md_kick(m, f, m.lf ? m.acc[i] : v, v, na);
-        m.acc[i] = na;
+        // VelocityVerlet reads accelerations only after a second half alone
+        if (m.lf) m.acc[i] = na;
         md_drift(m, na, v, p);
         m.vel[i] = v;
     }
@@ -3200,7 +3246,7 @@ __global__ __launch_bounds__(512, 2) void k_oct_step(OctForce a, OctStep s, OctR
             double4 na4 = make_double4(0, 0, 0, 0);
             if (live) {
                 md_kick(s.m, f, ac, v, na4);
-                s.m.acc[i] = na4;
+                if (s.m.lf || s.then != OCT_FUSED) s.m.acc[i] = na4;
             }
             if (s.then == OCT_FUSED) {
                 if (live) {
