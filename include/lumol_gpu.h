@@ -347,10 +347,10 @@ int lg_system_get_tuning(lg_system* sys, lg_tuning* tuning);
 enum {
     LG_KERNEL_NLIST = 0,        /* displacement check + cell list + Verlet list */
     LG_KERNEL_PAIRS = 1,        /* k_pairs: LJ + Ewald real space / Wolf, and, in
-                                   the FP64 form, the intra-molecular terms (extra
+                                   forces, the intra-molecular terms (extra
                                    blocks of the same launch)                     */
     LG_KERNEL_MOLECULES = 2,    /* the intra-molecular terms in a launch of their own
-                                   or with the list build (mixed form)            */
+                                   (energies without rho(k))                      */
     LG_KERNEL_KSPACE_RHO = 3,   /* rho(k) partials in a launch of their own       */
     LG_KERNEL_KSPACE_FORCE = 4, /* k-space forces, with the half-steps that follow
                                    them in MD and the rho(k) partials of the new

@@ -478,7 +478,6 @@ struct lg_system {
     DevBuf<int> mc_cell_count, mc_atom_cell;
     // snapshot for neighbour-list overflow recovery
     DevBuf<double4> snap_pos, snap_vel, snap_acc;
-    bool intra_done = false;  // launch_nlist ran the intra-molecular terms (k_direct_intra)
     // MD chunk captured as a HIP graph, with what it was captured for
     hipGraphExec_t md_exec = nullptr;
     uint64_t md_key[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -1600,9 +1599,8 @@ static IntraArgs intra_args(lg_system* s) {
     return ia;
 }
 
-int launch_nlist(lg_system* s, bool check, bool energy) {
+int launch_nlist(lg_system* s, bool check) {
     hipStream_t st = S(s);
-    s->intra_done = false;
     // profiled intervals only around launches (an empty event pair would
     // count the event packets' own dispatch as list time)
     long prof = -1;
@@ -1624,18 +1622,6 @@ int launch_nlist(lg_system* s, bool check, bool energy) {
                       s->nbr.p, s->nnbr.p, s->ref.p, s->sorted.p, flag, direct_split(s)};
         const bool nearest = s->periodic && (g.reach[0] == 0 || g.reach[1] == 0 || g.reach[2] == 0);
         prof_stop(s, prof);
-        // forces only: the intra-molecular terms ride as the last blocks of
-        // this launch, which most steps leave empty
-        s->intra_done = !energy && !s->gen_pairs && s->nterms > 0;
-        if (s->intra_done) {
-            const int ncb = direct_blocks(s), fib = blocks_for(s->nterms, kCellBlock);
-            auto go = [&](auto kernel) {
-                launch_timed(s, LG_KERNEL_MOLECULES, kernel, ncb + fib, kCellBlock, 0, da, ncb, intra_args(s));
-            };
-            if (nearest) go(k_direct_intra<true>);
-            else go(k_direct_intra<false>);
-            return LG_OK;
-        }
         long p2 = prof_start(s, LG_KERNEL_NLIST);
         if (nearest)
             k_nlist_direct<true><<<direct_blocks(s), kCellBlock, 0, st>>>(da);
@@ -1713,16 +1699,17 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
     // rho(k) partials first: their reduction runs as the last blocks of the
     // pair launch, and the k-space forces after it
     int nchunks = 0;
+    bool intra_done = false;  // the energy terms ran beside rho(k)
     if (oct) {
         if (!rho_done) {
             const OctRho ra = oct_rho_args(s, mixed);
             const int grid = int(xcd_grid(ra.ngroups, ra.nchunks));
             s->rho_nchunks = ra.nchunks;
-            // the intra-molecular terms ride along, unless the list launch ran them
-            const int ib = s->nterms > 0 && !s->gen_pairs && !s->intra_done ? blocks_for(s->nterms, 512) : 0;
+            // the intra-molecular terms ride along, when energies are formed
+            const int ib = s->nterms > 0 && !s->gen_pairs && energy ? blocks_for(s->nterms, 512) : 0;
             if (mixed) launch_rho_oct<float>(s, ra, grid, energy, ib, intra_args(s));
             else launch_rho_oct<double>(s, ra, grid, energy, ib, intra_args(s));
-            if (ib > 0) s->intra_done = true;
+            intra_done = ib > 0;
         }
         nchunks = s->rho_nchunks;
     } else if (kspace) {
@@ -1774,9 +1761,9 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
         // any other caller converts the current positions here
         launch_timed(s, LG_KERNEL_PAIRS, k_frac, blocks_for(n, 256), 256, 0, s->pos.p, n, cell_tags(s));
     }
-    // the intra-molecular terms run as the last blocks of the list launch
-    // (forces only, direct build) or of the rho(k) launch (intra_done), of
-    // the general pair launch, or in a launch of their own
+    // the intra-molecular terms run as blocks of the pair launch (forces, and
+    // the general pair kernel), or with energies beside rho(k) (intra_done) or
+    // in a launch of their own
     IntraArgs& ia = pa.intra;
     ia = intra_args(s);
     const int iblocks = s->nterms > 0 ? blocks_for(s->nterms, 256) : 0;
@@ -1814,7 +1801,7 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
         rr.epart = epk;
     }
     const bool intra_apart = !s->gen_pairs;
-    if (intra_apart && iblocks > 0 && !s->intra_done) {
+    if (intra_apart && iblocks > 0 && !intra_done && energy) {
         if (energy)
             launch_timed(s, LG_KERNEL_MOLECULES, k_intra_terms<true>, iblocks, 256, 0, ia);
         else
@@ -1822,18 +1809,21 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
     }
     const int pblocks = pair_blocks_of(size_t(n), s->tpa);
     pa.pair_blocks = pblocks;
-    pa.intra_blocks = intra_apart ? 0 : iblocks;
+    pa.intra_blocks = intra_apart && energy ? 0 : iblocks;
     const int nblocks = pblocks + pa.intra_blocks + rblocks;
     const int ck = coulomb_variant(s->coul);
+    const bool intra = pa.intra_blocks > 0;
     const bool lib = !s->hf_ok;  // FP64: the tables of h and erfcx missed their bound
 #define LG_PAIRS_CK(T, CK, LIB)                                                 \
     if (ck == CK) {                                                             \
         if (mixed && energy)                                                    \
             launch_timed(s, LG_KERNEL_PAIRS, k_pairs_mixed<true, T, CK>, nblocks, kPairBlock, 0, pa);     \
         else if (mixed)                                                         \
-            launch_timed(s, LG_KERNEL_PAIRS, k_pairs_mixed<false, T, CK>, nblocks, kPairBlock, 0, pa);    \
+            launch_timed(s, LG_KERNEL_PAIRS, intra ? k_pairs_mixed<false, T, CK, true> : k_pairs_mixed<false, T, CK>, nblocks, kPairBlock, 0, pa);    \
         else if (energy)                                                        \
             launch_timed(s, LG_KERNEL_PAIRS, lib ? k_pairs<true, T, LIB> : k_pairs<true, T, CK>, nblocks, kPairBlock, 0, pa);   \
+        else if (intra)                                                         \
+            launch_timed(s, LG_KERNEL_PAIRS, lib ? k_pairs<false, T, LIB, true> : k_pairs<false, T, CK, true>, nblocks, kPairBlock, 0, pa); \
         else                                                                    \
             launch_timed(s, LG_KERNEL_PAIRS, lib ? k_pairs<false, T, LIB> : k_pairs<false, T, CK>, nblocks, kPairBlock, 0, pa); \
     }
@@ -1922,7 +1912,7 @@ int check_overflow(lg_system* s, bool* overflowed, bool* nonfinite = nullptr) {
 int compute(lg_system* s, bool energy) {
     LG_TRY(prepare(s));
     for (int attempt = 0; attempt < 4; attempt++) {
-        LG_TRY(launch_nlist(s, true, energy));
+        LG_TRY(launch_nlist(s, true));
         LG_TRY(launch_forces(s, energy));
         bool ov = false;
         LG_TRY(check_overflow(s, &ov));
@@ -2867,7 +2857,7 @@ int lg_potential_energy_noalloc(lg_system* s, lg_energy_terms* out) {
     double* sums = s->ep_k_at + size_t(nbk) * 7;
     const uint32_t mask = s->prof_mask;
     s->prof_mask = 0;  // no event creation in this call
-    int rc = launch_nlist(s, true, true);
+    int rc = launch_nlist(s, true);
     if (rc == LG_OK) rc = launch_forces(s, true);
     s->prof_mask = mask;
     s->ep_pairs_at = s->ep_mol_at = s->ep_k_at = nullptr;
@@ -3098,7 +3088,7 @@ static int md_chunk(lg_system* s, uint64_t todo) {
             else
                 launch_timed(s, LG_KERNEL_INTEGRATE, k_md_first, nb, kMdBlock, 0, m, th);
         }
-        LG_TRY(launch_nlist(s, false, false));
+        LG_TRY(launch_nlist(s, false));
         LG_TRY(launch_forces(s, false, false, true, with_rho != 0));
         const bool fuse = !thermo && k + 1 < todo;
         if (oct)

@@ -1445,6 +1445,26 @@ __device__ __forceinline__ double rsqrt_newton(double x) {
     return y + y * e;
 }
 
+// The blocks behind the pair blocks: the intra-molecular terms (kIntra, force
+// evaluations of molecules), then the rho(k) reduction.  The terms' code needs
+// 104 VGPRs, which would hold every pair block to four waves per SIMD; the
+// kIntra instances are held to what the pairs need, and the few term blocks
+// spill.  They hide behind the pairs, where their own launch (or their place
+// in the list launch) took 5 to 7 us: SPC/E 3000 molecules, us per step,
+// mixed 48.5 -> 43.6, FP64 57.5 -> 52.9.  Other systems keep instances
+// without them: the spill space alone cost NaCl of 4096 ions 4%.
+template <bool kEnergy, bool kIntra>
+__device__ __forceinline__ void pair_extra_block(const PairArgs& a, unsigned char* lds) {
+    const int b = blockIdx.x - a.pair_blocks;
+    if constexpr (kIntra) {
+        if (b < a.intra_blocks) {
+            intra_block<kEnergy>(a.intra, b);
+            return;
+        }
+    }
+    kspace_reduce_block<kEnergy>(a, b - a.intra_blocks, lds);
+}
+
 // The pair kernel of LJ/Harmonic/Null systems, FP64.  TPA lanes share one
 // atom i and stride through its neighbour row; the group's partial forces
 // are combined with xor-shuffles (TPA divides 64).
@@ -1465,8 +1485,10 @@ __device__ __forceinline__ double rsqrt_newton(double x) {
 //   pieces (no exponential); energies keep exp(-x^2) erfcx(x).
 // SPC/E, 9000 atoms: 41 -> 21 us per launch against the reference's order with
 // library root, division and exponential.
-template <bool kEnergy, int TPA, int CK>
-__global__ __launch_bounds__(kPairBlock) void k_pairs(PairArgs a) {
+template <bool kEnergy, int TPA, int CK, bool kIntra = false>
+__global__ __launch_bounds__(kPairBlock)
+__attribute__((amdgpu_waves_per_eu(!kIntra ? 1 : CK == CK_NONE ? 8 : CK == CK_EWALD || CK == CK_WOLF ? 6 : 3)))
+void k_pairs(PairArgs a) {
     struct alignas(16) Lj {
         double A, B, r2c, shift;  // 48 eps s^12, 24 eps s^6, cutoff test (0: no term), energy shift
     };
@@ -1479,7 +1501,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs(PairArgs a) {
     __shared__ __align__(16) double hft[kTab ? kErfcxPieces * (kErfcxDeg64 + 1) : 2];
     __shared__ __align__(16) double ecx[kTab && kEnergy ? kErfcxPieces * (kErfcxDeg64 + 1) : 2];
     if ((int)blockIdx.x >= a.pair_blocks) {  // uniform over the block
-        kspace_reduce_block<kEnergy>(a, blockIdx.x - a.pair_blocks, lds);
+        pair_extra_block<kEnergy, kIntra>(a, lds);
         return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.rebuild) *a.rebuild = 0;
@@ -1807,11 +1829,10 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(2)))
 // energies keep exp(-x^2) erfcx(x).  1/r is the hardware reciprocal square
 // root (1 ulp).
 //
-// The launch carries the rho(k) reduction blocks but not the intra-molecular
-// terms: their code needs 104 VGPRs, which would hold every pair block of the
-// launch to four waves per SIMD, against eight for the pair code alone.
-template <bool kEnergy, int TPA, int CK>
-__global__ __launch_bounds__(kPairBlock) void k_pairs_mixed(PairArgs a) {
+// The launch carries the rho(k) reduction blocks and, in the kIntra instances,
+// the intra-molecular terms (pair_extra_block).
+template <bool kEnergy, int TPA, int CK, bool kIntra = false>
+__global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(kIntra ? 8 : 1))) void k_pairs_mixed(PairArgs a) {
     __shared__ double red[kPairBlock / 64][8];
     constexpr bool kTab = CK == CK_EWALD || CK == CK_WOLF;
     struct Tables {
@@ -1828,7 +1849,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pairs_mixed(PairArgs a) {
     float* const ecx = reinterpret_cast<float*>(tb.ecx);
     float* const hft = reinterpret_cast<float*>(tb.hft);
     if ((int)blockIdx.x >= a.pair_blocks) {  // uniform over the block
-        kspace_reduce_block<kEnergy>(a, blockIdx.x - a.pair_blocks, lds);
+        pair_extra_block<kEnergy, kIntra>(a, lds);
         return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.rebuild) *a.rebuild = 0;
@@ -2453,18 +2474,6 @@ __global__ __launch_bounds__(512, 2) void k_rho_oct(OctRho ra, int SA, const dou
     const int a0 = chunk * ra.width;
     oct_rho_group<T>(ra, SA, grp, chunk, min(ra.width, n - a0), false, reinterpret_cast<T*>(oct_smem),
                      [&](int at) { return pos[a0 + at]; });
-}
-
-// The direct Verlet build in the first ncb blocks; any blocks past those run
-// the intra-molecular terms (forces only, kCellBlock terms per block), which
-// need only the positions of the first half-step (mixed form).
-template <bool kMinImage>
-__global__ __launch_bounds__(kCellBlock) void k_direct_intra(DirectArgs da, int ncb, IntraArgs ia) {
-    __shared__ DirectLds lds;
-    if ((int)blockIdx.x < ncb)
-        nlist_direct_block<kMinImage>(da, blockIdx.x, ncb, lds);
-    else
-        intra_block<false>(ia, blockIdx.x - ncb);
 }
 
 // k-space forces of the row form: one lane per atom, rows of k-vectors (fixed ikx, iky;
