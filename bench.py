@@ -263,8 +263,8 @@ ROOFLINE_CLASSES = ("pairs", "kspace_rho", "kspace_force", "integrate")
 
 def class_work(cls, workload, form, natoms, n_pairs, nk, batch=1):
     """(bound, algorithmic work per launch, peak, unit, description) of a
-    kernel class: VALU FLOP for the pair and k-space kernels (FP32 peak in
-    the mixed form, FP64 otherwise), HBM bytes for the integrator."""
+    kernel class: FLOP for the pair and k-space kernels (FP32 peak in the
+    mixed form, FP64 otherwise), HBM bytes for the integrator."""
     peak = PEAK_TFLOPS[form]
     if cls == "pairs":
         # water: every O-O pair within rc also carries Coulomb; the pair set
@@ -273,8 +273,16 @@ def class_work(cls, workload, form, natoms, n_pairs, nk, batch=1):
         return ("valu", batch * n_pairs * flop / 1e12, peak, "TFLOP/s",
                 f"{flop} FLOP x {n_pairs} pairs within rc (forces only) x {batch} system(s) per launch")
     if cls == "kspace_force":
-        return ("valu", batch * nk * natoms * FLOP_KSPACE_FORCE / 1e12, peak, "TFLOP/s",
-                f"{FLOP_KSPACE_FORCE} FLOP x {nk} k-vectors x {natoms} atoms x {batch} system(s) per launch")
+        # without a thermostat the launch also forms rho(k) of the new
+        # positions; with one (NaCl) the first half-step's launch does
+        flop = FLOP_KSPACE_FORCE + (0 if workload == "nacl" else FLOP_KSPACE_RHO)
+        return ("mfma", batch * nk * natoms * flop / 1e12, peak, "TFLOP/s",
+                f"{flop} FLOP x {nk} k-vectors x {natoms} atoms x {batch} system(s) per launch (matrix cores; the "
+                f"octants' shared sums need a quarter of it)")
+    if cls == "integrate" and workload == "nacl":
+        return ("mfma", batch * nk * natoms * FLOP_KSPACE_RHO / 1e12, peak, "TFLOP/s",
+                f"{FLOP_KSPACE_RHO} FLOP x {nk} k-vectors x {natoms} atoms x {batch} system(s) per launch "
+                f"(the first half-step with rho(k))")
     if cls == "kspace_rho":
         return ("valu", batch * nk * natoms * FLOP_KSPACE_RHO / 1e12, peak, "TFLOP/s",
                 f"{FLOP_KSPACE_RHO} FLOP x {nk} k-vectors x {natoms} atoms x {batch} system(s) per launch "
@@ -294,7 +302,8 @@ def roofline_of(prof, steps, workload, form, natoms, n_pairs, nk, batch=1, timin
     bound, work, peak, unit, per = class_work(dom, workload, form, natoms, n_pairs, nk, batch)
     achieved = work / avg_s
     return {"bound": bound, "achieved": achieved, "peak": peak, "unit": unit, "frac": achieved / peak,
-            "traffic": load_traffic(workload, form, dom), "kernel": dom, "avg_launch_us": avg_s * 1e6,
+            # the committed counters of the k-space classes are of other kernels
+            "traffic": load_traffic(workload, form, dom) if dom == "pairs" else None, "kernel": dom, "avg_launch_us": avg_s * 1e6,
             "launches": launches, "work": per, "timing": timing}, {c: round(v, 2) for c, v in per_step.items()}
 
 
