@@ -380,10 +380,9 @@ struct lg_system {
     int cap = 0;
     DevBuf<int> cellid, slot, count, start, tmp, sorted, nbr, nnbr, flags;  // flags[0] rebuild, [1] overflow
     DevBuf<float4> cpos;  // list-build candidate records in sorted order
-    int listed_precision = 0;  // of the copies below
     bool slot_rows = false;  // list entries name sorted places (slot_form), and
     DevBuf<int> rank;        // where each atom is
-    DevBuf<double4> spos;    // FP64: the positions in that order
+    DevBuf<double4> spos;    // the positions in that order, as the FP64 kernel reads them
     DevBuf<float4> frac;  // positions as the mixed pair kernel reads them (frac_pos)
     double3 frac_origin = make_double3(0.0, 0.0, 0.0);  // infinite cells: atom 0 at the last set
     // parameters
@@ -1399,12 +1398,13 @@ int prepare_nlist(lg_system* s) {
     LG_HIP(hipMemcpyAsync(s->flags.p, init, sizeof(init), hipMemcpyHostToDevice, S(s)));
     LG_HIP(hipMemsetAsync(s->count.p, 0, g.ncell * sizeof(int), S(s)));
     s->slot_rows = slot_form(s);
-    s->listed_precision = s->precision;
     if (s->slot_rows) {
         // any valid place until the first build sets them
         LG_TRY(s->rank.ensure(n));
         LG_HIP(hipMemsetAsync(s->rank.p, 0, n * sizeof(int), S(s)));
-        if (s->precision != LG_PRECISION_MIXED) LG_TRY(s->spos.ensure(n));
+        // in the mixed form too: the precision may change without a call that
+        // may allocate in between (lg_potential_energy_noalloc)
+        LG_TRY(s->spos.ensure(n));
     }
     s->nlist_dirty = false;
     return LG_OK;
@@ -1413,9 +1413,6 @@ int prepare_nlist(lg_system* s) {
 
 int prepare(lg_system* s) {
     if (s->n == 0) return fail(LG_E_INVALID, "empty system");
-    // the lists hold another form of entries, or lack the copies that the
-    // other precision reads
-    if (s->listed_precision != s->precision && s->slot_rows) s->nlist_dirty = true;
     if (s->topo_dirty || s->meta_dirty || s->params_dirty || s->kspace_dirty || s->nlist_dirty) {
         s->cfg_epoch++;
         s->mc_ready = false;

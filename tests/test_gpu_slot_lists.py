@@ -3,11 +3,14 @@ kernels gather copies of the positions kept in that order): everything that
 reads the lists, against the oracle, in both precisions and across what
 changes the order or the copies: steps with rebuilds, new positions, a change
 of precision, Monte Carlo moves."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import lumol_oracle as lo
 from lumol_amd import MolecularDynamics, Simulation, VelocityVerlet
+from lumol_amd import _native as nat
 from lumol_amd._native import LG_PRECISION_FP64, LG_PRECISION_MIXED
 from lumol_amd.workloads import lj_mc_chain, spce
 
@@ -63,3 +66,21 @@ def test_many_cells(rho):
     # 210 000 and 11 000 cells: several passes of the cell scan, and one
     s, _, _ = lj_mc_chain(33000, seed=6, rho_star=rho)
     check(s, 1e-10, full=False)
+
+
+def test_precision_change_without_allocation():
+    # the evaluation that may not allocate, in each precision after the other
+    # alone was evaluated
+    L = nat.lib()
+    for first, then in ((LG_PRECISION_MIXED, LG_PRECISION_FP64), (LG_PRECISION_FP64, LG_PRECISION_MIXED)):
+        s, _, _ = lj_mc_chain(33000, seed=8)
+        s.set_precision(first)
+        s.potential_energy()
+        h = s._sync()
+        nat.check(L.lg_system_set_precision(h, then))
+        t, u = nat.EnergyTerms(), nat.EnergyTerms()
+        assert L.lg_potential_energy_noalloc(h, ctypes.byref(t)) == nat.LG_OK
+        nat.check(L.lg_potential_energy(h, ctypes.byref(u)))
+        assert [getattr(t, f) for f, _ in t._fields_] == [getattr(u, f) for f, _ in u._fields_]
+        eo = lo.OracleSystem(s, nthreads=16).potential_energy()
+        assert abs(t.total - eo) <= BARS[then] * abs(eo)
