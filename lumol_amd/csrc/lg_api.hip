@@ -874,8 +874,9 @@ static double fit_erfcx(double xmax, int deg, std::vector<T>& out) {
 
 // Least double x with sqrt(x) >= rc (sqrt(x) > rc when `beyond`): the square
 // root rounds monotonically, so the reference's cutoff tests on r = sqrt(x)
-// are tests of x.
+// are tests of x.  An infinite cutoff (infinite cells) has no such x.
 double r2_bound(double rc, bool beyond) {
+    if (!(rc < INFINITY)) return INFINITY;
     auto out = [&](double x) { return beyond ? std::sqrt(x) > rc : std::sqrt(x) >= rc; };
     double x = rc * rc;
     while (out(x) && x > 0.0) x = std::nextafter(x, 0.0);

@@ -98,3 +98,19 @@ def test_argument_and_state_errors():
     assert L.lg_md_setup(h, 0, 1.0, 300.0, 0.5) == nat.LG_E_INVALID  # tau < 1
     assert L.lg_md_setup(h, 0, -1.0, -1.0, 1.0) == nat.LG_E_INVALID
     L.lg_system_destroy(h)
+
+
+def test_infinite_coulomb_cutoff_in_an_infinite_cell():
+    # both sums accept the cutoff there; Ewald then refuses the cell, Wolf's
+    # constants are not finite
+    L = nat.lib()
+    h = new_system(cell=(0.0, 0.0, 0.0))
+    t = nat.EnergyTerms()
+    assert L.lg_coulomb_ewald(h, float("inf"), 5, 0.3, 0) == nat.LG_OK
+    rc, msg = status_and_message(L.lg_potential_energy(h, ctypes.byref(t)))
+    assert rc == nat.LG_E_INVALID and "infinite unit cell" in msg
+    assert L.lg_coulomb_wolf(h, float("inf"), 0, 1.0) == nat.LG_OK
+    assert L.lg_potential_energy(h, ctypes.byref(t)) == nat.LG_E_NONFINITE
+    assert L.lg_coulomb_wolf(h, 9.0, 0, 1.0) == nat.LG_OK
+    assert L.lg_potential_energy(h, ctypes.byref(t)) == nat.LG_OK
+    L.lg_system_destroy(h)
