@@ -427,11 +427,14 @@ struct lg_system {
     double ecx_inv_h = 0.0;
     // the mixed pair kernel's real-space force factor
     // h(r) = erfc(alpha r) + (2 alpha / sqrt(pi)) r exp(-alpha^2 r^2) on
-    // [0, rc], FP32 pieces (hforce_ld); hf_ok when the fit met 1e-7
+    // [0, rc], FP32 pieces (hforce_ld); hf_ok when the fit met 1e-7 of h
     DevBuf<float> hf32;
-    DevBuf<double> hf64;  // the same in FP64 pieces
     double hf_inv_h = 0.0;
     bool hf_ok = false;
+    // the same in FP64 pieces (hforce_tab); hf64_ok when the fit met 2e-15 of h
+    DevBuf<double> hf64;
+    double hf64_inv_h = 0.0;
+    bool hf64_ok = false;
     bool ecx_ok = false;
     double kg[3] = {0, 0, 0};    // 2 pi / L per axis
     DevBuf<double> efac, vfac;
@@ -786,19 +789,19 @@ int prepare_meta(lg_system* s) {
     return LG_OK;
 }
 
-// A function f on [0, xmax] as kErfcxPieces polynomials of degree `deg` in
-// t in [-1, 1] per piece: the piece's Chebyshev interpolant (deg + 1
-// Chebyshev nodes, long double), expanded in powers of t.  Returns the
-// largest relative (or absolute) error against f (long double) over 64 points per piece.
+// A function f on M pieces of width h from 0 as polynomials of degree `deg`
+// in t in [-1, 1] per piece, `stride` coefficients apart: the piece's
+// Chebyshev interpolant (deg + 1 Chebyshev nodes, long double), expanded in
+// powers of t.  Returns the largest relative error against f (long double)
+// over 64 points per piece.
 // Used for erfcx(x) = exp(x^2) erfc(x) and for the real-space force factor
 // of the mixed pair kernel (hforce_ld).
 static long double erfcx_ld(long double x) { return erfcl(x) * expl(x * x); }
 template <typename T, typename F>
-static double fit_pieces(double xmax, int deg, F fn, std::vector<T>& out, bool absolute = false) {
-    const int M = kErfcxPieces, D = deg;
+static double fit_pieces(long double h, int M, int deg, int stride, F fn, std::vector<T>& out) {
+    const int D = deg;
     const long double pi = 3.141592653589793238462643383279502884L;
-    const long double h = (long double)xmax / M;
-    out.assign(size_t(M) * (D + 1), T(0));
+    out.assign(size_t(M) * stride, T(0));
     double worst = 0.0;
     std::vector<long double> f(D + 1), c(D + 1), mono(D + 1), tprev(D + 1), tcur(D + 1), tnext(D + 1);
     for (int k = 0; k < M; k++) {
@@ -828,13 +831,13 @@ static double fit_pieces(double xmax, int deg, F fn, std::vector<T>& out, bool a
             tprev = tcur;
             tcur = tnext;
         }
-        for (int q = 0; q <= D; q++) out[size_t(k) * (D + 1) + q] = T(mono[q]);
+        for (int q = 0; q <= D; q++) out[size_t(k) * stride + q] = T(mono[q]);
         for (int z = 0; z < 64; z++) {
             const long double t = -1.0L + 2.0L * (z + 0.5L) / 64.0L;
-            long double p = (long double)out[size_t(k) * (D + 1) + D];
-            for (int q = D - 1; q >= 0; q--) p = p * t + (long double)out[size_t(k) * (D + 1) + q];
+            long double p = (long double)out[size_t(k) * stride + D];
+            for (int q = D - 1; q >= 0; q--) p = p * t + (long double)out[size_t(k) * stride + q];
             const long double ref = fn(mid + half * t);
-            worst = std::max(worst, double(fabsl(p - ref) / (absolute ? 1.0L : ref)));
+            worst = std::max(worst, double(fabsl(p - ref) / ref));
         }
     }
     return worst;
@@ -844,14 +847,14 @@ static double fit_pieces(double xmax, int deg, F fn, std::vector<T>& out, bool a
 // stream of one water model) fit once.  A fit is a pure function of the key,
 // so a cached table is the table the fit would return.
 template <typename T, typename F>
-static double fit_cached(int fn_id, double param, double xmax, int deg, F fn, std::vector<T>& out,
-                         bool absolute = false) {
+static double fit_cached(int fn_id, double param, double range, long double h, int pieces, int deg, int stride, F fn,
+                         std::vector<T>& out) {
     using Key = std::tuple<int, uint64_t, uint64_t, int>;
     static std::mutex mu;
     static std::map<Key, std::pair<std::vector<T>, double>> cache;
     uint64_t pb, xb;
     std::memcpy(&pb, &param, sizeof(pb));
-    std::memcpy(&xb, &xmax, sizeof(xb));
+    std::memcpy(&xb, &range, sizeof(xb));
     const Key key{fn_id, pb, xb, deg};
     {
         std::lock_guard<std::mutex> lk(mu);
@@ -861,14 +864,19 @@ static double fit_cached(int fn_id, double param, double xmax, int deg, F fn, st
             return it->second.second;
         }
     }
-    const double err = fit_pieces(xmax, deg, fn, out, absolute);
+    const double err = fit_pieces(h, pieces, deg, stride, fn, out);
     std::lock_guard<std::mutex> lk(mu);
     cache.emplace(key, std::make_pair(out, err));
     return err;
 }
+// kErfcxPieces pieces over [0, xmax] (erfcx_tab).
+template <typename T, typename F>
+static double fit_range(int fn_id, double param, double xmax, int deg, F fn, std::vector<T>& out) {
+    return fit_cached(fn_id, param, xmax, (long double)xmax / kErfcxPieces, kErfcxPieces, deg, deg + 1, fn, out);
+}
 template <typename T>
 static double fit_erfcx(double xmax, int deg, std::vector<T>& out) {
-    return fit_cached(0, 0.0, xmax, deg, erfcx_ld, out);
+    return fit_range(0, 0.0, xmax, deg, erfcx_ld, out);
 }
 
 
@@ -949,7 +957,7 @@ int prepare_params(lg_system* s) {
     // erfcx tables for the pair kernels' real-space erfc (Ewald and Wolf);
     // kept only if the fit meets 1e-14 (FP64) and 1e-7 (FP32) relative
     s->ecx_ok = false;
-    s->hf_ok = false;
+    s->hf_ok = s->hf64_ok = false;
     if ((s->coul_kind == COUL_EWALD || s->coul_kind == COUL_WOLF) && c.alpha > 0.0 && c.rc > 0.0) {
         const double xmax = c.alpha * c.rc * (1.0 + 1e-9);
         std::vector<double> t64;
@@ -969,17 +977,25 @@ int prepare_params(lg_system* s) {
         auto hforce_ld = [al, g0](long double r) { return erfcl(al * r) + g0 * r * expl(-al * al * r * r); };
         const double rmax = c.rc * (1.0 + 1e-9);
         std::vector<float> th;
-        const double eh = fit_cached(1, c.alpha, rmax, kErfcxDeg32, hforce_ld, th);
-        // FP64: the largest error against h itself, whose tail (5e-5 at the
-        // cutoff) a relative bound would overrate
-        std::vector<double> th64;
-        const double eh64 = fit_cached(2, c.alpha, rmax, kErfcxDeg64, hforce_ld, th64, true);
-        s->hf_ok = false;
-        if (s->ecx_ok && eh < 1e-7 && eh64 < 2e-15) {
+        const double eh = fit_range(1, c.alpha, rmax, kErfcxDeg32, hforce_ld, th);
+        if (s->ecx_ok && eh < 1e-7) {
             LG_TRY(upload(s->hf32, th, S(s)));
-            LG_TRY(upload(s->hf64, th64, S(s)));
             s->hf_inv_h = kErfcxPieces / rmax;
             s->hf_ok = true;
+        }
+        // FP64: relative too, to what exp and the erfcx table leave (3e-15 at
+        // alpha rc = pi, 4e-15 at 4); beyond it those two run
+        float inv_h = float(kHfPieces / rmax);
+        if (double(inv_h) * rmax > double(kHfPieces)) inv_h = std::nextafter(inv_h, 0.0f);
+        if (s->ecx_ok && std::isfinite(inv_h) && inv_h > 1e-30f) {
+            std::vector<double> th64;
+            const double eh64 = fit_cached(2, c.alpha, double(inv_h), 1.0L / inv_h, kHfPieces, kHfDeg, kHfStride,
+                                           hforce_ld, th64);
+            if (eh64 < 2e-15) {
+                LG_TRY(upload(s->hf64, th64, S(s)));
+                s->hf64_inv_h = inv_h;
+                s->hf64_ok = true;
+            }
         }
     }
     s->params_dirty = false;
@@ -1748,7 +1764,8 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
     pa.ecx32 = s->ecx_ok ? s->ecx32.p : nullptr;
     pa.ecx_inv_h = s->ecx_inv_h;
     pa.hf32 = s->hf_ok ? s->hf32.p : nullptr;
-    pa.hf64 = s->hf_ok ? s->hf64.p : nullptr;
+    pa.hf64 = s->hf64_ok ? s->hf64.p : nullptr;
+    pa.hf64_inv_h = s->hf64_inv_h;
     pa.tie = s->periodic && max_cutoff(s) > (0.5 - 1e-6) * std::min(s->L[0], std::min(s->L[1], s->L[2]));
     pa.hf_inv_h = s->hf_inv_h;
     pa.frac = s->frac.p;
@@ -1811,26 +1828,26 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
     const int nblocks = pblocks + pa.intra_blocks + rblocks;
     const int ck = coulomb_variant(s->coul);
     const bool intra = pa.intra_blocks > 0;
-    const bool lib = !s->hf_ok;  // FP64: the tables of h and erfcx missed their bound
-#define LG_PAIRS_CK(T, CK, LIB)                                                 \
+    const bool hexp = !s->hf64_ok;  // FP64: the table of h missed its bound
+#define LG_PAIRS_CK(T, CK, EXP)                                                 \
     if (ck == CK) {                                                             \
         if (mixed && energy)                                                    \
             launch_timed(s, LG_KERNEL_PAIRS, k_pairs_mixed<true, T, CK>, nblocks, kPairBlock, 0, pa);     \
         else if (mixed)                                                         \
             launch_timed(s, LG_KERNEL_PAIRS, intra ? k_pairs_mixed<false, T, CK, true> : k_pairs_mixed<false, T, CK>, nblocks, kPairBlock, 0, pa);    \
         else if (energy)                                                        \
-            launch_timed(s, LG_KERNEL_PAIRS, lib ? k_pairs<true, T, LIB> : k_pairs<true, T, CK>, nblocks, kPairBlock, 0, pa);   \
+            launch_timed(s, LG_KERNEL_PAIRS, hexp ? k_pairs<true, T, EXP> : k_pairs<true, T, CK>, nblocks, kPairBlock, 0, pa);   \
         else if (intra)                                                         \
-            launch_timed(s, LG_KERNEL_PAIRS, lib ? k_pairs<false, T, LIB, true> : k_pairs<false, T, CK, true>, nblocks, kPairBlock, 0, pa); \
+            launch_timed(s, LG_KERNEL_PAIRS, hexp ? k_pairs<false, T, EXP, true> : k_pairs<false, T, CK, true>, nblocks, kPairBlock, 0, pa); \
         else                                                                    \
-            launch_timed(s, LG_KERNEL_PAIRS, lib ? k_pairs<false, T, LIB> : k_pairs<false, T, CK>, nblocks, kPairBlock, 0, pa); \
+            launch_timed(s, LG_KERNEL_PAIRS, hexp ? k_pairs<false, T, EXP> : k_pairs<false, T, CK>, nblocks, kPairBlock, 0, pa); \
     }
 #define LG_PAIRS_CASE(T)                 \
     case T:                              \
         LG_PAIRS_CK(T, CK_NONE, CK_NONE)          \
-        LG_PAIRS_CK(T, CK_EWALD, CK_EWALD_LIB)         \
+        LG_PAIRS_CK(T, CK_EWALD, CK_EWALD_EXP)         \
         LG_PAIRS_CK(T, CK_EWALD_ERF, CK_EWALD_ERF)     \
-        LG_PAIRS_CK(T, CK_WOLF, CK_WOLF_LIB)          \
+        LG_PAIRS_CK(T, CK_WOLF, CK_WOLF_EXP)          \
         break;
     if (s->gen_pairs) {
         // any pair potential kind or a table: the general FP64 instance, in
@@ -2731,7 +2748,9 @@ __global__ void k_energy_gather(const double* __restrict__ pp, int nbp, const do
 static bool small_steps(const lg_system* s) {
     return s->n <= size_t(small_max(s->precision == LG_PRECISION_MIXED)) && !s->gen_pairs && s->nterms == 0 &&
            s->nmol == int(s->n) &&
-           (s->coul_kind == COUL_NONE || (s->coul_kind == COUL_WOLF && (s->hf_ok || s->coul.inter_excl))) &&
+           (s->coul_kind == COUL_NONE ||
+            (s->coul_kind == COUL_WOLF &&
+             ((s->precision == LG_PRECISION_MIXED ? s->hf_ok : s->hf64_ok) || s->coul.inter_excl))) &&
            s->tune.nlist_build == 0 && s->tune.pair_lanes == 0;
 }
 template <bool kMixed>
@@ -2772,7 +2791,7 @@ static int small_chunk(lg_system* s, uint64_t todo) {
     a.fo = s->frac_origin;
     a.hf64 = s->hf64.p;
     a.hf32 = s->hf32.p;
-    a.hf_inv_h = s->hf_inv_h;
+    a.hf_inv_h = mixed ? s->hf_inv_h : s->hf64_inv_h;
     a.tie = s->periodic && max_cutoff(s) > (0.5 - 1e-6) * std::min(s->L[0], std::min(s->L[1], s->L[2]));
     a.th = Thermo{nullptr, 0, double(3 * s->n), s->berendsen_T, s->berendsen_tau, nullptr};
     if (n <= small_loop_max(mixed)) {

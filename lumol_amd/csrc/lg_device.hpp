@@ -345,6 +345,48 @@ __host__ __device__ __forceinline__ float erfcx_tab(const float* __restrict__ c,
     return p;
 }
 
+// The real-space force factor h(r) of the FP64 pair kernels (see lg_api.hip)
+// by pieces of a degree that keeps the fit's error below an ulp or two of h
+// itself up to alpha rc = 3.9, the default alpha rc = pi among them.  inv_h
+// has 24 bits, so the argument within a piece is rounded once only; with
+// pieces placed by a rounded product, that rounding alone is a few ulps of h
+// near the cutoff, where h falls steeply.  A piece takes kHfStride doubles:
+// lanes in neighbouring pieces then read different LDS banks.
+constexpr int kHfPieces = 128;
+constexpr int kHfDeg = 7;
+constexpr int kHfStride = 10;
+constexpr int kHfDoubles = kHfPieces * kHfStride;
+__host__ __device__ __forceinline__ double hforce_tab(const double* __restrict__ c, double r, double inv_h) {
+    const int k = (int)fmin(fmax(r * inv_h, 0.0), (double)(kHfPieces - 1));
+    const double t = fma(r, 2.0 * inv_h, -(double)(2 * k + 1));
+    const double* q = c + k * kHfStride;
+    double p = q[kHfDeg];
+#pragma unroll
+    for (int d = kHfDeg - 1; d >= 0; d--) p = p * t + q[d];
+    return p;
+}
+
+// 1 / x by the hardware estimate and two Newton steps, each of whose residuals
+// is one fused product: rounded to about half an ulp.
+__device__ __forceinline__ double recip_newton(double x) {
+    double y = __builtin_amdgcn_rcp(x);
+    y = fma(y, fma(-x, y, 1.0), y);
+    return fma(y, fma(-x, y, 1.0), y);
+}
+// sqrt(x) and 1 / x, both to about half an ulp: the hardware estimate of 1 /
+// sqrt(x), one coupled step for the root g and half its inverse h, and a
+// correction of each by its fused residual.  Not a number for x = 0.
+__device__ __forceinline__ void root_recip(double x, double& root, double& recip) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    root = fma(fma(-g, g, x), h, g);
+    const double i = h + h, i2 = i * i;
+    recip = fma(i2, fma(-x, i2, 1.0), i2);
+}
+
 // erfc(x) for x >= 0 from the Chebyshev fit of Numerical Recipes in C, 2nd
 // ed., section 6.2 ("erfcc"): fractional error below 1.2e-7 everywhere.
 // `ex2` = exp(-x^2) is returned for the Ewald force term.

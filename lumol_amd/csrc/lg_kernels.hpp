@@ -1386,7 +1386,8 @@ struct PairArgs {
     const double* ecx64;
     const float* ecx32;
     double ecx_inv_h;
-    const double* hf64;  // h(r) as hf32 below, in FP64 pieces, or null
+    const double* hf64;  // h(r) as hf32 below, in FP64 pieces (hforce_tab), or null
+    double hf64_inv_h;
     int tie;             // a cutoff reaches half the box: images within 1e-9 of a tie are checked
     const double* tabs;  // TableComputation tables (general instance)
     const float4* frac;  // positions as frac_pos (mixed instance)
@@ -1425,24 +1426,13 @@ __device__ __forceinline__ int xcd_contiguous(int b, int P) { return (b & 7) * (
 // excludes (the -erf removal term only), Wolf.  A Wolf system whose
 // restriction excludes the pairs uses CK_NONE.  One variant per instance
 // keeps the registers of the unused paths out of the kernel.
-// The last two: Ewald and Wolf whose tables missed their bound (FP64 form).
-enum : int { CK_NONE = 0, CK_EWALD = 1, CK_EWALD_ERF = 2, CK_WOLF = 3, CK_EWALD_LIB = 4, CK_WOLF_LIB = 5 };
+// The last two: Ewald and Wolf whose FP64 table of h missed its bound.
+enum : int { CK_NONE = 0, CK_EWALD = 1, CK_EWALD_ERF = 2, CK_WOLF = 3, CK_EWALD_EXP = 4, CK_WOLF_EXP = 5 };
 
 __host__ __forceinline__ int coulomb_variant(const CoulParam& c) {
     if (c.kind == COUL_EWALD) return c.inter_excl ? CK_EWALD_ERF : CK_EWALD;
     if (c.kind == COUL_WOLF) return c.inter_excl ? CK_NONE : CK_WOLF;
     return CK_NONE;
-}
-
-// 1 / sqrt(x) to about an ulp: the hardware estimate and two Newton steps.
-__device__ __forceinline__ double rsqrt_newton(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    double t = x * y;
-    double e = 0.5 - 0.5 * t * y;
-    y = y + y * e;
-    t = x * y;
-    e = 0.5 - 0.5 * t * y;
-    return y + y * e;
 }
 
 // The blocks behind the pair blocks: the intra-molecular terms (kIntra, force
@@ -1478,13 +1468,20 @@ __device__ __forceinline__ void pair_extra_block(const PairArgs& a, unsigned cha
 // * the cutoffs as tests of r^2 against the least double whose square root
 //   fails the reference's test (`r < rc`, `r <= rc`; the square root rounds
 //   monotonically), so the pair set stays the reference's without a root;
-// * 1 / r by the hardware estimate and Newton steps, no root or division;
+// * r and 1 / r^2 by the hardware estimate and Newton steps (root_recip, or
+//   recip_newton where no term needs r), no root or division; they are
+//   rounded no worse than the library's, and 1 / r^2 better than the square
+//   of a rounded 1 / r;
 // * Lennard-Jones as (A r^-6 - B) r^-8, formed for every pair and selected;
 // * the real-space Ewald or Wolf force as h(r) r^-3 with h(r) = erfc(alpha r)
 //   + (2 alpha / sqrt(pi)) r exp(-alpha^2 r^2) from a table of polynomial
-//   pieces (no exponential); energies keep exp(-x^2) erfcx(x).
-// SPC/E, 9000 atoms: 41 -> 21 us per launch against the reference's order with
-// library root, division and exponential.
+//   pieces (no exponential); energies, and forces where that table misses its
+//   bound (alpha rc above 3.9), keep exp(-x^2) erfcx(x).
+// Relative error of the force factor against 128 bits, rms over distances
+// from 1.5 A to a cutoff of 9 A, reference's order / this: Lennard-Jones 3.5
+// to 13e-16 / 1.6 to 4.3e-16, Ewald at alpha rc = pi 1.8 to 9.5e-16 / 1.4 to
+// 4.6e-16.  SPC/E, 9000 atoms: 41 -> 21 us per launch against the
+// reference's order with library root, division and exponential.
 template <bool kEnergy, int TPA, int CK, bool kIntra = false>
 __global__ __launch_bounds__(kPairBlock)
 __attribute__((amdgpu_waves_per_eu(!kIntra ? 1 : CK == CK_NONE ? 8 : CK == CK_EWALD || CK == CK_WOLF ? 6 : 3)))
@@ -1498,8 +1495,9 @@ void k_pairs(PairArgs a) {
     double2* const hmt = reinterpret_cast<double2*>(lds + sizeof(Lj) * kMaxKinds * kMaxKinds);  // Harmonic {k, x0}, k = 0 otherwise
     __shared__ double red[kPairBlock / 64][8];
     constexpr bool kTab = CK == CK_EWALD || CK == CK_WOLF;
-    __shared__ __align__(16) double hft[kTab ? kErfcxPieces * (kErfcxDeg64 + 1) : 2];
-    __shared__ __align__(16) double ecx[kTab && kEnergy ? kErfcxPieces * (kErfcxDeg64 + 1) : 2];
+    constexpr bool kExp = CK == CK_EWALD_EXP || CK == CK_WOLF_EXP, kEcx = kExp || (kTab && kEnergy);
+    __shared__ __align__(16) double hft[kTab ? kHfDoubles : 2];
+    __shared__ __align__(16) double ecx[kEcx ? kErfcxPieces * (kErfcxDeg64 + 1) : 2];
     if ((int)blockIdx.x >= a.pair_blocks) {  // uniform over the block
         pair_extra_block<kEnergy, kIntra>(a, lds);
         return;
@@ -1516,13 +1514,13 @@ void k_pairs(PairArgs a) {
         hmt[x] = make_double2(hm ? pp.p0 : 0.0, hm ? pp.p1 : 0.0);
         harmonic |= hm;
     }
-    if (kTab) {
-        constexpr int n2 = kErfcxPieces * (kErfcxDeg64 + 1) / 2;
-        for (int x = threadIdx.x; x < n2; x += blockDim.x) {
+    if (kTab)
+        for (int x = threadIdx.x; x < kHfDoubles / 2; x += blockDim.x)
             reinterpret_cast<double2*>(hft)[x] = reinterpret_cast<const double2*>(a.hf64)[x];
-            if (kEnergy) reinterpret_cast<double2*>(ecx)[x] = reinterpret_cast<const double2*>(a.ecx64)[x];
-        }
-    }
+    const bool use_ecx = kEcx && a.ecx64 != nullptr;  // uniform
+    if (use_ecx)
+        for (int x = threadIdx.x; x < kErfcxPieces * (kErfcxDeg64 + 1) / 2; x += blockDim.x)
+            reinterpret_cast<double2*>(ecx)[x] = reinterpret_cast<const double2*>(a.ecx64)[x];
     harmonic = __syncthreads_or(harmonic);  // also the barrier of the LDS tables
 
     // XCD-contiguous order of the pair blocks (the launch has a multiple of 8)
@@ -1565,40 +1563,50 @@ void k_pairs(PairArgs a) {
                 dz = image_rint(dz, Lz, iz);
             }
             const double r2 = norm2_ordered(dx, dy, dz);
-            const double inv_r = rsqrt_newton(r2), i2 = inv_r * inv_r, i6 = i2 * i2 * i2;
+            double r = 0.0, i2;
+            if constexpr (CK == CK_NONE)
+                i2 = recip_newton(r2);
+            else
+                root_recip(r2, r, i2);
+            const double i6 = i2 * i2 * i2;
             const Lj P = ljrow[kj];
             const bool in_pair = r2 < P.r2c;
             double fp = (P.A * i6 - P.B) * (i6 * i2), e_p = 0.0, e_c = 0.0;
             if (kEnergy) e_p = i6 * (P.A * (1.0 / 12.0) * i6 - P.B * (1.0 / 6.0));
             if (harmonic) {  // uniform
                 const double2 H = hmrow[kj];
-                const double r = r2 * inv_r;
-                fp += H.x * (H.y - r) * inv_r;
-                if (kEnergy) e_p += 0.5 * H.x * (r - H.y) * (r - H.y);
+                double rh = r, ih;
+                if constexpr (CK == CK_NONE) root_recip(r2, rh, ih);
+                fp += H.x * (H.y - rh) * (rh * i2);
+                if (kEnergy) e_p += 0.5 * H.x * (rh - H.y) * (rh - H.y);
             }
             double fs = in_pair ? fp : 0.0;
             if (kEnergy) e_p = in_pair ? e_p - P.shift : 0.0;
             if (CK != CK_NONE) {
                 const double pref = qi * pj.w;  // 0 adds an exact 0
                 const bool in_coul = r2 < c.r2c;
-                const double r = r2 * inv_r;
-                double fc, ec = 0.0;
+                double fc = 0.0, ec = 0.0;
                 if constexpr (kTab) {
-                    const double h3 = erfcx_tab(hft, r, a.hf_inv_h) * (inv_r * i2);
-                    fc = CK == CK_EWALD ? pref * h3 : pref * (h3 - c.f_const * inv_r);
+                    const double h3 = hforce_tab(hft, r, a.hf64_inv_h) * (r * (i2 * i2));
+                    fc = CK == CK_EWALD ? pref * h3 : pref * (h3 - c.f_const * (r * i2));
                     if (kEnergy) {
                         const double x = c.alpha * r;
-                        const double er = exp(-x * x) * erfcx_tab(ecx, x, a.ecx_inv_h) * inv_r;
+                        const double er = exp(-x * x) * erfcx_tab(ecx, x, a.ecx_inv_h) * (r * i2);
                         ec = CK == CK_EWALD ? pref * er : pref * (er - c.e_const);
                     }
                 } else if (in_coul) {
-                    // the library's erf and erfc
-                    if (CK == CK_WOLF_LIB)
-                        wolf_pair(c, qi * kFourPiEps0 * pj.w, r, inv_r, ec, fc);
-                    else
-                        ewald_real(c.alpha, qi * kFourPiEps0 * pj.w, r, inv_r, CK == CK_EWALD_ERF, ec, fc);
-                } else {
-                    fc = 0.0;
+                    const double inv_r = r * i2;
+                    if (kExp && use_ecx) {  // uniform
+                        // ewald.rs:387-428 / wolf.rs:90-117 with erfc = exp(-x^2) erfcx(x)
+                        const double x = c.alpha * r, ex = exp(-x * x), er = ex * erfcx_tab(ecx, x, a.ecx_inv_h);
+                        const double f = (er * inv_r + c.alpha * kFrac2SqrtPi * ex) * i2;
+                        fc = CK == CK_EWALD_EXP ? pref * f : pref * (f - c.f_const * inv_r);
+                        if (kEnergy) ec = CK == CK_EWALD_EXP ? pref * er * inv_r : pref * (er * inv_r - c.e_const);
+                    } else if (CK == CK_WOLF_EXP) {  // the library's erf and erfc
+                        wolf_pair(c, pi.w * pj.w, r, inv_r, ec, fc);
+                    } else {
+                        ewald_real(c.alpha, pi.w * pj.w, r, inv_r, CK == CK_EWALD_ERF, ec, fc);
+                    }
                 }
                 const bool on = in_coul && pref != 0.0;
                 fs += on ? fc : 0.0;
@@ -2877,7 +2885,7 @@ struct SmallArgs {
     double3 fo;        // origin of the FP32 coordinates in an infinite cell
     const double* hf64;
     const float* hf32;
-    double hf_inv_h;
+    double hf_inv_h;  // of the one that the form reads
 };
 // Atoms of the largest system in each form; past them the all-pairs work
 // costs more than the list's launches.  us per step, list / one launch:
@@ -2892,12 +2900,17 @@ constexpr int small_loop_max(bool mixed) { return mixed ? 96 : 64; }
 template <int CK>
 __device__ __forceinline__ double small_pair(double4 P, double2 H, int harmonic, double r2, double pref,
                                              const CoulParam& c, const double* hft, double hf_inv_h) {
-    const double inv_r = rsqrt_newton(r2), i2 = inv_r * inv_r, i6 = i2 * i2 * i2;
+    double r = 0.0, i2;
+    if (CK == CK_WOLF || harmonic)  // uniform
+        root_recip(r2, r, i2);
+    else
+        i2 = recip_newton(r2);
+    const double i6 = i2 * i2 * i2;
     double fp = (P.x * i6 - P.y) * (i6 * i2);
-    if (harmonic) fp += H.x * (H.y - r2 * inv_r) * inv_r;  // uniform
+    if (harmonic) fp += H.x * (H.y - r) * (r * i2);  // uniform
     double fs = r2 < P.z ? fp : 0.0;
     if constexpr (CK == CK_WOLF) {
-        const double fc = pref * (erfcx_tab(hft, r2 * inv_r, hf_inv_h) * (inv_r * i2) - c.f_const * inv_r);
+        const double fc = pref * (hforce_tab(hft, r, hf_inv_h) * (r * (i2 * i2)) - c.f_const * (r * i2));
         fs += r2 < c.r2c && pref != 0.0 ? fc : 0.0;
     }
     return fs;
@@ -2932,7 +2945,7 @@ __global__ __launch_bounds__(kLoop ? 1024 : 256) void k_small_step(SmallArgs a) 
     __shared__ unsigned char ks[NMAX];
     __shared__ T4 ljt[kMaxKinds * kMaxKinds];
     __shared__ T2 hmt[kMaxKinds * kMaxKinds];
-    __shared__ __align__(16) T hft[CK == CK_WOLF ? kErfcxPieces * ((kMixed ? kErfcxDeg32 : kErfcxDeg64) + 1) : 4];
+    __shared__ __align__(16) T hft[CK != CK_WOLF ? 4 : kMixed ? kErfcxPieces * (kErfcxDeg32 + 1) : kHfDoubles];
     __shared__ double4 own_p[OWN], own_v[OWN];
     __shared__ double ke_red[16];
     const int tid = threadIdx.x, n = a.n;

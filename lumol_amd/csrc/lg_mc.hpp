@@ -717,9 +717,7 @@ __device__ __forceinline__ double mc_wave_sum(double v) {
 
 // Pair energy at r2 from {4 eps s^12, 4 eps s^6, r2 bound, shift}.
 __device__ __forceinline__ double mc_lj(double4 P, double r2) {
-    double y = __builtin_amdgcn_rcp(r2);
-    y += y * (1.0 - r2 * y);
-    y += y * (1.0 - r2 * y);
+    const double y = recip_newton(r2);
     const double i6 = y * y * y, e = (P.x * i6 - P.y) * i6 - P.w;
     return r2 < P.z ? e : 0.0;
 }

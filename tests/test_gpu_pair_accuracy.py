@@ -1,0 +1,90 @@
+"""Relative error of the FP64 real-space pair forces, of isolated pairs of sites
+at many distances, against 50 digits: Ewald without k-vectors (kmax 1) over
+the alphas of each of its forms (the table of the force factor, exp and the
+table of erfcx, the library), Wolf, and Lennard-Jones.
+
+Bounds, u = 2^-53: the distance is rounded by u and the force factor falls as
+r^(2 x^2), x = alpha r, so 2 x^2 u; the argument of the exponential rounds
+its x and x^2 once more each, 3 x^2 u (not in the table form); ten more
+roundings of products and sums; and the fits' bounds, 2e-15 of the force
+factor or 1e-14 of erfcx, whichever the alpha takes (the former is met to 2e-16
+up to alpha rc = 3.5)."""
+import numpy as np
+import pytest
+
+from lumol_amd import Ewald, LennardJones, PairInteraction, System, UnitCell, Wolf
+from lumol_amd.consts import FOUR_PI_EPSILON_0
+
+mp = pytest.importorskip("mpmath").mp
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -53
+M = 6  # pairs on an axis
+RC = 9.0
+
+
+def dimers(coulomb, pair=None):
+    """M^3 pairs along x, 4 rc apart; distances of 20 bits, so that their
+    squares are exact.  Returns the force on each first site and r."""
+    g = 4.0 * RC * np.array([(i, j, k) for i in range(M) for j in range(M) for k in range(M)], float)
+    r = np.round(np.linspace(1.25, RC - 2.0 ** -16, M ** 3) * 2 ** 16) / 2 ** 16
+    pos = np.repeat(g, 2, axis=0)
+    pos[1::2, 0] += r
+    q = np.tile([1.0, -1.0], M ** 3)
+    s = System.from_arrays(["A"] * (2 * M ** 3), pos, UnitCell.ortho(*[4.0 * RC * M] * 3),
+                           charges=q if coulomb is not None else 0 * q, masses=np.ones(2 * M ** 3))
+    if pair is not None:
+        s.set_pair_potential(("A", "A"), PairInteraction(pair, RC))
+    if coulomb is not None:
+        s.set_coulomb_potential(coulomb)
+    f = s.forces()
+    assert (f[:, 1:] == 0).all()
+    assert (f[0::2, 0] == -f[1::2, 0]).all()
+    return f[0::2, 0], r
+
+
+def ewald_factor(alpha, r):
+    """erfc(alpha r) / r^2 + 2 alpha / sqrt(pi) exp(-alpha^2 r^2) / r"""
+    return mp.erfc(alpha * r) / r ** 2 + 2 * alpha / mp.sqrt(mp.pi) * mp.exp(-(alpha * r) ** 2) / r
+
+
+@pytest.mark.parametrize("arc", [0.5, 2.5, float(np.pi), 3.5, 4.0, 4.6, 5.6, 7.5])
+def test_ewald(arc):
+    mp.dps = 50
+    alpha = arc / RC
+    f, r = dimers(Ewald(RC, 1, alpha))
+    worst = 0.0
+    for a, b in zip(f, r):
+        ref = ewald_factor(mp.mpf(alpha), mp.mpf(b)) / mp.mpf(FOUR_PI_EPSILON_0)
+        x2 = (alpha * b) ** 2
+        bound = (2 * x2 + 10) * U + (2e-16 if arc <= 3.5 else 3 * x2 * U + 1e-14)
+        err = abs(float((mp.mpf(float(a)) - ref) / ref))
+        worst = max(worst, err / bound)
+        assert err <= bound, (b, err, bound)
+    print(f"alpha rc {arc}: {worst:.2f} of the bound")
+
+
+def test_wolf():
+    mp.dps = 50
+    f, r = dimers(Wolf(RC))
+    alpha = mp.pi / RC
+    fc = ewald_factor(alpha, mp.mpf(RC))
+    for a, b in zip(f, r):
+        whole = ewald_factor(alpha, mp.mpf(b)) / mp.mpf(FOUR_PI_EPSILON_0)
+        ref = whole - fc / mp.mpf(FOUR_PI_EPSILON_0)
+        x2 = (np.pi / RC * b) ** 2
+        # relative to the unshifted force, plus the constant's own rounding
+        assert abs(float((mp.mpf(float(a)) - ref) / whole)) <= (2 * x2 + 10) * U + 2e-16 + 25 * U * float(
+            fc / FOUR_PI_EPSILON_0 / whole)
+
+
+def test_lennard_jones():
+    mp.dps = 50
+    sigma, eps = 3.1, 1.3e-4
+    f, r = dimers(None, LennardJones(sigma, eps))
+    for a, b in zip(f, r):
+        s6 = (mp.mpf(sigma) / mp.mpf(b)) ** 6
+        up, down = 48 * mp.mpf(eps) * s6 * s6 / b, 24 * mp.mpf(eps) * s6 / b
+        # 14 powers of the rounded 1 / r^2 by halves, six products and sums,
+        # sigma^12 (eleven)
+        assert abs(float((mp.mpf(float(a)) - (down - up)) / (up + down))) <= (7 + 6 + 11) * U
+
