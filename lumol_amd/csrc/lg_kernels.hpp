@@ -1507,7 +1507,7 @@ void k_pairs(PairArgs a) {
     int harmonic = 0;
     for (int x = threadIdx.x; x < nk2; x += blockDim.x) {
         const PairParam pp = a.table[x];
-        const bool on = pp.pot > POT_NULL && !pp.inter_excl, lj = pp.pot == POT_LJ;
+        const bool lj = pp.pot == POT_LJ, on = (lj || (pp.pot > POT_NULL && pp.p0 != 0.0)) && !pp.inter_excl;
         const double s2 = pp.p0 * pp.p0, s6 = lj ? s2 * s2 * s2 : 0.0;
         ljt[x] = Lj{lj ? 48.0 * pp.p1 * (s6 * s6) : 0.0, lj ? 24.0 * pp.p1 * s6 : 0.0, on ? pp.r2c : 0.0, pp.shift};
         const bool hm = on && pp.pot == POT_HARMONIC;
@@ -1577,8 +1577,10 @@ void k_pairs(PairArgs a) {
                 const double2 H = hmrow[kj];
                 double rh = r, ih;
                 if constexpr (CK == CK_NONE) root_recip(r2, rh, ih);
-                fp += H.x * (H.y - rh) * (rh * i2);
-                if (kEnergy) e_p += 0.5 * H.x * (rh - H.y) * (rh - H.y);
+                rh = r2 > 0.0 ? rh : 0.0;  // sites at one place have an energy
+                const bool hm = H.x != 0.0;
+                fp = hm ? H.x * (H.y - rh) * (rh * i2) : fp;
+                if (kEnergy) e_p = hm ? 0.5 * H.x * (rh - H.y) * (rh - H.y) : e_p;
             }
             double fs = in_pair ? fp : 0.0;
             if (kEnergy) e_p = in_pair ? e_p - P.shift : 0.0;
@@ -2907,7 +2909,7 @@ __device__ __forceinline__ double small_pair(double4 P, double2 H, int harmonic,
         i2 = recip_newton(r2);
     const double i6 = i2 * i2 * i2;
     double fp = (P.x * i6 - P.y) * (i6 * i2);
-    if (harmonic) fp += H.x * (H.y - r) * (r * i2);  // uniform
+    if (harmonic) fp = H.x != 0.0 ? H.x * (H.y - r) * (r * i2) : fp;
     double fs = r2 < P.z ? fp : 0.0;
     if constexpr (CK == CK_WOLF) {
         const double fc = pref * (hforce_tab(hft, r, hf_inv_h) * (r * (i2 * i2)) - c.f_const * (r * i2));
@@ -2952,7 +2954,8 @@ __global__ __launch_bounds__(kLoop ? 1024 : 256) void k_small_step(SmallArgs a) 
     int harmonic = 0;
     for (int x = tid; x < a.nkinds * a.nkinds; x += BLOCK) {
         const PairParam pp = a.table[x];
-        const bool on = pp.pot > POT_NULL && !pp.inter_excl, lj = pp.pot == POT_LJ, hm = on && pp.pot == POT_HARMONIC;
+        const bool lj = pp.pot == POT_LJ, on = (lj || (pp.pot > POT_NULL && pp.p0 != 0.0)) && !pp.inter_excl,
+                   hm = on && pp.pot == POT_HARMONIC;
         const double s2 = pp.p0 * pp.p0, s6 = lj ? s2 * s2 * s2 : 0.0;
         const float rcf = (float)pp.rc;
         ljt[x].x = (T)(lj ? 48.0 * pp.p1 * (s6 * s6) : 0.0);

@@ -12,7 +12,8 @@ up to alpha rc = 3.5)."""
 import numpy as np
 import pytest
 
-from lumol_amd import Ewald, LennardJones, PairInteraction, System, UnitCell, Wolf
+import lumol_oracle as lo
+from lumol_amd import Ewald, Harmonic, LennardJones, PairInteraction, System, UnitCell, Wolf
 from lumol_amd.consts import FOUR_PI_EPSILON_0
 
 mp = pytest.importorskip("mpmath").mp
@@ -88,3 +89,12 @@ def test_lennard_jones():
         # sigma^12 (eleven)
         assert abs(float((mp.mpf(float(a)) - (down - up)) / (up + down))) <= (7 + 6 + 11) * U
 
+
+def test_harmonic_sites_at_one_place():
+    # an energy, k x0^2 / 2, without a direction of the force
+    pos = np.array([[1.0, 1.0, 1.0], [1.0, 1.0, 1.0], [9.0, 9.0, 9.0], [9.0, 9.0, 12.5]])
+    s = System.from_arrays(["A"] * 4, pos, UnitCell.ortho(20.0, 20.0, 20.0), masses=np.ones(4))
+    s.set_pair_potential(("A", "A"), PairInteraction(Harmonic(2e-4, 4.0), 8.0))
+    e, eo = s.potential_energy(), lo.OracleSystem(s, nthreads=1).potential_energy()
+    assert abs(e - eo) <= 1e-14 * abs(eo)
+    assert abs(e - (0.5 * 2e-4 * 16.0 + 0.5 * 2e-4 * 0.25)) <= 1e-14 * abs(e)
