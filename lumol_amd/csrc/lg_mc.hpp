@@ -754,6 +754,10 @@ __device__ __forceinline__ uint2 mc_span(double rc, double d, double L) {
     return make_uint2(a, a + b);
 }
 typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
+// A half of a fraction word.  Moves write halves and the next attempt reads
+// words, with no barrier in between: the type tells the compiler that they
+// are the same memory.
+typedef unsigned short __attribute__((may_alias)) mc_half;
 // Zero half words where base <= f <= base + width (modulo 2^16).
 __device__ __forceinline__ unsigned mc_outside(unsigned f, unsigned base, unsigned width) {
     const ushort2v d = __builtin_bit_cast(ushort2v, f) - __builtin_bit_cast(ushort2v, base);
@@ -775,8 +779,8 @@ __global__ __launch_bounds__(kMcAtomBlock) void k_mc_atoms(const McChain* __rest
     // a wave's list holds all atoms that it tests
     unsigned short* const list = reinterpret_cast<unsigned short*>(FZ + rows * BLOCK) + wave * rows * 128;
     unsigned char* const kind = reinterpret_cast<unsigned char*>(FZ + rows * BLOCK) + rows * BLOCK * 4;
-    unsigned short *const fx = reinterpret_cast<unsigned short*>(FX), *const fy = reinterpret_cast<unsigned short*>(FY),
-                          *const fz = reinterpret_cast<unsigned short*>(FZ);
+    mc_half *const fx = reinterpret_cast<mc_half*>(FX), *const fy = reinterpret_cast<mc_half*>(FY),
+                   *const fz = reinterpret_cast<mc_half*>(FZ);
     const bool periodic = c.box.periodic != 0;
     const double Lx = c.box.L[0], Ly = c.box.L[1], Lz = c.box.L[2];
     const double ix = c.box.inv[0], iy = c.box.inv[1], iz = c.box.inv[2];
@@ -793,9 +797,9 @@ __global__ __launch_bounds__(kMcAtomBlock) void k_mc_atoms(const McChain* __rest
         X[i] = p.x;
         Y[i] = p.y;
         Z[i] = p.z;
-        fx[i] = (unsigned short)mc_frac16(p.x, ix);
-        fy[i] = (unsigned short)mc_frac16(p.y, iy);
-        fz[i] = (unsigned short)mc_frac16(p.z, iz);
+        fx[i] = (mc_half)mc_frac16(p.x, ix);
+        fy[i] = (mc_half)mc_frac16(p.y, iy);
+        fz[i] = (mc_half)mc_frac16(p.z, iz);
         kind[i] = (unsigned char)c.meta[i].x;
     }
     // test results of a lane: bit rows - 1 - r and 16 above it for the atoms
@@ -920,9 +924,9 @@ __global__ __launch_bounds__(kMcAtomBlock) void k_mc_atoms(const McChain* __rest
                     X[i] = qx;
                     Y[i] = qy;
                     Z[i] = qz;
-                    fx[i] = (unsigned short)hx;
-                    fy[i] = (unsigned short)hy;
-                    fz[i] = (unsigned short)hz;
+                    fx[i] = (mc_half)hx;
+                    fy[i] = (mc_half)hy;
+                    fz[i] = (mc_half)hz;
                 }
                 if (i2 == i) {
                     px2 = qx;

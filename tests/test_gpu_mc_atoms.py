@@ -92,6 +92,23 @@ def test_switching_amplitude():
     assert np.array_equal(s.positions, o.positions())
 
 
+def test_every_move_decides_the_next():
+    # a few sites, most moves accepted: an attempt tests sites whose fractions
+    # the attempt before has just written
+    for n in (2, 4, 7):
+        s = chain(n, box=(4.0 * SIGMA,) * 3, rc=1.9 * SIGMA, seed=5)
+        o = lo.OracleSystem(s, nthreads=1)
+        o.cache_init()
+        s.cache_init()
+        beta, t = 0.05 / EPS, 0
+        for k in (1, 2, 61, 400, 1500):
+            a = s.mc_run(31, t, k, beta, 1.2 * SIGMA)
+            assert a == o.mc_run(31, t, k, beta, 1.2 * SIGMA)
+            t += k
+            assert np.array_equal(s.positions, o.positions())
+        assert a > 1000
+
+
 def test_same_bits_however_divided():
     out = []
     for parts in ([900], [100] * 9, [450, 450]):
