@@ -482,7 +482,7 @@ struct lg_system {
     DevBuf<double4> snap_pos, snap_vel, snap_acc;
     // MD chunk captured as a HIP graph, with what it was captured for
     hipGraphExec_t md_exec = nullptr;
-    uint64_t md_key[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    std::array<uint64_t, 11> md_key{};
     uint64_t cfg_epoch = 0;  // bumped by prepare() whenever anything was re-derived
     // kernel timing (lg_profile_*)
     uint32_t prof_mask = 0;
@@ -3163,12 +3163,14 @@ int lg_md_run(lg_system* s, uint64_t nsteps) {
         const bool graph = s->tune.md_graph == 2 && s->prof_mask == 0;
         if (graph) {
             // captured once per (chunk length, configuration, buffer set,
-            // integrator settings) and replayed
-            const uint64_t key[8] = {todo, s->cfg_epoch, g_alloc_epoch.load(), uint64_t(s->integrator),
-                                     uint64_t(s->precision), bits_of(s->dt),
-                                     s->thermostat ? bits_of(s->berendsen_T) : ~uint64_t(0),
-                                     bits_of(s->berendsen_tau)};
-            if (!s->md_exec || !std::equal(key, key + 8, s->md_key)) {
+            // integrator settings, in an infinite cell the origin of the FP32
+            // coordinates, which new positions move) and replayed
+            const double3 fo = s->periodic ? make_double3(0.0, 0.0, 0.0) : s->frac_origin;
+            const std::array<uint64_t, 11> key = {todo, s->cfg_epoch, g_alloc_epoch.load(), uint64_t(s->integrator),
+                                                  uint64_t(s->precision), bits_of(s->dt),
+                                                  s->thermostat ? bits_of(s->berendsen_T) : ~uint64_t(0),
+                                                  bits_of(s->berendsen_tau), bits_of(fo.x), bits_of(fo.y), bits_of(fo.z)};
+            if (!s->md_exec || key != s->md_key) {
                 if (s->md_exec) (void)hipGraphExecDestroy(s->md_exec);
                 s->md_exec = nullptr;
                 hipGraph_t g = nullptr;
@@ -3186,7 +3188,7 @@ int lg_md_run(lg_system* s, uint64_t nsteps) {
                     s->md_exec = nullptr;
                     return fail(LG_E_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
                 }
-                std::copy(key, key + 8, s->md_key);
+                s->md_key = key;
             }
             LG_HIP(hipGraphLaunch(s->md_exec, st));
         } else {
