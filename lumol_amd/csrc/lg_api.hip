@@ -1023,10 +1023,21 @@ static int oct_step_atoms_t(const lg_system* s) {
 static int oct_step_atoms(const lg_system* s, bool mixed) {
     return mixed ? oct_step_atoms_t<float>(s) : oct_step_atoms_t<double>(s);
 }
-// Whether k_oct_step also forms the rho partials: one set per block is
-// written, so beyond 512 blocks the separate pass, with up to 512 atoms per
-// set, takes over.
-static bool oct_step_rho(const lg_system* s, bool mixed) { return blocks_for(s->n, oct_step_atoms(s, mixed)) <= 512; }
+constexpr size_t kOctItemBytes = 4 * 64 * sizeof(double4);  // rho partials of an item
+
+// Whether k_oct_step also forms the rho partials.  It writes one set per
+// block, the separate pass one per up to 512 atoms, so the step's are written
+// and read again from 16 atoms a block on; against that stands the separate
+// launch, which forms the phase rows anew.  us per step, in the step /
+// separate, mixed: 4096 ions kmax 9 (12 MB) 27 / 26, 12 (22 MB) 35 / 30, 16 (46
+// MB) 43 / 34, 32 285 / 222; 8000 ions (32 atoms a block) kmax 9 33 / 33, 16 54
+// / 49, 32 396 / 354; from 64 atoms a block on 13 824 ions kmax 12 50 / 48, 24
+// (152 MB) 272 / 299, 48 (1 GB) 2107 / 1910, 32 768 ions kmax 16 105 / 113, 24
+// 436 / 474.  Beyond 512 blocks (a narrow rho_width) the separate pass too.
+static bool oct_step_rho(const lg_system* s, bool mixed) {
+    const int c = oct_step_atoms(s, mixed), blocks = blocks_for(s->n, c);
+    return blocks <= 512 && size_t(blocks) * s->oct_nitems * kOctItemBytes <= size_t(c >= 64 ? 256 : 16) << 20;
+}
 
 // The octant form's tables from the k set (see lg_kspace.hpp): pairs (p, q) =
 // (ikx, |iky|) sorted by how many ikz they need, row tiles of four pairs,

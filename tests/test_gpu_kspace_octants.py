@@ -5,6 +5,8 @@ the sizes where a row tile gains a step or a column tile (2, 4, 7, 8, 9, 16,
 k set is not symmetric (-kmax without +kmax on the long axes), atom counts
 around the 16 of a matrix tile, and MD steps with every number of atom groups
 per block."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -82,3 +84,27 @@ def test_md_groups(width, thermostat, kmax):
     o.md_run(0, 1.0, 6, *((300.0, 50.0) if thermostat else ()))
     assert np.abs(s.positions - o.positions()).max() < 1e-10
     assert np.abs(run(LG_PRECISION_MIXED).positions - s.positions).max() < 1e-6
+
+
+def test_partial_sums_stay_small():
+    # steps of 4096 ions at 40 k-vectors an axis: one set of partial sums of
+    # rho(k) per 16 atoms would be 700 MB
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    s = ions(4096, (45.0, 45.0, 45.0), 40)
+    # what does not depend on the k-vectors is allocated first
+    s.set_coulomb_potential(Ewald(18.0, 2))
+    md = Simulation(MolecularDynamics(VelocityVerlet(1.0)))
+    md.run(s, 2)
+    before = free()
+    s.set_coulomb_potential(Ewald(18.0, 40))
+    md.run(s, 2)
+    assert before - free() < 300 << 20
+    o = lo.OracleSystem(s, nthreads=16)
+    f, fo = s.forces(), o.forces()
+    assert np.abs(f - fo).max() < 1e-10 * np.abs(fo).max()
