@@ -300,7 +300,7 @@ int lg_mc_run_batch(lg_system* const* systems, size_t count, const uint64_t* see
  *                 16 for systems with a pair potential other than LJ,
  *                 Harmonic and Null, or a table)
  *   kspace_split  row ranges of the k-space force kernel of the row form
- *                 (1..32; kmax above 64; no effect on the octant form)
+ *                 (1..32; no effect on the octant form, see rho_kind)
  *   rho_width     atoms per block of the rho(k) kernel (a multiple of 64 up to
  *                 512); a quarter of it in the MD kernel that forms rho(k)
  *                 with the half-steps
@@ -317,9 +317,10 @@ int lg_mc_run_batch(lg_system* const* systems, size_t count, const uint64_t* see
  *                 the replay measured 4-18% slower than eager launches, so
  *                 it is off by default.
  *   rho_kind      1 (default), 2 or 3: the three forms that earlier versions
- *                 of rho(k) had.  All run the octant form on the matrix cores
- *                 now (kmax up to 64, the row form above), with the same bits;
- *                 the knob is kept for saved choices.
+ *                 of rho(k) had.  All run one form now, with the same bits:
+ *                 octants on the matrix cores up to kmax 32, and up to kmax 64
+ *                 with 2048 atoms or more (FP64: 1280, from kmax
+ *                 44 on 512), else rows; the knob is kept for saved choices.
  * lumol_amd.tuning picks them per size bucket by timing the candidates.
  * Results do not depend on them beyond summation order. */
 typedef struct lg_tuning {

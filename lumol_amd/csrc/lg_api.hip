@@ -406,9 +406,8 @@ struct lg_system {
     DevBuf<double4> fk;  // k-space partial forces [ksplit][n]
     DevBuf<int4> kidx;
     DevBuf<KRow> rows;
-    // octant form (kmax <= kOctMaxK): (p, q) pairs and their row tiles, work
-    // items of the rho pass, output tiles, k map, force coefficients, partials
-    bool oct = false;
+    // octant form (oct_pays): (p, q) pairs and their row tiles, work items of
+    // the rho pass, output tiles, k map, force coefficients, partials
     int oct_nrt = 0, oct_nst = 0, oct_steps = 0, oct_zcols = 0, oct_nitems = 0, oct_ntiles = 0;
     int oct_width = 0, oct_nchunks = 0, oct_ngroups = 0, oct_ipg = 0, oct_asplit = 1;
     int rho_nchunks = 0;  // partial sums of the last rho pass
@@ -418,7 +417,7 @@ struct lg_system {
     DevBuf<float> ocoef32;
     DevBuf<double> ocoef64;
     DevBuf<double4> opart;
-    // row form (kmax above it)
+    // row form (the others)
     DevBuf<KUnit> units;         // rho pass work units (up to 5 k-vectors of a row)
     DevBuf<int> kslot;           // k -> slot of the rho partials (j * nunits + unit)
     // erfcx tables of the real-space erfc (empty: library erfc)
@@ -1003,6 +1002,23 @@ int prepare_params(lg_system* s) {
     return LG_OK;
 }
 
+// Which systems' k-space runs in the octant form.  A block of it holds 16 atoms
+// or more and takes every row tile of the k set in turn, so few atoms leave
+// most CUs idle; above kmax 32, where the operands of a row no longer stay in
+// registers, that costs more than the products save.  us per MD step, octants /
+// rows, mixed: 512 ions kmax 32 78 / 112, 48 471 / 386, 64 1239 / 1152; 1728 ions 32
+// 87 / 145, 48 571 / 529, 64 1254 / 1170; 2744 ions 48 569 / 581, 64 1253 / 1291.  FP64:
+// 216 ions 48 532 / 411, 64 1236 / 1225; 512 ions 33 191 / 138, 48 520 / 546, 64 1440
+// / 1829; 1000 ions 48 615 / 815.
+static bool oct_pays(const lg_system* s, bool mixed) {
+    const int kmax = s->coul_kmax;
+    if (s->nk <= 0 || kmax > kOctMaxK) return false;
+    return kmax <= 32 || s->n >= size_t(mixed ? 2048 : kmax < 44 ? 1280 : 512);
+}
+static bool oct_form(const lg_system* s) {
+    return s->coul_kind == COUL_EWALD && oct_pays(s, s->precision == LG_PRECISION_MIXED);
+}
+
 // Atoms per block of k_oct_step: the 16-atom groups dealt evenly to one block
 // per CU (256), at most as many as the LDS holds.  One block more than there
 // are CUs would double the time of the kernel, which is bound by the matrix
@@ -1030,10 +1046,9 @@ constexpr size_t kOctItemBytes = 4 * 64 * sizeof(double4);  // rho partials of a
 // and read again from 16 atoms a block on; against that stands the separate
 // launch, which forms the phase rows anew.  us per step, in the step /
 // separate, mixed: 4096 ions kmax 9 (12 MB) 27 / 26, 12 (22 MB) 35 / 30, 16 (46
-// MB) 43 / 34, 32 285 / 222; 8000 ions (32 atoms a block) kmax 9 33 / 33, 16 54
-// / 49, 32 396 / 354; from 64 atoms a block on 13 824 ions kmax 12 50 / 48, 24
-// (152 MB) 272 / 299, 48 (1 GB) 2107 / 1910, 32 768 ions kmax 16 105 / 113, 24
-// 436 / 474.  Beyond 512 blocks (a narrow rho_width) the separate pass too.
+// MB) 43 / 34; 8000 ions (32 atoms a block) kmax 9 33 / 33, 16 54 / 49; from 64
+// atoms a block on 13 824 ions kmax 12 50 / 48, 48 (1 GB) 2107 / 1910, 32 768 ions
+// kmax 16 105 / 113, with NST 0 at kmax 24 436 / 474.  Beyond 512 blocks (a narrow rho_width) the separate pass too.
 static bool oct_step_rho(const lg_system* s, bool mixed) {
     const int c = oct_step_atoms(s, mixed), blocks = blocks_for(s->n, c);
     return blocks <= 512 && size_t(blocks) * s->oct_nitems * kOctItemBytes <= size_t(c >= 64 ? 256 : 16) << 20;
@@ -1238,8 +1253,11 @@ int prepare_kspace(lg_system* s) {
     LG_TRY(upload(s->vfac, vflat, st));
     LG_TRY(s->rho.ensure(s->nk));
     if (kmax > 1000) return fail(LG_E_UNSUPPORTED, "kmax too large");
-    s->oct = kmax <= kOctMaxK && s->nk > 0;
-    if (s->oct) return prepare_octants(s, idx);
+    // the tables of both forms where they differ by precision, which may
+    // change without a call that may allocate
+    const bool both = oct_pays(s, true) != oct_pays(s, false);
+    if (both || oct_pays(s, true)) LG_TRY(prepare_octants(s, idx));
+    if (!both && oct_pays(s, true)) return LG_OK;
     std::vector<KRow> rows;
     for (int k = 0; k < s->nk; k++) {
         if (rows.empty() || rows.back().ikx != idx[k].x || rows.back().iky != idx[k].y ||
@@ -1488,7 +1506,7 @@ static int direct_blocks(const lg_system* s) { return s->grid.ncell * direct_spl
 // that keeps the grid at or below ~2048 blocks, so that per-block work stays
 // substantial while the partials stay few; the tuning knob overrides.
 static int rho_chunk(const lg_system* s) {
-    if (s->oct) return s->oct_width;
+    if (oct_form(s)) return s->oct_width;
     if (s->tune.rho_width > 0) return s->tune.rho_width;
     int nub = blocks_for(s->nunits, 64);
     int w = 64;
@@ -1499,7 +1517,7 @@ static int rho_chunk(const lg_system* s) {
 // Blocks of the rho(k) reduction (and of its energy partials).
 static int kspace_reduce_blocks(const lg_system* s) {
     if (s->coul_kind != COUL_EWALD || s->nk <= 0) return 0;
-    return s->oct ? 4 * s->oct_ntiles : blocks_for(s->nk, kRhoReduceK);
+    return oct_form(s) ? 4 * s->oct_ntiles : blocks_for(s->nk, kRhoReduceK);
 }
 
 // Arguments of the octant rho pass.
@@ -1534,7 +1552,13 @@ static void launch_rho_oct(lg_system* s, const OctRho& ra, int grid, bool energy
     else go(k_rho_oct<T, false>);
 }
 
-// k_oct_step: NST by the steps of the longest row (0 above eight steps).
+// k_oct_step: NST by the steps of the longest row (0 above 16).  The rows'
+// operands in registers and a coefficient load one unit ahead are what the
+// instances are for: us per mixed MD step with NST 0 / 12 or 16, 512 ions kmax 20
+// 62 / 42, 32 166 / 78, 4096 ions 65 / 45, 222 / 134.  Among them a row shorter
+// than its instance loads and skips steps: kmax 10 with NST 8 / 5, FP64, 512
+// ions 23.5 / 22.9, 32 768 ions 85.3 / 82.1; kmax 8 with NST 5 / 4 13 824 ions 39.9 /
+// 39.1; mixed 0 to 1.5%.
 template <typename T, int NST>
 static void launch_oct_step_c(lg_system* s, int cls, const OctForce& a, const OctStep& st, const OctRho& ra, int c) {
     launch_timed(s, cls, k_oct_step<T, NST>, blocks_for(s->n, c), 512, uint32_t(oct_step_lds<T>(ra.kmax, ra.zcols, c)),
@@ -1543,13 +1567,17 @@ static void launch_oct_step_c(lg_system* s, int cls, const OctForce& a, const Oc
 template <typename T>
 static void launch_oct_step_t(lg_system* s, int cls, const OctForce& a, const OctStep& st, const OctRho& ra, int c) {
     // an instance reads NST steps of every row tile, which holds oct_nst =
-    // 4 ceil(extent / 8) of them: 4 for at most 4 steps, 8 for 5 to 8
+    // 4 ceil(extent / 8) of them: 4 for at most 4 steps, 8 for 5 to 8, 12, 16
     if (s->oct_steps <= 4)
         launch_oct_step_c<T, 4>(s, cls, a, st, ra, c);
     else if (s->oct_steps <= 5)
         launch_oct_step_c<T, 5>(s, cls, a, st, ra, c);
     else if (s->oct_steps <= 8)
         launch_oct_step_c<T, 8>(s, cls, a, st, ra, c);
+    else if (s->oct_steps <= 12)
+        launch_oct_step_c<T, 12>(s, cls, a, st, ra, c);
+    else if (s->oct_steps <= 16)
+        launch_oct_step_c<T, 16>(s, cls, a, st, ra, c);
     else
         launch_oct_step_c<T, 0>(s, cls, a, st, ra, c);
 }
@@ -1720,7 +1748,7 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
     int n = int(s->n);
     bool mixed = s->precision == LG_PRECISION_MIXED;
     const bool kspace = s->coul_kind == COUL_EWALD && s->nk > 0;
-    const bool oct = kspace && s->oct;
+    const bool oct = kspace && oct_form(s);
     // rho(k) partials first: their reduction runs as the last blocks of the
     // pair launch, and the k-space forces after it
     int nchunks = 0;
@@ -2971,7 +2999,7 @@ int lg_molecular_virial(lg_system* s, double* w9) {
     a.part = s->molvir_part.p;
     k_mol_pairs<<<nbp, 256, 0, st>>>(a);
     if (kspace)
-        k_mol_kspace<<<nbp, 256, 0, st>>>(s->pos.p, s->meta.p, s->fk.p, s->oct ? 1 : s->ksplit, s->oct ? 1 : 0, n, s->mol_com.p,
+        k_mol_kspace<<<nbp, 256, 0, st>>>(s->pos.p, s->meta.p, s->fk.p, oct_form(s) ? 1 : s->ksplit, oct_form(s) ? 1 : 0, n, s->mol_com.p,
                                           s->molvir_part.p + size_t(nbp) * 6);
     LG_HIP(hipGetLastError());
     std::vector<double> h(size_t(nbp) * (6 + (kspace ? 9 : 0)));
@@ -3085,7 +3113,7 @@ static int md_chunk(lg_system* s, uint64_t todo) {
     const int n = int(s->n);
     const bool thermo = s->thermostat;
     const bool kspace = s->coul_kind == COUL_EWALD && s->nk > 0;
-    const bool oct = kspace && s->oct;
+    const bool oct = kspace && oct_form(s);
     const int nb = blocks_for(n, kMdBlock);
     // kinetic-energy partials: one per block of the kernel with the second half
     const int nke = oct ? oct_ke_parts(s) : nb;

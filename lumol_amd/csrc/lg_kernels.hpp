@@ -2284,8 +2284,8 @@ __global__ __launch_bounds__(256) void k_mol_kspace(const double4* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------------
-// Ewald k-space (ewald.rs:633-733) of the row form, for kmax above kOctMaxK
-// (below: lg_kspace.hpp).  k_phase computes, once per evaluation,
+// Ewald k-space (ewald.rs:633-733) of the row form, which runs where the
+// octant form (lg_kspace.hpp) does not pay (oct_pays).  k_phase computes, once per evaluation,
 // e^{i n k_axis . r_i} for every atom and axis by the reference's recursion
 // (polar for n = 1, products for |n| >= 2, conjugates for n < 0) into a
 // table in HBM; the rho and force kernels read the rows they use from it and
@@ -2383,7 +2383,7 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
     return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-// ---- row form (kmax above kOctMaxK) ---------------------------------------------
+// ---- row form (oct_pays says where) -----------------------------------------------
 // rho partial sums by row units.  A unit is up to kRhoUnitK (5) consecutive
 // k-vectors of one row (fixed ikx, iky; consecutive ikz): per atom, the lane
 // forms q e^{i k0.r} = q (Ex * Ey) * Ez[ikz0] and steps to the next ikz by

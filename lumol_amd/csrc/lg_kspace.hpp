@@ -56,7 +56,8 @@ __device__ __forceinline__ oct_d4 oct_mfma(double a, double b, oct_d4 c) {
 
 // Largest kmax of the octant form: the phase rows of 16 atoms fit the LDS of
 // its launches with room to spare (FP64, kmax 64: 404 rows of 17 x 8 B = 55 KB).
-// Beyond it (half a million k-vectors) the row kernels run.
+// Beyond it (half a million k-vectors) the row kernels run, as they do for few
+// atoms from kmax 33 on (oct_pays).
 constexpr int kOctMaxK = 64;
 
 // (cos, sin) of 2 pi u, u in turns: the reduction to an eighth of a turn is
