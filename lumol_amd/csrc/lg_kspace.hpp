@@ -179,7 +179,8 @@ __device__ __forceinline__ void oct_stage_rows(T* sm, const double* inv3, int km
 // The rho partials of chunk `chunk` for the items of group `grp`: per stage
 // of SA atoms (the rows are formed in `sm`, or stand there already when
 // `staged`: one stage), each of the 8 waves sums its item.  Mixed form: FP32
-// sums of 32 atoms, added in FP64.  na atoms in the chunk; pos(at).
+// sums of 32 atoms, whatever the stages, added in FP64.  na atoms in the
+// chunk; pos(at).
 template <typename T, typename F>
 __device__ __forceinline__ void oct_rho_group(const OctRho& a, int SA, int grp, int chunk, int na, bool staged, T* sm,
                                               F pos) {
@@ -213,6 +214,7 @@ __device__ __forceinline__ void oct_rho_group(const OctRho& a, int SA, int grp, 
             acc[u] = acc_t{0, 0, 0, 0};
         }
     };
+    int held = 0;  // trips in the FP32 sums, over the stages
     for (int s0 = 0; s0 < na; s0 += SA) {
         const int ns = min(SA, na - s0);
         if (!staged) {
@@ -227,7 +229,7 @@ __device__ __forceinline__ void oct_rho_group(const OctRho& a, int SA, int grp, 
                 for (int q = q0; q < q1; q++) {
                     step(sm + 8 * q);
                     step(sm + 8 * q + 4);
-                    if (sizeof(T) == 4 && ((q - q0) & 3) == 3) flush();
+                    if (sizeof(T) == 4 && (++held & 3) == 0) flush();
                 }
             };
             if (shape == 0)

@@ -12,7 +12,7 @@ import pytest
 
 import lumol_oracle as lo
 from lumol_amd import Ewald, LennardJones, MolecularDynamics, PairInteraction, Simulation, System, UnitCell, VelocityVerlet
-from lumol_amd._native import LG_PRECISION_MIXED
+from lumol_amd._native import LG_PRECISION_FP64, LG_PRECISION_MIXED
 from lumol_amd.system import BerendsenThermostat
 
 pytestmark = pytest.mark.gpu
@@ -108,3 +108,22 @@ def test_partial_sums_stay_small():
     o = lo.OracleSystem(s, nthreads=16)
     f, fo = s.forces(), o.forces()
     assert np.abs(f - fo).max() < 1e-10 * np.abs(fo).max()
+
+
+@pytest.mark.parametrize("width", [0, 64, 320, 512])
+@pytest.mark.parametrize("kmax", [9, 16, 24, 26, 28, 32])
+def test_mixed_sums_hold_32_atoms(kmax, width):
+    # a lattice whose structure factors are n q at every eighth k-vector and
+    # nothing between, with charges of 19 bits: sums of up to 32 of them are
+    # exact in FP32 and longer ones are not.  The rest is the phases' own
+    # FP32 rounding, off by a thousandth of 1e-7 of n q, squared
+    g = np.array([(i, j, k) for i in range(8) for j in range(8) for k in range(8)], float) * 4.0
+    e = []
+    for precision in (LG_PRECISION_FP64, LG_PRECISION_MIXED):
+        s = System.from_arrays(["Ar"] * 512, g, UnitCell.cubic(32.0), charges=np.full(512, 2.0 ** 19 - 1.0),
+                               masses=np.ones(512))
+        s.set_coulomb_potential(Ewald(9.0, kmax, 2.0))
+        s.set_precision(precision)
+        s.set_tuning(rho_width=width)
+        e.append(s.energy_terms().coulomb_kspace)
+    assert abs(e[1] - e[0]) <= 1e-11 * e[0]
