@@ -1045,7 +1045,7 @@ constexpr size_t kOctItemBytes = 4 * 64 * sizeof(double4);  // rho partials of a
 // block, the separate pass one per up to 512 atoms, so the step's are written
 // and read again from 16 atoms a block on; against that stands the separate
 // launch, which forms the phase rows anew.  us per step, in the step /
-// separate, mixed: 4096 ions kmax 9 (12 MB) 27 / 26, 12 (22 MB) 35 / 30, 16 (46
+// separate, mixed: 4096 ions kmax 9 (12 MB) 27 / 26, 12 (26 MB) 35 / 30, 16 (48
 // MB) 43 / 34; 8000 ions (32 atoms a block) kmax 9 33 / 33, 16 54 / 49; from 64
 // atoms a block on 13 824 ions kmax 12 50 / 48, 48 (1 GB) 2107 / 1910, 32 768 ions
 // kmax 16 105 / 113, with NST 0 at kmax 24 436 / 474.  Beyond 512 blocks (a narrow rho_width) the separate pass too.

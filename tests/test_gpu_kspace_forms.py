@@ -3,12 +3,16 @@ octants up to kmax 32 and, up to kmax 64, for systems of enough atoms (fewer in
 FP64); rows elsewhere.  Told apart by the launches of an MD segment without a
 thermostat: the octant form carries the half-steps between two force
 evaluations in its k-space launch, the row form has them in launches of their
-own.  Forces of either side against the oracle."""
+own.  Forces of either side against the oracle.  And both forms at the ends of
+their ranges: the octants' largest kmax, steps of more blocks than their
+partial sums are kept for, evaluations and steps in rows, in both
+precisions."""
 import numpy as np
 import pytest
 
 import lumol_oracle as lo
-from lumol_amd import Ewald, LennardJones, MolecularDynamics, PairInteraction, Simulation, System, UnitCell, VelocityVerlet
+from lumol_amd import (BerendsenThermostat, Ewald, LeapFrog, LennardJones, MolecularDynamics, PairInteraction, Simulation,
+                       System, UnitCell, VelocityVerlet)
 from lumol_amd._native import LG_PRECISION_FP64, LG_PRECISION_MIXED
 
 pytestmark = pytest.mark.gpu
@@ -51,3 +55,65 @@ def test_form(n, kmax, mixed, fp64):
         sim.run(s, 8)
         launches = s.profile_end()["integrate"][1]
         assert launches == (1 if octants else 9)
+
+
+def md(s, precision, integrator, thermostat, steps, width=0):
+    s.set_precision(precision)
+    s.set_tuning(rho_width=width)
+    prop = MolecularDynamics((LeapFrog if integrator else VelocityVerlet)(1.0))
+    if thermostat:
+        prop.set_thermostat(BerendsenThermostat(300.0, 50.0))
+    Simulation(prop).run(s, steps)
+    return s
+
+
+def check_md(make, integrator, thermostat, steps, width=0):
+    o = lo.OracleSystem(make(), nthreads=16)
+    o.md_reset()
+    o.md_run(integrator, 1.0, steps, *((300.0, 50.0) if thermostat else ()))
+    a = md(make(), LG_PRECISION_FP64, integrator, thermostat, steps, width)
+    assert np.abs(a.positions - o.positions()).max() < 1e-10
+    assert np.abs(a.velocities - o.velocities()).max() < 1e-10
+    b = md(make(), LG_PRECISION_MIXED, integrator, thermostat, steps, width)
+    assert np.abs(b.positions - a.positions).max() < 1e-6
+
+
+def check_evaluation(s):
+    o = lo.OracleSystem(s, nthreads=16)
+    fo, eo, wo = o.forces(), o.energy_terms(), o.virial()
+    scale = max(abs(eo[k]) for k in ("pairs", "coulomb", "total"))
+    for precision, bar in ((LG_PRECISION_FP64, 1e-10), (LG_PRECISION_MIXED, 1e-4)):
+        s.set_precision(precision)
+        assert np.abs(s.forces() - fo).max() <= bar * np.abs(fo).max()
+        assert abs(s.energy_terms().total - eo["total"]) <= bar * scale
+        assert np.abs(s.virial() - wo).max() <= bar * np.abs(wo).max()
+
+
+@pytest.mark.parametrize("kmax", [24, 63, 64])
+def test_largest_octants(kmax):
+    # FP64 above kmax 32: stages of 16 atoms, hundreds of item groups
+    check_evaluation(ions(2060, kmax))
+
+
+@pytest.mark.parametrize("n,kmax", [(7, 33), (65, 40), (300, 33), (48, 65)])
+def test_rows(n, kmax):
+    check_evaluation(ions(n, kmax))
+
+
+@pytest.mark.parametrize("thermostat", [False, True])
+@pytest.mark.parametrize("integrator", [0, 1])
+@pytest.mark.parametrize("n,kmax", [(65, 33), (48, 65)])
+def test_rows_md(n, kmax, integrator, thermostat):
+    check_md(lambda: ions(n, kmax), integrator, thermostat, 4)
+
+
+@pytest.mark.parametrize("thermostat", [False, True])
+def test_md_of_more_than_512_blocks(thermostat):
+    # 16 atoms a block: the half-steps do not form rho(k)
+    check_md(lambda: ions(8208, 4), 0, thermostat, 3, width=64)
+
+
+@pytest.mark.parametrize("thermostat", [False, True])
+def test_md_of_large_partial_sums(thermostat):
+    # 30 MB of them in the half-steps: rho(k) in a launch of its own
+    check_md(lambda: ions(4100, 13), 0, thermostat, 3)
