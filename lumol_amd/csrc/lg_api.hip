@@ -1407,9 +1407,10 @@ int prepare_nlist(lg_system* s) {
     // capacity from the mean density, with margin; exact sizes are checked
     // after every build (overflow flag) and grown on demand.
     size_t capacity = n;
+    double expect = double(n);  // entries of a list
     if (s->periodic && s->rlist > 0) {
         double volume = s->L[0] * s->L[1] * s->L[2];
-        double expect = 4.0 / 3.0 * kPi * s->rlist * s->rlist * s->rlist * double(n) / volume;
+        expect = 4.0 / 3.0 * kPi * s->rlist * s->rlist * s->rlist * double(n) / volume;
         capacity = size_t(std::ceil(expect * 1.5 + 64));
         capacity = std::min(capacity, n);
     }
@@ -1432,11 +1433,20 @@ int prepare_nlist(lg_system* s) {
     // lists; not fewer than 8 (1M-atom Kob-Andersen: 4 lanes 660/720 us per
     // mixed/FP64 step, 8 lanes 562/625 us; lumol_amd.tuning picks per bucket)
     s->tpa = n <= 8192 ? 64 : n <= 32768 ? 32 : n <= 131072 ? 16 : 8;
-    // lists without Coulomb pairs are short (75 entries in liquid argon), and
-    // half of 64 lanes would idle: 16 against 64 lanes 14.2 / 15.8 us per
-    // step at 7919 atoms, 20.8 / 30.4 at 32 000 (8 lanes 14.9 / 20.7); above, 8
-    // against 16 lanes 48.3 / 53.9 at 100 000
-    if (s->coul_kind == COUL_NONE) s->tpa = n <= 32768 ? std::min(s->tpa, 16) : 8;
+    // without Coulomb pairs an entry is little work, and lanes beyond those
+    // that fill the card only shorten what each has to do: 2^17 lanes in all
+    // for lists of less than 128 entries, twice that below 400 and four times
+    // from there on, at least 8 an atom.  us per step of Lennard-Jones argon,
+    // mixed, with 8 / 16 / 32 / 64 lanes, cutoff 8.5 A (68 entries): 1600 atoms 11.1 /
+    // 10.1 / 9.7 / 9.7, 8000 11.4 / 10.7 / 11.1 / 12.8, 32 000 18.5 / 20.2 / 22.7 / 29.1,
+    // 131 000 46 / 55 / 76 / 116; 12 A (193): 1600 14.7 / 11.8 / 10.4 / 10.1, 8000 14.7
+    // / 12.2 / 11.8 / 13.3, 32 000 20.8 / 20.9 / 23.4 / 29.6; 17 A (548): 1600 28.5 / 18.9
+    // / 15.0 / 13.4, 8000 24.8 / 17.5 / 15.0 / 15.7, 32 000 35.5 / 30.8 / 33.4 / 40.5
+    if (s->coul_kind == COUL_NONE) {
+        const size_t lanes = size_t(expect < 128.0 ? 1 : expect < 400.0 ? 2 : 4) << 17;
+        s->tpa = 64;
+        while (s->tpa > 8 && size_t(s->tpa) * n > lanes) s->tpa /= 2;
+    }
     if (s->tune.pair_lanes > 0) s->tpa = s->tune.pair_lanes;
     if (s->gen_pairs) s->tpa = 16;  // the general pair kernel has one instance
     LG_TRY(s->epart_pairs.ensure(size_t(pair_blocks_of(n, s->tpa)) * 8));
@@ -1700,8 +1710,9 @@ int launch_nlist(lg_system* s, bool check) {
             s->slot_rows ? s->rank.p : nullptr, cell_tags(s));
     }
     // the build by lanes pays for each run of cells once per lane group: 4
-    // lanes against 8, 10^6 Kob-Andersen atoms: 314 / 328 us per step, 36 000
-    // atoms (too few waves) 28.3 / 27.9
+    // lanes against 8, 10^6 Kob-Andersen atoms: 314 / 328 us per step, argon of
+    // 150 000 and 300 000 atoms 50.9 / 50.2 and 82.8 / 85.3 (cutoff 8.5 A), 62.5 /
+    // 63.8 and 137.6 / 140.0 (12 A), 36 000 atoms (too few waves) 28.3 / 27.9
     const int lanes = s->tune.pair_lanes == 0 && n > 131072 ? std::min(s->tpa, 4) : s->tpa;
     int nb = blocks_for(size_t(n) * lanes, 256);
     // FP32 candidate test with a 1e-4 relative margin on rlist

@@ -63,3 +63,18 @@ def test_trajectory(case):
         Simulation(MolecularDynamics(VelocityVerlet(2.0))).run(s, 60)
         out.append(s.positions.copy())
     assert np.abs(out[0] - out[1]).max() < 1e-8
+
+
+# atoms of argon's density, cutoff, lanes per atom: by the entries of a list
+# (24, 68, 193, 548 at 6, 8.5, 12, 17 A) and the lanes that fill the card
+@pytest.mark.parametrize("n,rc,lanes", [(1600, 8.5, 64), (1600, 17.0, 64), (4000, 8.5, 32), (4000, 12.0, 64),
+                                        (4000, 17.0, 64), (8000, 8.5, 16), (8192, 6.0, 16), (8193, 6.0, 8),
+                                        (8000, 12.0, 32), (8000, 17.0, 64), (32000, 8.5, 8), (32000, 17.0, 16),
+                                        (50000, 8.5, 8)])
+def test_lanes_without_coulomb(n, rc, lanes):
+    s = fluid(n, [(n / 0.02115) ** (1.0 / 3.0)] * 3, rc)
+    assert s.tuning()["pair_lanes"] == lanes
+    if n <= 8193:
+        f, fo = s.forces(), lo.OracleSystem(s, nthreads=8).forces()
+        assert np.abs(f - fo).max() <= 1e-10 * np.abs(fo).max()
+
