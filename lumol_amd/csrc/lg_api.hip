@@ -1310,7 +1310,8 @@ double max_cutoff(lg_system* s) {
 }
 
 constexpr size_t kDirectMax = 32768;  // atoms of the direct list build
-constexpr int kDenseCells = 27;       // cells of the per-cell list builds
+constexpr int kDenseCells = 27;       // cells of the per-cell list builds; above kDirectMax, where
+                                      // a cell has one workgroup, 128
 
 // Neighbour-list maintenance.  `check` runs the displacement test here; the
 // MD step does it inside the integrator's first half instead.  Every kernel
@@ -1330,7 +1331,7 @@ static bool direct_fits(const lg_system* s) {
     return s->n <= kDirectMax && s->grid.n[0] <= 1023 && s->grid.n[1] <= 1023 && s->grid.n[2] <= 1023;
 }
 static bool cells_dense(const lg_system* s) {
-    return s->grid.ncell >= kDenseCells && s->n >= size_t(8) * s->grid.ncell;
+    return s->grid.ncell >= (s->n <= kDirectMax ? kDenseCells : 128) && s->n >= size_t(8) * s->grid.ncell;
 }
 static bool direct_build(const lg_system* s) {
     if (!direct_fits(s)) return false;

@@ -78,3 +78,10 @@ def test_lanes_without_coulomb(n, rc, lanes):
         f, fo = s.forces(), lo.OracleSystem(s, nthreads=8).forces()
         assert np.abs(f - fo).max() <= 1e-10 * np.abs(fo).max()
 
+
+def test_few_large_cells():
+    # 36 cells: workgroups per cell up to the direct build's largest system,
+    # lanes per atom above it, where a cell has one workgroup
+    for n, build in ((3000, 3), (33000, 1)):
+        s = fluid(n, (30.0, 30.0, 24.0), 9.0)
+        assert s.tuning()["nlist_build"] == build
