@@ -1,8 +1,8 @@
 """Per-size-bucket autotuner of the device launch knobs.
 
 The knobs (``lg_tuning``): lanes per atom of the pair and neighbour-list
-kernels, row ranges of the k-space force kernel, the form of the rho(k)
-kernel (rows, with its atoms per block, or the matrix cores).  They are
+kernels, atoms per block of the rho(k) kernel, and row ranges of the k-space
+force kernel where the row form may run (kmax above 32).  They are
 tuned one after the other: every candidate value is timed with the
 library's HIP-event profiler over `reps` force evaluations of the system
 itself, in `rounds` interleaved passes of which the fastest counts -- the
@@ -21,10 +21,13 @@ import time
 from . import _native as nat
 
 PAIR_LANES = (8, 16, 32, 64)
-KSPACE_SPLITS = (2, 4, 8, 16, 32)
+# row ranges of the k-space forces: the octant form, the only one up to kmax
+# 32, does not use them, so there is nothing to choose (8 is its report)
+KSPACE_SPLITS = (8,)
+ROW_KSPACE_SPLITS = (2, 4, 8, 16, 32)
 RHO_WIDTHS = (64, 128, 192, 256, 512)
 NLIST_BUILDS = (0, 2)  # automatic, cell list (lg_tuning.nlist_build)
-RHO_KINDS = (1, 2, 3)  # one octant form now (lg_tuning.rho_kind); timed as before for saved choices
+RHO_KINDS = (1,)  # one form, whatever the value (lg_tuning.rho_kind); saved choices of 2 and 3 are accepted
 
 _cache = {}
 _lock = threading.Lock()
@@ -36,6 +39,10 @@ def bucket(system):
     nk = system.ewald_kvector_count() if ewald else 0
     p2 = lambda x: 0 if x <= 0 else 1 << int(math.ceil(math.log2(x)))
     return (ewald, int(system.precision), p2(n), p2(nk))
+
+
+def _splits(system):
+    return KSPACE_SPLITS if system.coulomb.kmax <= 32 else ROW_KSPACE_SPLITS
 
 
 def _time_all(system, reps, classes=None, step=None):
@@ -60,10 +67,10 @@ def _time_all(system, reps, classes=None, step=None):
 _KNOB_CLASSES = {
     "pair_lanes": ("nlist", "pairs"),
     "kspace_split": ("kspace_force",),
-    "rho_width": ("kspace_rho", "pairs"),  # the rho reduction runs in the pair launch
-    "rho_kind": ("kspace_rho", "pairs"),
+    # the rho reduction runs in the pair launch, and the atoms per block of the
+    # octant forces follow the width
+    "rho_width": ("kspace_rho", "pairs", "kspace_force"),
 }
-
 
 
 def autotune(system, reps=5, use_cache=True, rounds=3, step=None):
@@ -92,39 +99,25 @@ def autotune(system, reps=5, use_cache=True, rounds=3, step=None):
         warm()  # builds the lists and tables once
         best = {"pair_lanes": 0, "kspace_split": 0, "rho_width": 0, "rho_kind": 0}
 
-        def pick(field, values, **extra):
+        def pick(field, values):
             # each candidate timed in `rounds` interleaved passes, the
             # fastest pass kept: a single short timing flips the choice
             # between runs on small systems
+            if len(values) == 1:
+                return values[0]
             times = {v: float("inf") for v in values}
             for _ in range(rounds):
                 for v in values:
-                    trial = dict(best, **{field: v}, **extra)
-                    apply(trial)
+                    apply(dict(best, **{field: v}))
                     warm()
                     times[v] = min(times[v], _time_all(system, reps, classes[field], step))
-            return min(times, key=times.get), times
+            return min(times, key=times.get)
 
-        # pair kernel lanes
-        best["pair_lanes"], _ = pick("pair_lanes", PAIR_LANES)
+        best["pair_lanes"] = pick("pair_lanes", PAIR_LANES)
         if key[0]:
-            best["kspace_split"], _ = pick("kspace_split", KSPACE_SPLITS)
-            # rho(k): each width of the row form, then at the best width
-            # the row form without its LDS staging, then the matrix-core form
-            width, times = pick("rho_width", RHO_WIDTHS, rho_kind=1)
-            kind, t_kind = 1, times[width]
-            for k in (3, 2):
-                trial = dict(best, rho_width=width if k != 2 else 0, rho_kind=k)
-                apply(trial)
-                warm()
-                t = float("inf")
-                if system.tuning()["rho_kind"] == k:
-                    for _ in range(rounds):
-                        t = min(t, _time_all(system, reps, classes["rho_kind"], step))
-                if t < t_kind:
-                    kind, t_kind = k, t
-            best["rho_kind"] = kind
-            best["rho_width"] = width if kind != 2 else 0
+            best["kspace_split"] = pick("kspace_split", _splits(system))
+            best["rho_kind"] = RHO_KINDS[0]
+            best["rho_width"] = pick("rho_width", RHO_WIDTHS)
         hit = best
         with _lock:
             _cache[key] = hit
@@ -138,10 +131,10 @@ def autotune_concurrent(systems, run, rounds=2, passes=2):
     not those for several sharing the device (four SPC/E systems: wider rho
     blocks).  `run()` advances every system by the same fixed work,
     concurrently, and returns its wall time.  The knobs are chosen in turn
-    (the list build, pair lanes, then the k-space split, rho width and rho
-    form; `passes` rounds of this coordinate descent), every candidate timed
-    in `rounds` interleaved passes and the fastest pass kept.  Returns the
-    knobs (dict)."""
+    (the list build, pair lanes, then the k-space split and rho width;
+    `passes` rounds of this coordinate descent), every candidate timed in
+    `rounds` interleaved passes and the fastest pass kept.  Returns the knobs
+    (dict)."""
     graphs = [getattr(s, "tuning_", (0, 0, 0, 0, 0, 0))[4] for s in systems]
     best = {"pair_lanes": 0, "kspace_split": 0, "rho_width": 0, "nlist_build": 0, "rho_kind": 0}
 
@@ -157,9 +150,7 @@ def autotune_concurrent(systems, run, rounds=2, passes=2):
     # more launch per step
     fields = [("nlist_build", NLIST_BUILDS), ("pair_lanes", PAIR_LANES)]
     if bucket(systems[0])[0]:
-        # the matrix-core rho(k) leaves the vector ALU to the other systems'
-        # kernels: it can win in a batch where it loses alone
-        fields += [("kspace_split", KSPACE_SPLITS), ("rho_width", RHO_WIDTHS), ("rho_kind", RHO_KINDS)]
+        fields += [("kspace_split", _splits(systems[0])), ("rho_width", RHO_WIDTHS), ("rho_kind", RHO_KINDS)]
     # coordinate descent, `passes` times over the knobs: the first pass
     # tunes each knob with the later ones still at their built-in choice
     for _ in range(passes):

@@ -104,3 +104,25 @@ def test_autotune_concurrent_applies_one_choice():
         s.set_tuning(pair_lanes=best["pair_lanes"], kspace_split=best["kspace_split"], rho_width=best["rho_width"],
                      nlist_build=best["nlist_build"], rho_kind=best["rho_kind"])
         assert frel(s.forces(), f) < 1e-12
+
+
+def test_autotune_times_only_what_differs():
+    # up to kmax 32 the k-space split has no effect and all kinds of rho(k) are
+    # one form: timing them would let noise choose
+    from lumol_amd import MolecularDynamics, Simulation, VelocityVerlet
+    s = spce(nmol=300, L=20.8, cutoff=8.0, kmax=7, seed=14)
+    sim = Simulation(MolecularDynamics(VelocityVerlet(0.5)))
+    calls = []
+
+    def step():
+        sim.run(s, 2)
+        calls.append(1)
+
+    best = tuning.autotune(s, use_cache=False, rounds=1, step=step)
+    # one call before, then a call to warm up and a timed one per candidate
+    assert len(calls) == 1 + 2 * (len(tuning.PAIR_LANES) + len(tuning.RHO_WIDTHS))
+    assert best["rho_kind"] == 1 and best["rho_width"] in tuning.RHO_WIDTHS
+    # choices saved when there were more are accepted
+    for kind in (2, 3):
+        s.set_tuning(best["pair_lanes"], 16, 128, rho_kind=kind)
+        assert np.isfinite(s.forces()).all() and s.tuning()["rho_kind"] == kind
