@@ -41,6 +41,12 @@ def bucket(system):
     return (ewald, int(system.precision), p2(n), p2(nk))
 
 
+def _lanes(system):
+    """Without Coulomb also the built-in choice: it takes small systems'
+    steps without a list, which any set value keeps."""
+    return PAIR_LANES if bucket(system)[0] else (0,) + PAIR_LANES
+
+
 def _splits(system):
     return KSPACE_SPLITS if system.coulomb.kmax <= 32 else ROW_KSPACE_SPLITS
 
@@ -113,7 +119,7 @@ def autotune(system, reps=5, use_cache=True, rounds=3, step=None):
                     times[v] = min(times[v], _time_all(system, reps, classes[field], step))
             return min(times, key=times.get)
 
-        best["pair_lanes"] = pick("pair_lanes", PAIR_LANES)
+        best["pair_lanes"] = pick("pair_lanes", _lanes(system))
         if key[0]:
             best["kspace_split"] = pick("kspace_split", _splits(system))
             best["rho_kind"] = RHO_KINDS[0]
@@ -148,7 +154,7 @@ def autotune_concurrent(systems, run, rounds=2, passes=2):
     # cell-list build, whose rebuilds cost the vector ALU less (the direct
     # build reads every atom's cell tag in every cell's workgroup) at one
     # more launch per step
-    fields = [("nlist_build", NLIST_BUILDS), ("pair_lanes", PAIR_LANES)]
+    fields = [("nlist_build", NLIST_BUILDS), ("pair_lanes", _lanes(systems[0]))]
     if bucket(systems[0])[0]:
         fields += [("kspace_split", _splits(systems[0])), ("rho_width", RHO_WIDTHS), ("rho_kind", RHO_KINDS)]
     # coordinate descent, `passes` times over the knobs: the first pass

@@ -126,3 +126,17 @@ def test_autotune_times_only_what_differs():
     for kind in (2, 3):
         s.set_tuning(best["pair_lanes"], 16, 128, rho_kind=kind)
         assert np.isfinite(s.forces()).all() and s.tuning()["rho_kind"] == kind
+
+
+def test_autotune_leaves_small_steps():
+    # a set number of lanes keeps the list kernels: without Coulomb the tuner
+    # has the built-in choice, steps of one launch, among its candidates
+    from lumol_amd import MolecularDynamics, Simulation, VelocityVerlet
+    from lumol_amd.workloads import argon
+    s = argon(ncell=4, cutoff=8.5)
+    sim = Simulation(MolecularDynamics(VelocityVerlet(1.0)))
+    best = tuning.autotune(s, use_cache=False, rounds=3, step=lambda: sim.run(s, 200))
+    s.profile_begin(["nlist", "pairs", "integrate"])
+    sim.run(s, 20)
+    launches = {k: n for k, (_, n) in s.profile_end().items()}
+    assert best["pair_lanes"] == 0 and launches["pairs"] == 0 and launches["integrate"] == 20
