@@ -1867,12 +1867,8 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
         rr.epart = epk;
     }
     const bool intra_apart = !s->gen_pairs;
-    if (intra_apart && iblocks > 0 && !intra_done && energy) {
-        if (energy)
-            launch_timed(s, LG_KERNEL_MOLECULES, k_intra_terms<true>, iblocks, 256, 0, ia);
-        else
-            launch_timed(s, LG_KERNEL_MOLECULES, k_intra_terms<false>, iblocks, 256, 0, ia);
-    }
+    if (intra_apart && iblocks > 0 && !intra_done && energy)
+        launch_timed(s, LG_KERNEL_MOLECULES, k_intra_terms, iblocks, 256, 0, ia);
     const int pblocks = pair_blocks_of(size_t(n), s->tpa);
     pa.pair_blocks = pblocks;
     pa.intra_blocks = intra_apart && energy ? 0 : iblocks;

@@ -128,19 +128,6 @@ __device__ __forceinline__ void min_image(const Box& b, double& dx, double& dy, 
 // image1 without its check of near-halves (see PairArgs.tie).
 __device__ __forceinline__ double image_rint(double d, double L, double inv) { return d - rint(d * inv) * L; }
 
-// Minimum image for the mixed form, whose distance is rounded to FP32 next:
-// d - rint(d / a) a with the reciprocal, 3 operations per axis.  It differs
-// from image1 only for |d| within ulps of a half box length, where both
-// images are equally near and, the cutoff being at most half the box, no
-// pair within it lies.
-__device__ __forceinline__ void min_image_fast(const Box& b, double& dx, double& dy, double& dz) {
-    if (b.periodic) {
-        dx -= rint(dx * b.inv[0]) * b.L[0];
-        dy -= rint(dy * b.inv[1]) * b.L[1];
-        dz -= rint(dz * b.inv[2]) * b.L[2];
-    }
-}
-
 // Vector3D::norm2 order: x*x + y*y + z*z, left to right, unfused.
 __device__ __forceinline__ double norm2_ordered(double x, double y, double z) {
     double a = x * x;

@@ -1259,10 +1259,8 @@ __device__ __forceinline__ void intra_block(const IntraArgs& a, int blk) {
     }
 }
 
-template <bool kEnergy>
-__global__ __launch_bounds__(256) void k_intra_terms(IntraArgs a) {
-    intra_block<kEnergy>(a, blockIdx.x);
-}
+// The terms with their energies alone.
+__global__ __launch_bounds__(256) void k_intra_terms(IntraArgs a) { intra_block<true>(a, blockIdx.x); }
 
 // Per k-vector record of the force kernels: rho(k) (written by
 // k_rho_reduce) and g = 2 factor_k, gz = g * ikz.  The reference's force
@@ -2309,14 +2307,11 @@ __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
 // with L mod 8 == by mod 8, so all blocks that read row by's data (an atom
 // chunk of the phase table) share one L2 and the chunk is fetched from HBM
 // once.  False for the padding blocks (whole block; call before any barrier).
-__device__ __forceinline__ bool xcd_block_at(int L, int gx, int gy, int& bx, int& by) {
-    int q = L >> 3;
+__device__ __forceinline__ bool xcd_block(int gx, int gy, int& bx, int& by) {
+    const int L = blockIdx.x, q = L >> 3;
     by = (q / gx) * 8 + (L & 7);
     bx = q - (q / gx) * gx;
     return by < gy;
-}
-__device__ __forceinline__ bool xcd_block(int gx, int gy, int& bx, int& by) {
-    return xcd_block_at(blockIdx.x, gx, gy, bx, by);
 }
 __host__ __forceinline__ unsigned xcd_grid(int gx, int gy) { return unsigned(gx) * unsigned((gy + 7) / 8 * 8); }
 
@@ -3300,9 +3295,5 @@ __global__ __launch_bounds__(512, 2) void k_oct_step(OctForce a, OctStep s, OctR
     }
 }
 #pragma clang fp contract(on)
-
-__global__ void k_set_scalar(double* __restrict__ p, double v) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
-}
 
 }  // namespace lg
