@@ -309,7 +309,8 @@ int lg_mc_run_batch(lg_system* const* systems, size_t count, const uint64_t* see
  *                 per cell over the atoms' cell tags, no cell list (up to
  *                 32768 atoms; a box of fewer than 256 cells deals each
  *                 cell's home atoms to up to 8 workgroups).  Default: 3 when
- *                 there are >= 27 cells and >= 8 atoms per cell and it
+ *                 there are >= 27 cells (128 above 32768 atoms) and
+ *                 >= 8 atoms per cell and it
  *                 applies, else 2 there, else 1
  *   md_graph      lg_md_run: 1 (default) launches every kernel; 2 captures a
  *                 chunk of steps in a HIP graph once and replays it (eager

@@ -1313,20 +1313,13 @@ constexpr size_t kDirectMax = 32768;  // atoms of the direct list build
 constexpr int kDenseCells = 27;       // cells of the per-cell list builds; above kDirectMax, where
                                       // a cell has one workgroup, 128
 
-// Neighbour-list maintenance.  `check` runs the displacement test here; the
-// MD step does it inside the integrator's first half instead.  Every kernel
-// returns at once when flags[0] (rebuild) is clear; the build kernel clears
-// it again.
-// Which list-build kernel runs: one workgroup per cell (k_nlist_cells) when
-// there are enough cells to fill the device and enough atoms per cell to keep
-// its waves busy, else TPA lanes per atom (k_nlist_build); the tuning knob
-// nlist_build overrides (1 lanes per atom, 2 cells).
-// Verlet build: 1 lanes per atom over the cell list, 2 one workgroup per
-// cell over the cell list, 3 workgroups per cell (direct_split) over the
-// atoms' cell tags (no cell list; up to 32768 atoms and 1023 cells per axis).  Default:
-// the per-cell builds when there are >= 27 cells (kDenseCells; argon of 1600
-// atoms in 64 cells: 18.0 us per step by lanes, 13.8 direct) and >= 8 atoms
-// per cell, the direct one where it applies.
+// Which list build runs (the knob nlist_build overrides): 1 lanes per atom
+// over the cell list (k_nlist_build), 2 one workgroup per cell over the cell
+// list (k_nlist_cells), 3 workgroups per cell (direct_split) over the atoms'
+// cell tags (k_nlist_direct; no cell list; up to 32768 atoms and 1023 cells
+// per axis).  Default: the per-cell builds when there are cells enough
+// (cells_dense; argon of 1600 atoms in 64 cells: 18.0 us per step by lanes,
+// 13.8 direct) and 8 atoms or more in one, the direct one where it applies.
 static bool direct_fits(const lg_system* s) {
     return s->n <= kDirectMax && s->grid.n[0] <= 1023 && s->grid.n[1] <= 1023 && s->grid.n[2] <= 1023;
 }
@@ -1663,6 +1656,10 @@ static IntraArgs intra_args(lg_system* s) {
     return ia;
 }
 
+// Neighbour-list maintenance.  `check` runs the displacement test here; the
+// MD step does it inside the integrator's first half instead.  Every kernel
+// returns at once when flags[0] (rebuild) is clear; the pair kernel that
+// follows clears it again.
 int launch_nlist(lg_system* s, bool check) {
     hipStream_t st = S(s);
     // profiled intervals only around launches (an empty event pair would

@@ -79,7 +79,7 @@ __host__ __device__ __forceinline__ int cell_coord(double x, double L, double in
 
 // Cell coordinates of every atom for the direct Verlet build, written by the
 // kernels that see each new position (the displacement test, the first half
-// of an MD step): cx | cy << 10 | cz << 20 (cells per axis <= 256).  Off
+// of an MD step): cx | cy << 10 | cz << 20 (cells per axis <= 1023).  Off
 // when tag is null.
 // What the MD half-steps write beside a new position: the cell tag of the
 // direct Verlet build (tag, or null) and the position as the mixed pair
