@@ -2790,7 +2790,8 @@ __global__ void k_energy_gather(const double* __restrict__ pp, int nbp, const do
 // tables, of at most small_max atoms.  A set knob of the list kernels keeps
 // the list.
 static bool small_steps(const lg_system* s) {
-    return s->n <= size_t(small_max(s->precision == LG_PRECISION_MIXED)) && !s->gen_pairs && s->nterms == 0 &&
+    const bool wolf = coulomb_variant(s->coul) == CK_WOLF;
+    return s->n <= size_t(small_max(s->precision == LG_PRECISION_MIXED, wolf)) && !s->gen_pairs && s->nterms == 0 &&
            s->nmol == int(s->n) &&
            (s->coul_kind == COUL_NONE ||
             (s->coul_kind == COUL_WOLF &&

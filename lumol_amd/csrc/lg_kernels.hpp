@@ -2888,7 +2888,12 @@ struct SmallArgs {
 // costs more than the list's launches.  us per step, list / one launch:
 // FP64 1024 atoms 13.6 / 9.4, 1200 13.9 / 18.1 (its blocks pass the 256
 // compute units); mixed 1500 13.8 / 11.3, 2048 13.8 / 13.7.
-constexpr int small_max(bool mixed) { return mixed ? 1536 : 1024; }
+// Wolf pairs cost half as much again: 200 steps in one call, list / one launch,
+// mixed 1100 atoms 9.4 / 11.4, 1500 atoms 9.5 / 13.4 on a host that launches in
+// 3 us (12.4 for the list where it takes 4); FP64 800 atoms 9.4 / 10.6, 1000
+// 9.4 / 11.7; a call of one step 50 / 37 us at any of these sizes.
+// Its lines lie between those of long calls on a fast host and of short ones.
+constexpr int small_max(bool mixed, bool wolf) { return wolf ? (mixed ? 1200 : 900) : mixed ? 1536 : 1024; }
 // The same for the loop, one launch per step / loop: FP64 64 atoms 4.6 / 3.4,
 // 80 atoms 4.8 / 5.2; mixed 96 atoms 4.8 / 3.8, 112 atoms 4.9 / 4.8.
 constexpr int small_loop_max(bool mixed) { return mixed ? 96 : 64; }
@@ -2933,7 +2938,7 @@ __global__ __launch_bounds__(kLoop ? 1024 : 256) void k_small_step(SmallArgs a) 
     typedef typename std::conditional<kMixed, float4, double4>::type T4;
     typedef typename std::conditional<kMixed, float2, double2>::type T2;
     constexpr int BLOCK = kLoop ? 1024 : 256, TPA = kLoop ? (kMixed ? 8 : 16) : 64, OWN = BLOCK / TPA;
-    constexpr int NMAX = kLoop ? small_loop_max(kMixed) : small_max(kMixed);
+    constexpr int NMAX = kLoop ? small_loop_max(kMixed) : small_max(kMixed, CK == CK_WOLF);
     // positions: fixed-point fractions (or FP32 coordinates) and charge in the
     // mixed form, coordinates in FP64
     __shared__ float4 xf[kMixed ? NMAX : 1];

@@ -100,3 +100,19 @@ def test_energy_after_steps():
     o = lo.OracleSystem(s, nthreads=8)
     assert abs(s.potential_energy() - o.potential_energy()) <= 1e-10 * abs(o.potential_energy())
     assert np.abs(s.forces() - o.forces()).max() <= 1e-10 * np.abs(o.forces()).max()
+
+
+@pytest.mark.parametrize("n,wolf,mixed,small", [(900, True, False, True), (901, True, False, False), (1200, True, True, True),
+                                                (1201, True, True, False), (1024, False, False, True),
+                                                (1536, False, True, True), (1537, False, True, False)])
+def test_line_between_the_paths(n, wolf, mixed, small):
+    s = system(n, wolf)
+    if mixed:
+        s.set_precision(LG_PRECISION_MIXED)
+    sim = dynamics()
+    sim.run(s, 1)
+    s.profile_begin(["pairs"])
+    sim.run(s, 5)
+    assert (s.profile_end()["pairs"][1] == 0) == small
+    if wolf:
+        check(system(n, wolf), mixed)
