@@ -302,8 +302,7 @@ def roofline_of(prof, steps, workload, form, natoms, n_pairs, nk, batch=1, timin
     bound, work, peak, unit, per = class_work(dom, workload, form, natoms, n_pairs, nk, batch)
     achieved = work / avg_s
     return {"bound": bound, "achieved": achieved, "peak": peak, "unit": unit, "frac": achieved / peak,
-            # the committed counters of the k-space classes are of other kernels
-            "traffic": load_traffic(workload, form, dom) if dom == "pairs" else None, "kernel": dom, "avg_launch_us": avg_s * 1e6,
+            "traffic": load_traffic(workload, form, dom), "kernel": dom, "avg_launch_us": avg_s * 1e6,
             "launches": launches, "work": per, "timing": timing}, {c: round(v, 2) for c, v in per_step.items()}
 
 

@@ -243,7 +243,7 @@ __global__ void k_cell_scatter(const int* __restrict__ cellid, const int* __rest
 // that order.  The atoms of a run of cells then lie in a row, and a wave's
 // gather touches a few cache lines instead of one per lane: 10^6 Kob-Andersen
 // atoms, mixed, pair kernel 363 -> 215 us (its
-// address units are busy 80% of that, its arithmetic 60%).  The copies and the atoms'
+// address units are busy 74% of that, its arithmetic 56%).  The copies and the atoms'
 // places (rank) are rewritten here with the order.
 constexpr int kRankBlocks = 4096;
 __global__ __launch_bounds__(256) void k_cell_rank(const int* __restrict__ tmp, const int* __restrict__ start,
@@ -1478,7 +1478,7 @@ __device__ __forceinline__ void pair_extra_block(const PairArgs& a, unsigned cha
 // Relative error of the force factor against 128 bits, rms over distances
 // from 1.5 A to a cutoff of 9 A, reference's order / this: Lennard-Jones 3.5
 // to 13e-16 / 1.6 to 4.3e-16, Ewald at alpha rc = pi 1.8 to 9.5e-16 / 1.4 to
-// 4.6e-16.  SPC/E, 9000 atoms: 41 -> 21 us per launch against the
+// 4.6e-16.  SPC/E, 9000 atoms: 41 -> 22 us per launch against the
 // reference's order with library root, division and exponential.
 template <bool kEnergy, int TPA, int CK, bool kIntra = false>
 __global__ __launch_bounds__(kPairBlock)
