@@ -408,6 +408,8 @@ struct lg_system {
     DevBuf<KRow> rows;
     // octant form (oct_pays): (p, q) pairs and their row tiles, work items of
     // the rho pass, output tiles, k map, force coefficients, partials
+    std::vector<int4> oct_idx;  // the k set of the tables, for oct_kmax
+    int oct_kmax = 0;
     int oct_nrt = 0, oct_nst = 0, oct_steps = 0, oct_zcols = 0, oct_nitems = 0, oct_ntiles = 0;
     int oct_width = 0, oct_nchunks = 0, oct_ngroups = 0, oct_ipg = 0, oct_asplit = 1;
     int rho_nchunks = 0;  // partial sums of the last rho pass
@@ -1058,21 +1060,21 @@ static bool oct_step_rho(const lg_system* s, bool mixed) {
 // (ikx, |iky|) sorted by how many ikz they need, row tiles of four pairs,
 // work items of four output tiles, and for every output column of a tile the
 // k-vectors it completes.
-static int prepare_octants(lg_system* s, const std::vector<int4>& idx) {
-    std::map<std::pair<int, int>, int> extent;  // pair -> largest |ikz| + 1
-    for (const int4& k : idx) {
-        int& z = extent[{k.x, std::abs(k.y)}];
-        z = std::max(z, std::abs(k.z) + 1);
-    }
+static int octant_tables(lg_system* s, const std::vector<int4>& idx) {
+    const int K1 = s->coul_kmax + 1;
+    auto pq = [&](const int4& k) { return size_t(k.x) * K1 + std::abs(k.y); };
+    std::vector<int> extent(size_t(K1) * K1, 0);  // by pair: largest |ikz| + 1
+    for (const int4& k : idx) extent[pq(k)] = std::max(extent[pq(k)], std::abs(k.z) + 1);
     std::vector<std::array<int, 3>> pairs;  // extent, p, q
-    for (auto& [pq, z] : extent) pairs.push_back({z, pq.first, pq.second});
+    for (int j = 0; j < K1 * K1; j++)
+        if (extent[j] > 0) pairs.push_back({extent[j], j / K1, j % K1});
     std::stable_sort(pairs.begin(), pairs.end(), [](auto& a, auto& b) { return a[0] > b[0]; });
     const int nrt = int((pairs.size() + 3) / 4);
     std::vector<int> opairs(size_t(nrt) * 4, 0), steps(nrt), ncol(nrt);
-    std::map<std::pair<int, int>, int> at;
+    std::vector<int> at(size_t(K1) * K1, 0);
     for (size_t j = 0; j < pairs.size(); j++) {
         opairs[j] = pairs[j][1] | pairs[j][2] << 16;
-        at[{pairs[j][1], pairs[j][2]}] = int(j);
+        at[size_t(pairs[j][1]) * K1 + pairs[j][2]] = int(j);
     }
     for (int t = 0; t < nrt; t++) {
         const int z = pairs[size_t(t) * 4][0];
@@ -1118,13 +1120,12 @@ static int prepare_octants(lg_system* s, const std::vector<int4>& idx) {
     for (size_t e = 0; e < slots.size(); e++) tile_of[size_t(slots[e].y) * ncol[0] + slots[e].z] = int(e);
     std::vector<int> kmap(slots.size() * 4 * 16 * 2, -1);
     for (size_t k = 0; k < idx.size(); k++) {
-        const int j = at[{idx[k].x, std::abs(idx[k].y)}], r = std::abs(idx[k].z);
+        const int j = at[pq(idx[k])], r = std::abs(idx[k].z);
         const int e = tile_of[size_t(j / 4) * ncol[0] + r / 8];
         const int col = 2 * (r % 8) + (idx[k].z < 0 ? 1 : 0);
         kmap[((size_t(e) * 4 + j % 4) * 16 + col) * 2 + (idx[k].y < 0 ? 1 : 0)] = int(k);
     }
     // the X and Y phase rows of every matrix row of an item (see OctRho)
-    const int K1 = s->coul_kmax + 1;
     std::vector<int4> rows32, rows64;
     for (const OctItem& it : items)
         for (int i = 0; i < 16; i++) {
@@ -1152,21 +1153,6 @@ static int prepare_octants(lg_system* s, const std::vector<int4>& idx) {
     s->oct_steps = steps[0];  // of the longest row
     s->oct_nitems = int(items.size());
     s->oct_ntiles = int(slots.size());
-    // about one block per CU: the widest chunk of atoms (fewer partial sums),
-    // then fewer items per block (their waves share the atoms), then narrower
-    // chunks
-    const int nitems = int(items.size());
-    int ng = blocks_for(nitems, 8), w = 512;
-    auto blocks = [&]() { return ng * blocks_for(s->n, w); };
-    while (w > 128 && blocks() < 200) w -= 64;
-    while (ng < nitems && 2 * ng <= blocks_for(nitems, 2) && blocks() < 128) ng *= 2;
-    while (w > 64 && blocks() < 128) w -= 64;
-    if (s->tune.rho_width > 0) w = s->tune.rho_width;
-    s->oct_ipg = blocks_for(nitems, ng);
-    s->oct_ngroups = blocks_for(nitems, s->oct_ipg);
-    s->oct_asplit = 8 / s->oct_ipg;
-    s->oct_width = w;
-    s->oct_nchunks = blocks_for(s->n, w);
     hipStream_t st = S(s);
     LG_TRY(upload(s->opairs, opairs, st));
     LG_TRY(upload(s->osteps, steps, st));
@@ -1179,6 +1165,36 @@ static int prepare_octants(lg_system* s, const std::vector<int4>& idx) {
     const std::vector<double> zero(size_t(nrt) * s->oct_nst * 64, 0.0);
     LG_TRY(upload(s->ocoef64, zero, st));
     LG_TRY(upload(s->ocoef32, std::vector<float>(zero.size(), 0.f), st));
+    LG_HIP(hipStreamSynchronize(st));  // the tables above are local
+    return LG_OK;
+}
+
+// The tables follow from the k set alone.  A cell that changes by little (a
+// barostat's steps) keeps it, and then only the launch shape is looked at.
+static int prepare_octants(lg_system* s, const std::vector<int4>& idx) {
+    const bool same = s->oct_kmax == s->coul_kmax && s->oct_idx.size() == idx.size() &&
+                      std::memcmp(s->oct_idx.data(), idx.data(), idx.size() * sizeof(int4)) == 0;
+    if (!same) {
+        s->oct_kmax = 0;
+        LG_TRY(octant_tables(s, idx));
+        s->oct_idx = idx;
+        s->oct_kmax = s->coul_kmax;
+    }
+    // about one block per CU: the widest chunk of atoms (fewer partial sums),
+    // then fewer items per block (their waves share the atoms), then narrower
+    // chunks
+    const int nitems = s->oct_nitems;
+    int ng = blocks_for(nitems, 8), w = 512;
+    auto blocks = [&]() { return ng * blocks_for(s->n, w); };
+    while (w > 128 && blocks() < 200) w -= 64;
+    while (ng < nitems && 2 * ng <= blocks_for(nitems, 2) && blocks() < 128) ng *= 2;
+    while (w > 64 && blocks() < 128) w -= 64;
+    if (s->tune.rho_width > 0) w = s->tune.rho_width;
+    s->oct_ipg = blocks_for(nitems, ng);
+    s->oct_ngroups = blocks_for(nitems, s->oct_ipg);
+    s->oct_asplit = 8 / s->oct_ipg;
+    s->oct_width = w;
+    s->oct_nchunks = blocks_for(s->n, w);
     size_t sets = size_t(s->oct_nchunks);
     for (int m = 0; m < 2; m++)
         if (oct_step_rho(s, m == 1)) sets = std::max(sets, size_t(blocks_for(s->n, oct_step_atoms(s, m == 1))));
@@ -1186,7 +1202,6 @@ static int prepare_octants(lg_system* s, const std::vector<int4>& idx) {
     LG_TRY(s->epart_k.ensure(size_t(s->oct_ntiles) * 4 * 7));
     s->ksplit = s->tune.kspace_split > 0 ? s->tune.kspace_split : 8;
     LG_TRY(s->fk.ensure(s->n));
-    LG_HIP(hipStreamSynchronize(st));  // the tables above are local
     return LG_OK;
 }
 

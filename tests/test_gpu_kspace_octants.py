@@ -127,3 +127,31 @@ def test_mixed_sums_hold_32_atoms(kmax, width):
         s.set_tuning(rho_width=width)
         e.append(s.energy_terms().coulomb_kspace)
     assert abs(e[1] - e[0]) <= 1e-11 * e[0]
+
+
+def test_tables_follow_the_k_set():
+    # the octant tables are kept while the k set stays: cells that scale, cells
+    # that change its members, another kmax, launch shape and precision
+    s = ions(300, (20.0, 24.0, 31.0), 9)
+
+    def same(bar=1e-10):
+        o = lo.OracleSystem(s, nthreads=8)
+        f, fo = s.forces(), o.forces()
+        assert np.abs(f - fo).max() < bar * np.abs(fo).max()
+        w, wo = s.virial(), o.virial()
+        assert np.abs(w - wo).max() <= bar * np.abs(wo).max()
+
+    same()
+    for box in ((20.2, 24.24, 31.31), (20.0, 24.0, 36.0), (28.0, 20.0, 20.0), (20.0, 24.0, 31.0)):
+        s.cell = UnitCell.ortho(*box)
+        s.cell_changed()
+        same()
+    for kmax in (8, 17, 9):
+        s.set_coulomb_potential(Ewald(8.0, kmax))
+        same()
+    s.set_tuning(rho_width=64)
+    same()
+    s.set_precision(LG_PRECISION_MIXED)
+    s.cell = UnitCell.ortho(20.2, 24.24, 31.31)
+    s.cell_changed()
+    same(1e-4)
