@@ -413,9 +413,10 @@ struct lg_system {
     int oct_nrt = 0, oct_nst = 0, oct_steps = 0, oct_zcols = 0, oct_nitems = 0, oct_ntiles = 0;
     int oct_width = 0, oct_nchunks = 0, oct_ngroups = 0, oct_ipg = 0, oct_asplit = 1;
     int rho_nchunks = 0;  // partial sums of the last rho pass
-    DevBuf<int> opairs, osteps, okmap, omask;
-    DevBuf<OctItem> oitems;
-    DevBuf<int4> oslots, orows32, orows64;
+    DevBuf<unsigned char> otab;  // the tables, one upload
+    const int *opairs = nullptr, *osteps = nullptr, *okmap = nullptr, *omask = nullptr;
+    const OctItem* oitems = nullptr;
+    const int4 *oslots = nullptr, *orows32 = nullptr, *orows64 = nullptr;
     DevBuf<float> ocoef32;
     DevBuf<double> ocoef64;
     DevBuf<double4> opart;
@@ -794,12 +795,16 @@ int prepare_meta(lg_system* s) {
 // in t in [-1, 1] per piece, `stride` coefficients apart: the piece's
 // Chebyshev interpolant (deg + 1 Chebyshev nodes, long double), expanded in
 // powers of t.  Returns the largest relative error against f (long double)
-// over 64 points per piece.
+// over `checks` points per piece.
 // Used for erfcx(x) = exp(x^2) erfc(x) and for the real-space force factor
 // of the mixed pair kernel (hforce_ld).
 static long double erfcx_ld(long double x) { return erfcl(x) * expl(x * x); }
 template <typename T, typename F>
-static double fit_pieces(long double h, int M, int deg, int stride, F fn, std::vector<T>& out) {
+static double fit_pieces(long double h, int M, int deg, int stride, F fn, std::vector<T>& out,
+                         std::vector<long double>* refs, int checks) {
+    // f at the points of every piece, formed once for fits that share them
+    const bool have = refs && !refs->empty();
+    if (refs && !have) refs->resize(size_t(M) * checks);
     const int D = deg;
     const long double pi = 3.141592653589793238462643383279502884L;
     out.assign(size_t(M) * stride, T(0));
@@ -833,11 +838,12 @@ static double fit_pieces(long double h, int M, int deg, int stride, F fn, std::v
             tcur = tnext;
         }
         for (int q = 0; q <= D; q++) out[size_t(k) * stride + q] = T(mono[q]);
-        for (int z = 0; z < 64; z++) {
-            const long double t = -1.0L + 2.0L * (z + 0.5L) / 64.0L;
+        for (int z = 0; z < checks; z++) {
+            const long double t = -1.0L + 2.0L * (z + 0.5L) / checks;
             long double p = (long double)out[size_t(k) * stride + D];
             for (int q = D - 1; q >= 0; q--) p = p * t + (long double)out[size_t(k) * stride + q];
-            const long double ref = fn(mid + half * t);
+            const long double ref = have ? (*refs)[size_t(k) * checks + z] : fn(mid + half * t);
+            if (refs && !have) (*refs)[size_t(k) * checks + z] = ref;
             worst = std::max(worst, double(fabsl(p - ref) / ref));
         }
     }
@@ -849,7 +855,7 @@ static double fit_pieces(long double h, int M, int deg, int stride, F fn, std::v
 // so a cached table is the table the fit would return.
 template <typename T, typename F>
 static double fit_cached(int fn_id, double param, double range, long double h, int pieces, int deg, int stride, F fn,
-                         std::vector<T>& out) {
+                         std::vector<T>& out, std::vector<long double>* refs = nullptr, int checks = 64) {
     using Key = std::tuple<int, uint64_t, uint64_t, int>;
     static std::mutex mu;
     static std::map<Key, std::pair<std::vector<T>, double>> cache;
@@ -865,19 +871,20 @@ static double fit_cached(int fn_id, double param, double range, long double h, i
             return it->second.second;
         }
     }
-    const double err = fit_pieces(h, pieces, deg, stride, fn, out);
+    const double err = fit_pieces(h, pieces, deg, stride, fn, out, refs, checks);
     std::lock_guard<std::mutex> lk(mu);
     cache.emplace(key, std::make_pair(out, err));
     return err;
 }
 // kErfcxPieces pieces over [0, xmax] (erfcx_tab).
 template <typename T, typename F>
-static double fit_range(int fn_id, double param, double xmax, int deg, F fn, std::vector<T>& out) {
-    return fit_cached(fn_id, param, xmax, (long double)xmax / kErfcxPieces, kErfcxPieces, deg, deg + 1, fn, out);
+static double fit_range(int fn_id, double param, double xmax, int deg, F fn, std::vector<T>& out,
+                        std::vector<long double>* refs = nullptr) {
+    return fit_cached(fn_id, param, xmax, (long double)xmax / kErfcxPieces, kErfcxPieces, deg, deg + 1, fn, out, refs);
 }
 template <typename T>
-static double fit_erfcx(double xmax, int deg, std::vector<T>& out) {
-    return fit_range(0, 0.0, xmax, deg, erfcx_ld, out);
+static double fit_erfcx(double xmax, int deg, std::vector<T>& out, std::vector<long double>* refs) {
+    return fit_range(0, 0.0, xmax, deg, erfcx_ld, out, refs);
 }
 
 
@@ -963,8 +970,9 @@ int prepare_params(lg_system* s) {
         const double xmax = c.alpha * c.rc * (1.0 + 1e-9);
         std::vector<double> t64;
         std::vector<float> t32;
-        const double e64 = fit_erfcx(xmax, kErfcxDeg64, t64);
-        const double e32 = fit_erfcx(xmax, kErfcxDeg32, t32);
+        std::vector<long double> refs;
+        const double e64 = fit_erfcx(xmax, kErfcxDeg64, t64, &refs);
+        const double e32 = fit_erfcx(xmax, kErfcxDeg32, t32, &refs);
         if (xmax < 27.0 && e64 < 1e-14 && e32 < 1e-7) {
             LG_TRY(upload(s->ecx64, t64, S(s)));
             LG_TRY(upload(s->ecx32, t32, S(s)));
@@ -991,7 +999,7 @@ int prepare_params(lg_system* s) {
         if (s->ecx_ok && std::isfinite(inv_h) && inv_h > 1e-30f) {
             std::vector<double> th64;
             const double eh64 = fit_cached(2, c.alpha, double(inv_h), 1.0L / inv_h, kHfPieces, kHfDeg, kHfStride,
-                                           hforce_ld, th64);
+                                           hforce_ld, th64, nullptr, 24);
             if (eh64 < 2e-15) {
                 LG_TRY(upload(s->hf64, th64, S(s)));
                 s->hf64_inv_h = inv_h;
@@ -1154,18 +1162,30 @@ static int octant_tables(lg_system* s, const std::vector<int4>& idx) {
     s->oct_nitems = int(items.size());
     s->oct_ntiles = int(slots.size());
     hipStream_t st = S(s);
-    LG_TRY(upload(s->opairs, opairs, st));
-    LG_TRY(upload(s->osteps, steps, st));
-    LG_TRY(upload(s->okmap, kmap, st));
-    LG_TRY(upload(s->oitems, items, st));
-    LG_TRY(upload(s->oslots, slots, st));
-    LG_TRY(upload(s->omask, mask, st));
-    LG_TRY(upload(s->orows32, rows32, st));
-    LG_TRY(upload(s->orows64, rows64, st));
-    const std::vector<double> zero(size_t(nrt) * s->oct_nst * 64, 0.0);
-    LG_TRY(upload(s->ocoef64, zero, st));
-    LG_TRY(upload(s->ocoef32, std::vector<float>(zero.size(), 0.f), st));
-    LG_HIP(hipStreamSynchronize(st));  // the tables above are local
+    std::vector<unsigned char> tab;
+    std::vector<std::pair<size_t, const void**>> places;
+    auto put = [&](const auto& v, auto& where) {
+        tab.resize((tab.size() + 255) / 256 * 256);
+        places.push_back({tab.size(), reinterpret_cast<const void**>(&where)});
+        const auto* b = reinterpret_cast<const unsigned char*>(v.data());
+        tab.insert(tab.end(), b, b + v.size() * sizeof(v[0]));
+    };
+    put(opairs, s->opairs);
+    put(steps, s->osteps);
+    put(kmap, s->okmap);
+    put(items, s->oitems);
+    put(slots, s->oslots);
+    put(mask, s->omask);
+    put(rows32, s->orows32);
+    put(rows64, s->orows64);
+    LG_TRY(upload(s->otab, tab, st));
+    for (auto& [at, where] : places) *where = s->otab.p + at;
+    const size_t ncoef = size_t(nrt) * s->oct_nst * 64;
+    LG_TRY(s->ocoef64.ensure(ncoef));
+    LG_TRY(s->ocoef32.ensure(ncoef));
+    LG_HIP(hipMemsetAsync(s->ocoef64.p, 0, ncoef * sizeof(double), st));
+    LG_HIP(hipMemsetAsync(s->ocoef32.p, 0, ncoef * sizeof(float), st));
+    LG_HIP(hipStreamSynchronize(st));  // the table above is local
     return LG_OK;
 }
 
@@ -1545,9 +1565,9 @@ static OctRho oct_rho_args(const lg_system* s, bool mixed) {
     for (int d = 0; d < 3; d++) a.inv[d] = s->box.inv[d];
     a.kmax = s->coul_kmax;
     a.zcols = s->oct_zcols;
-    a.items = s->oitems.p;
-    a.rows = mixed ? s->orows32.p : s->orows64.p;
-    a.mask = s->omask.p;
+    a.items = s->oitems;
+    a.rows = mixed ? s->orows32 : s->orows64;
+    a.mask = s->omask;
     a.nitems = s->oct_nitems;
     a.ngroups = s->oct_ngroups;
     a.ipg = s->oct_ipg;
@@ -1611,8 +1631,8 @@ static void launch_oct_step(lg_system* s, int what, int then, double* ke_part, c
     OctForce a{};
     for (int d = 0; d < 3; d++) a.kg[d] = s->kg[d];
     a.coef = mixed ? static_cast<const void*>(s->ocoef32.p) : static_cast<const void*>(s->ocoef64.p);
-    a.pairs = s->opairs.p;
-    a.steps = s->osteps.p;
+    a.pairs = s->opairs;
+    a.steps = s->osteps;
     a.nrt = s->oct_nrt;
     a.nst = s->oct_nst;
     OctRho ra = oct_rho_args(s, mixed);
@@ -1854,8 +1874,8 @@ int launch_forces(lg_system* s, bool energy, bool combine = true, bool frac_done
         rr.partial = s->opart.p;
         rr.nchunks = nchunks;
         rr.nslots = 4 * s->oct_nitems;
-        rr.slots = s->oslots.p;
-        rr.kmap = s->okmap.p;
+        rr.slots = s->oslots;
+        rr.kmap = s->okmap;
         rr.nk = s->nk;
         rr.nst = s->oct_nst;
         rr.rho = s->rho.p;
@@ -2393,13 +2413,10 @@ int lg_system_destroy(lg_system* s) {
     DevBuf<int>* ibufs[] = {&s->cellid, &s->slot, &s->count, &s->start, &s->tmp, &s->sorted, &s->nbr, &s->nnbr,
 
                             &s->flags, &s->pair_restr, &s->slot_start, &s->d_mol_start,
-                            &s->mc_cell_count, &s->mc_atom_cell, &s->kslot, &s->opairs, &s->osteps, &s->okmap, &s->omask};
+                            &s->mc_cell_count, &s->mc_atom_cell, &s->kslot};
     for (auto* b : ibufs) b->release();
     s->units.release();
-    s->oitems.release();
-    s->oslots.release();
-    s->orows32.release();
-    s->orows64.release();
+    s->otab.release();
     s->ocoef32.release();
     s->ocoef64.release();
     s->opart.release();
