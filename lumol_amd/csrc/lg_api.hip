@@ -2137,9 +2137,10 @@ int pull_packed(lg_system* s, const double* src, size_t rows, int width, int pit
         const size_t cap = std::min(2 * need, 2 * kStageDoubles);
         if (hipHostMalloc(reinterpret_cast<void**>(&ctx->stage), cap * sizeof(double), hipHostMallocDefault) == hipSuccess)
             ctx->stage_cap = cap;
-        else
+        else {
             ctx->stage = nullptr;
-        (void)hipGetLastError();
+            (void)hipGetLastError();  // its own; an error from before is not cleared
+        }
     }
     if (!ctx->stage) {
         std::vector<double> h(rows * size_t(pitch));
