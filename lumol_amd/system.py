@@ -471,8 +471,8 @@ class System:
         lanes per atom, 2 one workgroup per cell over the cell list, 3 direct
         (workgroups per cell over the atoms' cell tags, up to 32768 atoms);
         md_graph: 1 eager launches (default), 2 HIP-graph replay of MD chunks;
-        rho_kind: 1, 2 or 3, one and the same octant form on the matrix cores
-        now (kept for saved choices)."""
+        rho_kind: 1, 2 or 3, one and the same form now (kept for saved
+        choices); kspace_split has no effect on its octants."""
         self.tuning_ = (int(pair_lanes), int(kspace_split), int(rho_width), int(nlist_build), int(md_graph),
                         int(rho_kind))
         if self._handle is not None and not self._dirty:
